@@ -49,7 +49,8 @@ typedef struct lh_mpnn lh_mpnn;  /* learned preconditioner (weights on device) *
 typedef struct lh_stats {
     int32_t iterations;      /* outer iterations                              */
     int32_t converged;       /* number of converged wanted pairs / rhs        */
-    int32_t fallback_used;   /* 1 if the learned preconditioner was replaced  */
+    int32_t fallback_used;   /* 1 if the learned preconditioner or the linear
+                                solver's multigrid cycle was replaced         */
     int32_t precision_mode;  /* LH_PREC_*                                     */
     double  max_resid;       /* largest final relative residual               */
     double  t_setup_us;      /* host-measured phase times (microseconds)      */
@@ -297,11 +298,14 @@ typedef struct lh_pcg_opts {
     int32_t poly_degree;   /* LH_PRECOND_JACOBI: degree of the Chebyshev-Jacobi
                               polynomial z = p(D^-1 K) D^-1 r (symmetric
                               positive definite, on [bmax / (2 deg^2), bmax],
-                              bmax the Gershgorin bound of D^-1 K); 0 or 1:
-                              plain Jacobi (the default: on one right-hand
-                              side each Chebyshev step costs ~0.4 of a
-                              Jacobi-CG iteration, so fewer iterations save
-                              little time); at most 256                      */
+                              bmax the Gershgorin bound of D^-1 K); at most
+                              256.  1: plain Jacobi.  0 (the default): a
+                              smoothed-aggregation multigrid cycle where
+                              Jacobi-CG is expected to take more than ~350
+                              iterations (about 4,200 rows of a surface's
+                              stiffness, 14,400 of a volume's), plain Jacobi
+                              elsewhere, where the cycle finds no hierarchy,
+                              and from iteration 200 on (fallback_used = 1)  */
     int32_t reserved;
 } lh_pcg_opts;
 int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta,

@@ -671,7 +671,8 @@ class EigHandle:
 def pcg(ctx: Context, A: DeviceCSR, B, alpha: float, beta: float, b, x0=None, dmask=None, rtol=1e-12,
         max_iter=0, precond=LH_PRECOND_JACOBI, verbose=0, no_fallback=False, poly_degree=0):
     """Solve (alpha*B + beta*A) x = b (b: (n,) or (n, nrhs)); returns (x, stats).
-    poly_degree (Jacobi): Chebyshev-Jacobi polynomial degree (0 or 1: plain Jacobi)."""
+    poly_degree (Jacobi): Chebyshev-Jacobi polynomial degree (1: plain Jacobi,
+    0: a multigrid cycle on large ill-conditioned systems, else plain Jacobi)."""
     b = np.asarray(b, dtype=np.float64)
     squeeze = b.ndim == 1
     b2 = b[:, None] if squeeze else b

@@ -41,6 +41,7 @@ SOURCES = {
     "lh_poly.hip": [],
     "lh_reorder.hip": [],
     "lh_eigs.hip": [],
+    "lh_amg.hip": [],
     "lh_pcg.hip": [],
     "lh_mpnn.hip": [],
     "lh_rrlib.hip": [],

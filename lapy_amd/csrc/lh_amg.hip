@@ -1,0 +1,1051 @@
+// Smoothed-aggregation multigrid for the linear solves' operator K
+// (symmetric, sparse, Laplacian-like: stiffness, Dirichlet-masked stiffness,
+// mass + t stiffness).
+//
+// Setup (once per solve, all on the device, deterministic), level by level:
+//  * lambda_max of D^-1 K from ten power steps;
+//  * aggregates around the roots of a maximal independent set of distance 2
+//    in the graph of strong connections (k_ij^2 > theta^2 k_ii k_jj), found
+//    with hashed keys in a fixed number of rounds; the roots are numbered in
+//    row order, so the coarse rows keep the fine rows' locality;
+//  * P = (I - w D^-1 K) P_0, P_0 the aggregates' indicator, w = 4 / (3
+//    lambda_max): the smoothing that makes the interpolated coarse functions
+//    continuous, without which the cycle's quality decays with every level;
+//  * K_c = P^T (K P): two sparse products, one wave per output row, the
+//    row's entries gathered in a hash table in LDS whose values are summed
+//    in the order of the first factor's entries (so the result does not
+//    depend on scheduling).
+//
+// Cycle: V(1,1) with the Chebyshev polynomial of degree 2 on [bmax / 6, bmax]
+// as the smoother before and after, hence a symmetric positive definite
+// preconditioner, as conjugate gradients need.  A level is six launches; all
+// levels of at most kTailRows rows run in one workgroup per column with
+// their vectors in LDS (one launch instead of six a level, which at these
+// sizes are nothing but launch latency), and the last level (at most 128
+// rows) multiplies with its inverse.
+//
+// The coarsest matrix of a pure Neumann operator is singular (constants):
+// its unit diagonal is raised by 1e-9, which leaves the other components
+// unchanged to that accuracy and bounds the constant one, which the
+// right-hand sides of such systems do not have.
+#include "lh_amg.hpp"
+
+#include <cmath>
+
+namespace lh {
+
+namespace {
+
+constexpr double kTheta = 0.05;      // strength threshold of the finest level, halved on each coarser one
+constexpr int kPowerSteps = 10;
+constexpr int kMisRounds = 8;
+constexpr int kMaxLevels = 12;
+constexpr int kCoarsest = 128;       // rows of the inverted level at most (kCholMax)
+constexpr int kTailRows = 2048;      // rows of a one-workgroup level at most
+constexpr int kTailNnz = 24576;      // and its entries: one CU reads them from L2 for every product
+constexpr int kTailSum = 2560;       // rows of all of them together at most
+constexpr int kLongRow = 20;         // mean row length from which a wave forms a row of P
+constexpr double kSmoothRatio = 6.0; // the smoother's interval is [bmax / ratio, bmax]
+
+static_assert(kCoarsest <= kCholMax, "the coarsest level is factorised by cholinv");
+
+// coefficients of the degree-2 Chebyshev smoother on [bmax / ratio, bmax]:
+// y = x + s D^-1 (b - K x), x' = y + c1 (y - x) + c2 D^-1 (b - K y)
+struct Cheb2 {
+    double s, c1, c2;
+};
+__host__ __device__ inline Cheb2 cheb2(double bmax) {
+    const double amin = bmax / kSmoothRatio;
+    const double th = 0.5 * (bmax + amin), de = 0.5 * (bmax - amin), sig = th / de;
+    const double rho0 = 1.0 / sig, rho1 = 1.0 / (2.0 * sig - rho0);
+    return Cheb2{1.0 / th, rho1 * rho0, 2.0 * rho1 / de};
+}
+
+__device__ __forceinline__ uint32_t mix32(uint32_t x) {
+    x ^= x >> 16;
+    x *= 0x7feb352du;
+    x ^= x >> 15;
+    x *= 0x846ca68bu;
+    x ^= x >> 16;
+    return x;
+}
+
+// ---- setup ------------------------------------------------------------------
+// dinv; bad[0] set when a row's diagonal is negative, missing or zero beside
+// non-zero entries; start vector of the power iteration (0 on zero rows)
+__global__ void k_amg_diag(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                           const double* __restrict__ kv, double* __restrict__ dinv, double* __restrict__ x,
+                           int* __restrict__ bad) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double d = 0.0, other = 0.0;
+    for (int32_t s = rp[i]; s < rp[i + 1]; ++s) {
+        if (cl[s] == (int32_t)i) d = kv[s];
+        else other = fmax(other, fabs(kv[s]));
+    }
+    if (!(d >= 0.0) || (d == 0.0 && other != 0.0)) bad[0] = 1;  // every writer stores the same value
+    const bool pos = d > 0.0;
+    dinv[i] = pos ? 1.0 / d : 0.0;
+    x[i] = pos ? (double)(mix32((uint32_t)i * 2654435761u + 12345u) >> 8) * (1.0 / 8388608.0) - 1.0 : 0.0;
+}
+// y = D^-1 K x, one thread per row
+__global__ void k_amg_power(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                            const double* __restrict__ kv, const double* __restrict__ dinv,
+                            const double* __restrict__ x, double* __restrict__ y) {
+    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double a = 0.0;
+    for (int32_t s = rp[i]; s < rp[i + 1]; ++s) a += kv[s] * x[cl[s]];
+    y[i] = dinv[i] * a;
+}
+// block partials of x^T D x and x^T D y (y = D^-1 K x): 2 doubles a block
+__global__ void __launch_bounds__(256)
+k_amg_rayleigh(int64_t n, const double* __restrict__ dinv, const double* __restrict__ x, const double* __restrict__ y,
+               double* __restrict__ part) {
+    __shared__ double sh[2][4];
+    double a = 0.0, b = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        if (dinv[i] > 0.0) {
+            const double d = 1.0 / dinv[i];
+            a += x[i] * d * x[i];
+            b += x[i] * d * y[i];
+        }
+    }
+    a = wave_sum64(a);
+    b = wave_sum64(b);
+    if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = a;
+        sh[1][threadIdx.x >> 6] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) part[2 * blockIdx.x + threadIdx.x] = (sh[threadIdx.x][0] + sh[threadIdx.x][1]) + (sh[threadIdx.x][2] + sh[threadIdx.x][3]);
+}
+
+// independent set: key = state (0 out, 1 undecided, 2 in) << 62 | hash | row
+constexpr unsigned long long kOut = 0ull, kUndecided = 1ull << 62, kIn = 2ull << 62;
+
+__global__ void k_mis_init(int64_t n, const double* __restrict__ dinv, unsigned long long* __restrict__ t) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    // zero rows (Dirichlet) take no part
+    t[i] = dinv[i] > 0.0
+               ? kUndecided | ((unsigned long long)(mix32((uint32_t)i + 0x9e3779b9u) >> 2) << 32) | (unsigned)i
+               : kOut;
+}
+__device__ __forceinline__ bool strong(double k, double di, double dj, double th2) { return k * k * di * dj > th2; }
+
+// largest key among the row and its strong neighbours
+__device__ __forceinline__ unsigned long long mis_max(int64_t i, const int32_t* __restrict__ rp,
+                                                      const int32_t* __restrict__ cl, const double* __restrict__ kv,
+                                                      const double* __restrict__ dinv, double th2,
+                                                      const unsigned long long* __restrict__ t) {
+    unsigned long long best = t[i];
+    const double di = dinv[i];
+    for (int32_t s = rp[i]; s < rp[i + 1]; ++s) {
+        const int32_t j = cl[s];
+        if (strong(kv[s], di, dinv[j], th2)) {
+            const unsigned long long q = t[j];
+            best = q > best ? q : best;
+        }
+    }
+    return best;
+}
+__global__ void k_mis_spread(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                             const double* __restrict__ kv, const double* __restrict__ dinv, double th2,
+                             const unsigned long long* __restrict__ t, unsigned long long* __restrict__ a) {
+    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = mis_max(i, rp, cl, kv, dinv, th2, t);
+}
+// second spreading step and the decision: a row whose key is the largest
+// within distance 2 joins, one with a member within distance 2 leaves
+__global__ void k_mis_decide(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                             const double* __restrict__ kv, const double* __restrict__ dinv, double th2,
+                             const unsigned long long* __restrict__ a, unsigned long long* __restrict__ t) {
+    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const unsigned long long own = t[i];
+    if ((own >> 62) != 1) return;
+    const unsigned long long best = mis_max(i, rp, cl, kv, dinv, th2, a);
+    if (best == own) t[i] = kIn | (own & ~(3ull << 62));
+    else if ((best >> 62) == 2) t[i] = kOut;
+}
+__global__ void k_mis_flag(int64_t n, const unsigned long long* __restrict__ t, int32_t* __restrict__ flag) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) flag[i] = (t[i] >> 62) == 2 ? 1 : 0;
+}
+__global__ void k_agg_roots(int64_t n, const int32_t* __restrict__ flag, const int32_t* __restrict__ id,
+                            int32_t* __restrict__ agg) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) agg[i] = flag[i] ? id[i] : -1;
+}
+// an unassigned row joins the aggregate of its strongest assigned neighbour
+// (the first of equals); in: the assignment before this pass
+__global__ void k_agg_join(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                           const double* __restrict__ kv, const double* __restrict__ dinv, double th2,
+                           const int32_t* __restrict__ in, int32_t* __restrict__ out) {
+    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    int32_t g = in[i];
+    const double di = dinv[i];
+    if (g < 0 && di > 0.0) {
+        double best = 0.0;
+        for (int32_t s = rp[i]; s < rp[i + 1]; ++s) {
+            const int32_t j = cl[s];
+            const double w = fabs(kv[s]);
+            if (in[j] >= 0 && w > best && strong(w, di, dinv[j], th2)) {
+                best = w;
+                g = in[j];
+            }
+        }
+    }
+    out[i] = g;
+}
+
+// P = (I - w D^-1 K) P_0 row by row: first the number of distinct aggregates
+// among a row's columns, then the entries in the order of first appearance.
+// One thread per row for short rows; for long ones (below) the quadratic
+// search is spread over a wave.
+template <bool FILL>
+__global__ void k_prolongator(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                              const double* __restrict__ kv, const double* __restrict__ dinv, double w,
+                              const int32_t* __restrict__ agg, const int32_t* __restrict__ pp,
+                              int32_t* __restrict__ count_or_cols, double* __restrict__ pv) {
+    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int32_t r0 = rp[i], r1 = rp[i + 1];
+    const double wd = w * dinv[i];
+    const int32_t own = agg[i];
+    int32_t at = FILL ? pp[i] : 0;
+    if (wd > 0.0) {
+        for (int32_t s = r0; s < r1; ++s) {
+            const int32_t g = agg[cl[s]];
+            if (g < 0) continue;
+            bool seen = false;
+            for (int32_t q = r0; q < s && !seen; ++q) seen = agg[cl[q]] == g;
+            if (seen) continue;
+            if (FILL) {
+                double v = 0.0;
+                for (int32_t q = s; q < r1; ++q)
+                    if (agg[cl[q]] == g) v += kv[q];
+                count_or_cols[at] = g;
+                pv[at] = (g == own ? 1.0 : 0.0) - wd * v;
+            }
+            ++at;
+        }
+    }
+    if (!FILL) count_or_cols[i] = at;
+}
+// one wave per row: each lane holds one entry of a chunk of 64 and meets all
+// entries of the row in order (lane reads), summing those of its aggregate;
+// the first lane of an aggregate writes.  Sums and order as above.
+template <bool FILL>
+__global__ void __launch_bounds__(256)
+k_prolongator_wave(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                   const double* __restrict__ kv, const double* __restrict__ dinv, double w,
+                   const int32_t* __restrict__ agg, const int32_t* __restrict__ pp, int32_t* __restrict__ count_or_cols,
+                   double* __restrict__ pv) {
+    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (i >= n) return;  // whole wave
+    const int lane = threadIdx.x & 63;
+    const int32_t r0 = rp[i], r1 = rp[i + 1];
+    const double wd = w * dinv[i];
+    const int32_t own = agg[i];
+    int32_t at = FILL ? pp[i] : 0;
+    if (wd > 0.0) {
+        for (int32_t a = r0; a < r1; a += 64) {
+            const int32_t g = (a + lane < r1) ? agg[cl[a + lane]] : -1;
+            bool seen = g < 0;
+            double v = 0.0;
+            for (int32_t b = r0; b < r1; b += 64) {
+                const bool in = b + lane < r1;
+                const int32_t gq = in ? agg[cl[b + lane]] : -1;
+                const double kq = in ? kv[b + lane] : 0.0;
+                const int cnt = r1 - b < 64 ? r1 - b : 64;
+                for (int o = 0; o < cnt; ++o) {
+                    const int32_t go = __builtin_amdgcn_readlane(gq, o);
+                    const double ko = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(kq), o),
+                                                       __builtin_amdgcn_readlane(__double2loint(kq), o));
+                    if (go == g) {
+                        v += ko;
+                        seen = seen || b + o < a + lane;
+                    }
+                }
+            }
+            const unsigned long long first = __ballot(!seen);
+            if (FILL && !seen) {
+                const int32_t q = at + __popcll(first & ((1ull << lane) - 1));
+                count_or_cols[q] = g;
+                pv[q] = (g == own ? 1.0 : 0.0) - wd * v;
+            }
+            at += __popcll(first);
+        }
+    }
+    if (!FILL && lane == 0) count_or_cols[i] = at;
+}
+
+// transpose of P: entries per coarse row, then each entry to a free place of
+// its row (in any order), then each row sorted by the fine row
+__global__ void k_count_cols(int64_t nnz, const int32_t* __restrict__ pc, int32_t* __restrict__ cnt) {
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < nnz) atomicAdd(cnt + pc[s], 1);
+}
+__global__ void k_scatter_cols(int64_t n, const int32_t* __restrict__ pp, const int32_t* __restrict__ pc,
+                               const double* __restrict__ pv, const int32_t* __restrict__ tp, int32_t* __restrict__ fill,
+                               int32_t* __restrict__ tc, double* __restrict__ tv) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    for (int32_t s = pp[i]; s < pp[i + 1]; ++s) {
+        const int32_t g = pc[s];
+        const int32_t q = tp[g] + atomicAdd(fill + g, 1);
+        tc[q] = (int32_t)i;
+        tv[q] = pv[s];
+    }
+}
+// one wave per row: an entry's place is the number of smaller ones (a row's
+// entries are distinct)
+__global__ void __launch_bounds__(256)
+k_sort_rows(int64_t nc, const int32_t* __restrict__ tp, const int32_t* __restrict__ ti, const double* __restrict__ vi,
+            int32_t* __restrict__ to, double* __restrict__ vo) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= nc) return;
+    const int32_t a = tp[r], b = tp[r + 1];
+    for (int32_t e = a + (int32_t)(threadIdx.x & 63); e < b; e += 64) {
+        const int32_t key = ti[e];
+        int32_t rank = 0;
+        for (int32_t q = a; q < b; ++q) rank += ti[q] < key;
+        to[a + rank] = key;
+        vo[a + rank] = vi[e];
+    }
+}
+
+// ---- C = X Y, one wave per row of X --------------------------------------------
+// The row's distinct columns live in a hash table of HS slots in LDS (linear
+// probing).  Counting: lanes insert the rows of Y in any order.  Filling:
+// the rows of Y are added one after another, the lanes of a step holding
+// distinct columns, so a value's terms are summed in the order of X's
+// entries; an entry's place in the output row is the number of smaller
+// columns.  A row with more than 3/4 HS distinct columns sets over[0].
+// Bound by the latency of its dependent LDS steps (one per entry of X's row).
+template <int HS>
+__device__ __forceinline__ int hash_slot(volatile int32_t* keys, int32_t key) {
+    int h = (int)(mix32((uint32_t)key) & (HS - 1));
+    for (int tries = 0; tries < HS; ++tries) {
+        const int32_t q = keys[h];
+        if (q == key) return h;
+        if (q < 0) {
+            const int32_t was = atomicCAS(const_cast<int32_t*>(keys) + h, -1, key);
+            if (was < 0 || was == key) return h;
+        }
+        h = (h + 1) & (HS - 1);
+    }
+    return -1;
+}
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int HS, bool FILL>
+__global__ void __launch_bounds__(256)
+k_spgemm(int64_t n, const int32_t* __restrict__ xp, const int32_t* __restrict__ xc, const double* __restrict__ xv,
+         const int32_t* __restrict__ yp, const int32_t* __restrict__ yc, const double* __restrict__ yv,
+         const int32_t* __restrict__ cp, int32_t* __restrict__ count_or_cols, double* __restrict__ cv,
+         int* __restrict__ over) {
+    __shared__ int32_t s_keys[4][HS];
+    __shared__ double s_vals[FILL ? 4 : 1][FILL ? HS : 1];
+    __shared__ int32_t s_list[FILL ? 4 : 1][FILL ? HS : 1], s_slot[FILL ? 4 : 1][FILL ? HS : 1];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + wv;
+    if (row >= n) return;  // no workgroup barrier follows
+    volatile int32_t* keys = s_keys[wv];
+    volatile double* vals = s_vals[FILL ? wv : 0];
+    for (int h = lane; h < HS; h += 64) {
+        keys[h] = -1;
+        if (FILL) vals[h] = 0.0;
+    }
+    wave_fence();
+    const int32_t a = xp[row], b = xp[row + 1];
+    if (!FILL) {
+        int mine = 0;
+        // lanes over X's entries; more than HS distinct columns: hash_slot gives up
+        for (int32_t e = a + lane; e < b; e += 64) {
+            const int32_t j = xc[e];
+            for (int32_t q = yp[j]; q < yp[j + 1]; ++q)
+                if (hash_slot<HS>(keys, yc[q]) < 0) mine = 1;
+        }
+        wave_fence();
+        int cnt = 0;
+        for (int h = lane; h < HS; h += 64) cnt += keys[h] >= 0;
+        for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
+        if (__any(mine) || cnt > HS * 3 / 4) {
+            if (lane == 0) over[0] = 1;
+        }
+        if (lane == 0) count_or_cols[row] = cnt;
+        return;
+    }
+    for (int32_t e = a; e < b; ++e) {
+        const int32_t j = xc[e];
+        const double x = xv[e];
+        for (int32_t q = yp[j] + lane; q < yp[j + 1]; q += 64) {
+            const int h = hash_slot<HS>(keys, yc[q]);
+            if (h >= 0) vals[h] = vals[h] + x * yv[q];
+        }
+        wave_fence();
+    }
+    // the table's columns packed into a list, then ranked against it
+    const int32_t base = cp[row], cnt = cp[row + 1] - base;
+    volatile int32_t* list = s_list[FILL ? wv : 0];
+    volatile int32_t* slot = s_slot[FILL ? wv : 0];
+    int c = 0;
+    for (int h0 = 0; h0 < HS; h0 += 64) {
+        const int32_t key = keys[h0 + lane];
+        const unsigned long long bal = __ballot(key >= 0);
+        const int at = c + __popcll(bal & ((1ull << lane) - 1));
+        if (key >= 0) {
+            list[at] = key;
+            slot[at] = h0 + lane;
+        }
+        c += __popcll(bal);
+    }
+    wave_fence();
+    for (int q = lane; q < c; q += 64) {
+        const int32_t key = list[q];
+        int32_t rank = 0;
+        for (int o = 0; o < c; ++o) rank += list[o] < key;
+        if (rank < cnt) {
+            count_or_cols[base + rank] = key;
+            cv[base + rank] = vals[slot[q]];
+        }
+    }
+}
+
+// dense copy of the coarsest matrix
+__global__ void k_amg_dense(int n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                            const double* __restrict__ kv, double* __restrict__ g) {
+    const int i = blockIdx.x;
+    for (int j = threadIdx.x; j < n; j += blockDim.x) g[i * n + j] = 0.0;
+    __syncthreads();
+    for (int32_t s = rp[i] + (int32_t)threadIdx.x; s < rp[i + 1]; s += blockDim.x) g[i * n + cl[s]] = kv[s];
+}
+// inverse = T T^T from the upper triangular T with T^T G T = I
+__global__ void k_amg_inverse(int n, const double* __restrict__ t, double* __restrict__ g) {
+    const int i = blockIdx.x;
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        double a = 0.0;
+        for (int k = i > j ? i : j; k < n; ++k) a += t[i * n + k] * t[j * n + k];
+        g[i * n + j] = a;
+    }
+}
+
+// ---- cycle --------------------------------------------------------------------
+// Every kernel works on row-major blocks of m columns, rows in XCD-contiguous
+// ranges, G lanes for each row and column.  The finest level's ELL rows take
+// one lane (its slots are loaded, then the gathers go out together; bound by
+// HBM); CSR rows take 1 to 16 by their mean length, a lane every G-th entry
+// and the sums combined in a fixed order: with one lane a row of 12 entries
+// took 4.7 us a launch and one of 70 entries 35 us on levels that fill a
+// fraction of the chip, all of it latency.
+
+// this lane's share of sum over row i of K of kv * f(column); W > 0: ELL rows
+// of W slots (G == 1)
+template <int W, int G, typename F>
+__device__ __forceinline__ double row_part(int64_t i, int lane, const int32_t* __restrict__ rp,
+                                           const int32_t* __restrict__ cl, const double* __restrict__ kv, F&& f) {
+    double a = 0.0;
+    if constexpr (W > 0) {
+#pragma unroll
+        for (int k0 = 0; k0 < W; k0 += 8) {
+            const int4 ca = *reinterpret_cast<const int4*>(cl + i * W + k0);
+            const int4 cb = *reinterpret_cast<const int4*>(cl + i * W + k0 + 4);
+            const double2* vp = reinterpret_cast<const double2*>(kv + i * W + k0);
+            const double2 v0 = vp[0], v1 = vp[1], v2 = vp[2], v3 = vp[3];
+            const double g0 = f(ca.x), g1 = f(ca.y), g2 = f(ca.z), g3 = f(ca.w);
+            const double g4 = f(cb.x), g5 = f(cb.y), g6 = f(cb.z), g7 = f(cb.w);
+            a += v0.x * g0;
+            a += v0.y * g1;
+            a += v1.x * g2;
+            a += v1.y * g3;
+            a += v2.x * g4;
+            a += v2.y * g5;
+            a += v3.x * g6;
+            a += v3.y * g7;
+        }
+    } else {
+        int32_t s = rp[i] + lane;
+        const int32_t r1 = rp[i + 1];
+        for (; s + 3 * G < r1; s += 4 * G) {
+            const double g0 = f(cl[s]), g1 = f(cl[s + G]), g2 = f(cl[s + 2 * G]), g3 = f(cl[s + 3 * G]);
+            a += kv[s] * g0;
+            a += kv[s + G] * g1;
+            a += kv[s + 2 * G] * g2;
+            a += kv[s + 3 * G] * g3;
+        }
+        for (; s < r1; s += G) a += kv[s] * f(cl[s]);
+    }
+    return a;
+}
+// the row's sum, in every one of its G lanes
+template <int W, int G, typename F>
+__device__ __forceinline__ double row_sum(int64_t i, int lane, const int32_t* __restrict__ rp,
+                                          const int32_t* __restrict__ cl, const double* __restrict__ kv, F&& f) {
+    double a = row_part<W, G>(i, lane, rp, cl, kv, f);
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+    return a;
+}
+// row, column and lane of a thread; false beyond the block's end
+template <int G>
+__device__ __forceinline__ bool place(int64_t n, int m, int64_t& i, int& c, int& lane) {
+    const int64_t gid = xcd_block() * 256 + threadIdx.x;
+    const int64_t t = gid / G;
+    lane = (int)(gid % G);
+    i = m == 1 ? t : t / m;
+    c = m == 1 ? 0 : (int)(t - i * m);
+    return i < n;
+}
+
+// the degree-2 smoother from x = 0: with x1 = s D^-1 b,
+// x = (1 + c1) x1 + c2 D^-1 (b - K x1)
+template <int W, int G>
+__global__ void __launch_bounds__(256)
+k_amg_pre(int64_t n, int m, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+          const double* __restrict__ kv, const double* __restrict__ dinv, const double* __restrict__ b,
+          double* __restrict__ x, double s, double c1, double c2, const int* __restrict__ status) {
+    if (status && status[0]) return;
+    int64_t i;
+    int c, lane;
+    if (!place<G>(n, m, i, c, lane)) return;
+    const double di = dinv[i], bi = b[i * m + c];
+    const double a = row_sum<W, G>(i, lane, rp, cl, kv, [&](int32_t j) { return dinv[j] * b[(int64_t)j * m + c]; });
+    if (lane == 0) x[i * m + c] = (1.0 + c1) * s * di * bi + c2 * di * (bi - s * a);
+}
+// MODE 0: out = b - K x; 1: out = x + g D^-1 (b - K x);
+// 2: out = w0 x + w1 out + g D^-1 (b - K x); 3: as 2, and the workgroup's
+// partial sums of b . out per column (m <= 4) into part[block * m + column]
+template <int W, int G, int MODE>
+__global__ void __launch_bounds__(256)
+k_amg_step(int64_t n, int m, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+           const double* __restrict__ kv, const double* __restrict__ dinv, const double* __restrict__ b,
+           const double* __restrict__ x, double* __restrict__ out, double w0, double w1, double g,
+           double* __restrict__ part, const int* __restrict__ status) {
+    if (status && status[0]) return;
+    int64_t i;
+    int c, lane;
+    const bool in = place<G>(n, m, i, c, lane);
+    double dot = 0.0;
+    if (in) {
+        const int64_t o = i * m + c;
+        const double bi = b[o];
+        const double r = bi - row_sum<W, G>(i, lane, rp, cl, kv, [&](int32_t j) { return x[(int64_t)j * m + c]; });
+        if (lane == 0) {
+            double v = r;
+            if (MODE >= 1) v = (MODE == 1 ? x[o] : w0 * x[o] + w1 * out[o]) + g * dinv[i] * r;
+            out[o] = v;
+            dot = bi * v;
+        }
+    }
+    if constexpr (MODE == 3) {
+        __shared__ double sh[4][4];
+        for (int q = 0; q < m; ++q) {
+            const double t = wave_sum64(in && c == q ? dot : 0.0);
+            if ((threadIdx.x & 63) == 0) sh[q][threadIdx.x >> 6] = t;
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < m)
+            part[(int64_t)blockIdx.x * m + threadIdx.x] =
+                (sh[threadIdx.x][0] + sh[threadIdx.x][1]) + (sh[threadIdx.x][2] + sh[threadIdx.x][3]);
+    }
+}
+// out (+)= M in for the transfer operators
+template <bool ADD, int G>
+__global__ void __launch_bounds__(256)
+k_amg_transfer(int64_t n, int m, const int32_t* __restrict__ mp, const int32_t* __restrict__ mc,
+               const double* __restrict__ mv, const double* __restrict__ in, double* __restrict__ out,
+               const int* __restrict__ status) {
+    if (status && status[0]) return;
+    int64_t i;
+    int c, lane;
+    if (!place<G>(n, m, i, c, lane)) return;
+    const double a = row_sum<0, G>(i, lane, mp, mc, mv, [&](int32_t j) { return in[(int64_t)j * m + c]; });
+    if (lane == 0) {
+        if (ADD) out[i * m + c] += a;
+        else out[i * m + c] = a;
+    }
+}
+
+// the tail: every level from `first` on for one column per workgroup, the
+// vectors in LDS.  A level's vectors start at `off` (rows of the tail's
+// levels before it).
+struct TailLevel {
+    int n, off;
+    const int32_t *rp, *cl;
+    const double *kv, *dinv;
+    const int32_t *pp, *pc, *tp, *tc;
+    const double *pv, *tv;
+    double s, c1, c2;
+};
+struct TailDesc {
+    int count;  // levels, the last one with the inverse
+    TailLevel lv[kMaxLevels];
+    const double* ginv;
+};
+constexpr int kTailThreads = 1024;
+
+// put(i, sum over row i of kv * v) for the rows of a CSR matrix, v in LDS,
+// four lanes a row
+template <typename P>
+__device__ __forceinline__ void tail_rows(int n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+                                          const double* __restrict__ kv, const double* v, P&& put) {
+    constexpr int G = 4;
+    for (int t = threadIdx.x; t < n * G; t += kTailThreads) {
+        const int i = t / G, lane = t % G;
+        const double a = row_sum<0, G>(i, lane, rp, cl, kv, [&](int32_t j) { return v[j]; });
+        if (lane == 0) put(i, a);
+    }
+}
+
+__global__ void __launch_bounds__(kTailThreads)
+k_amg_tail(int m, const TailDesc* __restrict__ desc, const double* __restrict__ b, double* __restrict__ x,
+           const int* __restrict__ status) {
+    if (status && status[0]) return;
+    __shared__ double sb[kTailSum], sx[kTailSum], sy[kTailSum];
+    __shared__ double red[kTailThreads];
+    const int tid = threadIdx.x, col = blockIdx.x;
+    const int count = desc->count;
+    {
+        const int n = desc->lv[0].n;
+        for (int i = tid; i < n; i += kTailThreads) sb[i] = b[(int64_t)i * m + col];
+    }
+    __syncthreads();
+    // down: smooth from zero, restrict the residual
+    for (int l = 0; l + 1 < count; ++l) {
+        const TailLevel& lv = desc->lv[l];
+        const double* bl = sb + lv.off;
+        double* xl = sx + lv.off;
+        double* yl = sy + lv.off;
+        for (int i = tid; i < lv.n; i += kTailThreads) yl[i] = lv.s * lv.dinv[i] * bl[i];
+        __syncthreads();
+        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, yl, [&](int i, double a) {
+            xl[i] = (1.0 + lv.c1) * yl[i] + lv.c2 * lv.dinv[i] * (bl[i] - a);
+        });
+        __syncthreads();
+        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, xl, [&](int i, double a) { yl[i] = bl[i] - a; });
+        __syncthreads();
+        const TailLevel& nx = desc->lv[l + 1];
+        tail_rows(nx.n, lv.tp, lv.tc, lv.tv, yl, [&](int i, double a) { sb[nx.off + i] = a; });
+        __syncthreads();
+    }
+    // the last level: x = K^-1 b, 8 threads a row
+    {
+        const TailLevel& lv = desc->lv[count - 1];
+        const int n = lv.n;  // <= 128
+        const int i = tid & 127, part = tid >> 7;
+        double a = 0.0;
+        if (i < n)
+            for (int k = part; k < n; k += kTailThreads / 128) a += desc->ginv[k * n + i] * sb[lv.off + k];
+        red[tid] = a;
+        __syncthreads();
+        if (tid < n) {
+            double t = 0.0;
+#pragma unroll
+            for (int p = 0; p < kTailThreads / 128; ++p) t += red[tid + 128 * p];
+            sx[lv.off + tid] = t;
+        }
+        __syncthreads();
+    }
+    // up: correct, smooth
+    for (int l = count - 2; l >= 0; --l) {
+        const TailLevel& lv = desc->lv[l];
+        const double* bl = sb + lv.off;
+        const double* xc = sx + desc->lv[l + 1].off;
+        double* xl = sx + lv.off;
+        double* yl = sy + lv.off;
+        for (int i = tid; i < lv.n; i += kTailThreads)
+            xl[i] += row_sum<0, 1>(i, 0, lv.pp, lv.pc, lv.pv, [&](int32_t j) { return xc[j]; });
+        __syncthreads();
+        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, xl,
+                  [&](int i, double a) { yl[i] = xl[i] + lv.s * lv.dinv[i] * (bl[i] - a); });
+        __syncthreads();
+        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, yl, [&](int i, double a) {
+            xl[i] = (1.0 + lv.c1) * yl[i] - lv.c1 * xl[i] + lv.c2 * lv.dinv[i] * (bl[i] - a);
+        });
+        __syncthreads();
+    }
+    const int n = desc->lv[0].n;
+    for (int i = tid; i < n; i += kTailThreads) x[(int64_t)i * m + col] = sx[i];
+}
+
+__global__ void k_fill_one(int64_t n, const double* __restrict__ dinv, double* __restrict__ x) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) x[i] = dinv[i] > 0.0 ? 1.0 : 0.0;
+}
+
+constexpr int kRB = 256;  // blocks of the Rayleigh quotient
+
+}  // namespace
+
+double amg_condition(lh_ctx* ctx, int64_t n, const int32_t* rp, const int32_t* cl, const double* kv,
+                     const double* dinv) {
+    DevBuf x(n * 8), y(n * 8), part(2 * kRB * 8);
+    k_fill_one<<<nblocks(n, 256), 256, 0, ctx->stream>>>(n, dinv, x.as<double>());
+    k_amg_power<<<nblocks_xcd(n, 256), 256, 0, ctx->stream>>>(n, rp, cl, kv, dinv, x.as<double>(), y.as<double>());
+    k_amg_rayleigh<<<kRB, 256, 0, ctx->stream>>>(n, dinv, x.as<double>(), y.as<double>(), part.as<double>());
+    LH_CHECK_LAUNCH();
+    double hp[2 * kRB], d = 0.0, k = 0.0;
+    d2h(ctx, hp, part.p, sizeof(hp));
+    for (int q = 0; q < kRB; ++q) {
+        d += hp[2 * q];
+        k += hp[2 * q + 1];
+    }
+    return k > 0.0 ? 2.0 * d / k : 1e30;
+}
+
+template <typename X>
+X* Amg::own(size_t count) {
+    keep.emplace_back(std::max<size_t>(count, 1) * sizeof(X));
+    return keep.back().as<X>();
+}
+
+bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const int32_t* cl0, const double* kv0,
+                int ell_w, const int32_t* ecl, const double* ekv) {
+    ctx = c;
+    levels.clear();
+    keep.clear();
+    hipStream_t st = ctx->stream;
+    DevBuf flags(64);         // [0] bad diagonal, [1] hash table too small
+    memset_d(ctx, flags.p, 0, 64);
+    int* bad = flags.as<int>();
+    int* over = bad + 1;
+    int64_t n = n0, nnz = nnz0;
+    const int32_t *rp = rp0, *cl = cl0;
+    const double* kv = kv0;
+    DevBuf x(n0 * 8), y(n0 * 8), part(2 * kRB * 8), key(n0 * 8), key2(n0 * 8), agg(n0 * 4), agg2(n0 * 4),
+        cnt((n0 + 1) * 4), idx((n0 + 1) * 4);
+    double theta = kTheta;
+    for (int l = 0; l < kMaxLevels; ++l) {
+        levels.emplace_back();
+        AmgLevel& lv = levels.back();
+        lv.n = n;
+        lv.nnz = nnz;
+        lv.rp = rp;
+        lv.cl = cl;
+        lv.d.kv = kv;
+        double* dinv = own<double>(n);
+        lv.d.dinv = dinv;
+        if (l == 0 && ell_w) {
+            lv.W = ell_w;
+            lv.ecl = ecl;
+            lv.d.kv = ekv;
+        }
+        const unsigned nb = nblocks(n, 256), nbx = nblocks_xcd(n, 256);
+        k_amg_diag<<<nb, 256, 0, st>>>(n, rp, cl, kv, dinv, x.as<double>(), bad);
+        LH_CHECK_LAUNCH();
+        if (n <= kCoarsest) {
+            // last level: its inverse
+            DevBuf g((size_t)n * n * 8), t((size_t)n * n * 8), stt(64);
+            ginv.alloc((size_t)n * n * 8);
+            k_amg_dense<<<(unsigned)n, 128, 0, st>>>((int)n, rp, cl, kv, g.as<double>());
+            LH_CHECK_LAUNCH();
+            cholinv(ctx, (int)n, g.as<double>(), t.as<double>(), 1e-9, stt.as<int>());
+            k_amg_inverse<<<(unsigned)n, 128, 0, st>>>((int)n, t.as<double>(), ginv.as<double>());
+            LH_CHECK_LAUNCH();
+            int hs = 0, hb[2] = {0, 0};
+            const Xfer q[2] = {{&hs, stt.p, 4}, {hb, flags.p, 8}};
+            d2h_n(ctx, q, 2);
+            if (hs || hb[0] || hb[1] || l == 0) return false;
+            break;
+        }
+        double *xa = x.as<double>(), *ya = y.as<double>();
+        for (int q = 0; q < kPowerSteps; ++q) {
+            k_amg_power<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, xa, ya);
+            if (q + 1 < kPowerSteps) std::swap(xa, ya);
+        }
+        k_amg_rayleigh<<<kRB, 256, 0, st>>>(n, dinv, xa, ya, part.as<double>());
+        LH_CHECK_LAUNCH();
+        // aggregates
+        const double th2 = theta * theta;
+        theta *= 0.5;
+        auto* ta = key.as<unsigned long long>();
+        auto* tb = key2.as<unsigned long long>();
+        k_mis_init<<<nb, 256, 0, st>>>(n, dinv, ta);
+        for (int r = 0; r < kMisRounds; ++r) {
+            k_mis_spread<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, th2, ta, tb);
+            k_mis_decide<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, th2, tb, ta);
+        }
+        k_mis_flag<<<nb, 256, 0, st>>>(n, ta, cnt.as<int32_t>());
+        LH_CHECK_LAUNCH();
+        exclusive_scan_i32(ctx, cnt.as<int32_t>(), idx.as<int32_t>(), n);
+        k_agg_roots<<<nb, 256, 0, st>>>(n, cnt.as<int32_t>(), idx.as<int32_t>(), agg.as<int32_t>());
+        int32_t *ga = agg.as<int32_t>(), *gb = agg2.as<int32_t>();
+        for (int r = 0; r < 3; ++r) {
+            k_agg_join<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, th2, ga, gb);
+            std::swap(ga, gb);
+        }
+        LH_CHECK_LAUNCH();
+        double hp[2 * kRB];
+        int32_t nc32 = 0;
+        int hb[2] = {0, 0};
+        {
+            const Xfer q[3] = {{hp, part.p, sizeof(hp)}, {&nc32, idx.as<int32_t>() + n, 4}, {hb, flags.p, 8}};
+            d2h_n(ctx, q, 3);
+        }
+        double xdx = 0.0, xkx = 0.0;
+        for (int q = 0; q < kRB; ++q) {
+            xdx += hp[2 * q];
+            xkx += hp[2 * q + 1];
+        }
+        const double lmax = xdx > 0.0 ? xkx / xdx : 0.0;
+        const int64_t nc = nc32;
+        // a stalled coarsening, a bad diagonal or a meaningless estimate: no hierarchy
+        if (hb[0] || hb[1] || nc < 1 || nc > n * 7 / 10 || !(lmax > 0.0) || !std::isfinite(lmax)) return false;
+        lv.bmax = 1.1 * lmax;
+        const double w = 4.0 / (3.0 * lv.bmax);
+        // P
+        int32_t* pp = own<int32_t>(n + 1);
+        const bool long_rows = nnz > kLongRow * n;
+        if (long_rows)
+            k_prolongator_wave<false><<<nblocks(n, 4), 256, 0, st>>>(n, rp, cl, kv, dinv, w, ga, nullptr,
+                                                                     cnt.as<int32_t>(), nullptr);
+        else
+            k_prolongator<false><<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, w, ga, nullptr, cnt.as<int32_t>(), nullptr);
+        LH_CHECK_LAUNCH();
+        exclusive_scan_i32(ctx, cnt.as<int32_t>(), pp, n);
+        // one entry per distinct aggregate of a row: at most nnz
+        int32_t* pc = own<int32_t>(nnz);
+        double* pv = own<double>(nnz);
+        if (long_rows)
+            k_prolongator_wave<true><<<nblocks(n, 4), 256, 0, st>>>(n, rp, cl, kv, dinv, w, ga, pp, pc, pv);
+        else
+            k_prolongator<true><<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, w, ga, pp, pc, pv);
+        LH_CHECK_LAUNCH();
+        int32_t pnnz = 0;
+        d2h(ctx, &pnnz, pp + n, 4);
+        // P^T
+        int32_t* tp = own<int32_t>(nc + 1);
+        int32_t* tc = own<int32_t>(pnnz);
+        double* tv = own<double>(pnnz);
+        {
+            DevBuf fill((nc + 1) * 4), t2((size_t)std::max(pnnz, 1) * 4), v2((size_t)std::max(pnnz, 1) * 8);
+            memset_d(ctx, cnt.p, 0, nc * 4);
+            memset_d(ctx, fill.p, 0, nc * 4);
+            k_count_cols<<<nblocks(std::max(pnnz, 1), 256), 256, 0, st>>>(pnnz, pc, cnt.as<int32_t>());
+            LH_CHECK_LAUNCH();
+            exclusive_scan_i32(ctx, cnt.as<int32_t>(), tp, nc);
+            k_scatter_cols<<<nb, 256, 0, st>>>(n, pp, pc, pv, tp, fill.as<int32_t>(), t2.as<int32_t>(), v2.as<double>());
+            k_sort_rows<<<nblocks(nc, 4), 256, 0, st>>>(nc, tp, t2.as<int32_t>(), v2.as<double>(), tc, tv);
+            LH_CHECK_LAUNCH();
+            if (!fill.pooled || !t2.pooled || !v2.pooled) HIPX(hipStreamSynchronize(st));  // they go out of scope
+        }
+        lv.nc = nc;
+        lv.pnnz = pnnz;
+        lv.pp = pp;
+        lv.pc = pc;
+        lv.d.pv = pv;
+        lv.tp = tp;
+        lv.tc = tc;
+        lv.d.rv = tv;
+        // K P, then P^T (K P): tables of 256 columns, of 1,024 where a row
+        // overflows them
+        auto product = [&](int64_t rows, const int32_t* xp, const int32_t* xc, const double* xv, const int32_t* yp,
+                           const int32_t* yc, const double* yv, int32_t*& op, int32_t*& oc, double*& ov,
+                           std::vector<DevBuf>& into) -> int32_t {
+            const unsigned g = nblocks(rows, 4);
+            auto get = [&](size_t bytes) -> void* {
+                into.emplace_back(bytes);
+                return into.back().p;
+            };
+            op = static_cast<int32_t*>(get((rows + 1) * 4));
+            bool wide = false;
+            int32_t total = 0;
+            for (;;) {
+                if (wide)
+                    k_spgemm<1024, false><<<g, 256, 0, st>>>(rows, xp, xc, xv, yp, yc, yv, nullptr, cnt.as<int32_t>(),
+                                                             nullptr, over);
+                else
+                    k_spgemm<256, false><<<g, 256, 0, st>>>(rows, xp, xc, xv, yp, yc, yv, nullptr, cnt.as<int32_t>(),
+                                                            nullptr, over);
+                LH_CHECK_LAUNCH();
+                exclusive_scan_i32(ctx, cnt.as<int32_t>(), op, rows);
+                int o = 0;
+                const Xfer q[2] = {{&total, op + rows, 4}, {&o, over, 4}};
+                d2h_n(ctx, q, 2);
+                if (!o) break;
+                if (wide) return -1;
+                wide = true;
+                memset_d(ctx, over, 0, 4);
+            }
+            oc = static_cast<int32_t*>(get((size_t)std::max(total, 1) * 4));
+            ov = static_cast<double*>(get((size_t)std::max(total, 1) * 8));
+            if (wide)
+                k_spgemm<1024, true><<<g, 256, 0, st>>>(rows, xp, xc, xv, yp, yc, yv, op, oc, ov, over);
+            else
+                k_spgemm<256, true><<<g, 256, 0, st>>>(rows, xp, xc, xv, yp, yc, yv, op, oc, ov, over);
+            LH_CHECK_LAUNCH();
+            return total;
+        };
+        std::vector<DevBuf> tmp;
+        int32_t *ap = nullptr, *ac = nullptr, *np_ = nullptr, *nc_ = nullptr;
+        double *av = nullptr, *nv_ = nullptr;
+        if (product(n, rp, cl, kv, pp, pc, pv, ap, ac, av, tmp) < 0) return false;
+        const int32_t cnnz = product(nc, tp, tc, tv, ap, ac, av, np_, nc_, nv_, keep);
+        if (cnnz < 0) return false;
+        for (const DevBuf& t : tmp)
+            if (!t.pooled) {
+                HIPX(hipStreamSynchronize(st));  // K P goes out of scope
+                break;
+            }
+        n = nc;
+        nnz = cnnz;
+        rp = np_;
+        cl = nc_;
+        kv = nv_;
+        if (l + 1 == kMaxLevels) return false;
+    }
+    // the tail: the levels of at most kTailRows rows, kTailSum together
+    const int last = (int)levels.size() - 1;
+    tail = last;
+    int64_t sum = levels[last].n;
+    while (tail > 1 && levels[tail - 1].n <= kTailRows && levels[tail - 1].nnz <= kTailNnz &&
+           sum + levels[tail - 1].n <= kTailSum)
+        sum += levels[--tail].n;
+    TailDesc d{};
+    d.count = last - tail + 1;
+    d.ginv = ginv.as<double>();
+    int off = 0;
+    for (int l = tail; l <= last; ++l) {
+        const AmgLevel& lv = levels[l];
+        TailLevel& t = d.lv[l - tail];
+        t.n = (int)lv.n;
+        t.off = off;
+        off += (int)lv.n;
+        t.rp = lv.rp;
+        t.cl = lv.cl;
+        t.kv = lv.d.kv;
+        t.dinv = lv.d.dinv;
+        t.pp = lv.pp;
+        t.pc = lv.pc;
+        t.pv = lv.d.pv;
+        t.tp = lv.tp;
+        t.tc = lv.tc;
+        t.tv = lv.d.rv;
+        const Cheb2 k = cheb2(lv.bmax);
+        t.s = k.s;
+        t.c1 = k.c1;
+        t.c2 = k.c2;
+    }
+    tail_desc.alloc(sizeof(TailDesc));
+    h2d(ctx, tail_desc.p, &d, sizeof(TailDesc));
+    return true;
+}
+
+void Amg::prepare(int m_) {
+    m = m_;
+    size_t total = 0;
+    for (int l = 0; l <= tail; ++l) total += 4 * (size_t)levels[l].n * m;
+    work.alloc(total * 8);
+    double* p = work.as<double>();
+    wb.clear();
+    wx.clear();
+    wy.clear();
+    wr.clear();
+    for (int l = 0; l <= tail; ++l) {
+        const size_t s = (size_t)levels[l].n * m;
+        wb.push_back(p);
+        wx.push_back(p + s);
+        wy.push_back(p + 2 * s);
+        wr.push_back(p + 3 * s);
+        p += 4 * s;
+    }
+}
+
+namespace {
+
+template <int V>
+struct IntC {
+    static constexpr int v = V;
+};
+// lanes for a row of the mean length: about four entries a lane
+int lanes_for(int64_t nnz, int64_t n) {
+    const int64_t avg = n > 0 ? nnz / n : 0;
+    return avg >= 40 ? 16 : avg >= 20 ? 8 : avg >= 8 ? 4 : 1;
+}
+template <typename F>
+void with_lanes(int g, F&& f) {
+    switch (g) {
+        case 1: f(IntC<1>{}); break;
+        case 4: f(IntC<4>{}); break;
+        case 8: f(IntC<8>{}); break;
+        default: f(IntC<16>{}); break;
+    }
+}
+
+}  // namespace
+
+void Amg::cycle(int l, const double* b, double* x, double* part, const int* status) {
+    hipStream_t st = ctx->stream;
+    if (l == tail) {
+        k_amg_tail<<<(unsigned)m, kTailThreads, 0, st>>>(m, tail_desc.as<TailDesc>(), b, x, status);
+        LH_CHECK_LAUNCH();
+        return;
+    }
+    const AmgLevel& lv = levels[l];
+    const Cheb2 k = cheb2(lv.bmax);
+    double *y = wy[l], *r = wr[l];
+    const int gk = lv.W ? 1 : lanes_for(lv.nnz, lv.n);
+    const unsigned nk = nblocks_xcd(lv.n * m * gk, 256);
+    const int32_t* cl = lv.W ? lv.ecl : lv.cl;
+    // f(W, G) with the level's slots per row and lanes per row
+    auto with_k = [&](auto&& f) {
+        switch (lv.W) {
+            case 8: f(IntC<8>{}, IntC<1>{}); break;
+            case 16: f(IntC<16>{}, IntC<1>{}); break;
+            case 24: f(IntC<24>{}, IntC<1>{}); break;
+            case 32: f(IntC<32>{}, IntC<1>{}); break;
+            default: with_lanes(gk, [&](auto g) { f(IntC<0>{}, g); });
+        }
+        LH_CHECK_LAUNCH();
+    };
+    with_k([&](auto w, auto g) {
+        k_amg_pre<w.v, g.v><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, x, k.s, k.c1, k.c2, status);
+    });
+    with_k([&](auto w, auto g) {
+        k_amg_step<w.v, g.v, 0><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, x, r, 0.0, 0.0, 0.0,
+                                                    nullptr, status);
+    });
+    const int gt = lanes_for(lv.pnnz, lv.nc), gp = lanes_for(lv.pnnz, lv.n);
+    with_lanes(gt, [&](auto g) {
+        k_amg_transfer<false, g.v><<<nblocks_xcd(lv.nc * m * gt, 256), 256, 0, st>>>(lv.nc, m, lv.tp, lv.tc, lv.d.rv, r,
+                                                                                   wb[l + 1], status);
+    });
+    LH_CHECK_LAUNCH();
+    cycle(l + 1, wb[l + 1], wx[l + 1], nullptr, status);
+    with_lanes(gp, [&](auto g) {
+        k_amg_transfer<true, g.v><<<nblocks_xcd(lv.n * m * gp, 256), 256, 0, st>>>(lv.n, m, lv.pp, lv.pc, lv.d.pv,
+                                                                                 wx[l + 1], x, status);
+    });
+    LH_CHECK_LAUNCH();
+    with_k([&](auto w, auto g) {
+        k_amg_step<w.v, g.v, 1><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, x, y, 0.0, 0.0, k.s,
+                                                    nullptr, status);
+    });
+    if (part)
+        with_k([&](auto w, auto g) {
+            k_amg_step<w.v, g.v, 3><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, y, x, 1.0 + k.c1,
+                                                        -k.c1, k.c2, part, status);
+        });
+    else
+        with_k([&](auto w, auto g) {
+            k_amg_step<w.v, g.v, 2><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, y, x, 1.0 + k.c1,
+                                                        -k.c1, k.c2, nullptr, status);
+        });
+}
+
+int Amg::dot_blocks() const {
+    if (m > 4) return 0;
+    const AmgLevel& lv = levels[0];
+    return (int)nblocks_xcd(lv.n * m * (lv.W ? 1 : lanes_for(lv.nnz, lv.n)), 256);
+}
+
+void Amg::apply(const double* R, double* Z, double* part, const int* status) { cycle(0, R, Z, part, status); }
+
+}  // namespace lh

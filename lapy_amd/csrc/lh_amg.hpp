@@ -1,0 +1,67 @@
+// Smoothed-aggregation multigrid (lh_amg.hip): the preconditioner of the
+// linear solves on large systems.
+#pragma once
+#include "lh_dense.hpp"
+
+namespace lh {
+
+// one level's operators in the precision T of the cycle
+template <typename T>
+struct AmgOps {
+    const T* kv = nullptr;    // K (the level's CSR slots; level 0 with an ELL copy: its slots)
+    const T* dinv = nullptr;  // 1 / diag K (0 on a zero row)
+    const T* pv = nullptr;    // P
+    const T* rv = nullptr;    // P^T
+};
+
+struct AmgLevel {
+    int64_t n = 0, nnz = 0;
+    const int32_t* rp = nullptr;  // K: CSR
+    const int32_t* cl = nullptr;
+    int W = 0;  // level 0 with an ELL copy: slots per row (columns at ecl); 0: CSR
+    const int32_t* ecl = nullptr;
+    double bmax = 2.0;  // upper end of the smoother's interval (estimate of lambda_max(D^-1 K))
+    // transfer to the next level (absent on the last one)
+    int64_t nc = 0, pnnz = 0;
+    const int32_t *pp = nullptr, *pc = nullptr;  // P (n x nc), CSR
+    const int32_t *tp = nullptr, *tc = nullptr;  // P^T (nc x n), CSR
+    AmgOps<double> d;
+};
+
+struct Amg {
+    // Hierarchy of the n x n operator with CSR slots (rp, cl, kv); symmetric,
+    // diagonal positive except on zero rows.  ell_w > 0: an ELL copy (ecl,
+    // ekv) for the products of the finest level.  Returns false (nothing to
+    // free) when no useful hierarchy exists: a negative diagonal, coarsening
+    // that stalls, or a coarsest matrix that does not factorise.
+    bool setup(lh_ctx* ctx, int64_t n, int64_t nnz, const int32_t* rp, const int32_t* cl, const double* kv, int ell_w,
+               const int32_t* ecl, const double* ekv);
+    // work blocks for m columns in double precision
+    void prepare(int m);
+    // Z <- M R, row-major n x m; a set status[0] makes every launch return at
+    // once.  part (not null; m <= 4): dot_blocks() partial sums of each
+    // column of R . Z, part[block * m + column]
+    void apply(const double* R, double* Z, double* part, const int* status);
+    int dot_blocks() const;  // 0: more than four columns
+
+    std::vector<AmgLevel> levels;
+
+   private:
+    lh_ctx* ctx = nullptr;
+    int m = 0;
+    int tail = 0;  // first level of the one-launch tail
+    std::vector<DevBuf> keep;  // every level's arrays
+    DevBuf ginv;               // inverse of the coarsest matrix (nl x nl)
+    DevBuf work;
+    DevBuf tail_desc;          // the tail's levels, for its kernel
+    std::vector<double*> wb, wx, wy, wr;  // per level: right-hand side, iterate, second iterate, residual
+    template <typename X> X* own(size_t count);
+    void cycle(int l, const double* b, double* x, double* part, const int* status);
+};
+
+// 2 tr(D) / 1^T K 1: a lower bound of the condition number of D^-1 K for an
+// operator with a mass term (close to it when the mass is spread evenly)
+double amg_condition(lh_ctx* ctx, int64_t n, const int32_t* rp, const int32_t* cl, const double* kv,
+                     const double* dinv);
+
+}  // namespace lh

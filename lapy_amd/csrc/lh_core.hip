@@ -67,7 +67,8 @@ static void scan_rec(lh_ctx* ctx, const int32_t* in, int32_t* out, int64_t n) {
         k_scan_add<<<nblocks(n, 256), 256, 0, ctx->stream>>>(out, n, sums_scan.as<int32_t>());
         LH_CHECK_LAUNCH();
     }
-    HIPX(hipStreamSynchronize(ctx->stream));  // sums buffers go out of scope
+    // the buffers go out of scope: arena memory is next written in stream order
+    if (!sums.pooled || !sums_scan.pooled) HIPX(hipStreamSynchronize(ctx->stream));
 }
 
 void exclusive_scan_i32(lh_ctx* ctx, const int32_t* in, int32_t* out, int64_t n) {

@@ -741,6 +741,7 @@ int lh_eigs(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const lh_eig
     HIPX(hipSetDevice(ctx->device));
     lh_stats st{};
     int code = LH_OK;
+    CallArena arena(ctx, arena_bytes(A->n(), block_width(k, opts)));
     *out = eigs_impl(ctx, A, B, k, sigma, opts, st, code);
     if (stats) *stats = st;
     if (code == LH_ERR_NOCONV) {

@@ -159,6 +159,42 @@ struct lh_ctx {
     std::shared_ptr<TuneTable> tune = std::make_shared<TuneTable>();
 };
 
+// A solve's temporaries from its context's own arena (bounded by kMost, kept
+// until the context ends): without it a small solve spends as long in
+// hipMalloc and hipFree as on the device.  Does nothing where the thread has
+// an arena already (the batched solver's workers).  What does not fit comes
+// from hipMalloc as before.  One call at a time uses a context and its stream,
+// so the memory is reused in stream order.
+struct CallArena {
+    static constexpr size_t kLeast = size_t(64) << 20, kMost = size_t(1) << 30;
+    lh_ctx* ctx = nullptr;
+    CallArena(lh_ctx* c, size_t want) {
+        if (lh_thread_arena) return;
+        want = want < kLeast ? kLeast : want > kMost ? kMost : want;
+        if (c->arena_mem.bytes < want) {
+            c->arena.base = nullptr;
+            try {
+                c->arena_mem.alloc(want);
+            } catch (const lh_error&) {  // no room: plain allocations, which may still fit
+                (void)hipGetLastError();
+                return;
+            }
+        }
+        c->arena.base = c->arena_mem.as<char>();
+        c->arena.cap = c->arena_mem.bytes;
+        c->arena.top = 0;
+        lh_thread_arena = &c->arena;
+        ctx = c;
+    }
+    ~CallArena() {
+        if (!ctx) return;
+        lh_thread_arena = nullptr;
+        ctx->arena.top = 0;
+    }
+    CallArena(const CallArena&) = delete;
+    CallArena& operator=(const CallArena&) = delete;
+};
+
 // frees ctx->blas (lh_rrlib.hip)
 void release_blas(lh_ctx* ctx);
 

@@ -18,6 +18,16 @@
 // such an A is regular (its smallest eigenvalue ~1e-9) and is solved as it
 // stands, as SuperLU does, with no projection.
 //
+// Large ill-conditioned systems are preconditioned by a multigrid cycle
+// (lh_amg.hip), the others by Jacobi.  Against Jacobi-CG, a whole call: a
+// singular Poisson solve on a closed surface of 163,842 vertices 2,496 -> 32
+// iterations (46 -> 7 ms on the device), a Dirichlet one of 40,962 1,168 -> 24
+// (17.4 -> 4.0 ms), three columns of mass + stiffness at 10,242 715 -> 28 (28 ->
+// 5 ms), and the solutions' error against 64-bit references is 2 to 10 times
+// smaller, since the residual left over lies in the high frequencies.  Below
+// ~350 Jacobi iterations the hierarchy's setup (1.5 ms at 40,962 rows, bound
+// by the latency of ~400 small launches) costs more than it saves.
+//
 // One iteration is two launches (Jacobi or no preconditioner), and no kernel
 // waits for another's blocks: each kernel reads the block partials the
 // previous one wrote, every block summing them itself in the same fixed order
@@ -45,7 +55,7 @@
 // gathered by a range then sit in that XCD's L2.  The host checks the done
 // flag once per chunk of iterations; iterations enqueued after convergence
 // exit at once.
-#include "lh_dense.hpp"
+#include "lh_amg.hpp"
 
 #include <chrono>
 #include <cmath>
@@ -57,6 +67,8 @@ namespace {
 constexpr int kBS = 256;    // threads per block of the set-up kernels
 constexpr int kIBS = 1024;  // threads per block of the iteration kernels
 constexpr int kMC = 8;      // right-hand sides per launch (wider blocks: several launches)
+constexpr double kAmgMinIters = 350.0;  // expected Jacobi-CG iterations from which the multigrid cycle takes over
+constexpr int kAmgMaxIters = 200;       // iterations with the cycle before Jacobi takes over again
 
 // K = beta * A + alpha * B on A's pattern
 template <typename VT>
@@ -191,7 +203,7 @@ struct CgState {
     double* rr[2];       // partials of r.r (nb_upd x m)
     double* pq;          // partials of p.q (nb_dir x m)
     double* sr;          // partials of sum(r) (nb_dir x m, singular systems)
-    int nb_upd, nb_dir;
+    int nb_upd, nb_dir, nb_rz;  // partials of r.r, of p.q and sum(r), of r.z
     int* status;         // [0]: done, [1]: iterations done (written by block 0)
     double* rr_out;      // r.r of the latest iterate (written by block 0)
 };
@@ -219,7 +231,7 @@ k_cg_dir(int64_t n, int m, int c0, int mc, int par, const int32_t* __restrict__ 
             // beta_k = rz_k / rz_{k-1}; 0 for a converged column (and at k = 0,
             // where P and Q hold zeros anyway)
             const double* const pp[3] = {s.rz[par], s.rz[par ^ 1], s.rr[par]};
-            const int np[3] = {s.nb_upd, s.nb_upd, s.nb_upd};
+            const int np[3] = {s.nb_rz, s.nb_rz, s.nb_upd};
             double v[3];
             allsum_partials_k<3>(pp, np, m, c0 + c, sh, v);
             const double rzk = v[0], rzo = v[1], rrk = v[2];
@@ -293,7 +305,7 @@ k_cg_dir_ell(int64_t n, int m, int c0, int mc, int par, const int32_t* __restric
         pq[c] = sr[c] = 0.0;
         if (c < mc) {
             const double* const pp[3] = {s.rz[par], s.rz[par ^ 1], s.rr[par]};
-            const int np[3] = {s.nb_upd, s.nb_upd, s.nb_upd};
+            const int np[3] = {s.nb_rz, s.nb_rz, s.nb_upd};
             double v[3];
             allsum_partials_k<3>(pp, np, m, c0 + c, sh, v);
             const double rzk = v[0], rzo = v[1], rrk = v[2];
@@ -376,13 +388,13 @@ k_cg_dir_ell(int64_t n, int m, int c0, int mc, int par, const int32_t* __restric
 
 // ---- update: x += alpha p, r = r - mean - alpha q, (z = D^-1 r) -------------
 // alpha_k = rz_k / p.q for an active column (r_k.r_k > tol2), else 0
-template <int MC, bool SING, bool JAC>
-__global__ void __launch_bounds__(kIBS)
+template <int BS, int MC, bool SING, bool JAC>
+__global__ void __launch_bounds__(BS)
 k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict__ dinv, const double* __restrict__ P,
             const double* __restrict__ Q, double* __restrict__ X, double* __restrict__ R, double* __restrict__ Z,
             CgState s, int last_chunk) {
     if (s.status[0]) return;
-    __shared__ double sh[4 * kIBS / 64];
+    __shared__ double sh[4 * BS / 64];
     // contiguous rows per block, an even count; a thread takes two adjacent
     // rows per step (one 16-byte load per operand for one column)
     int64_t rpb = (n + gridDim.x - 1) / gridDim.x;
@@ -396,7 +408,7 @@ k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict_
         if (c < mc) {
             const int cc = c0 + c;
             const double* const pp[4] = {s.rz[par], s.rr[par], s.pq, s.sr};
-            const int np[4] = {s.nb_upd, s.nb_upd, s.nb_dir, SING ? s.nb_dir : 0};
+            const int np[4] = {s.nb_rz, s.nb_upd, s.nb_dir, SING ? s.nb_dir : 0};
             double v[4];
             allsum_partials_k<4>(pp, np, m, cc, sh, v);
             const double rzk = v[0], rrk = v[1], pqk = v[2];
@@ -407,7 +419,7 @@ k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict_
             if (blockIdx.x == 0 && threadIdx.x == 0) s.rr_out[cc] = rrk;
         }
     }
-    for (int64_t i = rb + 2 * (int64_t)threadIdx.x; i < re; i += 2 * kIBS) {
+    for (int64_t i = rb + 2 * (int64_t)threadIdx.x; i < re; i += 2 * BS) {
         const bool two = i + 1 < re;
         double vr[2][MC], vq[2][MC], vp[2][MC], vx[2][MC], vd[2];
         if (MC == 1 && m == 1 && two) {
@@ -705,6 +717,7 @@ struct Launcher {
     int m;
     int lpr;
     unsigned nb;      // blocks of the row-wise kernels (partials per column)
+    bool small;       // k_cg_update in workgroups of 256 instead of 1,024 threads
     unsigned nb_dir;  // blocks of k_cg_dir
     const int32_t* rp;
     const int32_t* cl;
@@ -756,8 +769,9 @@ struct Launcher {
     template <int MC>
     void update_mc(int c0, int mc, int par, bool sing, bool jac, const double* dinv, const double* P,
                    const double* Q, double* X, double* R, double* Z, const CgState& s, int last) {
-#define LH_UPD(S, J) \
-    k_cg_update<MC, S, J><<<nb, kIBS, 0, ctx->stream>>>(n, m, c0, mc, par, dinv, P, Q, X, R, Z, s, last)
+#define LH_UPD(S, J)                                                                                              \
+    (small ? k_cg_update<kBS, MC, S, J><<<nb, kBS, 0, ctx->stream>>>(n, m, c0, mc, par, dinv, P, Q, X, R, Z, s, last) \
+           : k_cg_update<kIBS, MC, S, J><<<nb, kIBS, 0, ctx->stream>>>(n, m, c0, mc, par, dinv, P, Q, X, R, Z, s, last))
         if (sing) { if (jac) LH_UPD(true, true); else LH_UPD(true, false); }
         else { if (jac) LH_UPD(false, true); else LH_UPD(false, false); }
 #undef LH_UPD
@@ -885,6 +899,9 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
         LH_THROW(LH_ERR_ARG, "LH_PRECOND_LEARNED needs a network on the context (lh_ctx_set_mpnn)");
     if ((size_t)m * 16 + 64 > ctx->host_small_bytes) LH_THROW(LH_ERR_ARG, "too many right-hand sides (%d)", m);
     lh_stats st{};
+    // values, reordered and ELL copies, the multigrid hierarchy (~100 bytes an
+    // entry) and the block vectors
+    CallArena arena(ctx, (size_t)nnz * 100 + (size_t)n * 8 * (20 + 14 * (size_t)m));
     // operator values on A's pattern
     DevBuf kv(nnz * 8), missing(8);
     memset_d(ctx, missing.p, 0, 4);
@@ -963,7 +980,10 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     L.n = n;
     L.m = m;
     L.lpr = lanes_per_row(n > 0 ? (double)nnz / (double)n : 1.0);
-    L.nb = std::max(1u, std::min<unsigned>(nblocks(n, 2 * kIBS), (unsigned)ctx->n_cu));
+    // workgroups of 1,024 threads use a CU each only from 2,048 rows a CU on;
+    // below that, smaller ones spread over four times as many
+    L.small = nblocks(n, 2 * kIBS) < (unsigned)ctx->n_cu;
+    L.nb = std::max(1u, std::min<unsigned>(nblocks(n, 2 * (L.small ? kBS : kIBS)), (unsigned)ctx->n_cu));
     L.nb_dir = std::max<unsigned>(kXCDs, std::min<unsigned>(nblocks_xcd(n * L.lpr, kIBS), (unsigned)ctx->n_cu * 2));
     L.nb_dir = (L.nb_dir + kXCDs - 1) / kXCDs * kXCDs;
     L.rp = kpat->rowptr.as<int32_t>();
@@ -1002,6 +1022,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     s.sr = s.pq + pd;
     s.nb_upd = (int)L.nb;
     s.nb_dir = (int)L.nb_dir;
+    s.nb_rz = s.nb_upd;
     double* tol2 = scal.as<double>();
     double* sums = tol2 + m;
     double* rrout = sums + m;
@@ -1034,6 +1055,37 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
         for (double v : hg) g = std::max(g, v);
         cheb_bmax = g > 0.0 ? g : 2.0;
         cheb_amin = cheb_bmax / (2.0 * pdeg * pdeg);
+    }
+    // automatic (degree 0): the multigrid cycle where Jacobi-CG would take
+    // long, from the iterations it is expected to take: c n^(1/dim) without a
+    // mass term (surfaces 5.4 sqrt(n): 548 at 10,242 vertices, 1,076 at
+    // 40,962; volumes, told by their longer rows, 14.4 n^(1/3)), and from the
+    // condition estimate 2 tr(D) / 1^T K 1 with one
+    Amg amg;
+    bool amg_on = false;
+    if (precond == LH_PRECOND_JACOBI && pdeg_opt == 0) {
+        const double dn = (double)n;
+        double expect = (double)nnz > 10.0 * dn ? 14.4 * std::cbrt(dn) : 5.4 * std::sqrt(dn);
+        expect *= std::log(2.0 / rtol) / std::log(2e12);
+        if (expect > kAmgMinIters && alpha != 0.0) {
+            const double kappa = amg_condition(ctx, n, L.rp, L.cl, L.kv, dinv.as<double>());
+            expect = std::min(expect, 0.5 * std::sqrt(kappa) * std::log(2.0 / rtol));
+        }
+        if (expect > kAmgMinIters) {
+            amg_on = amg.setup(ctx, n, nnz, L.rp, L.cl, L.kv, L.ew, L.ecols, L.ev);
+            if (amg_on) amg.prepare(m);
+        }
+    }
+    // up to four columns: the cycle's last launch leaves the partials of r.z
+    DevBuf rzbuf;
+    double* const rz_plain[2] = {s.rz[0], s.rz[1]};
+    const int amg_dots = amg_on ? amg.dot_blocks() : 0;
+    if (amg_dots) {
+        rzbuf.alloc((size_t)amg_dots * m * 16);
+        memset_d(ctx, rzbuf.p, 0, rzbuf.bytes);
+        s.rz[0] = rzbuf.as<double>();
+        s.rz[1] = s.rz[0] + (size_t)amg_dots * m;
+        s.nb_rz = amg_dots;
     }
     DevBuf dT;
     if (pdeg > 1) dT.alloc((size_t)n * m * 8);
@@ -1099,7 +1151,9 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     // a first direction at iteration k: z = M^-1 r and the partials of r.z
     // into parity k % 2, P = Q = 0 (so p = z, q = K z whatever beta is)
     auto start_direction = [&](bool jac, int64_t k) {
-        if (jac && pdeg > 1) {
+        if (amg_on) {
+            amg.apply(dR.as<double>(), dZ.as<double>(), amg_dots ? s.rz[k & 1] : nullptr, nullptr);
+        } else if (jac && pdeg > 1) {
             L.cheb(pdeg, cheb_amin, cheb_bmax, dinv.as<double>(), dR.as<double>(), dZ.as<double>(), dT.as<double>(),
                    nullptr);
         } else if (jac) {
@@ -1108,7 +1162,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
         } else {
             apply_learned();
         }
-        L.rz(dR.as<double>(), dZ.as<double>(), s.rz[k & 1], nullptr);
+        if (!amg_on || !amg_dots) L.rz(dR.as<double>(), dZ.as<double>(), s.rz[k & 1], nullptr);
         HIPX(hipMemsetAsync(dP.p, 0, blk, ctx->stream));
         HIPX(hipMemsetAsync(dQ.p, 0, blk, ctx->stream));
     };
@@ -1120,15 +1174,18 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     int* hstat = static_cast<int*>(ctx->host_small);
     double* hrr_pin = reinterpret_cast<double*>(static_cast<char*>(ctx->host_small) + 64);
     while (!done && enq < max_iter) {
-        const int chunk = (int)std::min<int64_t>(learned_on ? 4 : 16, max_iter - enq);
+        const int chunk = (int)std::min<int64_t>(learned_on || amg_on ? 4 : 16, max_iter - enq);
         for (int kk = 0; kk < chunk; ++kk) {
             const int par = (int)((enq + kk) & 1);
             L.dir(par, singular, dZ.as<double>(), dP.as<double>(), dQ.as<double>(), dR.as<double>(), s);
-            L.update(par, singular, !learned_on && pdeg == 1, dinv.as<double>(), dP.as<double>(), dQ.as<double>(),
+            L.update(par, singular, !learned_on && !amg_on && pdeg == 1, dinv.as<double>(), dP.as<double>(), dQ.as<double>(),
                      dX.as<double>(), dR.as<double>(), dZ.as<double>(), s);
             if (learned_on) {
                 apply_learned();
                 L.rz(dR.as<double>(), dZ.as<double>(), s.rz[par ^ 1], s.status);
+            } else if (amg_on) {
+                amg.apply(dR.as<double>(), dZ.as<double>(), amg_dots ? s.rz[par ^ 1] : nullptr, s.status);
+                if (!amg_dots) L.rz(dR.as<double>(), dZ.as<double>(), s.rz[par ^ 1], s.status);
             } else if (pdeg > 1) {
                 L.cheb(pdeg, cheb_amin, cheb_bmax, dinv.as<double>(), dR.as<double>(), dZ.as<double>(),
                        dT.as<double>(), s.status);
@@ -1156,6 +1213,15 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
                 st.fallback_used = 1;
                 start_direction(true, enq);
             }
+        }
+        // an operator that the cycle does not suit: on with Jacobi (CG restarted)
+        if (amg_on && !done && enq >= kAmgMaxIters) {
+            amg_on = false;
+            s.rz[0] = rz_plain[0];
+            s.rz[1] = rz_plain[1];
+            s.nb_rz = s.nb_upd;
+            st.fallback_used = 1;
+            start_direction(true, enq);
         }
         prev_worst = worst;
         if (verbose && (enq % 256 == 0)) fprintf(stderr, "[pcg] it %d worst %.3e\n", iters, worst);

@@ -1,0 +1,125 @@
+"""The multigrid preconditioner of the linear solves (taken by the automatic
+choice on large systems): solutions against scipy's splu, and the systems it
+has to leave to Jacobi.
+
+Tolerance: both solves end at a relative residual of 1e-12 or below, so they
+differ by at most a few 1e-12 times the condition number in the norm of
+x: 1e-12 * 1e4 for the regular systems here (the largest condition number is
+that of the Jacobi-scaled 16,000-row ones); the true residual is held to 1e-11,
+ten times the recurrence's, for what rounding adds to it."""
+
+import numpy as np
+import pytest
+from scipy import sparse
+from scipy.sparse.linalg import splu
+
+from lapy_amd import Solver, TetMesh, TriaMesh, _lib, meshgen
+
+pytestmark = pytest.mark.gpu
+
+
+def _cap(level, keep):
+    """Open surface with an odd number of vertices."""
+    v, t = meshgen.perturbed_sphere(level, np.random.default_rng(4), axes=(1.3, 0.8, 1.0), sigma=0.02)
+    t = t[(v[:, 2] > np.quantile(v[:, 2], 1 - keep))[t].all(axis=1)]
+    used, t = np.unique(t, return_inverse=True)
+    return v[used], t.reshape(-1, 3)
+
+
+def _systems():
+    v, t = _cap(5, 0.43)  # 4,3xx rows: just above the smallest system that takes the cycle
+    yield "cap", Solver(TriaMesh(v, t), lump=True), 20
+    yield "closed", Solver(TriaMesh(*meshgen.perturbed_sphere(5, np.random.default_rng(3), sigma=0.05)), lump=True), 1
+    yield "tets", Solver(TetMesh(*meshgen.tet_cube(25, jitter=0.15)), lump=True), 40
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 9])  # partials in the cycle up to 4 columns, their own launch beyond
+def test_dirichlet_systems_against_splu(m):
+    ctx = _lib.default_context()
+    rng = np.random.default_rng(m)
+    for name, fem, nd in _systems():
+        a = sparse.csr_matrix(fem.stiffness)
+        n = a.shape[0]
+        dmask = np.zeros(n, np.uint8)
+        dmask[rng.choice(n, nd, replace=False)] = 1
+        free = np.flatnonzero(dmask == 0)
+        b = rng.standard_normal((n, m))
+        x, st = _lib.pcg(ctx, fem.device_matrices()[0], None, 0.0, 1.0, b, dmask=dmask, rtol=1e-12)
+        _, st_j = _lib.pcg(ctx, fem.device_matrices()[0], None, 0.0, 1.0, b[:, 0], dmask=dmask, rtol=1e-12,
+                           poly_degree=1)
+        print(name, n, "columns", m, "iterations", st.iterations, "jacobi", st_j.iterations, flush=True)
+        assert st.fallback_used == 0 and 4 * st.iterations < st_j.iterations  # the cycle ran
+        af = a[free][:, free]
+        xo = splu(sparse.csc_matrix(af)).solve(b[free])
+        for c in range(m):
+            assert np.linalg.norm(b[free, c] - af @ x[free, c]) <= 1e-11 * np.linalg.norm(b[free, c])
+            assert np.linalg.norm(x[free, c] - xo[:, c]) <= 1e-8 * np.linalg.norm(xo[:, c])
+        assert np.all(x[dmask == 1] == 0.0)
+
+
+def test_singular_and_mass_systems():
+    ctx = _lib.default_context()
+    rng = np.random.default_rng(2)
+    for name, fem, _ in _systems():
+        a, b = fem.device_matrices()
+        A, B = sparse.csr_matrix(fem.stiffness), sparse.csr_matrix(fem.mass)
+        n = A.shape[0]
+        f = rng.standard_normal((n, 2))
+        x, st = _lib.pcg(ctx, a, None, 0.0, 1.0, f, rtol=1e-12)  # constants: the null space
+        p = f - f.mean(axis=0)
+        assert st.fallback_used == 0 and st.iterations < 120
+        for c in range(2):
+            assert abs(x[:, c].mean()) <= 1e-12 * np.abs(x[:, c]).max()
+            assert np.linalg.norm(p[:, c] - A @ x[:, c]) <= 1e-11 * np.linalg.norm(p[:, c])
+        t = 1.0  # a long time step: mass + t stiffness, ill-conditioned
+        h, st = _lib.pcg(ctx, a, b, 1.0, t, f, rtol=1e-12)
+        k = sparse.csc_matrix(B + t * A)
+        ho = splu(k).solve(f)
+        print(name, "mass system iterations", st.iterations, flush=True)
+        for c in range(2):
+            assert np.linalg.norm(f[:, c] - k @ h[:, c]) <= 1e-11 * np.linalg.norm(f[:, c])
+            assert np.linalg.norm(h[:, c] - ho[:, c]) <= 1e-8 * np.linalg.norm(ho[:, c])
+
+
+def test_repeated_solves_are_bit_identical():
+    """Hierarchy, cycle and reductions are summed in fixed orders."""
+    ctx = _lib.default_context()
+    _, fem, _ = next(_systems())
+    b = np.random.default_rng(1).standard_normal(fem.device_matrices()[0].n)
+    x = [_lib.pcg(ctx, fem.device_matrices()[0], None, 0.0, 1.0, b, rtol=1e-12)[0] for _ in range(2)]
+    assert np.array_equal(x[0], x[1])
+
+
+def test_systems_left_to_jacobi():
+    """A negative definite matrix, a diagonal one and one whose rows couple to
+    nothing strongly: solved as before, without the cycle."""
+    ctx = _lib.default_context()
+    n = 6000
+    rng = np.random.default_rng(5)
+    lap = sparse.diags([-np.ones(n - 1), 2.0 * np.ones(n) + 0.5, -np.ones(n - 1)], [-1, 0, 1], format="csr")
+    weak = sparse.diags([-1e-3 * np.ones(n - 1), np.ones(n), -1e-3 * np.ones(n - 1)], [-1, 0, 1], format="csr")
+    b = rng.standard_normal(n)
+    for m in (-lap, sparse.csr_matrix(sparse.diags(rng.uniform(1, 2, n))), weak):
+        x, _ = _lib.pcg(ctx, _lib.DeviceCSR.from_scipy(ctx, m), None, 0.0, 1.0, b, rtol=1e-12)
+        assert np.linalg.norm(b - m @ x) <= 1e-11 * np.linalg.norm(b)
+
+
+def test_rows_with_many_entries():
+    """A graph Laplacian with rows of 3 to ~60 entries, not from a mesh: CSR
+    products, long rows in every setup kernel, hash tables of both sizes."""
+    ctx = _lib.default_context()
+    n = 5003
+    rng = np.random.default_rng(6)
+    i = np.repeat(np.arange(n), 14)
+    j = (i + np.rint(rng.normal(0, 60, len(i))).astype(int)) % n
+    hub = rng.choice(n, 40, replace=False)
+    i = np.concatenate([i, np.repeat(hub, 30)])
+    j = np.concatenate([j, rng.integers(0, n, 40 * 30)])
+    keep = i != j
+    w = sparse.coo_matrix((rng.uniform(0.5, 1.5, keep.sum()), (i[keep], j[keep])), shape=(n, n)).tocsr()
+    w = w + w.T
+    a = sparse.csr_matrix(sparse.diags(np.asarray(w.sum(axis=1)).ravel() + 1e-3) - w)
+    b = rng.standard_normal(n)
+    x, st = _lib.pcg(ctx, _lib.DeviceCSR.from_scipy(ctx, a), None, 0.0, 1.0, b, rtol=1e-12)
+    print("iterations", st.iterations, "longest row", np.diff(a.indptr).max())
+    assert np.linalg.norm(b - a @ x) <= 1e-11 * np.linalg.norm(b)
