@@ -181,6 +181,10 @@ struct Reorder {
     void unpermute(lh_ctx* ctx, const double* in, int ldi, double* out, int ldo, int64_t n, int m) const;
 };
 
+// the columns of a row-major n x m block (leading dimension ldi), one after
+// another, in the order before ro's permutation (ro null: as they are)
+void columns_out(lh_ctx* ctx, const double* in, int ldi, const Reorder* ro, double* out, int64_t n, int m);
+
 // the locality order of a pattern: built on the first request (outside any
 // call arena) and kept with the pattern; concurrent first requests build it
 // once

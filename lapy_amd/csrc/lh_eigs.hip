@@ -443,8 +443,7 @@ struct Lobpcg {
         }
         const Reorder* order = ext_ro ? ext_ro : (reordered ? ro.get() : nullptr);
         if constexpr (sizeof(T) == 8) {
-            if (order) order->unpermute(ctx, Sp(), ld, out_vecs->as<double>(), k, n, k);
-            else copy_block<double, double>(ctx, n, k, Sp(), ld, out_vecs->as<double>(), k);
+            columns_out(ctx, Sp(), ld, order, out_vecs->as<double>(), n, k);
         } else {
             LH_THROW(LH_ERR_ARG, "FP32 blocks are not returned");
         }
@@ -493,7 +492,7 @@ void dense_eigs(lh_ctx* ctx, const lh_csr* A, const lh_csr* B, int k, double* ev
         ArenaOff keep;  // the result outlives the solver's buffers
         evecs.alloc((size_t)n * k * 8);
     }
-    HIPX(hipMemcpyAsync(evecs.p, C.p, (size_t)n * k * 8, hipMemcpyDeviceToDevice, ctx->stream));
+    columns_out(ctx, C.as<double>(), k, nullptr, evecs.as<double>(), n, k);
     HIPX(hipStreamSynchronize(ctx->stream));
     st.iterations = 1;
     st.converged = k;
@@ -900,14 +899,7 @@ int lh_eig_download(lh_eig* e, double* evals, double* evecs) {
     LH_API_BEGIN(ctx)
     HIPX(hipSetDevice(ctx->device));
     if (evals) for (int j = 0; j < e->k; ++j) evals[j] = e->evals[j];
-    if (evecs) {
-        // device row-major n x k == host column-major k x n transposed; the
-        // caller wants evecs[:, j] contiguous (Fortran order), so transpose.
-        std::vector<double> h((size_t)e->n * e->k);
-        d2h(ctx, h.data(), e->evecs.p, h.size() * 8);
-        for (int64_t i = 0; i < e->n; ++i)
-            for (int j = 0; j < e->k; ++j) evecs[(int64_t)j * e->n + i] = h[i * e->k + j];
-    }
+    if (evecs) d2h(ctx, evecs, e->evecs.p, (size_t)e->n * e->k * 8);  // evecs[:, j] contiguous, as on the device
     LH_API_END(ctx)
 }
 

@@ -265,7 +265,7 @@ struct lh_eig {
     int64_t n = 0;
     int k = 0;
     std::vector<double> evals;
-    DevBuf evecs;        // n x k row-major on device
+    DevBuf evecs;        // k columns of n on the device
 };
 
 // --------------------------------------------------------------------------

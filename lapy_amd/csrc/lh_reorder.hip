@@ -306,6 +306,43 @@ __global__ void k_unpermute_block(const double* __restrict__ in, int ldi, const 
     out[i * ldo + c] = in[(int64_t)iperm[i] * ldi + c];
 }
 
+// out[c * n + i] = in[src(i) * ldi + c], src = iperm or the identity: a tile of
+// 64 rows and 32 columns passes through LDS, so that reads run along the
+// block's rows (256 contiguous bytes) and writes along its columns (512).  The
+// row stride of 65 keeps both sides free of repeated bank conflicts.  Bound by
+// HBM: it moves the block once each way, with the unpermutation that a
+// row-major result needs as well.
+__global__ void __launch_bounds__(256)
+k_columns_out(const double* __restrict__ in, int ldi, const int32_t* __restrict__ iperm, double* __restrict__ out,
+              int64_t n, int m) {
+    __shared__ double tile[32][65];
+    const int64_t r0 = (int64_t)blockIdx.x * 64;
+    const int c0 = blockIdx.y * 32;
+    {
+        const int c = threadIdx.x & 31, rg = threadIdx.x >> 5;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int r = rg + 8 * q;
+            const int64_t i = r0 + r;
+            if (i < n && c0 + c < m) tile[c][r] = in[(int64_t)(iperm ? iperm[i] : i) * ldi + c0 + c];
+        }
+    }
+    __syncthreads();
+    const int r = threadIdx.x & 63, cg = threadIdx.x >> 6;
+    if (r0 + r >= n) return;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int c = cg + 4 * q;
+        if (c0 + c < m) out[(int64_t)(c0 + c) * n + r0 + r] = tile[c][r];
+    }
+}
+
+void columns_out(lh_ctx* ctx, const double* in, int ldi, const Reorder* ro, double* out, int64_t n, int m) {
+    k_columns_out<<<dim3(nblocks(n, 64), nblocks(m, 32)), 256, 0, ctx->stream>>>(
+        in, ldi, ro ? ro->iperm.as<int32_t>() : nullptr, out, n, m);
+    LH_CHECK_LAUNCH();
+}
+
 void Reorder::unpermute(lh_ctx* ctx, const double* in, int ldi, double* out, int ldo, int64_t n, int m) const {
     k_unpermute_block<<<nblocks(n * m, 256), 256, 0, ctx->stream>>>(in, ldi, iperm.as<int32_t>(), out, ldo, n, m);
     LH_CHECK_LAUNCH();
