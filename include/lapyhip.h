@@ -49,8 +49,8 @@ typedef struct lh_mpnn lh_mpnn;  /* learned preconditioner (weights on device) *
 typedef struct lh_stats {
     int32_t iterations;      /* outer iterations                              */
     int32_t converged;       /* number of converged wanted pairs / rhs        */
-    int32_t fallback_used;   /* 1 if the learned preconditioner or the linear
-                                solver's multigrid cycle was replaced         */
+    int32_t fallback_used;   /* 1 if the learned preconditioner or the
+                                multigrid cycle was replaced                  */
     int32_t precision_mode;  /* LH_PREC_*                                     */
     double  max_resid;       /* largest final relative residual               */
     double  t_setup_us;      /* host-measured phase times (microseconds)      */
@@ -65,8 +65,8 @@ typedef struct lh_stats {
     int32_t restarts;
     int32_t iterations_fp32; /* LH_PREC_MIXED: iterations of the FP32 phase
                                 (included in `iterations`)                    */
-    int32_t poly_columns;    /* eigensolver: block columns the Chebyshev
-                                polynomial ran on, summed over iterations
+    int32_t poly_columns;    /* eigensolver: block columns the multigrid cycles
+                                (the polynomial) ran on, summed over iterations
                                 (converged wanted pairs get plain Jacobi)     */
 } lh_stats;
 
@@ -77,7 +77,8 @@ typedef struct lh_stats {
                               falling or reach 1e-5, then FP64 iterations from
                               its X block to the requested tolerance        */
 
-#define LH_PRECOND_JACOBI  0   /* Jacobi with the automatic Chebyshev polynomial */
+#define LH_PRECOND_JACOBI  0   /* the built-in one: multigrid, Jacobi with a
+                                  Chebyshev polynomial, or Jacobi (poly_degree) */
 #define LH_PRECOND_LEARNED 1   /* the context's network (lh_ctx_set_mpnn)        */
 #define LH_PRECOND_NONE    2
 #define LH_PRECOND_AUTO    3   /* eigensolver: the network where the automatic
@@ -210,8 +211,12 @@ typedef struct lh_eig_opts {
     int32_t verbose;
     int32_t poly_degree;   /* with LH_PRECOND_JACOBI: degree of the Chebyshev
                               polynomial in D^-1 (A - sigma B) applied on top
-                              of Jacobi; 0: automatic (~sqrt(n)/6.3, at most
-                              128), 1: plain Jacobi                          */
+                              of Jacobi; 1: plain Jacobi; 0: automatic: two or
+                              three smoothed-aggregation multigrid cycles, and
+                              where those find no hierarchy, or have not
+                              converged after 80 iterations (fallback_used =
+                              1), the polynomial of degree ~sqrt(n)/6.3, at
+                              most 128                                       */
     double  poly_ratio;    /* Chebyshev interval [lmax/ratio, lmax]
                               (0: automatic, 2 * degree^2)                   */
     int32_t poly_storage;  /* LH_STORE_* for the Chebyshev work blocks        */

@@ -447,12 +447,13 @@ __global__ void k_amg_inverse(int n, const double* __restrict__ t, double* __res
 // fraction of the chip, all of it latency.
 
 // this lane's share of sum over row i of K of kv * f(column); W > 0: ELL rows
-// of W slots (G == 1)
-template <int W, int G, typename F>
-__device__ __forceinline__ double row_part(int64_t i, int lane, const int32_t* __restrict__ rp,
-                                           const int32_t* __restrict__ cl, const double* __restrict__ kv, F&& f) {
-    double a = 0.0;
+// of W slots (double, G == 1)
+template <int W, int G, typename T, typename F>
+__device__ __forceinline__ T row_part(int64_t i, int lane, const int32_t* __restrict__ rp,
+                                      const int32_t* __restrict__ cl, const T* __restrict__ kv, F&& f) {
+    T a = T(0);
     if constexpr (W > 0) {
+        static_assert(sizeof(T) == 8, "the block kernels have their own ELL rows");
 #pragma unroll
         for (int k0 = 0; k0 < W; k0 += 8) {
             const int4 ca = *reinterpret_cast<const int4*>(cl + i * W + k0);
@@ -474,7 +475,7 @@ __device__ __forceinline__ double row_part(int64_t i, int lane, const int32_t* _
         int32_t s = rp[i] + lane;
         const int32_t r1 = rp[i + 1];
         for (; s + 3 * G < r1; s += 4 * G) {
-            const double g0 = f(cl[s]), g1 = f(cl[s + G]), g2 = f(cl[s + 2 * G]), g3 = f(cl[s + 3 * G]);
+            const T g0 = f(cl[s]), g1 = f(cl[s + G]), g2 = f(cl[s + 2 * G]), g3 = f(cl[s + 3 * G]);
             a += kv[s] * g0;
             a += kv[s + G] * g1;
             a += kv[s + 2 * G] * g2;
@@ -485,10 +486,10 @@ __device__ __forceinline__ double row_part(int64_t i, int lane, const int32_t* _
     return a;
 }
 // the row's sum, in every one of its G lanes
-template <int W, int G, typename F>
-__device__ __forceinline__ double row_sum(int64_t i, int lane, const int32_t* __restrict__ rp,
-                                          const int32_t* __restrict__ cl, const double* __restrict__ kv, F&& f) {
-    double a = row_part<W, G>(i, lane, rp, cl, kv, f);
+template <int W, int G, typename T, typename F>
+__device__ __forceinline__ T row_sum(int64_t i, int lane, const int32_t* __restrict__ rp,
+                                     const int32_t* __restrict__ cl, const T* __restrict__ kv, F&& f) {
+    T a = row_part<W, G>(i, lane, rp, cl, kv, f);
 #pragma unroll
     for (int o = G / 2; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
     return a;
@@ -576,77 +577,80 @@ k_amg_transfer(int64_t n, int m, const int32_t* __restrict__ mp, const int32_t* 
 // the tail: every level from `first` on for one column per workgroup, the
 // vectors in LDS.  A level's vectors start at `off` (rows of the tail's
 // levels before it).
+template <typename T>
 struct TailLevel {
     int n, off;
     const int32_t *rp, *cl;
-    const double *kv, *dinv;
+    const T *kv, *dinv;
     const int32_t *pp, *pc, *tp, *tc;
-    const double *pv, *tv;
-    double s, c1, c2;
+    const T *pv, *tv;
+    T s, c1, c2;
 };
+template <typename T>
 struct TailDesc {
     int count;  // levels, the last one with the inverse
-    TailLevel lv[kMaxLevels];
-    const double* ginv;
+    TailLevel<T> lv[kMaxLevels];
+    const T* ginv;
 };
 constexpr int kTailThreads = 1024;
 
 // put(i, sum over row i of kv * v) for the rows of a CSR matrix, v in LDS,
 // four lanes a row
-template <typename P>
+template <typename T, typename P>
 __device__ __forceinline__ void tail_rows(int n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
-                                          const double* __restrict__ kv, const double* v, P&& put) {
+                                          const T* __restrict__ kv, const T* v, P&& put) {
     constexpr int G = 4;
     for (int t = threadIdx.x; t < n * G; t += kTailThreads) {
         const int i = t / G, lane = t % G;
-        const double a = row_sum<0, G>(i, lane, rp, cl, kv, [&](int32_t j) { return v[j]; });
+        const T a = row_sum<0, G>(i, lane, rp, cl, kv, [&](int32_t j) { return v[j]; });
         if (lane == 0) put(i, a);
     }
 }
 
+template <typename T>
 __global__ void __launch_bounds__(kTailThreads)
-k_amg_tail(int m, const TailDesc* __restrict__ desc, const double* __restrict__ b, double* __restrict__ x,
+k_amg_tail(int ld, const TailDesc<T>* __restrict__ desc, const T* __restrict__ b, T* __restrict__ x,
            const int* __restrict__ status) {
     if (status && status[0]) return;
-    __shared__ double sb[kTailSum], sx[kTailSum], sy[kTailSum];
-    __shared__ double red[kTailThreads];
+    __shared__ T sb[kTailSum], sx[kTailSum], sy[kTailSum];
+    __shared__ T red[kTailThreads];
     const int tid = threadIdx.x, col = blockIdx.x;
     const int count = desc->count;
     {
         const int n = desc->lv[0].n;
-        for (int i = tid; i < n; i += kTailThreads) sb[i] = b[(int64_t)i * m + col];
+        for (int i = tid; i < n; i += kTailThreads) sb[i] = b[(int64_t)i * ld + col];
     }
     __syncthreads();
     // down: smooth from zero, restrict the residual
     for (int l = 0; l + 1 < count; ++l) {
-        const TailLevel& lv = desc->lv[l];
-        const double* bl = sb + lv.off;
-        double* xl = sx + lv.off;
-        double* yl = sy + lv.off;
+        const TailLevel<T>& lv = desc->lv[l];
+        const T* bl = sb + lv.off;
+        T* xl = sx + lv.off;
+        T* yl = sy + lv.off;
         for (int i = tid; i < lv.n; i += kTailThreads) yl[i] = lv.s * lv.dinv[i] * bl[i];
         __syncthreads();
-        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, yl, [&](int i, double a) {
-            xl[i] = (1.0 + lv.c1) * yl[i] + lv.c2 * lv.dinv[i] * (bl[i] - a);
+        tail_rows<T>(lv.n, lv.rp, lv.cl, lv.kv, yl, [&](int i, T a) {
+            xl[i] = (T(1) + lv.c1) * yl[i] + lv.c2 * lv.dinv[i] * (bl[i] - a);
         });
         __syncthreads();
-        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, xl, [&](int i, double a) { yl[i] = bl[i] - a; });
+        tail_rows<T>(lv.n, lv.rp, lv.cl, lv.kv, xl, [&](int i, T a) { yl[i] = bl[i] - a; });
         __syncthreads();
-        const TailLevel& nx = desc->lv[l + 1];
-        tail_rows(nx.n, lv.tp, lv.tc, lv.tv, yl, [&](int i, double a) { sb[nx.off + i] = a; });
+        const TailLevel<T>& nx = desc->lv[l + 1];
+        tail_rows<T>(nx.n, lv.tp, lv.tc, lv.tv, yl, [&](int i, T a) { sb[nx.off + i] = a; });
         __syncthreads();
     }
     // the last level: x = K^-1 b, 8 threads a row
     {
-        const TailLevel& lv = desc->lv[count - 1];
+        const TailLevel<T>& lv = desc->lv[count - 1];
         const int n = lv.n;  // <= 128
         const int i = tid & 127, part = tid >> 7;
-        double a = 0.0;
+        T a = T(0);
         if (i < n)
             for (int k = part; k < n; k += kTailThreads / 128) a += desc->ginv[k * n + i] * sb[lv.off + k];
         red[tid] = a;
         __syncthreads();
         if (tid < n) {
-            double t = 0.0;
+            T t = T(0);
 #pragma unroll
             for (int p = 0; p < kTailThreads / 128; ++p) t += red[tid + 128 * p];
             sx[lv.off + tid] = t;
@@ -655,24 +659,183 @@ k_amg_tail(int m, const TailDesc* __restrict__ desc, const double* __restrict__ 
     }
     // up: correct, smooth
     for (int l = count - 2; l >= 0; --l) {
-        const TailLevel& lv = desc->lv[l];
-        const double* bl = sb + lv.off;
-        const double* xc = sx + desc->lv[l + 1].off;
-        double* xl = sx + lv.off;
-        double* yl = sy + lv.off;
+        const TailLevel<T>& lv = desc->lv[l];
+        const T* bl = sb + lv.off;
+        const T* xc = sx + desc->lv[l + 1].off;
+        T* xl = sx + lv.off;
+        T* yl = sy + lv.off;
         for (int i = tid; i < lv.n; i += kTailThreads)
             xl[i] += row_sum<0, 1>(i, 0, lv.pp, lv.pc, lv.pv, [&](int32_t j) { return xc[j]; });
         __syncthreads();
-        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, xl,
-                  [&](int i, double a) { yl[i] = xl[i] + lv.s * lv.dinv[i] * (bl[i] - a); });
+        tail_rows<T>(lv.n, lv.rp, lv.cl, lv.kv, xl,
+                     [&](int i, T a) { yl[i] = xl[i] + lv.s * lv.dinv[i] * (bl[i] - a); });
         __syncthreads();
-        tail_rows(lv.n, lv.rp, lv.cl, lv.kv, yl, [&](int i, double a) {
-            xl[i] = (1.0 + lv.c1) * yl[i] - lv.c1 * xl[i] + lv.c2 * lv.dinv[i] * (bl[i] - a);
+        tail_rows<T>(lv.n, lv.rp, lv.cl, lv.kv, yl, [&](int i, T a) {
+            xl[i] = (T(1) + lv.c1) * yl[i] - lv.c1 * xl[i] + lv.c2 * lv.dinv[i] * (bl[i] - a);
         });
         __syncthreads();
     }
     const int n = desc->lv[0].n;
-    for (int i = tid; i < n; i += kTailThreads) x[(int64_t)i * m + col] = sx[i];
+    for (int i = tid; i < n; i += kTailThreads) x[(int64_t)i * ld + col] = sx[i];
+}
+
+// ---- block cycle: FP32 blocks of the eigensolver ------------------------------
+// Rows of ld columns (ld a multiple of 4), LPR lanes of four columns a row, the
+// entries of a row taken four at a time so that four gathers are in flight;
+// E8: the finest level's ELL rows of 8 slots, staged in LDS by one coalesced
+// load of the workgroup.  Bound by HBM on the finest level (a block of 64
+// columns of 655,362 rows is 168 MB; the gathers of the locality-ordered rows
+// hit L2) and by launch latency on the others.
+enum { kBlkPre = 0, kBlkRes = 1, kBlkSt1 = 2, kBlkSt2 = 3, kBlkMix = 4 };
+
+__device__ __forceinline__ float4 f4mul(float w, const float4& a) {
+    return make_float4(w * a.x, w * a.y, w * a.z, w * a.w);
+}
+__device__ __forceinline__ void f4add(float4& y, float w, const float4& a) {
+    y.x += w * a.x;
+    y.y += w * a.y;
+    y.z += w * a.z;
+    y.w += w * a.w;
+}
+// sum over `len` entries (cols, vals) of vals * v[cols, c0 .. c0 + 3], times
+// dscale[col] when given; a partial last group repeats `self` with weight 0
+template <bool DS>
+__device__ __forceinline__ float4 blk_gather(const int32_t* cols, const float* vals, int len, int32_t self,
+                                             const float* __restrict__ dscale, const float* __restrict__ v, int ld,
+                                             int c0) {
+    float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), a1 = a0;
+    for (int s = 0; s < len; s += 4) {
+        int32_t j[4];
+        float w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool in = s + q < len;
+            j[q] = in ? cols[s + q] : self;
+            w[q] = in ? vals[s + q] : 0.f;
+            if (DS) w[q] *= dscale[j[q]];
+        }
+        float4 x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const float4*>(v + (int64_t)j[q] * ld + c0);
+        f4add(a0, w[0], x[0]);
+        f4add(a1, w[1], x[1]);
+        f4add(a0, w[2], x[2]);
+        f4add(a1, w[3], x[3]);
+    }
+    f4add(a0, 1.f, a1);
+    return a0;
+}
+
+// kBlkPre: out = w0 D^-1 b + g D^-1 (b - w1 K D^-1 b); kBlkRes: out = b - g K x;
+// kBlkMix: out = w0 out + w1 b - g K x;
+// kBlkSt1: out = x + g D^-1 (b - K x); kBlkSt2: out = w0 x + w1 out + g D^-1 (b - K x)
+template <int MODE, int LPR, bool E8>
+__global__ void __launch_bounds__(256)
+k_blk_step(int64_t n, int ld, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
+           const float* __restrict__ kv, const float* __restrict__ dinv, const float* __restrict__ b,
+           const float* __restrict__ x, float* __restrict__ out, float w0, float w1, float g) {
+    constexpr int kRows = 256 / LPR;
+    __shared__ __align__(16) int32_t s_cols[E8 ? kRows * 8 : 4];
+    __shared__ __align__(16) float s_kv[E8 ? kRows * 8 : 4];
+    const int64_t blk = xcd_block();
+    const int64_t row = (blk * 256 + threadIdx.x) / LPR;
+    if (E8) {
+        const int64_t base = blk * kRows * 8;
+        for (int t = threadIdx.x; t < kRows * 8; t += 256) {
+            const bool in = base + t < n * 8;
+            s_cols[t] = in ? cl[base + t] : 0;
+            s_kv[t] = in ? kv[base + t] : 0.f;
+        }
+        __syncthreads();
+    }
+    if (row >= n) return;
+    const int32_t r0 = E8 ? 0 : rp[row];
+    const int len = E8 ? 8 : rp[row + 1] - r0;
+    const int32_t* cols = E8 ? s_cols + (threadIdx.x / LPR) * 8 : cl + r0;
+    const float* vals = E8 ? s_kv + (threadIdx.x / LPR) * 8 : kv + r0;
+    const float di = dinv[row];
+    for (int c0 = (int)(threadIdx.x % LPR) * 4; c0 < ld; c0 += LPR * 4) {
+        const int64_t o = row * ld + c0;
+        const float4 bi = *reinterpret_cast<const float4*>(b + o);
+        float4 y;
+        if (MODE == kBlkPre) {
+            const float4 a = blk_gather<true>(cols, vals, len, (int32_t)row, dinv, b, ld, c0);
+            y = f4mul(w0 * di + g * di, bi);
+            f4add(y, -g * di * w1, a);
+        } else {
+            const float4 a = blk_gather<false>(cols, vals, len, (int32_t)row, nullptr, x, ld, c0);
+            if (MODE == kBlkRes) {
+                y = bi;
+                f4add(y, -g, a);
+            } else if (MODE == kBlkMix) {
+                y = f4mul(w0, *reinterpret_cast<const float4*>(out + o));
+                f4add(y, w1, bi);
+                f4add(y, -g, a);
+            } else {
+                const float4 xi = *reinterpret_cast<const float4*>(x + o);
+                float4 r = bi;
+                f4add(r, -1.f, a);
+                if (MODE == kBlkSt1) {
+                    y = xi;
+                } else {
+                    y = f4mul(w0, xi);
+                    f4add(y, w1, *reinterpret_cast<const float4*>(out + o));
+                }
+                f4add(y, g * di, r);
+            }
+        }
+        *reinterpret_cast<float4*>(out + o) = y;
+    }
+}
+// out (+)= M in for the transfer operators
+template <bool ADD, int LPR>
+__global__ void __launch_bounds__(256)
+k_blk_transfer(int64_t n, int ld, const int32_t* __restrict__ mp, const int32_t* __restrict__ mc,
+               const float* __restrict__ mv, const float* __restrict__ in, float* __restrict__ out) {
+    const int64_t row = (xcd_block() * 256 + threadIdx.x) / LPR;
+    if (row >= n) return;
+    const int32_t r0 = mp[row];
+    const int len = mp[row + 1] - r0;
+    for (int c0 = (int)(threadIdx.x % LPR) * 4; c0 < ld; c0 += LPR * 4) {
+        const int64_t o = row * ld + c0;
+        float4 y = ADD ? *reinterpret_cast<const float4*>(out + o) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if (len > 0) f4add(y, 1.f, blk_gather<false>(mc + r0, mv + r0, len, mc[r0], nullptr, in, ld, c0));
+        *reinterpret_cast<float4*>(out + o) = y;
+    }
+}
+// b = W in FP32, columns m .. ld - 1 zero
+template <typename WT>
+__global__ void k_blk_in(int64_t n, int m, int ld, const WT* __restrict__ W, int ldw, float* __restrict__ b) {
+    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid >= n * ld) return;
+    const int64_t i = gid / ld;
+    const int c = (int)(gid - i * ld);
+    b[gid] = c < m ? (float)W[i * ldw + c] : 0.f;
+}
+// W = w1 x1 + w2 x2 (+ w3 x3)
+template <typename WT>
+__global__ void k_blk_out(int64_t n, int m, int ld, const float* __restrict__ x1, const float* __restrict__ x2,
+                          const float* __restrict__ x3, double w1, double w2, double w3, WT* __restrict__ W, int ldw) {
+    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid >= n * m) return;
+    const int64_t i = gid / m;
+    const int c = (int)(gid - i * m);
+    const int64_t o = i * ld + c;
+    double v = w1 * (double)x1[o] + w2 * (double)x2[o];
+    if (x3) v += w3 * (double)x3[o];
+    W[i * ldw + c] = (WT)v;
+}
+__global__ void k_narrow(int64_t cnt, const double* __restrict__ s, float* __restrict__ d) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < cnt) d[i] = (float)s[i];
+}
+// K's values in the slots of an ELL copy of its pattern (padding: 0)
+__global__ void k_amg_ell(int64_t n, int W, const int32_t* __restrict__ rp, const double* __restrict__ kv,
+                          float* __restrict__ ekv) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int32_t r0 = rp[i], len = rp[i + 1] - r0;
+    for (int q = 0; q < W; ++q) ekv[i * W + q] = q < len ? (float)kv[r0 + q] : 0.f;
 }
 
 __global__ void k_fill_one(int64_t n, const double* __restrict__ dinv, double* __restrict__ x) {
@@ -735,7 +898,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         if (l == 0 && ell_w) {
             lv.W = ell_w;
             lv.ecl = ecl;
-            lv.d.kv = ekv;
+            lv.ekv = ekv;
         }
         const unsigned nb = nblocks(n, 256), nbx = nblocks_xcd(n, 256);
         k_amg_diag<<<nb, 256, 0, st>>>(n, rp, cl, kv, dinv, x.as<double>(), bad);
@@ -905,41 +1068,48 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
     const int last = (int)levels.size() - 1;
     tail = last;
     int64_t sum = levels[last].n;
-    while (tail > 1 && levels[tail - 1].n <= kTailRows && levels[tail - 1].nnz <= kTailNnz &&
+    while (tail > 0 && levels[tail - 1].n <= kTailRows && levels[tail - 1].nnz <= kTailNnz &&
            sum + levels[tail - 1].n <= kTailSum)
         sum += levels[--tail].n;
-    TailDesc d{};
+    return true;
+}
+
+template <typename T>
+void Amg::describe_tail(const T* inverse) {
+    const int last = (int)levels.size() - 1;
+    TailDesc<T> d{};
     d.count = last - tail + 1;
-    d.ginv = ginv.as<double>();
+    d.ginv = inverse;
     int off = 0;
     for (int l = tail; l <= last; ++l) {
         const AmgLevel& lv = levels[l];
-        TailLevel& t = d.lv[l - tail];
+        const AmgOps<T>& o = lv.ops(T());
+        TailLevel<T>& t = d.lv[l - tail];
         t.n = (int)lv.n;
         t.off = off;
         off += (int)lv.n;
         t.rp = lv.rp;
         t.cl = lv.cl;
-        t.kv = lv.d.kv;
-        t.dinv = lv.d.dinv;
+        t.kv = o.kv;
+        t.dinv = o.dinv;
         t.pp = lv.pp;
         t.pc = lv.pc;
-        t.pv = lv.d.pv;
+        t.pv = o.pv;
         t.tp = lv.tp;
         t.tc = lv.tc;
-        t.tv = lv.d.rv;
+        t.tv = o.rv;
         const Cheb2 k = cheb2(lv.bmax);
-        t.s = k.s;
-        t.c1 = k.c1;
-        t.c2 = k.c2;
+        t.s = (T)k.s;
+        t.c1 = (T)k.c1;
+        t.c2 = (T)k.c2;
     }
-    tail_desc.alloc(sizeof(TailDesc));
-    h2d(ctx, tail_desc.p, &d, sizeof(TailDesc));
-    return true;
+    tail_desc.alloc(sizeof(TailDesc<T>));
+    h2d(ctx, tail_desc.p, &d, sizeof(d));
 }
 
 void Amg::prepare(int m_) {
     m = m_;
+    describe_tail<double>(ginv.as<double>());
     size_t total = 0;
     for (int l = 0; l <= tail; ++l) total += 4 * (size_t)levels[l].n * m;
     work.alloc(total * 8);
@@ -979,12 +1149,26 @@ void with_lanes(int g, F&& f) {
     }
 }
 
+// lanes of four columns for a block row
+template <typename F>
+void with_row_lanes(int lpr, F&& f) {
+    switch (lpr) {
+        case 1: f(IntC<1>{}); break;
+        case 2: f(IntC<2>{}); break;
+        case 4: f(IntC<4>{}); break;
+        case 8: f(IntC<8>{}); break;
+        case 16: f(IntC<16>{}); break;
+        case 32: f(IntC<32>{}); break;
+        default: f(IntC<64>{}); break;
+    }
+}
+
 }  // namespace
 
 void Amg::cycle(int l, const double* b, double* x, double* part, const int* status) {
     hipStream_t st = ctx->stream;
     if (l == tail) {
-        k_amg_tail<<<(unsigned)m, kTailThreads, 0, st>>>(m, tail_desc.as<TailDesc>(), b, x, status);
+        k_amg_tail<double><<<(unsigned)m, kTailThreads, 0, st>>>(m, tail_desc.as<TailDesc<double>>(), b, x, status);
         LH_CHECK_LAUNCH();
         return;
     }
@@ -994,6 +1178,7 @@ void Amg::cycle(int l, const double* b, double* x, double* part, const int* stat
     const int gk = lv.W ? 1 : lanes_for(lv.nnz, lv.n);
     const unsigned nk = nblocks_xcd(lv.n * m * gk, 256);
     const int32_t* cl = lv.W ? lv.ecl : lv.cl;
+    const double* kv = lv.W ? lv.ekv : lv.d.kv;
     // f(W, G) with the level's slots per row and lanes per row
     auto with_k = [&](auto&& f) {
         switch (lv.W) {
@@ -1006,10 +1191,10 @@ void Amg::cycle(int l, const double* b, double* x, double* part, const int* stat
         LH_CHECK_LAUNCH();
     };
     with_k([&](auto w, auto g) {
-        k_amg_pre<w.v, g.v><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, x, k.s, k.c1, k.c2, status);
+        k_amg_pre<w.v, g.v><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, kv, lv.d.dinv, b, x, k.s, k.c1, k.c2, status);
     });
     with_k([&](auto w, auto g) {
-        k_amg_step<w.v, g.v, 0><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, x, r, 0.0, 0.0, 0.0,
+        k_amg_step<w.v, g.v, 0><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, kv, lv.d.dinv, b, x, r, 0.0, 0.0, 0.0,
                                                     nullptr, status);
     });
     const int gt = lanes_for(lv.pnnz, lv.nc), gp = lanes_for(lv.pnnz, lv.n);
@@ -1025,27 +1210,172 @@ void Amg::cycle(int l, const double* b, double* x, double* part, const int* stat
     });
     LH_CHECK_LAUNCH();
     with_k([&](auto w, auto g) {
-        k_amg_step<w.v, g.v, 1><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, x, y, 0.0, 0.0, k.s,
+        k_amg_step<w.v, g.v, 1><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, kv, lv.d.dinv, b, x, y, 0.0, 0.0, k.s,
                                                     nullptr, status);
     });
     if (part)
         with_k([&](auto w, auto g) {
-            k_amg_step<w.v, g.v, 3><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, y, x, 1.0 + k.c1,
+            k_amg_step<w.v, g.v, 3><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, kv, lv.d.dinv, b, y, x, 1.0 + k.c1,
                                                         -k.c1, k.c2, part, status);
         });
     else
         with_k([&](auto w, auto g) {
-            k_amg_step<w.v, g.v, 2><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, lv.d.kv, lv.d.dinv, b, y, x, 1.0 + k.c1,
+            k_amg_step<w.v, g.v, 2><<<nk, 256, 0, st>>>(lv.n, m, lv.rp, cl, kv, lv.d.dinv, b, y, x, 1.0 + k.c1,
                                                         -k.c1, k.c2, nullptr, status);
         });
 }
 
 int Amg::dot_blocks() const {
-    if (m > 4) return 0;
+    if (m > 4 || tail == 0) return 0;
     const AmgLevel& lv = levels[0];
     return (int)nblocks_xcd(lv.n * m * (lv.W ? 1 : lanes_for(lv.nnz, lv.n)), 256);
 }
 
 void Amg::apply(const double* R, double* Z, double* part, const int* status) { cycle(0, R, Z, part, status); }
+
+// ---- blocks ---------------------------------------------------------------------
+// Two or three cycles combined by the Chebyshev iteration on [lo, kBlkHi], where
+// the eigenvalues of M K lie (at most 1; the smallest 0.4 to 0.6 on smooth
+// surfaces, 0.1 on rough ones).  With d_1 = x_1 / theta, x_1 = M b:
+//   d_k = p_k d_{k-1} + q_k x_k, z_k = z_{k-1} + d_k, x_k = M r_k, r_k = b - K z_{k-1},
+// where K x_1 = theta (b - r_2) spares r_3 one product.  The eigensolver then
+// needs about the iterations that the exact inverse of K would give it (50
+// pairs at 10,242 vertices: 18 with two cycles or the inverse, 24 with one
+// cycle, 21 with the Chebyshev-Jacobi polynomial of degree 16; 10 pairs: 14, 13, 21
+// and 24; on a surface with noise of two edge lengths 15 with three cycles, 14
+// with the inverse, 21 with two).  Three from kManyRows rows on, where an
+// iteration's other work is ten times a cycle's; two below, where a cycle is
+// launch latency and costs a seventh of an iteration.
+constexpr double kBlkHi = 1.02, kBlkLo2 = 0.35, kBlkLo3 = 0.2;
+constexpr int64_t kManyRows = 65536;
+
+void Amg::prepare_blocks(int m_, int ell_w, const int32_t* ecl) {
+    m = m_;
+    ld = (m + 3) / 4 * 4;
+    hipStream_t st = ctx->stream;
+    auto narrow = [&](const double* s, int64_t cnt) {
+        float* d = own<float>(cnt);
+        k_narrow<<<nblocks(std::max<int64_t>(cnt, 1), 256), 256, 0, st>>>(cnt, s, d);
+        LH_CHECK_LAUNCH();
+        return d;
+    };
+    const int last = (int)levels.size() - 1;
+    for (int l = 0; l <= last; ++l) {
+        AmgLevel& lv = levels[l];
+        lv.f.kv = narrow(lv.d.kv, lv.nnz);
+        lv.f.dinv = narrow(lv.d.dinv, lv.n);
+        if (l < last) {
+            lv.f.pv = narrow(lv.d.pv, lv.pnnz);
+            lv.f.rv = narrow(lv.d.rv, lv.pnnz);
+        }
+    }
+    AmgLevel& l0 = levels[0];
+    if (ell_w == 8 && tail > 0) {
+        float* e = own<float>((size_t)l0.n * 8);
+        k_amg_ell<<<nblocks(l0.n, 256), 256, 0, st>>>(l0.n, 8, l0.rp, l0.d.kv, e);
+        LH_CHECK_LAUNCH();
+        l0.W = 8;
+        l0.ecl = ecl;
+        l0.ekv32 = e;
+    }
+    describe_tail<float>(narrow(ginv.as<double>(), levels[last].n * levels[last].n));
+    cycles = l0.n >= kManyRows ? 3 : 2;
+    size_t total = cycles * (size_t)l0.n * ld;
+    for (int l = 0; l <= tail; ++l) total += (l == 0 || l < tail ? 4 : 2) * (size_t)levels[l].n * ld;
+    work.alloc(total * 4);
+    float* p = work.as<float>();
+    auto take = [&](int64_t n) {
+        float* q = p;
+        p += (size_t)n * ld;
+        return q;
+    };
+    bin = take(l0.n);
+    bx1 = take(l0.n);
+    if (cycles == 3) bx2 = take(l0.n);
+    for (int l = 0; l <= tail; ++l) {
+        fb.push_back(take(levels[l].n));
+        fx.push_back(take(levels[l].n));
+        if (l == 0 || l < tail) {
+            fy.push_back(take(levels[l].n));
+            fr.push_back(take(levels[l].n));
+        }
+    }
+}
+
+template <int MODE>
+void Amg::blk_step(int l, int w, const float* b, const float* x, float* out, float w0, float w1, float g) {
+    const AmgLevel& lv = levels[l];
+    const bool e8 = lv.W == 8 && lv.ekv32;
+    const int lpr = std::min(64, vec_lanes(w, 4));
+    const unsigned nb = nblocks_xcd(lv.n * lpr, 256);
+    const int32_t* cl = e8 ? lv.ecl : lv.cl;
+    const float* kv = e8 ? lv.ekv32 : lv.f.kv;
+    auto go = [&](auto L) {
+        if (e8)
+            k_blk_step<MODE, L.v, true><<<nb, 256, 0, ctx->stream>>>(lv.n, w, lv.rp, cl, kv, lv.f.dinv, b, x, out, w0,
+                                                                     w1, g);
+        else
+            k_blk_step<MODE, L.v, false><<<nb, 256, 0, ctx->stream>>>(lv.n, w, lv.rp, cl, kv, lv.f.dinv, b, x, out, w0,
+                                                                      w1, g);
+        LH_CHECK_LAUNCH();
+    };
+    with_row_lanes(lpr, go);
+}
+
+void Amg::cycle_blocks(int l, int w, const float* b, float* x) {
+    if (l == tail) {
+        k_amg_tail<float><<<(unsigned)w, kTailThreads, 0, ctx->stream>>>(w, tail_desc.as<TailDesc<float>>(), b, x,
+                                                                        nullptr);
+        LH_CHECK_LAUNCH();
+        return;
+    }
+    const AmgLevel& lv = levels[l];
+    const Cheb2 k = cheb2(lv.bmax);
+    const int lpr = std::min(64, vec_lanes(w, 4));
+    blk_step<kBlkPre>(l, w, b, nullptr, x, (float)((1.0 + k.c1) * k.s), (float)k.s, (float)k.c2);
+    blk_step<kBlkRes>(l, w, b, x, fr[l], 0.f, 0.f, 1.f);
+    with_row_lanes(lpr, [&](auto L) {
+        k_blk_transfer<false, L.v><<<nblocks_xcd(lv.nc * lpr, 256), 256, 0, ctx->stream>>>(lv.nc, w, lv.tp, lv.tc, lv.f.rv,
+                                                                                         fr[l], fb[l + 1]);
+    });
+    LH_CHECK_LAUNCH();
+    cycle_blocks(l + 1, w, fb[l + 1], fx[l + 1]);
+    with_row_lanes(lpr, [&](auto L) {
+        k_blk_transfer<true, L.v><<<nblocks_xcd(lv.n * lpr, 256), 256, 0, ctx->stream>>>(lv.n, w, lv.pp, lv.pc, lv.f.pv,
+                                                                                       fx[l + 1], x);
+    });
+    LH_CHECK_LAUNCH();
+    blk_step<kBlkSt1>(l, w, b, x, fy[l], 0.f, 0.f, (float)k.s);
+    blk_step<kBlkSt2>(l, w, b, fy[l], x, (float)(1.0 + k.c1), (float)-k.c1, (float)k.c2);
+}
+
+template <typename WT>
+void Amg::apply_blocks(WT* W, int ldw, int cols) {
+    if (cols > m) LH_THROW(LH_ERR_ARG, "multigrid block width %d exceeds %d", cols, m);
+    const int w = (cols + 3) / 4 * 4;
+    const int64_t n = levels[0].n;
+    const double lo = cycles == 3 ? kBlkLo3 : kBlkLo2;
+    const double th = 0.5 * (kBlkHi + lo), de = 0.5 * (kBlkHi - lo), sig = th / de;
+    const double rho1 = 1.0 / sig, rho2 = 1.0 / (2.0 * sig - rho1), rho3 = 1.0 / (2.0 * sig - rho2);
+    const double p2 = rho2 * rho1, q2 = 2.0 * rho2 / de, p3 = rho3 * rho2, q3 = 2.0 * rho3 / de;
+    k_blk_in<<<nblocks(n * w, 256), 256, 0, ctx->stream>>>(n, cols, w, W, ldw, bin);
+    LH_CHECK_LAUNCH();
+    cycle_blocks(0, w, bin, bx1);
+    blk_step<kBlkRes>(0, w, bin, bx1, fb[0], 0.f, 0.f, (float)(1.0 / th));
+    const unsigned nb = nblocks(n * cols, 256);
+    if (cycles == 2) {
+        cycle_blocks(0, w, fb[0], fx[0]);
+        k_blk_out<<<nb, 256, 0, ctx->stream>>>(n, cols, w, bx1, fx[0], nullptr, (1.0 + p2) / th, q2, 0.0, W, ldw);
+    } else {
+        cycle_blocks(0, w, fb[0], bx2);
+        blk_step<kBlkMix>(0, w, fb[0], bx2, bin, (float)-p2, (float)(1.0 + p2), (float)q2);  // r_3 over b
+        cycle_blocks(0, w, bin, fx[0]);
+        k_blk_out<<<nb, 256, 0, ctx->stream>>>(n, cols, w, bx1, bx2, fx[0], (1.0 + p2 + p3 * p2) / th,
+                                               (1.0 + p3) * q2, q3, W, ldw);
+    }
+    LH_CHECK_LAUNCH();
+}
+template void Amg::apply_blocks<double>(double*, int, int);
+template void Amg::apply_blocks<float>(float*, int, int);
 
 }  // namespace lh

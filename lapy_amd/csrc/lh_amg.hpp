@@ -1,5 +1,6 @@
 // Smoothed-aggregation multigrid (lh_amg.hip): the preconditioner of the
-// linear solves on large systems.
+// linear solves on large systems (FP64) and of the block eigensolver (FP32
+// blocks, as its Chebyshev polynomial's arithmetic).
 #pragma once
 #include "lh_dense.hpp"
 
@@ -18,14 +19,19 @@ struct AmgLevel {
     int64_t n = 0, nnz = 0;
     const int32_t* rp = nullptr;  // K: CSR
     const int32_t* cl = nullptr;
-    int W = 0;  // level 0 with an ELL copy: slots per row (columns at ecl); 0: CSR
+    int W = 0;  // level 0 with an ELL copy: slots per row; 0: CSR
     const int32_t* ecl = nullptr;
+    const double* ekv = nullptr;
+    const float* ekv32 = nullptr;
     double bmax = 2.0;  // upper end of the smoother's interval (estimate of lambda_max(D^-1 K))
     // transfer to the next level (absent on the last one)
     int64_t nc = 0, pnnz = 0;
     const int32_t *pp = nullptr, *pc = nullptr;  // P (n x nc), CSR
     const int32_t *tp = nullptr, *tc = nullptr;  // P^T (nc x n), CSR
     AmgOps<double> d;
+    AmgOps<float> f;  // the block cycle's
+    const AmgOps<double>& ops(double) const { return d; }
+    const AmgOps<float>& ops(float) const { return f; }
 };
 
 struct Amg {
@@ -44,6 +50,16 @@ struct Amg {
     void apply(const double* R, double* Z, double* part, const int* status);
     int dot_blocks() const;  // 0: more than four columns
 
+    // the block cycle for at most m columns: FP32 copies and work blocks.
+    // ell_w == 8: the columns of an ELL copy of the finest level's pattern
+    void prepare_blocks(int m, int ell_w, const int32_t* ecl);
+    // W (n x cols, leading dimension ldw) <- p(M K) M W, in FP32
+    template <typename WT>  // double or float
+    void apply_blocks(WT* W, int ldw, int cols);
+
+    // products with the finest K in one application: four a cycle, one between two
+    int block_products() const { return 5 * cycles - 1; }
+
     std::vector<AmgLevel> levels;
 
    private:
@@ -55,6 +71,13 @@ struct Amg {
     DevBuf work;
     DevBuf tail_desc;          // the tail's levels, for its kernel
     std::vector<double*> wb, wx, wy, wr;  // per level: right-hand side, iterate, second iterate, residual
+    int ld = 0;                // block cycle: columns rounded up to 4
+    int cycles = 2;            // combined in one application
+    float *bin = nullptr, *bx1 = nullptr, *bx2 = nullptr;
+    std::vector<float*> fb, fx, fy, fr;
+    template <typename T> void describe_tail(const T* inverse);
+    template <int MODE> void blk_step(int l, int w, const float* b, const float* x, float* out, float w0, float w1, float g);
+    void cycle_blocks(int l, int w, const float* b, float* x);
     template <typename X> X* own(size_t count);
     void cycle(int l, const double* b, double* x, double* part, const int* status);
 };

@@ -10,7 +10,9 @@
 //                    block (more accurate than the usual GEMM recurrences and
 //                    not slower: the SpMM reads the block once, a GEMM update
 //                    reads the 3m-wide S)
-//   W = D^-1 (AX - BX Theta),  D = diag(A - sigma*B)      (Jacobi)
+//   W = M (AX - BX Theta)  with M two or three multigrid cycles for K = A -
+//                    sigma*B (lh_amg.hip), nearly K^-1; or D^-1 and a
+//                    Chebyshev polynomial in D^-1 K, D = diag(K) (lh_poly.hip)
 //   W <- W - X (BX)^T W (twice),  Cholesky-QR in the B inner product
 //   P <- P - X (BX)^T P - W (BW)^T P,  Cholesky-QR (dropped on breakdown)
 //   Rayleigh-Ritz on span(S) with the one-workgroup FP64 solver (lh_rr.hip)
@@ -23,7 +25,7 @@
 //
 // Convergence: ||A x_j - theta_j B x_j||_2 / ||B x_j||_2 <= tol * scale_j with
 // scale_j = max(|theta_j|, 1e-2 * |theta_{k-1}|) for the k wanted columns.
-#include "lh_dense.hpp"
+#include "lh_amg.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -44,6 +46,9 @@ double now_us() {
 // the polynomial skips the wanted pairs whose relative residual is at most
 // this many times the tolerance (they keep a plain Jacobi direction)
 constexpr double kPolyLockFactor = 1.0;
+// iterations with the multigrid cycle before the polynomial takes over (13 to
+// 25 are usual)
+constexpr int kAmgMaxIters = 80;
 
 // T: the block type.  double for the FP64 solve; float for the first phase
 // of the mixed-precision solve (FP32 blocks, FP32 SpMM, FP32 matrix-core
@@ -75,6 +80,11 @@ struct Lobpcg {
     ChebPrecond own_cheb;
     ChebPrecond* cheb = &own_cheb;  // a second phase shares the first one's
     bool cheb_ready = false;
+    bool use_amg = false;  // the multigrid cycle; the polynomial (or Jacobi) where it finds no hierarchy
+    Amg own_amg;
+    Amg* amg = &own_amg;   // a second phase shares the first one's
+    bool amg_ready = false;
+    DevBuf kshift;         // K = A - sigma B, what the cycle is built from
     // locality reordering (solver-internal)
     std::shared_ptr<Reorder> ro;      // the pattern's (kept with it)
     const Reorder* ext_ro = nullptr;  // a second phase's: the first phase's order
@@ -256,7 +266,18 @@ struct Lobpcg {
         res.assign(m, 0.0);
         HIPX(hipMemsetAsync(S.p, 0, n * ld * sizeof(T), ctx->stream));
         jacobi_diag(ctx, A, B, -sigma, 1.0, dinv.as<double>());
-        if (poly_degree > 1 && !cheb_ready) cheb->setup(ctx, A, B, sigma, poly_degree, poly_ratio, n, m, poly_half);
+        auto set_polynomial = [&]() {
+            if (poly_degree > 1 && !cheb_ready) cheb->setup(ctx, A, B, sigma, poly_degree, poly_ratio, n, m, poly_half);
+        };
+        bool amg_on = use_amg;
+        if (amg_on && !amg_ready) {
+            form_shifted(ctx, A, B, -sigma, 1.0, kshift);
+            amg_on = amg->setup(ctx, n, A->nnz(), A->pat->rowptr.as<int32_t>(), A->pat->cols.as<int32_t>(),
+                                kshift.as<double>(), 0, nullptr, nullptr);
+            if (amg_on) amg->prepare_blocks(m, ell.W, ell.cols.as<int32_t>());
+            amg_ready = amg_on;
+        }
+        if (!amg_on) set_polynomial();
         bool learned_on = false;
         if (precond == LH_PRECOND_LEARNED) {
             learned.setup(ctx, ctx->mpnn, A, B, -sigma, 1.0);  // K = A - sigma B
@@ -340,15 +361,22 @@ struct Lobpcg {
                 gm_hist.push_back(std::exp(lg / k));
                 if (it >= kMinFp32Iters && gm_hist[it] > 0.55 * gm_hist[it - 1]) break;
             }
+            // an operator that the cycle does not suit
+            if (amg_on && it >= kAmgMaxIters) {
+                amg_on = false;
+                st.fallback_used = 1;
+                set_polynomial();
+                if (verbose) fprintf(stderr, "[lobpcg] it %d: multigrid -> polynomial\n", it);
+            }
             // precondition W
             if (learned_on) {
                 learned.apply(Sp() + m, ld, m);
-            } else if (poly_degree > 1) {
-                // soft locking of the polynomial: the wanted pairs that pass
-                // the convergence test keep a plain Jacobi direction in W;
-                // the others and the guard columns k..m-1, gathered in front
-                // of W (ma of them, rounded up to 8), get the polynomial,
-                // when that saves 8 columns or more.  The order of W's
+            } else if (amg_on || poly_degree > 1) {
+                // soft locking of the cycle (the polynomial): the wanted pairs
+                // that pass the convergence test keep a plain Jacobi direction
+                // in W; the others and the guard columns k..m-1, gathered in
+                // front of W (ma of them, rounded up to 8), get the cycle, when
+                // that saves 8 columns or more.  The order of W's
                 // columns does not matter to the Rayleigh-Ritz step.
                 perm.clear();
                 for (int j = 0; j < m; ++j)
@@ -370,14 +398,16 @@ struct Lobpcg {
                     gather_cols<T>(ctx, n, m, W, ld, tmp, ld,
                                    reinterpret_cast<const int32_t*>(lockbuf.as<char>() + (size_t)m * 8));
                     copy_block<T, T>(ctx, n, m, tmp, ld, W, ld);
-                    cheb->apply(W, ld, ma, lockbuf.as<double>());
+                    if (amg_on) amg->apply_blocks<T>(W, ld, ma);
+                    else cheb->apply(W, ld, ma, lockbuf.as<double>());
                     rowscale<T>(ctx, n, m - ma, W + ma, ld, dinv.as<double>());
                     st.poly_columns += ma;
                 } else {
-                    cheb->apply(Sp() + m, ld, m, cs1.as<double>());  // cs1: ||w_c||^2 from the test above
+                    if (amg_on) amg->apply_blocks<T>(Sp() + m, ld, m);
+                    else cheb->apply(Sp() + m, ld, m, cs1.as<double>());  // cs1: ||w_c||^2 from the test above
                     st.poly_columns += m;
                 }
-                st.spmm_calls += poly_degree - 1;
+                st.spmm_calls += amg_on ? amg->block_products() : poly_degree - 1;
             } else if (precond != LH_PRECOND_NONE) {
                 rowscale<T>(ctx, n, m, Sp() + m, ld, dinv.as<double>());
             }
@@ -538,7 +568,12 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
     L.max_iter = (opts && opts->max_iter > 0) ? opts->max_iter : 20000;
     L.seed = opts ? opts->seed : 0;
     L.verbose = opts ? opts->verbose : 0;
-    // preconditioner: Jacobi, accelerated by a Chebyshev polynomial on
+    // preconditioner: by default the multigrid cycles.  Against the automatic
+    // polynomial, iterations and device time of a solve: 642 vertices, 10 pairs
+    // 21 -> 13, 8.4 -> 5.4 ms; 10,242, 10 pairs 27 -> 15, 13.7 -> 8.7; 29,000,
+    // 50 pairs 20 -> 19, 42.9 -> 41.0; 655,362, 50 pairs 25 -> 22, 402 -> 242
+    // (the polynomial's 128 products an iteration against 14 with FP32
+    // blocks).  Otherwise: Jacobi, accelerated by a Chebyshev polynomial on
     // [lmax / (2 d^2), lmax] whose degree d grows with sqrt(n) (the condition
     // number of a mesh Laplacian grows like n^(2/dim)) until the iteration
     // count stops falling (128 at 655k vertices: beyond it the block's own
@@ -560,6 +595,7 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
     L.no_fallback = opts && opts->no_fallback;
     const bool jac = pc == LH_PRECOND_JACOBI;
     int deg = opts ? opts->poly_degree : 0;
+    L.use_amg = jac && deg <= 0;
     if (!jac) deg = 1;
     if (deg <= 0) deg = auto_deg < 4 ? 1 : auto_deg;
     deg = std::max(1, std::min(deg, 1024));
@@ -602,6 +638,7 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
         L1.poly_degree = L.poly_degree;
         L1.poly_ratio = L.poly_ratio;
         L1.poly_half = L.poly_half;
+        L1.use_amg = L.use_amg;
         L1.phase_one = true;
         L1.run(nullptr, nullptr);
         DevBuf X0((size_t)n * m * 8);
@@ -611,6 +648,9 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
         L.ext_ro = L1.reordered ? L1.ro.get() : nullptr;
         L.cheb = L1.cheb;
         L.cheb_ready = L.poly_degree > 1;
+        L.amg = L1.amg;
+        L.amg_ready = L1.amg_ready;
+        L.use_amg = L1.amg_ready;
         L.x0 = X0.as<double>();
         L.x0_ld = m;
         L.max_iter = std::max(1, L.max_iter - L1.st.iterations);

@@ -13,7 +13,6 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("level,keep,k", [
-    (2, 1.0, 1),     # 162 rows: the dense path, one column
     (3, 1.0, 31),    # 642 rows: the caller's order, below one tile of columns
     (3, 0.61, 33),   # an odd number of rows, one column into the second tile
     (5, 0.413, 32),  # above 4,096 rows: the locality order undone

@@ -123,3 +123,48 @@ def test_rows_with_many_entries():
     x, st = _lib.pcg(ctx, _lib.DeviceCSR.from_scipy(ctx, a), None, 0.0, 1.0, b, rtol=1e-12)
     print("iterations", st.iterations, "longest row", np.diff(a.indptr).max())
     assert np.linalg.norm(b - a @ x) <= 1e-11 * np.linalg.norm(b)
+
+
+def _eig_problem(name):
+    if name == "tail":  # 642 rows: every level in the one-launch tail
+        return Solver(TriaMesh(*meshgen.perturbed_sphere(3, np.random.default_rng(1), axes=(1.3, 0.8, 1.0), sigma=0.02)))
+    if name == "one level":  # 2,562 rows: the finest level launched, lumped mass
+        return Solver(TriaMesh(*meshgen.perturbed_sphere(4, np.random.default_rng(2), axes=(1.3, 0.8, 1.0), sigma=0.05)),
+                      lump=True)
+    if name == "cap":  # odd rows, the locality order, 8 slots a row
+        return Solver(TriaMesh(*_cap(5, 0.43)))
+    return Solver(TetMesh(*meshgen.tet_cube(17, jitter=0.15)))  # 5,832 rows of ~15 entries
+
+
+@pytest.mark.parametrize("name,k,block", [("tail", 5, 0), ("tail", 10, 13), ("one level", 9, 18), ("one level", 33, 0),
+                                          ("cap", 3, 7), ("cap", 40, 66), ("tets", 12, 0)])
+def test_eigenpairs_with_the_block_cycle(name, k, block):
+    """Widths that are no multiples of the four columns a lane holds, one
+    lane to more than 16 lanes a row, each kind of finest level.  Held to the
+    solver's own bar: residuals of 1e-9 (ten times that for the host's
+    rounding), eigenvalues within 1e-10 of scipy's (their error is the
+    residual's square), B-orthonormal to 1e-9."""
+    from oracle import fem as ofem
+
+    fem = _eig_problem(name)
+    lam, x = fem.eigs(k=k, block=block)
+    st = fem.last_stats
+    print(name, x.shape, "block", block, "iterations", st.iterations)
+    assert st.fallback_used == 0 and st.iterations <= 60
+    a, b = fem.stiffness, fem.mass
+    bx = b @ x
+    res = np.linalg.norm(a @ x - bx * lam, axis=0) / np.linalg.norm(bx, axis=0)
+    assert np.all(res <= 1e-8 * np.maximum(np.abs(lam), 1e-2 * lam[-1]))
+    assert np.abs(x.T @ bx - np.eye(k)).max() <= 1e-9
+    lo = ofem.eigs(a, b, k=k)[0]
+    assert np.all(np.abs(lam - lo) <= 1e-10 * lo[-1])
+
+
+def test_eigenpairs_the_same_with_and_without_the_cycle():
+    """The mixed-precision solve shares one hierarchy between its phases; an
+    explicit degree keeps the polynomial."""
+    fem = _eig_problem("cap")
+    lam, _ = fem.eigs(k=12)
+    for opts in ({"precision": "mixed"}, {"poly_degree": 11}, {"poly_degree": 1}):
+        other, _ = fem.eigs(k=12, **opts)
+        assert np.all(np.abs(other - lam) <= 1e-10 * lam[-1])
