@@ -428,44 +428,146 @@ void rr_solve(lh_ctx* ctx, int N, int nev, double* GA, double* GM, double* C, do
 // T with T^T G T = I for a small SPD Gram G (m x m, m <= 128): G is
 // equilibrated to unit diagonal (D G D), optionally shifted, and T = D U
 // with U upper triangular and U^T G_s U = I, the inverse of G_s's Cholesky
-// factor transposed.  U comes from symmetric elimination on [G_s | I]:
-// step j takes the pivot p = S_jj of the Schur complement S (the square of
-// the Cholesky factor's diagonal), subtracts r r^T / p from S (r = row j of
-// S, zero at indices <= j) and U[:, j] r^T / p from U, and scales column j
-// of U by 1 / sqrt(p) at the end (Gram-Schmidt of the unit vectors in the
-// G_s inner product).  S and U live in registers: 512 threads form 16
-// half-waves, thread (hw, ln) holding entries [hw + 16a][ln + 32b].  Columns
-// are eliminated in pairs: rows j, j + 1 of S and columns j, j + 1 of U are
-// published to LDS, double-buffered by the pair's parity, so one barrier per
-// two columns suffices.  status 1 on a non-positive diagonal
-// or a pivot <= 1e-12 (reported in ((double*)status)[1]); otherwise the
-// smallest pivot is reported there (below 1e-2 the caller repeats the pass).
+// factor transposed.  U comes from elimination on [G_s | I] in place: step j
+// takes the pivot p = S_jj of the Schur complement S (the square of the
+// Cholesky factor's diagonal) and f = (row j of S beyond column j) / p, and
+// subtracts (column j) f from every other row: from the rows beyond j, which
+// still hold S, and from the rows before it, which hold U; row j itself, a
+// unit vector of U, becomes -f.  Column j of U is scaled by 1 / sqrt(p) at the
+// end.  One matrix serves both, since row i needs S while i > j and U after.
+// It lives in registers: 512 threads form 16 half-waves, thread (hw, ln)
+// holding entries [hw + 16a][ln + 32b].  Columns are eliminated in pairs; the
+// next pair's rows and columns are left in LDS by their owners right after
+// the update, double-buffered by the pair's parity: one barrier per two
+// columns.  The pairs of 32 columns form a phase compiled for the register
+// columns that are left.  Bound by the pair's dependent chain (two reciprocals,
+// LDS, barrier): with S and U apart, dynamic column skips and selects over all
+// register rows a 128-column factor took 176 us, now 79.  status 1 on a non-positive
+// diagonal or a pivot <= 1e-12 (reported in ((double*)status)[1]); otherwise
+// the smallest pivot is reported there (below 1e-2 the caller repeats the pass).
 constexpr int CHOL_NT = 512;
+
+template <int CB>
+struct CholShared {
+    double dsc[32 * CB], piv[32 * CB];
+    double rbuf[2][2][32 * CB], cbuf[2][2][32 * CB];
+    int flag;
+};
+
+// rows and columns j, j + 1 (j even, j / 32 == P) into the buffers of parity par
+template <int CB, int P>
+__device__ __forceinline__ void chol_publish(int j, int par, const double (&A)[2 * CB][CB], CholShared<CB>& S) {
+    const int hw = threadIdx.x >> 5, ln = threadIdx.x & 31;
+    const int hr = hw - (j & 15), hc = ln - (j & 31);
+    if (hr == 0 || hr == 1) {
+        if (j & 16) {
+#pragma unroll
+            for (int b = P; b < CB; ++b) S.rbuf[par][hr][ln + 32 * b] = A[2 * P + 1][b];
+        } else {
+#pragma unroll
+            for (int b = P; b < CB; ++b) S.rbuf[par][hr][ln + 32 * b] = A[2 * P][b];
+        }
+    }
+    if (hc == 0 || hc == 1) {
+#pragma unroll
+        for (int a = 0; a < 2 * CB; ++a) S.cbuf[par][hc][hw + 16 * a] = A[a][P];
+    }
+}
+
+// the pairs of columns 32 P .. 32 P + 31; false on a small pivot (in S.piv[0])
+template <int CB, int P>
+__device__ __forceinline__ bool chol_phase(int m, double (&A)[2 * CB][CB], CholShared<CB>& S) {
+    constexpr int RA = 2 * CB;
+    const int hw = threadIdx.x >> 5, ln = threadIdx.x & 31;
+    const int jend = m < 32 * P + 32 ? m : 32 * P + 32;
+    for (int j = 32 * P; j < jend; j += 2) {
+        const int par = (j >> 1) & 1;
+        const double p1 = S.rbuf[par][0][j], r12 = S.rbuf[par][0][j + 1], r22 = S.rbuf[par][1][j + 1];
+        double fc1[CB], fc2[CB], q1[RA], q2[RA];
+#pragma unroll
+        for (int b = P; b < CB; ++b) {
+            fc1[b] = S.rbuf[par][0][ln + 32 * b];
+            fc2[b] = S.rbuf[par][1][ln + 32 * b];
+        }
+#pragma unroll
+        for (int a = 0; a < RA; ++a) {
+            q1[a] = S.cbuf[par][0][hw + 16 * a];
+            q2[a] = S.cbuf[par][1][hw + 16 * a];
+        }
+        // 1e-12 < p <= ~1 (unit diagonal): the short-latency reciprocals
+        const double ip1 = rcp_nr(p1);
+        const double f = r12 * ip1;
+        const double p2 = r22 - f * r12;
+        if (!(p1 > 1e-12) || !(p2 > 1e-12)) {  // uniform; an odd m's partner is the padding's pivot 1
+            __syncthreads();
+            if (threadIdx.x == 0) S.piv[0] = p1 > 1e-12 ? p2 : p1;
+            return false;
+        }
+        const double ip2 = rcp_nr(p2);
+        if (threadIdx.x == 0) {
+            S.piv[j] = p1;
+            S.piv[j + 1] = p2;
+        }
+#pragma unroll
+        for (int b = P; b < CB; ++b) {
+            const double r1 = fc1[b];
+            fc1[b] = r1 * ip1;
+            fc2[b] = (fc2[b] - f * r1) * ip2;
+            if (b == P) {  // finished columns
+                const int c = ln + 32 * P;
+                fc1[b] = c > j ? fc1[b] : 0.0;
+                fc2[b] = c > j + 1 ? fc2[b] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < RA; ++a) {
+            q2[a] -= f * q1[a];
+            double keep = 1.0;
+            if (a == 2 * P || a == 2 * P + 1) {  // may hold rows j, j + 1: unit vectors of U from here on
+                const int i = hw + 16 * a;
+                const bool one = i == j, two = i == j + 1;
+                q1[a] = one ? 1.0 : two ? 0.0 : q1[a];
+                q2[a] = one ? -f : two ? 1.0 : q2[a];
+                keep = (one || two) ? 0.0 : 1.0;
+            }
+#pragma unroll
+            for (int b = P; b < CB; ++b) {
+                const double v = (a == 2 * P || a == 2 * P + 1) ? keep * A[a][b] : A[a][b];
+                A[a][b] = v - (q1[a] * fc1[b] + q2[a] * fc2[b]);
+            }
+        }
+        const int jn = j + 2;
+        if (jn < m) {
+            if (P + 1 < CB && (jn & 31) == 0) chol_publish<CB, (P + 1 < CB ? P + 1 : P)>(jn, par ^ 1, A, S);
+            else chol_publish<CB, P>(jn, par ^ 1, A, S);
+        }
+        __syncthreads();
+    }
+    return true;
+}
 
 template <int CB>
 __global__ void __launch_bounds__(CHOL_NT) k_cholinv(int m, const double* __restrict__ G, double* __restrict__ T,
                                                      double shift, int* __restrict__ status) {
     constexpr int RA = 2 * CB;
-    __shared__ double dsc[kCholMax], piv[kCholMax + 1];
-    __shared__ double rbuf[2][2][32 * CB], ubuf[2][2][32 * CB];
-    __shared__ int flag[1];
+    __shared__ CholShared<CB> S;
     const int tid = threadIdx.x, hw = tid >> 5, ln = tid & 31;
-    if (tid == 0) flag[0] = 0;
+    if (tid == 0) S.flag = 0;
     __syncthreads();
     for (int i = tid; i < m; i += CHOL_NT) {
         const double d = G[i * m + i];
-        dsc[i] = d > 0.0 ? 1.0 / sqrt(d) : 0.0;
-        if (!(d > 0.0)) flag[0] = 1;
+        S.dsc[i] = d > 0.0 ? 1.0 / sqrt(d) : 0.0;
+        if (!(d > 0.0)) S.flag = 1;
     }
     __syncthreads();
-    if (flag[0]) {
+    if (S.flag) {
         if (tid == 0) status[0] = 1;
         return;
     }
-    // S and U padded to 32 CB with the identity: the padding has zero
-    // coupling, is never a pivot and stays unchanged, so no bounds tests
-    // are needed inside the elimination
-    double S[RA][CB], U[RA][CB];
+    // padded to 32 CB with the identity: the padding has zero coupling, is
+    // never a pivot (but as an odd m's partner) and stays unchanged, so no
+    // bounds tests are needed inside the elimination
+    double A[RA][CB];
 #pragma unroll
     for (int a = 0; a < RA; ++a) {
         const int i = hw + 16 * a;
@@ -473,116 +575,44 @@ __global__ void __launch_bounds__(CHOL_NT) k_cholinv(int m, const double* __rest
         for (int b = 0; b < CB; ++b) {
             const int c = ln + 32 * b;
             double v = (i == c) ? 1.0 : 0.0;
-            if (i < m && c < m && i != c) v = 0.5 * (G[i * m + c] + G[c * m + i]) * dsc[i] * dsc[c];
+            if (i < m && c < m && i != c) v = 0.5 * (G[i * m + c] + G[c * m + i]) * S.dsc[i] * S.dsc[c];
             if (i == c && i < m) v = 1.0 + shift;
-            S[a][b] = v;
-            U[a][b] = (i == c) ? 1.0 : 0.0;
+            A[a][b] = v;
         }
     }
-    // two columns per step (one barrier): rows j and j + 1 of S and columns j
-    // and j + 1 of U are published; every thread corrects row j + 1 for the
-    // elimination of column j itself (r2' = r2 - f r1, f = S[j][j+1] / p1)
-    // and applies both rank-1 updates.  An odd m pairs its last column with
-    // the identity padding (pivot 1, no coupling).
-    for (int j = 0; j < m; j += 2) {
-        const int par = (j >> 1) & 1;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int jr = j + h;
-            if (hw == (jr & 15)) {
-                const int aj = jr >> 4;
-#pragma unroll
-                for (int a = 0; a < RA; ++a)
-                    if (a == aj) {
-#pragma unroll
-                        for (int b = 0; b < CB; ++b) {
-                            const int c = ln + 32 * b;
-                            rbuf[par][h][c] = (c >= jr) ? S[a][b] : 0.0;
-                        }
-                    }
-            }
-            if (ln == (jr & 31)) {
-                const int bj = jr >> 5;
-#pragma unroll
-                for (int b = 0; b < CB; ++b)
-                    if (b == bj) {
-#pragma unroll
-                        for (int a = 0; a < RA; ++a) ubuf[par][h][hw + 16 * a] = U[a][b];  // zero below row jr
-                    }
-            }
-        }
-        __syncthreads();
-        const double p1 = rbuf[par][0][j];
-        if (!(p1 > 1e-12)) {  // uniform
-            if (tid == 0) {
-                status[0] = 1;
-                reinterpret_cast<double*>(status)[1] = p1;
-            }
-            return;
-        }
-        const double ip1 = rcp_nr(p1);  // 1e-12 < p <= ~1 (unit diagonal): the short-latency form
-        const double f = rbuf[par][0][j + 1] * ip1;
-        const double p2 = rbuf[par][1][j + 1] - f * rbuf[par][0][j + 1];
-        if (!(p2 > 1e-12)) {  // uniform
-            if (tid == 0) {
-                status[0] = 1;
-                reinterpret_cast<double*>(status)[1] = p2;
-            }
-            return;
-        }
-        const double ip2 = rcp_nr(p2);
-        if (tid == 0) {
-            piv[j] = p1;
-            piv[j + 1] = p2;
-        }
-        double fc1[CB], fc2[CB];
-#pragma unroll
-        for (int b = 0; b < CB; ++b) {
-            const int c = ln + 32 * b;
-            const double r1 = rbuf[par][0][c];
-            fc1[b] = (c > j) ? r1 * ip1 : 0.0;
-            fc2[b] = (c > j + 1) ? (rbuf[par][1][c] - f * r1) * ip2 : 0.0;
-        }
-        // S -= r1 fc1^T + r2' fc2^T, U -= u1 fc1^T + u2' fc2^T (r1 and r2' are
-        // zero at rows before j; rows j and j + 1 are finished); columns <= j
-        // have zero coefficients
-        const int b_lo = (j >= 31) ? (j - 31) / 32 + 1 : 0;
-#pragma unroll
-        for (int a = 0; a < RA; ++a) {
-            const int i = hw + 16 * a;
-            const double r1i = rbuf[par][0][i];
-            const double r2i = (i > j) ? rbuf[par][1][i] - f * r1i : 0.0;
-            const double u1i = ubuf[par][0][i];
-            const double u2i = ubuf[par][1][i] - f * u1i;
-#pragma unroll
-            for (int b = 0; b < CB; ++b) {
-                if (b < b_lo) continue;
-                S[a][b] -= r1i * fc1[b] + r2i * fc2[b];
-                U[a][b] -= u1i * fc1[b] + u2i * fc2[b];
-            }
-        }
-    }
+    chol_publish<CB, 0>(0, 0, A, S);
     __syncthreads();
+    bool ok = chol_phase<CB, 0>(m, A, S);
+    if constexpr (CB > 1) ok = ok && chol_phase<CB, 1>(m, A, S);
+    if constexpr (CB > 2) ok = ok && chol_phase<CB, 2>(m, A, S);
+    if constexpr (CB > 3) ok = ok && chol_phase<CB, 3>(m, A, S);
+    if (!ok) {  // uniform
+        if (tid == 0) {
+            status[0] = 1;
+            reinterpret_cast<double*>(status)[1] = S.piv[0];
+        }
+        return;
+    }
     double isq[CB];
 #pragma unroll
     for (int b = 0; b < CB; ++b) {
         const int c = ln + 32 * b;
-        isq[b] = (c < m) ? 1.0 / sqrt(piv[c]) : 0.0;
+        isq[b] = (c < m) ? 1.0 / sqrt(S.piv[c]) : 0.0;
     }
 #pragma unroll
     for (int a = 0; a < RA; ++a) {
         const int i = hw + 16 * a;
         if (i >= m) continue;
-        const double di = dsc[i];
+        const double di = S.dsc[i];
 #pragma unroll
         for (int b = 0; b < CB; ++b) {
             const int c = ln + 32 * b;
-            if (c < m) T[i * m + c] = (c >= i) ? di * U[a][b] * isq[b] : 0.0;
+            if (c < m) T[i * m + c] = (c > i) ? di * A[a][b] * isq[b] : (c == i) ? di * isq[b] : 0.0;
         }
     }
     if (tid < 64) {  // the smallest pivot (a running minimum in the loop costs registers)
         double mp = 1.0;
-        for (int j = tid; j < m; j += 64) mp = fmin(mp, piv[j]);
+        for (int j = tid; j < m; j += 64) mp = fmin(mp, S.piv[j]);
         for (int off = 32; off > 0; off >>= 1) mp = fmin(mp, __shfl_xor(mp, off, 64));
         if (tid == 0) {
             status[0] = 0;

@@ -34,8 +34,8 @@ __device__ __forceinline__ double sqrt_nr(double x) {
 // same two numbers).
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
 // over the 16 lanes of a DPP row
@@ -45,6 +45,23 @@ __device__ __forceinline__ double row_sum16(double v) {
     v += dpp_f64<0x141>(v);  // row_half_mirror: 7 - lane within 8
     v += dpp_f64<0x140>(v);  // row_mirror: 15 - lane within 16
     return v;
+}
+// the same for the elements from FROM on of an array, stage by stage, so that
+// the dependent stages of different elements overlap
+template <int FROM, int N>
+__device__ __forceinline__ void row_sum16_each(double (&v)[N]) {
+#define LH_STAGE(CTRL)                                          \
+    {                                                           \
+        double t[N];                                            \
+        _Pragma("unroll") for (int a = FROM; a < N; ++a) t[a] = dpp_f64<CTRL>(v[a]); \
+        _Pragma("unroll") for (int a = FROM; a < N; ++a) v[a] += t[a];               \
+        __builtin_amdgcn_sched_barrier(0);                      \
+    }
+    LH_STAGE(0xB1)
+    LH_STAGE(0x4E)
+    LH_STAGE(0x141)
+    LH_STAGE(0x140)
+#undef LH_STAGE
 }
 // over the 32 lanes of a half-wave
 __device__ __forceinline__ double half_sum32(double v) {
@@ -59,6 +76,22 @@ __device__ __forceinline__ double wave_sum64(double v) {
     const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
     const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
     return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+// three at once, stage by stage
+__device__ __forceinline__ void wave_sum64_each(double (&v)[3]) {
+    row_sum16_each<0>(v);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v[a]), __double2loint(v[a]), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v[a]), __double2hiint(v[a]), false, false);
+        v[a] = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v[a]), __double2loint(v[a]), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v[a]), __double2hiint(v[a]), false, false);
+        v[a] = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
 }
 
 // C (p x q, ldc, FP64) = alpha * U^T V over n rows; sym (p == q): the
@@ -86,8 +119,10 @@ size_t rr_work_doubles(int N, int nev);
 // standard symmetric Rayleigh-Ritz (orthonormal basis), LDS-resident, N <= kRRStdMaxN
 constexpr int kRRStdMaxN = 192;
 size_t rr_std_work_doubles(int N, int nev);
+// H is the mean of G and its transpose; mirrored: the two are the same bits
+// outside the diagonal tiles of 64, as gram() with sym leaves them
 void rr_std(lh_ctx* ctx, int N, int nev, const double* G, int ldg, double* C, double* theta, double* work,
-            int* status, unsigned long long* prof = nullptr);
+            int* status, unsigned long long* prof = nullptr, bool mirrored = false);
 void rr_solve(lh_ctx* ctx, int N, int nev, double* GA, double* GM, double* C, double* theta, double* work,
               int* status);
 // the same generalized problem through rocSOLVER (sygvd) for trial bases

@@ -10,18 +10,19 @@
 //     in global memory.
 //  2. k_rr_bisect (one wave per wanted eigenvalue): multisection on T scaled
 //     by a power of two to ||T|| <= 1, the 64 lanes evaluating Sturm counts
-//     at 64 interior points (65-fold bracket reduction per round).
+//     (sign changes of the leading minors) at 64 interior points (65-fold
+//     bracket reduction per round).
 //  3. k_rr_invit (one wave per eigenvalue; only the first of a group of
 //     numerically equal eigenvalues works): inverse iteration with the LU
 //     factors of T - lambda I (same scaling) in LDS, Gram-Schmidt inside the
 //     group.
 //  4. k_rr_back (one wave per eigenvector): Z := Q Y, the reflectors applied
-//     in reverse order, loaded four steps ahead into registers.
+//     in reverse order, two at a time, loaded eight pairs ahead into registers.
 //  5. k_rr_polish (one workgroup): Newton-Schulz orthonormalisation of Z in
 //     the small space, Z := Z (3 I - Z^T Z) / 2 (inverse iteration leaves
 //     orthogonality errors ~ eps ||T|| / gap; each step squares them; up to
 //     three steps, none for a basis with ||Z^T Z - I|| >= 1/2), its products
-//     in 4 x 4 register tiles from 32 columns up.
+//     on the matrix cores from 32 columns up.
 //
 // Replaces the dense Rayleigh-Ritz step ARPACK performs inside eigsh
 // (lapy/solver.py:713-715) for the block solver.
@@ -37,32 +38,23 @@ constexpr int NB = 1024;
 constexpr int NMAX = kRRStdMaxN;
 constexpr int PK = NMAX * (NMAX + 1) / 2;
 
-__device__ __forceinline__ int rowbase(int i) { return i * (i + 1) / 2; }
-
 __device__ __forceinline__ double wsum(double v) { return wave_sum64(v); }
-__device__ double bsum(double v, double* red) {
-    v = wsum(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < NB / 64; ++i) s += red[i];
-    return s;
-}
 
 __device__ __forceinline__ void stamp(unsigned long long* prof, int slot) {
     if (prof && threadIdx.x == 0 && blockIdx.x == 0) prof[slot] = wall_clock64();
 }
 
-// work layout (doubles): reflectors R[k][i] (N x N), d (N), e (N), tau (N),
+// work layout (doubles): reflectors R[k][i] (N rows of NP = N rounded up to 32,
+// entry i > k of reflector k in place), d (N), e (N), tau (N),
 // bounds (4: lo, hi, ||T||, -), lam (nev), Y (nev x N, column g contiguous),
 // Z (N x nev row-major)
+__host__ __device__ constexpr int rr_stride(int N) { return (N + 31) / 32 * 32; }
+
 struct RRWork {
     double *R, *d, *e, *tau, *bnd, *lam, *Y, *Z;
     __host__ __device__ RRWork(double* w, int N, int nev) {
         R = w;
-        d = R + (size_t)N * N;
+        d = R + (size_t)N * rr_stride(N);
         e = d + N;
         tau = e + N;
         bnd = tau + N;
@@ -72,77 +64,127 @@ struct RRWork {
     }
 };
 
-// number of eigenvalues of T below x (negative pivots of T - x I).  The
-// caller scales T so that ||T|| <= 1: the pivots then lie between pivmin and
-// ~1 / pivmin, where the short-latency reciprocal is accurate
-__device__ int sturm(const double* d, const double* e2, int N, double x, double pivmin) {
+// number of eigenvalues of T below x: sign changes of the leading principal
+// minors p_{i+1} = (d_i - x) p_i - e_{i-1}^2 p_{i-1}.  The caller scales T so
+// that ||T|| <= 1 and raises e^2 to 1e-60 at least, so that a vanishing minor
+// (which counts as positive) is followed by one of the sign that its
+// predecessor's asks for; the pair is rescaled by a power of two every 8 steps,
+// in which it changes by 1e-240 to 1e4 at most.  Three FP64 instructions and the
+// sign's three a step; the quotient form q_i = (d_i - x) - e^2 / q_{i-1}, whose
+// reciprocal alone is a chain of nine, took 89 us a call at N = 192 against
+// 43 us.  N8: N rounded up to 8; d is padded with 2 there (no x is above 1).
+__device__ int sturm(const double* d, const double* e2, int N8, double x) {
     int cnt = 0;
-    double q = d[0] - x;
-    if (fabs(q) < pivmin) q = -pivmin;
-    cnt += q < 0.0;
-    for (int i = 1; i < N; ++i) {
-        q = (d[i] - x) - e2[i - 1] * rcp_nr(q);
-        if (fabs(q) < pivmin) q = -pivmin;
-        cnt += q < 0.0;
+    double pm = 0.0, p = 1.0;
+    for (int i0 = 0; i0 < N8; i0 += 8) {
+        double dd[8], ee[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            dd[u] = d[i0 + u];
+            ee[u] = e2[i0 + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const double q = fma(dd[u] - x, p, -(ee[u] * pm));
+            pm = p;
+            p = q;
+            cnt += (int)((unsigned)(__double2hiint(p) ^ __double2hiint(pm)) >> 31);
+        }
+        const int ex = ilogb(fmax(fabs(p), fabs(pm)));  // never both 0
+        p = ldexp(p, -ex);
+        pm = ldexp(pm, -ex);
     }
     return cnt;
 }
 
-// LU with partial pivoting of T - lam I into ws (1/u0, u1, u2, l, piv: 5N).
-// The caller scales T to ||T|| <= 1, so the pivots (a zero or sub-normal one
-// replaced by tiny) have ordinary magnitudes and their reciprocals come from
-// the short-latency form, stored for the solves
+// LU with partial pivoting of T - lam I into ws (1/u0, u1, u2, l, swapped: 5
+// arrays of NMAX).  The caller scales T to ||T|| <= 1, so the pivots (a zero or
+// sub-normal one replaced by tiny) have ordinary magnitudes and their
+// reciprocals come from the short-latency form, stored for the solves.  Eight
+// steps' entries of T are loaded ahead of their use, and branches are selects:
+// a step is its reciprocal's dependent chain, without the LDS round trips that
+// a load behind a store has to wait for.  d and e are readable to N + 8.
+constexpr int TB = 8;
 __device__ void tri_factor(const double* d, const double* e, int N, double lam, double tiny, double* ws) {
     double* iu0 = ws;
-    double* u1 = ws + N;
-    double* u2 = ws + 2 * N;
-    double* lm = ws + 3 * N;
-    double* pv = ws + 4 * N;
-    double c0 = d[0] - lam, c1 = (N > 1) ? e[0] : 0.0, c2 = 0.0;
-    for (int i = 0; i < N - 1; ++i) {
-        const double sub = e[i];
-        const double a1 = d[i + 1] - lam;
-        const double b1 = (i + 1 < N - 1) ? e[i + 1] : 0.0;
-        if (fabs(c0) >= fabs(sub) || !(fabs(sub) > 1e-300)) {
-            const double piv = (fabs(c0) > 1e-300) ? c0 : tiny;
+    double* u1 = ws + NMAX;
+    double* u2 = ws + 2 * NMAX;
+    double* lm = ws + 3 * NMAX;
+    double* pv = ws + 4 * NMAX;
+    double c0 = d[0] - lam, c1 = (N > 1) ? e[0] : 0.0;
+    for (int i0 = 0; i0 < N - 1; i0 += TB) {
+        double dn[TB], en[TB + 1];
+#pragma unroll
+        for (int u = 0; u < TB; ++u) dn[u] = d[i0 + u + 1] - lam;
+#pragma unroll
+        for (int u = 0; u <= TB; ++u) en[u] = (i0 + u < N - 1) ? e[i0 + u] : 0.0;
+#pragma unroll
+        for (int u = 0; u < TB; ++u) {
+            const int i = i0 + u;
+            if (i >= N - 1) break;
+            const double sub = en[u], a1 = dn[u], b1 = en[u + 1];
+            const bool sw = !(fabs(c0) >= fabs(sub) || !(fabs(sub) > 1e-300));
+            const double piv = sw ? sub : (fabs(c0) > 1e-300) ? c0 : tiny;
             const double ip = rcp_nr(piv);
-            const double l = sub * ip;
-            iu0[i] = ip; u1[i] = c1; u2[i] = c2; lm[i] = l; pv[i] = 0.0;
-            c0 = a1 - l * c1;
-            c1 = b1 - l * c2;
-        } else {
-            const double ip = rcp_nr(sub);
-            const double l = c0 * ip;
-            iu0[i] = ip; u1[i] = a1; u2[i] = b1; lm[i] = l; pv[i] = 1.0;
-            c0 = c1 - l * a1;
-            c1 = c2 - l * b1;
+            const double l = (sw ? c0 : sub) * ip;
+            const double x1 = sw ? a1 : c1, x2 = sw ? b1 : 0.0, y0 = sw ? c1 : a1, y1 = sw ? 0.0 : b1;
+            iu0[i] = ip;
+            u1[i] = x1;
+            u2[i] = x2;
+            lm[i] = l;
+            pv[i] = sw ? 1.0 : 0.0;
+            c0 = y0 - l * x1;
+            c1 = y1 - l * x2;
         }
-        c2 = 0.0;
     }
     iu0[N - 1] = rcp_nr((fabs(c0) > tiny) ? c0 : tiny);
 }
 
-// solve with the factorisation; y overwritten
+// solve with the factorisation; y overwritten, loads eight steps at a time as
+// in the factorisation
 __device__ void tri_lu_solve(const double* ws, int N, double* y) {
     const double* iu0 = ws;
-    const double* u1 = ws + N;
-    const double* u2 = ws + 2 * N;
-    const double* lm = ws + 3 * N;
-    const double* pv = ws + 4 * N;
+    const double* u1 = ws + NMAX;
+    const double* u2 = ws + 2 * NMAX;
+    const double* lm = ws + 3 * NMAX;
+    const double* pv = ws + 4 * NMAX;
     double a = y[0];
-    for (int i = 0; i < N - 1; ++i) {
-        double b = y[i + 1];
-        if (pv[i] != 0.0) { double t = a; a = b; b = t; }
-        y[i] = a;
-        a = b - lm[i] * a;
+    for (int i0 = 0; i0 < N - 1; i0 += TB) {
+        double b[TB], l[TB], s[TB];
+#pragma unroll
+        for (int u = 0; u < TB; ++u) {  // entries from N on are not used
+            const int i = i0 + u < N - 1 ? i0 + u : N - 2;
+            b[u] = y[i + 1];
+            l[u] = lm[i];
+            s[u] = pv[i];
+        }
+#pragma unroll
+        for (int u = 0; u < TB; ++u) {
+            const int i = i0 + u;
+            if (i >= N - 1) break;
+            const bool sw = s[u] != 0.0;
+            const double hi = sw ? b[u] : a, lo = sw ? a : b[u];
+            y[i] = hi;
+            a = lo - l[u] * hi;
+        }
     }
-    double x2 = a * iu0[N - 1];
-    y[N - 1] = x2;
-    if (N >= 2) {
-        double x1 = (y[N - 2] - u1[N - 2] * x2) * iu0[N - 2];
-        y[N - 2] = x1;
-        for (int i = N - 3; i >= 0; --i) {
-            double x0 = (y[i] - u1[i] * x1 - u2[i] * x2) * iu0[i];
+    double x1 = a * iu0[N - 1], x2 = 0.0;
+    y[N - 1] = x1;
+    for (int i0 = N - 2; i0 >= 0; i0 -= TB) {
+        double r[TB], c1[TB], c2[TB], p[TB];
+#pragma unroll
+        for (int u = 0; u < TB; ++u) {
+            const int i = i0 - u > 0 ? i0 - u : 0;
+            r[u] = y[i];
+            c1[u] = u1[i];
+            c2[u] = u2[i];
+            p[u] = iu0[i];
+        }
+#pragma unroll
+        for (int u = 0; u < TB; ++u) {
+            const int i = i0 - u;
+            if (i < 0) break;
+            const double x0 = (r[u] - c2[u] * x2 - c1[u] * x1) * p[u];
             y[i] = x0;
             x2 = x1;
             x1 = x0;
@@ -155,32 +197,150 @@ __device__ void tri_lu_solve(const double* ws, int N, double* y) {
 // row each), and the thread (group g, lane l) holds H[g + 32a][l + 16b] for
 // a < CB, b < 2 CB (CB = ceil(N / 32)), a block-cyclic layout in which every
 // row is spread over the 16 lanes of one group, so that row sums are DPP
-// sums within a row.  Step k (Householder reflector of row k = column k
-// below the diagonal) costs two barriers:
-//  A. the group owning row k forms the norm of H[k][k+1:], alpha, v0 and
-//     tau, and publishes v (zero at indices <= k) to LDS and to global
-//     memory (barrier 1);
+// sums within a row; rows and columns from N on are zero and stay zero.  Step
+// k (Householder reflector of row k = column k below the diagonal) costs two
+// barriers:
+//  A. the row's owner has left it in LDS (barrier 1); every group forms the
+//     norm, alpha, v_0 and tau by itself, each lane keeping its columns of v;
 //  B. every thread multiplies its block by v; row sums give p = tau H v for
-//     the group's rows, which is published with the group's share of p . v
-//     (barrier 2);
-//  C. every thread forms K = tau (p . v) / 2 and w = p - K v and applies
-//     H -= v w^T + w v^T to its block in registers.
-// v, p and the shares of p . v are double-buffered by the parity of k, so
-// step k + 1 may overwrite nothing that a thread still reads from step k.
-// Rows and columns <= k are finished: p is zero there, so the update leaves
-// them unchanged, and register rows that lie wholly in them are skipped.
-// The step's critical path is the owning group's reflector (a norm, a square
-// root and a division in one wave, ~4,000 cycles), which the other waves
-// wait for at barrier 1.
+//     the group's rows, which is published (barrier 2);
+//  C. every thread forms K = tau (p . v) / 2 and w = p - K v, applies
+//     H -= v w^T + w v^T to its block in registers, and the owner of row
+//     k + 1 leaves it in LDS.
+// The row and p are double-buffered by the parity of k, so step k + 1
+// overwrites nothing that a thread still reads from step k.
+// Step k belongs to phase A0 = (k + 1) / 32, in which the register rows below
+// A0 and columns below 2 A0 are finished: the phases are compiled one by one,
+// so that their loops run over what is left (42 % of the block on average),
+// the next row is register row A0, and only the first two register columns
+// and the first register row need comparisons with k.
+// Bound by the dependent steps of a column (~2,000 cycles at small N, of which
+// LDS and the barriers take ~500, four row sums ~430 and the reflector's scalars
+// ~300) and, at N = 192, by the FP64 instructions of two waves a SIMD: 303 us a
+// call at N = 192, 44 at 48.  Forming the reflector in its owner alone, with
+// selects over all register rows and the store to global memory before the
+// barrier, took ~4,000 cycles in which the other waves waited: 690 and 71 us.
 constexpr int TRI_NT = 512;
 
 template <int CB>
+struct TriShared {
+    double xbuf[2][32 * CB], pbuf[2][32 * CB];
+    double sd[32 * CB], se[32 * CB], stau[32 * CB];
+};
+
+// steps k of phase A0, up to N - 3
+template <int CB, int A0>
+__device__ __forceinline__ void tri_phase(int N, double (&h)[CB][2 * CB], TriShared<CB>& S, double* __restrict__ R) {
+    constexpr int RA = CB, CC = 2 * CB, B0 = 2 * A0, NP = 32 * CB;
+    const int tid = threadIdx.x, g = tid >> 4, l = tid & 15;
+    const int kend = (N - 2 < 32 * A0 + 31) ? N - 2 : 32 * A0 + 31;
+    for (int k = (A0 == 0) ? 0 : 32 * A0 - 1; k < kend; ++k) {
+        const int par = k & 1;
+        // A. the reflector; k + 1 lies in register columns B0, B0 + 1
+        double v[CC], vr[RA];
+#pragma unroll
+        for (int b = B0; b < CC; ++b) v[b] = S.xbuf[par][l + 16 * b];
+        const double x0 = S.xbuf[par][k + 1];
+#pragma unroll
+        for (int a = A0; a < RA; ++a) vr[a] = S.xbuf[par][g + 32 * a];
+        double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+        for (int b = B0; b < CC; b += 2) {
+            if (b == B0) {
+                v[b] = (l + 16 * b <= k) ? 0.0 : v[b];
+                v[b + 1] = (l + 16 * (b + 1) <= k) ? 0.0 : v[b + 1];
+            }
+            s0 += v[b] * v[b];
+            s1 += v[b + 1] * v[b + 1];
+        }
+        const double xn2 = row_sum16(s0 + s1);
+        double alpha = 0.0, v0 = 0.0, t = 0.0;
+        if (xn2 != 0.0) {
+            // the short-latency forms on the step's critical path (the
+            // exact ones for extreme magnitudes; xn2 is the same in every
+            // lane, so one branch runs)
+            if (xn2 > 1e-280 && xn2 < 1e280) {
+                const double sq = sqrt_nr(xn2);
+                alpha = (x0 >= 0.0) ? -sq : sq;
+                v0 = x0 - alpha;
+                t = 2.0 * rcp_nr(xn2 - x0 * x0 + v0 * v0);
+            } else {
+                alpha = (x0 >= 0.0) ? -sqrt(xn2) : sqrt(xn2);
+                v0 = x0 - alpha;
+                t = 2.0 / (xn2 - x0 * x0 + v0 * v0);
+            }
+        }
+#pragma unroll
+        for (int b = B0; b < B0 + 2; ++b) v[b] = (l + 16 * b == k + 1) ? v0 : v[b];
+        {
+            const int i = g + 32 * A0;
+            vr[A0] = (i <= k) ? 0.0 : (i == k + 1) ? v0 : vr[A0];
+        }
+        // B. p = tau H v for this group's rows
+        double p[RA];
+#pragma unroll
+        for (int a = A0; a < RA; ++a) {
+            double q0 = 0.0, q1 = 0.0;
+#pragma unroll
+            for (int b = B0; b < CC; b += 2) {
+                q0 += h[a][b] * v[b];
+                q1 += h[a][b + 1] * v[b + 1];
+            }
+            p[a] = q0 + q1;
+        }
+        row_sum16_each<A0>(p);
+#pragma unroll
+        for (int a = A0; a < RA; ++a) p[a] *= t;
+        if (g + 32 * A0 <= k) p[A0] = 0.0;
+        {
+            double mine = p[A0];
+#pragma unroll
+            for (int a = A0 + 1; a < RA; ++a) mine = (l == a - A0) ? p[a] : mine;
+            if (l < RA - A0) S.pbuf[par][g + 32 * (A0 + l)] = mine;
+        }
+        __syncthreads();
+        // C. rank-2 update
+        double w[CC];
+        double k0 = 0.0, k1 = 0.0;
+#pragma unroll
+        for (int b = B0; b < CC; ++b) w[b] = S.pbuf[par][l + 16 * b];
+#pragma unroll
+        for (int b = B0; b < CC; b += 2) {
+            k0 += w[b] * v[b];
+            k1 += w[b + 1] * v[b + 1];
+        }
+        const double K = 0.5 * t * row_sum16(k0 + k1);
+#pragma unroll
+        for (int b = B0; b < CC; ++b) w[b] -= K * v[b];
+#pragma unroll
+        for (int a = A0; a < RA; ++a) {
+            const double wr = p[a] - K * vr[a];
+#pragma unroll
+            for (int b = B0; b < CC; ++b) h[a][b] -= vr[a] * w[b] + wr * v[b];
+        }
+        if (g == ((k + 1) & 31)) {
+#pragma unroll
+            for (int b = B0; b < CC; ++b) S.xbuf[par ^ 1][l + 16 * b] = h[A0][b];
+            if (l == ((k + 1) & 15)) S.sd[k + 1] = S.xbuf[par ^ 1][k + 1];  // this lane's own entry
+        }
+        if (g == ((k + 17) & 31)) {  // another wave: the reflector for the back-transformation
+#pragma unroll
+            for (int b = B0; b < CC; ++b) R[(int64_t)k * NP + l + 16 * b] = v[b];
+            if (l == 0) {
+                S.se[k] = alpha;
+                S.stau[k] = t;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <int CB>
 __global__ void __launch_bounds__(TRI_NT)
-k_rr_tri(int N, int nev, const double* __restrict__ G, int ldg, double* __restrict__ work,
+k_rr_tri(int N, int nev, const double* __restrict__ G, int ldg, int sym, double* __restrict__ work,
          unsigned long long* __restrict__ prof) {
     constexpr int RA = CB, CC = 2 * CB;
-    __shared__ double vbuf[2][NMAX], pbuf[2][NMAX], kpart[2][32];
-    __shared__ double sd[NMAX], se[NMAX], stau[NMAX];
+    __shared__ TriShared<CB> S;
     RRWork W(work, N, nev);
     const int tid = threadIdx.x, g = tid >> 4, l = tid & 15;
     stamp(prof, 0);
@@ -191,121 +351,27 @@ k_rr_tri(int N, int nev, const double* __restrict__ G, int ldg, double* __restri
 #pragma unroll
         for (int b = 0; b < CC; ++b) {
             const int j = l + 16 * b;
-            h[a][b] = (i < N && j < N) ? 0.5 * (G[(int64_t)i * ldg + j] + G[(int64_t)j * ldg + i]) : 0.0;
+            const bool in = i < N && j < N;
+            double x = in ? G[(int64_t)i * ldg + j] : 0.0;
+            // the mirror image, read across the rows' cache lines, is the
+            // same bits outside a Gram's diagonal tiles of 64
+            if (in && (!sym || a / 2 == b / 4)) x = 0.5 * (x + G[(int64_t)j * ldg + i]);
+            h[a][b] = x;
         }
     }
     stamp(prof, 1);
-    for (int k = 0; k < N - 2; ++k) {
-        const int par = k & 1;
-        // A. reflector of row k (owned by group k % 32, register row k / 32)
-        if (g == (k & 31)) {
-            const int ak = k >> 5;
-            double x[CC];
+    if (g == 0) {  // row 0
 #pragma unroll
-            for (int b = 0; b < CC; ++b) x[b] = 0.0;
-#pragma unroll
-            for (int a = 0; a < RA; ++a)
-                if (a == ak) {
-#pragma unroll
-                    for (int b = 0; b < CC; ++b) x[b] = h[a][b];
-                }
-            if (l == (k & 15)) {
-#pragma unroll
-                for (int b = 0; b < CC; ++b)
-                    if (b == (k >> 4)) sd[k] = x[b];
-            }
-            double part = 0.0, x0l = 0.0;
-#pragma unroll
-            for (int b = 0; b < CC; ++b) {
-                const int j = l + 16 * b;
-                if (j <= k || j >= N) x[b] = 0.0;
-                part += x[b] * x[b];
-                if (b == ((k + 1) >> 4)) x0l = x[b];
-            }
-            const double xn2 = row_sum16(part);
-            const int src = ((g & 3) << 4) + ((k + 1) & 15);  // lane of H[k][k+1] in this wave
-            const double x0 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x0l), src),
-                                               __builtin_amdgcn_readlane(__double2loint(x0l), src));
-            double alpha = 0.0, v0 = 0.0, t = 0.0;
-            if (xn2 != 0.0) {
-                // the short-latency forms on the step's critical path (the
-                // exact ones for extreme magnitudes; xn2 is the same in every
-                // lane, so one branch runs)
-                if (xn2 > 1e-280 && xn2 < 1e280) {
-                    const double sq = sqrt_nr(xn2);
-                    alpha = (x0 >= 0.0) ? -sq : sq;
-                    v0 = x0 - alpha;
-                    t = 2.0 * rcp_nr(xn2 - x0 * x0 + v0 * v0);
-                } else {
-                    alpha = (x0 >= 0.0) ? -sqrt(xn2) : sqrt(xn2);
-                    v0 = x0 - alpha;
-                    t = 2.0 / (xn2 - x0 * x0 + v0 * v0);
-                }
-            }
-#pragma unroll
-            for (int b = 0; b < CC; ++b) {
-                const int j = l + 16 * b;
-                const double v = (t == 0.0) ? 0.0 : ((j == k + 1) ? v0 : x[b]);
-                if (j < N) vbuf[par][j] = v;
-                if (j > k && j < N) W.R[(int64_t)k * N + (j - k - 1)] = v;
-            }
-            if (l == 0) {
-                se[k] = alpha;
-                stau[k] = t;
-            }
-        }
-        __syncthreads();
-        const double t = stau[k];
-        if (t == 0.0) continue;  // H untouched (uniform)
-        // B. p = tau H v for this group's rows
-        // register rows a < a_lo hold rows <= k only and are skipped; within
-        // a row, finished columns get exact zero updates (v and w are zero
-        // there), which costs less than a branch per block
-        const int a_lo = (k >= 31) ? (k - 31) / 32 + 1 : 0;
-        double vc[CC];
-#pragma unroll
-        for (int b = 0; b < CC; ++b) {
-            const int j = l + 16 * b;
-            vc[b] = (j < N) ? vbuf[par][j] : 0.0;
-        }
-        double kp = 0.0;
-#pragma unroll
-        for (int a = 0; a < RA; ++a) {
-            const int i = g + 32 * a;
-            double p = 0.0;
-            if (a >= a_lo) {
-                double s = 0.0;
-#pragma unroll
-                for (int b = 0; b < CC; ++b) s += h[a][b] * vc[b];
-                p = t * row_sum16(s);
-            }
-            if (i <= k || i >= N) p = 0.0;
-            if (i < N) kp += p * vbuf[par][i];
-            if (l == a && i < N) pbuf[par][i] = p;
-        }
-        if (l == 0) kpart[par][g] = kp;
-        __syncthreads();
-        // C. rank-2 update H -= v w^T + w v^T, w = p - K v (v and p at this
-        // thread's rows read back from LDS); every half-wave holds the 32
-        // shares of p . v
-        const double K = 0.5 * t * half_sum32(kpart[par][tid & 31]);
-        double wc[CC];
-#pragma unroll
-        for (int b = 0; b < CC; ++b) {
-            const int j = l + 16 * b;
-            wc[b] = ((j < N) ? pbuf[par][j] : 0.0) - K * vc[b];
-        }
-#pragma unroll
-        for (int a = 0; a < RA; ++a) {
-            const int i = g + 32 * a;
-            if (a < a_lo || i >= N) continue;
-            const double vr = vbuf[par][i];
-            const double wr = pbuf[par][i] - K * vr;
-#pragma unroll
-            for (int b = 0; b < CC; ++b)
-                h[a][b] -= vr * wc[b] + wr * vc[b];
-        }
+        for (int b = 0; b < CC; ++b) S.xbuf[0][l + 16 * b] = h[0][b];
+        if (l == 0) S.sd[0] = h[0][0];
     }
+    __syncthreads();
+    tri_phase<CB, 0>(N, h, S, W.R);
+    if constexpr (CB > 1) tri_phase<CB, 1>(N, h, S, W.R);
+    if constexpr (CB > 2) tri_phase<CB, 2>(N, h, S, W.R);
+    if constexpr (CB > 3) tri_phase<CB, 3>(N, h, S, W.R);
+    if constexpr (CB > 4) tri_phase<CB, 4>(N, h, S, W.R);
+    if constexpr (CB > 5) tri_phase<CB, 5>(N, h, S, W.R);
     // the last 2 x 2 block (or the 1 x 1 matrix)
 #pragma unroll
     for (int a = 0; a < RA; ++a) {
@@ -313,33 +379,40 @@ k_rr_tri(int N, int nev, const double* __restrict__ G, int ldg, double* __restri
 #pragma unroll
         for (int b = 0; b < CC; ++b) {
             const int j = l + 16 * b;
-            if (N >= 2 && i == N - 2 && j == N - 2) sd[N - 2] = h[a][b];
-            if (N >= 2 && i == N - 1 && j == N - 2) se[N - 2] = h[a][b];
-            if (i == N - 1 && j == N - 1) sd[N - 1] = h[a][b];
+            if (N >= 2 && i == N - 1 && j == N - 2) S.se[N - 2] = h[a][b];
+            if (i == N - 1 && j == N - 1) S.sd[N - 1] = h[a][b];
         }
     }
     if (tid == 0) {
-        if (N >= 2) stau[N - 2] = 0.0;
-        stau[N - 1] = 0.0;
-        se[N - 1] = 0.0;
+        if (N >= 2) S.stau[N - 2] = 0.0;
+        S.stau[N - 1] = 0.0;
+        S.se[N - 1] = 0.0;
     }
     __syncthreads();
     for (int i = tid; i < N; i += TRI_NT) {
-        W.d[i] = sd[i];
-        W.e[i] = se[i];
-        W.tau[i] = stau[i];
+        W.d[i] = S.sd[i];
+        W.e[i] = S.se[i];
+        W.tau[i] = S.stau[i];
     }
-    if (tid == 0) {
-        double lo = sd[0], hi = sd[0], nrm = 0.0;
-        for (int i = 0; i < N; ++i) {
-            const double rr = (i > 0 ? fabs(se[i - 1]) : 0.0) + (i < N - 1 ? fabs(se[i]) : 0.0);
-            lo = fmin(lo, sd[i] - rr);
-            hi = fmax(hi, sd[i] + rr);
-            nrm = fmax(nrm, fabs(sd[i]) + rr);
+    // Gershgorin bounds, by the first wave
+    if (tid < 64) {
+        double lo = S.sd[0], hi = S.sd[0], nrm = 0.0;
+        for (int i = tid; i < N; i += 64) {
+            const double rr = (i > 0 ? fabs(S.se[i - 1]) : 0.0) + (i < N - 1 ? fabs(S.se[i]) : 0.0);
+            lo = fmin(lo, S.sd[i] - rr);
+            hi = fmax(hi, S.sd[i] + rr);
+            nrm = fmax(nrm, fabs(S.sd[i]) + rr);
         }
-        W.bnd[0] = lo;
-        W.bnd[1] = hi;
-        W.bnd[2] = fmax(nrm, 1e-300);
+        for (int o = 32; o > 0; o >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, o, 64));
+            hi = fmax(hi, __shfl_xor(hi, o, 64));
+            nrm = fmax(nrm, __shfl_xor(nrm, o, 64));
+        }
+        if (tid == 0) {
+            W.bnd[0] = lo;
+            W.bnd[1] = hi;
+            W.bnd[2] = fmax(nrm, 1e-300);
+        }
     }
     stamp(prof, 2);
 }
@@ -352,20 +425,21 @@ k_rr_bisect(int N, int nev, double* __restrict__ work, double* __restrict__ thet
     stamp(prof, 3);
     RRWork W(work, N, nev);
     const int j = blockIdx.x, q = threadIdx.x;
-    // T scaled by a power of two (exact) to ||T|| <= 1
+    const int N8 = (N + 7) & ~7;
+    // T scaled by a power of two (exact) to ||T|| <= 1; se2[i] couples i - 1 and i
     const double sc = ldexp(1.0, -ilogb(W.bnd[2]) - 1);
-    for (int i = q; i < N; i += 64) {
-        sd[i] = W.d[i] * sc;
-        se2[i] = (i < N - 1) ? (W.e[i] * sc) * (W.e[i] * sc) : 0.0;
+    for (int i = q; i < N8; i += 64) {
+        sd[i] = i < N ? W.d[i] * sc : 2.0;
+        const double e = (i > 0 && i < N) ? W.e[i - 1] * sc : 0.0;
+        se2[i] = fmax(e * e, 1e-60);
     }
     __syncthreads();
     const double glo = W.bnd[0] * sc, ghi = W.bnd[1] * sc, tnorm = W.bnd[2] * sc;
-    const double pivmin = 1e-290 + 1e-300 * tnorm;
     double a = glo - 1e-14 * tnorm, b = ghi + 1e-14 * tnorm;
     for (int it = 0; it < 24; ++it) {
         const double h = (b - a) / 65.0;
         const double x = a + (q + 1) * h;
-        const bool pred = sturm(sd, se2, N, x, pivmin) > j;
+        const bool pred = sturm(sd, se2, N8, x) > j;
         const unsigned long long bal = __ballot(pred);
         const int first = bal ? (__ffsll((long long)bal) - 1) : 64;
         const double nb = (first < 64) ? a + (first + 1) * h : b;
@@ -391,7 +465,7 @@ __device__ __forceinline__ double wave_dot3(const double* y, const double* z, in
 
 __global__ void __launch_bounds__(64)
 k_rr_invit(int N, int nev, double* __restrict__ work) {
-    __shared__ double sd[NMAX], se[NMAX], ws[5 * NMAX], y[NMAX];
+    __shared__ double sd[NMAX + TB], se[NMAX + TB], ws[5 * NMAX], y[NMAX];
     RRWork W(work, N, nev);
     const int j = blockIdx.x, q = threadIdx.x;
     const double tnorm = W.bnd[2];
@@ -434,50 +508,70 @@ k_rr_invit(int N, int nev, double* __restrict__ work) {
 
 // ---- 4. back-transformation Z = Q Y ----------------------------------------
 // One wave per eigenvector (rows q, q + 64, q + 128 in lane q), one
-// workgroup each, so the vectors spread over CUs.  The N - 2 reflector steps
-// are dependent; each one's entries are loaded BACK_PD steps ahead into a
-// register ring, which hides the L2 latency, and the wave sums are DPP sums.
-constexpr int BACK_PD = 4;
+// workgroup each, so the vectors spread over CUs.  The N - 2 reflectors are
+// applied in dependent pairs: with s1 = t1 v1.z, the second one's s2 =
+// t2 (v2.z - s1 v2.v1), and the three dot products of a pair run through the
+// cross-lane stages together.  The entries are loaded BACK_PD pairs ahead into
+// a register ring: they come from another XCD's L2, which takes ~1 us.  Bound by
+// the dependent stages of the pairs: 39 us a call at N = 192 (76 us with one
+// reflector at a time, four ahead, its loads behind branches).
+constexpr int BACK_PD = 8;
 
 __global__ void __launch_bounds__(64)
 k_rr_back(int N, int nev, double* __restrict__ work, unsigned long long* __restrict__ prof) {
-    __shared__ double tau[NMAX];
+    __shared__ double tau[NMAX + 2];
     stamp(prof, 4);
     RRWork W(work, N, nev);
     const int g = blockIdx.x, q = threadIdx.x;
-    for (int i = q; i < N; i += 64) tau[i] = W.tau[i];
+    for (int i = q; i < N; i += 64) tau[i + 1] = W.tau[i];
+    if (q == 0) tau[0] = 0.0;  // "reflector -1": the partner of an odd last one
     const double* yg = W.Y + (int64_t)g * N;
     double z0 = (q < N) ? yg[q] : 0.0;
     double z1 = (q + 64 < N) ? yg[q + 64] : 0.0;
     double z2 = (q + 128 < N) ? yg[q + 128] : 0.0;
-    // reflector k acts on rows k+1 .. N-1 with v_k[row - k - 1] = R[k][row - k - 1]
+    // reflector k acts on rows k+1 .. N-1: loaded without a branch, from a
+    // row and entry that exist, and masked when it is used
+    const int NP = rr_stride(N);
     auto vload = [&](int k, int row) -> double {
-        return (k >= 0 && row >= k + 1 && row < N) ? W.R[(int64_t)k * N + (row - k - 1)] : 0.0;
+        return W.R[(int64_t)(k > 0 ? k : 0) * NP + (row < NP ? row : NP - 1)];
     };
-    double ring[BACK_PD][3];
+    auto masked = [&](double v, int k, int row) -> double { return (row > k && row < N) ? v : 0.0; };
+    double ring[BACK_PD][6];
 #pragma unroll
     for (int d = 0; d < BACK_PD; ++d) {
-        const int k = N - 3 - d;
-        ring[d][0] = vload(k, q);
-        ring[d][1] = vload(k, q + 64);
-        ring[d][2] = vload(k, q + 128);
+        const int k = N - 3 - 2 * d;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            ring[d][c] = vload(k, q + 64 * c);
+            ring[d][3 + c] = vload(k - 1, q + 64 * c);
+        }
     }
     __syncthreads();  // tau staged
-    for (int k0 = N - 3; k0 >= 0; k0 -= BACK_PD) {
+    for (int k0 = N - 3; k0 >= 0; k0 -= 2 * BACK_PD) {
 #pragma unroll
         for (int d = 0; d < BACK_PD; ++d) {
-            const int k = k0 - d;
+            const int k = k0 - 2 * d;
             if (k < 0) break;
-            const double v0 = ring[d][0], v1 = ring[d][1], v2 = ring[d][2];
-            ring[d][0] = vload(k - BACK_PD, q);
-            ring[d][1] = vload(k - BACK_PD, q + 64);
-            ring[d][2] = vload(k - BACK_PD, q + 128);
-            const double t = tau[k];
-            if (t == 0.0) continue;
-            const double sdot = t * wsum(v0 * z0 + v1 * z1 + v2 * z2);
-            z0 -= sdot * v0;
-            z1 -= sdot * v1;
-            z2 -= sdot * v2;
+            double v[6];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                v[c] = masked(ring[d][c], k, q + 64 * c);
+                v[3 + c] = k > 0 ? masked(ring[d][3 + c], k - 1, q + 64 * c) : 0.0;
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                ring[d][c] = vload(k - 2 * BACK_PD, q + 64 * c);
+                ring[d][3 + c] = vload(k - 2 * BACK_PD - 1, q + 64 * c);
+            }
+            const double t1 = tau[k + 1], t2 = tau[k];
+            double s[3] = {v[0] * z0 + v[1] * z1 + v[2] * z2, v[3] * z0 + v[4] * z1 + v[5] * z2,
+                           v[3] * v[0] + v[4] * v[1] + v[5] * v[2]};
+            wave_sum64_each(s);
+            const double a1 = t1 * s[0];
+            const double a2 = t2 * (s[1] - a1 * s[2]);
+            z0 -= a1 * v[0] + a2 * v[3];
+            z1 -= a1 * v[1] + a2 * v[4];
+            z2 -= a1 * v[2] + a2 * v[5];
         }
     }
     if (q < N) W.Z[(int64_t)q * nev + g] = z0;
@@ -486,10 +580,11 @@ k_rr_back(int N, int nev, double* __restrict__ work, unsigned long long* __restr
 }
 
 // ---- 5. orthonormalisation in the small space and output --------------------
-// 4 x 4 tiles of Z in the update: with N nev + nev^2 <= PK and N <= NMAX
-// there are at most 864 (ceil(N/4) ceil(nev/4), maximised over the
-// admissible shapes), one per thread of the 1024
-constexpr int POL_UT = 1;
+typedef double d4_t __attribute__((ext_vector_type(4)));
+// rows of Z and E in LDS when the products run on the matrix cores: two
+// doubles longer than nev, against bank conflicts between rows
+__device__ __forceinline__ int pol_ld(int nev) { return nev >= 32 ? nev + 2 : nev; }
+
 __global__ void __launch_bounds__(NB)
 k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, int* __restrict__ status,
             unsigned long long* __restrict__ prof) {
@@ -498,53 +593,48 @@ k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, i
     stamp(prof, 5);
     RRWork W(work, N, nev);
     const int tid = threadIdx.x;
-    const int nz = N * nev;
-    if (nz + nev * nev <= PK && ((N + 3) / 4) * ((nev + 3) / 4) <= NB * POL_UT) {
-        double* E = Zs + nz;
-        for (int idx = tid; idx < nz; idx += NB) Zs[idx] = W.Z[idx];
+    const int nz = N * nev, ld = pol_ld(nev);
+    if ((N + nev) * ld <= PK && ((N + 15) / 16) * ((nev + 15) / 16) <= 3 * (NB / 64)) {
+        double* E = Zs + N * ld;
+        for (int idx = tid; idx < nz; idx += NB) Zs[(idx / nev) * ld + idx % nev] = W.Z[idx];
         __syncthreads();
         if (nev >= 32) {
-            // both products in 4 x 4 register tiles: every LDS value loaded serves
-            // four multiply-adds
-            const int nt = (nev + 3) / 4, nr = (N + 3) / 4;
+            // both products on the matrix cores (v_mfma_f64_16x16x4f64, operands
+            // from LDS): at N = 192, nev = 64 10 tiles of 48 instructions on the
+            // 16 waves for E, then 48 of 16, three a wave, for the update.  In
+            // 4 x 4 register tiles on the vector units the call took 53 us, now 28.
+            const int lane = tid & 63, wv = tid >> 6, il = lane & 15, kg = lane >> 4;
+            const int nt = (nev + 15) / 16, nr = (N + 15) / 16;
             const int ntri = nt * (nt + 1) / 2, nupd = nr * nt;
             for (int pass = 0; pass < 3; ++pass) {
                 // E = Z^T Z - I: lower-triangle tiles, mirrored
                 double emax = 0.0;
-                for (int t = tid; t < ntri; t += NB) {
-                    int ta = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-                    while ((ta + 1) * (ta + 2) / 2 <= t) ++ta;
-                    while (ta * (ta + 1) / 2 > t) --ta;
-                    const int a0 = 4 * ta, b0 = 4 * (t - ta * (ta + 1) / 2);
-                    double sacc[4][4];
-    #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-    #pragma unroll
-                        for (int w = 0; w < 4; ++w) sacc[u][w] = 0.0;
-                    for (int i = 0; i < N; ++i) {
-                        const double* zr = Zs + i * nev;
-                        double za[4], zb[4];
-    #pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            za[u] = (a0 + u < nev) ? zr[a0 + u] : 0.0;
-                            zb[u] = (b0 + u < nev) ? zr[b0 + u] : 0.0;
-                        }
-    #pragma unroll
-                        for (int u = 0; u < 4; ++u)
-    #pragma unroll
-                            for (int w = 0; w < 4; ++w) sacc[u][w] += za[u] * zb[w];
+                for (int t = wv; t < ntri; t += NB / 64) {
+                    int ta = 0, first = 0;
+                    while (first + ta + 1 <= t) first += ++ta;
+                    const int tb = t - first;
+                    const int ca = 16 * ta + il, cb = 16 * tb + il;
+                    const bool ina = ca < nev, inb = cb < nev;
+                    const double* za = Zs + (ina ? ca : 0);
+                    const double* zb = Zs + (inb ? cb : 0);
+                    d4_t acc = {0.0, 0.0, 0.0, 0.0};
+                    for (int i0 = 0; i0 < N; i0 += 4) {
+                        const int i = i0 + kg;
+                        const bool in = i < N;
+                        const int o = (in ? i : 0) * ld;
+                        const double x = za[o], y = zb[o];
+                        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ina && in ? x : 0.0, inb && in ? y : 0.0, acc, 0,
+                                                                   0, 0);
                     }
-    #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-    #pragma unroll
-                        for (int w = 0; w < 4; ++w) {
-                            const int a = a0 + u, b = b0 + w;
-                            if (a >= nev || b > a) continue;
-                            const double ev = sacc[u][w] - (a == b ? 1.0 : 0.0);
-                            E[a * nev + b] = ev;
-                            E[b * nev + a] = ev;
-                            emax = fmax(emax, fabs(ev));
-                        }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int i = 16 * ta + kg + 4 * r, j = cb;
+                        if (i >= nev || j >= nev || j > i) continue;
+                        const double ev = acc[r] - (i == j ? 1.0 : 0.0);
+                        E[i * ld + j] = ev;
+                        E[j * ld + i] = ev;
+                        emax = fmax(emax, fabs(ev));
+                    }
                 }
                 // block max of |E|
                 for (int off = 32; off > 0; off >>= 1) emax = fmax(emax, __shfl_xor(emax, off, 64));
@@ -552,50 +642,40 @@ k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, i
                 if ((tid & 63) == 0) red[tid >> 6] = emax;
                 __syncthreads();
                 double em = 0.0;
-    #pragma unroll
+#pragma unroll
                 for (int w = 0; w < NB / 64; ++w) em = fmax(em, red[w]);
                 // Newton-Schulz needs ||E|| < 1; a basis that far off is left as it is
                 if (em >= 0.5 || (pass > 0 && em <= 1e-8)) break;
-                // Z <- Z - Z E / 2: one 4 x 4 tile of Z per thread, written after a
-                // barrier once every tile has been read
-                const bool has = tid < nupd;
-                const int i0 = 4 * (tid / nt), c0 = 4 * (tid % nt);
-                double sacc[4][4];
-    #pragma unroll
-                for (int u = 0; u < 4; ++u)
-    #pragma unroll
-                    for (int w = 0; w < 4; ++w) sacc[u][w] = 0.0;
-                if (has) {
-                    for (int h = 0; h < nev; ++h) {
-                        const double* er = E + h * nev;
-                        double zi[4], eh[4];
-    #pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            zi[u] = (i0 + u < N) ? Zs[(i0 + u) * nev + h] : 0.0;
-                            eh[u] = (c0 + u < nev) ? er[c0 + u] : 0.0;
-                        }
-    #pragma unroll
-                        for (int u = 0; u < 4; ++u)
-    #pragma unroll
-                            for (int w = 0; w < 4; ++w) sacc[u][w] += zi[u] * eh[w];
+                // Z <- Z - Z E / 2: up to three 16 x 16 tiles a wave, written
+                // after a barrier once every tile has been read
+                d4_t acc[3];
+#pragma unroll
+                for (int u = 0; u < 3; ++u) {
+                    acc[u] = (d4_t){0.0, 0.0, 0.0, 0.0};
+                    const int t = wv + (NB / 64) * u;
+                    if (t >= nupd) continue;
+                    const int row = 16 * (t / nt) + il, col = 16 * (t % nt) + il;
+                    const bool inr = row < N, inc = col < nev;
+                    const double* zr = Zs + (inr ? row : 0) * ld;
+                    for (int k0 = 0; k0 < nev; k0 += 4) {
+                        const int k = k0 + kg;
+                        const bool in = k < nev;
+                        const double x = zr[in ? k : 0], y = E[(in ? k : 0) * ld + (inc ? col : 0)];
+                        acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(inr && in ? x : 0.0, inc && in ? y : 0.0, acc[u],
+                                                                      0, 0, 0);
                     }
-    #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-    #pragma unroll
-                        for (int w = 0; w < 4; ++w) {
-                            const int i = i0 + u, c = c0 + w;
-                            sacc[u][w] = (i < N && c < nev) ? Zs[i * nev + c] - 0.5 * sacc[u][w] : 0.0;
-                        }
                 }
                 __syncthreads();
-                if (has) {
-    #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-    #pragma unroll
-                        for (int w = 0; w < 4; ++w) {
-                            const int i = i0 + u, c = c0 + w;
-                            if (i < N && c < nev) Zs[i * nev + c] = sacc[u][w];
-                        }
+#pragma unroll
+                for (int u = 0; u < 3; ++u) {
+                    const int t = wv + (NB / 64) * u;
+                    if (t >= nupd) continue;
+                    const int col = 16 * (t % nt) + il;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int row = 16 * (t / nt) + kg + 4 * r;
+                        if (row < N && col < nev) Zs[row * ld + col] -= 0.5 * acc[u][r];
+                    }
                 }
                 __syncthreads();
                 if (em <= 1e-8) break;  // one step leaves ~ em^2: rounding level
@@ -654,7 +734,7 @@ k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, i
                 if (em <= 1e-8) break;  // one step leaves ~ em^2: rounding level
             }
         }
-        for (int idx = tid; idx < nz; idx += NB) C[idx] = Zs[idx];
+        for (int idx = tid; idx < nz; idx += NB) C[idx] = Zs[(idx / nev) * ld + idx % nev];
     } else {
         for (int idx = tid; idx < nz; idx += NB) C[idx] = W.Z[idx];
     }
@@ -664,19 +744,20 @@ k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, i
 
 }  // namespace
 
-size_t rr_std_work_doubles(int N, int nev) { return (size_t)N * N + 3 * (size_t)N + 4 + nev + 2 * (size_t)N * nev + 64; }
+size_t rr_std_work_doubles(int N, int nev) { return (size_t)N * rr_stride(N) + 3 * (size_t)N + 4 + nev + 2 * (size_t)N * nev + 64; }
 
 void rr_std(lh_ctx* ctx, int N, int nev, const double* G, int ldg, double* C, double* theta, double* work,
-            int* status, unsigned long long* prof) {
+            int* status, unsigned long long* prof, bool mirrored) {
+    const int sym = mirrored ? 1 : 0;
     if (N > kRRStdMaxN || nev > N || N < 1 || nev < 1)
         LH_THROW(LH_ERR_ARG, "rr_std: N=%d nev=%d out of range", N, nev);
     switch ((N + 31) / 32) {
-        case 1: k_rr_tri<1><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, work, prof); break;
-        case 2: k_rr_tri<2><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, work, prof); break;
-        case 3: k_rr_tri<3><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, work, prof); break;
-        case 4: k_rr_tri<4><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, work, prof); break;
-        case 5: k_rr_tri<5><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, work, prof); break;
-        default: k_rr_tri<6><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, work, prof); break;
+        case 1: k_rr_tri<1><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, sym, work, prof); break;
+        case 2: k_rr_tri<2><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, sym, work, prof); break;
+        case 3: k_rr_tri<3><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, sym, work, prof); break;
+        case 4: k_rr_tri<4><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, sym, work, prof); break;
+        case 5: k_rr_tri<5><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, sym, work, prof); break;
+        default: k_rr_tri<6><<<1, TRI_NT, 0, ctx->stream>>>(N, nev, G, ldg, sym, work, prof); break;
     }
     LH_CHECK_LAUNCH();
     k_rr_bisect<<<nev, 64, 0, ctx->stream>>>(N, nev, work, theta, prof);
