@@ -99,6 +99,12 @@ int  lh_sync(lh_ctx* ctx);
 /* Number of visible HIP devices (0 when no GPU is present). */
 int  lh_device_count(void);
 
+/* 122-bit content hash of a host array (no counterpart in the reference: it
+ * tells whether a mesh object's arrays are those of its device copy).  The
+ * values depend on keys drawn at random once per process and are only to be
+ * compared within it. */
+int lh_content_hash(const void* data, uint64_t bytes, uint64_t* out /* 2 */);
+
 /* ---- mesh ---------------------------------------------------------------- */
 /* Uploads the arrays LaPy's Solver reads from a mesh: geometry.v (nv x 3,
  * float32 or float64 -- the element math runs in this dtype, as numpy does at

@@ -89,6 +89,7 @@ SIGNATURES = {
     "lh_ctx_destroy": (None, [_vp]),
     "lh_last_error": (C.c_char_p, [_vp]),
     "lh_sync": (C.c_int, [_vp]),
+    "lh_content_hash": (C.c_int, [_vp, C.c_uint64, C.POINTER(C.c_uint64)]),
     "lh_mesh_create": (C.c_int, [_vp, _vp, C.c_int, _i64, _vp, _i64, C.c_int, C.POINTER(_vp)]),
     "lh_mesh_create_device": (C.c_int, [_vp, _vp, C.c_int, _i64, _vp, _i64, C.c_int, C.POINTER(_vp)]),
     "lh_mesh_clone": (C.c_int, [_vp, C.POINTER(_vp)]),
@@ -248,6 +249,13 @@ class Context:
         """Row order of the triangle assembly (LH_ASM_ORDER_*); the values
         do not depend on it."""
         check(lib().lh_ctx_set_assembly_order(self.handle, int(order)), self, "lh_ctx_set_assembly_order")
+
+
+def content_hash(a):
+    """lh_content_hash of a contiguous array: two integers."""
+    out = (C.c_uint64 * 2)()
+    check(lib().lh_content_hash(_ptr(a), a.nbytes, out), None, "lh_content_hash")
+    return out[0], out[1]
 
 
 _default_ctx = None

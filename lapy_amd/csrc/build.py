@@ -33,6 +33,7 @@ COMMON = [
 ]
 SOURCES = {
     "lh_core.hip": [],
+    "lh_hash.hip": [],
     "lh_assembly.hip": ["-ffp-contract=off"],
     "lh_sparse.hip": [],
     "lh_dense.hip": [],

@@ -116,13 +116,10 @@ def _vertex_scalar(mesh, value):
 # ---------------------------------------------------------------------------
 
 def _fingerprint(v, t):
-    import hashlib
-
-    h = hashlib.blake2b(digest_size=16)
+    key = []
     for a in (np.ascontiguousarray(v), np.ascontiguousarray(t)):
-        h.update(str((a.dtype.str, a.shape)).encode())
-        h.update(memoryview(a).cast("B"))
-    return h.hexdigest()
+        key.append((a.dtype.str, a.shape, *_lib.content_hash(a)))
+    return tuple(key)
 
 
 def device_mesh(geometry, ctx=None) -> "_lib.DeviceMesh":
