@@ -787,20 +787,52 @@ k_blk_step(int64_t n, int ld, const int32_t* __restrict__ rp, const int32_t* __r
         *reinterpret_cast<float4*>(out + o) = y;
     }
 }
-// out (+)= M in for the transfer operators
-template <bool ADD, int LPR>
+// out += P in: a fine row has at most a few entries
+template <int LPR>
 __global__ void __launch_bounds__(256)
-k_blk_transfer(int64_t n, int ld, const int32_t* __restrict__ mp, const int32_t* __restrict__ mc,
-               const float* __restrict__ mv, const float* __restrict__ in, float* __restrict__ out) {
+k_blk_prolong(int64_t n, int ld, const int32_t* __restrict__ mp, const int32_t* __restrict__ mc,
+              const float* __restrict__ mv, const float* __restrict__ in, float* __restrict__ out) {
     const int64_t row = (xcd_block() * 256 + threadIdx.x) / LPR;
     if (row >= n) return;
     const int32_t r0 = mp[row];
     const int len = mp[row + 1] - r0;
     for (int c0 = (int)(threadIdx.x % LPR) * 4; c0 < ld; c0 += LPR * 4) {
         const int64_t o = row * ld + c0;
-        float4 y = ADD ? *reinterpret_cast<const float4*>(out + o) : make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 y = *reinterpret_cast<const float4*>(out + o);
         if (len > 0) f4add(y, 1.f, blk_gather<false>(mc + r0, mv + r0, len, mc[r0], nullptr, in, ld, c0));
         *reinterpret_cast<float4*>(out + o) = y;
+    }
+}
+// out = R in: a coarse row gathers the fine rows of its whole neighbourhood
+// (some 60 of a triangle mesh, 200 to 400 of a tet mesh) and there are few of
+// them, so a row is one serial chain of gathers unless its entries are split:
+// a wave a row, whose 64 / LPR groups of lanes take contiguous parts; their
+// sums are added pairwise by shuffles (35,937 tet vertices, 30 pairs: a whole solve
+// 39.6 -> 32.6 ms, of which one lane group a row spent 3.6 ms here).
+template <int LPR>
+__global__ void __launch_bounds__(256)
+k_blk_restrict(int64_t n, int ld, const int32_t* __restrict__ mp, const int32_t* __restrict__ mc,
+               const float* __restrict__ mv, const float* __restrict__ in, float* __restrict__ out) {
+    constexpr int kParts = 64 / LPR;
+    const int64_t row = xcd_block() * 4 + (threadIdx.x >> 6);
+    if (row >= n) return;  // whole wave exits together
+    const int lane = (int)(threadIdx.x & 63), part = lane / LPR;
+    const int32_t r0 = mp[row];
+    const int len = mp[row + 1] - r0;
+    const int per = ((len + kParts - 1) / kParts + 3) / 4 * 4;
+    const int s0 = min(part * per, len), cnt = min(per, len - s0);
+    for (int cb = 0; cb < ld; cb += LPR * 4) {
+        const int c0 = cb + (lane % LPR) * 4;
+        float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (c0 < ld && cnt > 0) y = blk_gather<false>(mc + r0 + s0, mv + r0 + s0, cnt, mc[r0 + s0], nullptr, in, ld, c0);
+#pragma unroll
+        for (int d = LPR; d < 64; d *= 2) {
+            y.x += __shfl_xor(y.x, d);
+            y.y += __shfl_xor(y.y, d);
+            y.z += __shfl_xor(y.z, d);
+            y.w += __shfl_xor(y.w, d);
+        }
+        if (c0 < ld && part == 0) *reinterpret_cast<float4*>(out + row * ld + c0) = y;
     }
 }
 // b = W in FP32, columns m .. ld - 1 zero
@@ -1335,14 +1367,14 @@ void Amg::cycle_blocks(int l, int w, const float* b, float* x) {
     blk_step<kBlkPre>(l, w, b, nullptr, x, (float)((1.0 + k.c1) * k.s), (float)k.s, (float)k.c2);
     blk_step<kBlkRes>(l, w, b, x, fr[l], 0.f, 0.f, 1.f);
     with_row_lanes(lpr, [&](auto L) {
-        k_blk_transfer<false, L.v><<<nblocks_xcd(lv.nc * lpr, 256), 256, 0, ctx->stream>>>(lv.nc, w, lv.tp, lv.tc, lv.f.rv,
-                                                                                         fr[l], fb[l + 1]);
+        k_blk_restrict<L.v><<<nblocks_xcd(lv.nc * 64, 256), 256, 0, ctx->stream>>>(lv.nc, w, lv.tp, lv.tc, lv.f.rv, fr[l],
+                                                                                 fb[l + 1]);
     });
     LH_CHECK_LAUNCH();
     cycle_blocks(l + 1, w, fb[l + 1], fx[l + 1]);
     with_row_lanes(lpr, [&](auto L) {
-        k_blk_transfer<true, L.v><<<nblocks_xcd(lv.n * lpr, 256), 256, 0, ctx->stream>>>(lv.n, w, lv.pp, lv.pc, lv.f.pv,
-                                                                                       fx[l + 1], x);
+        k_blk_prolong<L.v><<<nblocks_xcd(lv.n * lpr, 256), 256, 0, ctx->stream>>>(lv.n, w, lv.pp, lv.pc, lv.f.pv,
+                                                                                fx[l + 1], x);
     });
     LH_CHECK_LAUNCH();
     blk_step<kBlkSt1>(l, w, b, x, fy[l], 0.f, 0.f, (float)k.s);
