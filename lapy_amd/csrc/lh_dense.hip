@@ -705,8 +705,8 @@ template void colsq<float>(lh_ctx*, int64_t, int, const float*, int, double*, De
 
 // R = AX - MX diag(theta) fused with the squared column norms of R and of
 // MX (per-workgroup partials, summed in fixed order by k_colsq_reduce).
-// 16-byte lanes: LPR = m / V lanes per row (V = 2 doubles or 4 floats),
-// 256 / LPR rows per pass of the workgroup over its row range.
+// 16-byte lanes: LPR >= m / V lanes per row (V = 2 doubles or 4 floats; a power
+// of two, the lanes beyond m / V idle), 256 / LPR rows per pass of the workgroup over its row range.
 template <typename T, int LPR>
 __global__ void __launch_bounds__(256)
 k_residual_norms(int64_t n, int m, const T* __restrict__ AX, const T* __restrict__ MX, int ldx,
@@ -768,9 +768,8 @@ void residual_norms(lh_ctx* ctx, int64_t n, int m, const T* AX, const T* MX, int
                     int ldr, double* r2, double* mx2, DevBuf& ws) {
     constexpr int VN = Vec16<T>::n;
     auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) % 16) == 0; };
-    const int lanes = m / VN;
-    const bool vec = m % VN == 0 && ldx % VN == 0 && ldr % VN == 0 && al(AX) && al(MX) && al(R) &&
-                     (lanes == 4 || lanes == 8 || lanes == 16 || lanes == 32 || lanes == 64);
+    const int lanes = std::max(4, vec_lanes(m, VN));
+    const bool vec = m % VN == 0 && ldx % VN == 0 && ldr % VN == 0 && al(AX) && al(MX) && al(R) && lanes <= 64;
     if (!vec) {
         residual<T>(ctx, n, m, AX, MX, ldx, theta, R, ldr);
         colsq<T>(ctx, n, m, R, ldr, r2, ws);

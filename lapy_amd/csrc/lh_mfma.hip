@@ -26,6 +26,7 @@
 #include "lh_dense.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 namespace lh {
 
@@ -165,72 +166,95 @@ k_gram_mfma(int64_t n, int64_t rows_per_wave, int nwaves, const T* __restrict__ 
 // (bi, bj) holds the contiguous columns 16 bi .. 16 bi + 15 of U and 16 bj ..
 // 16 bj + 15 of V, so the blocks wholly beyond p or q are skipped (a 16-column
 // Gram runs one matrix-core block instead of 16).  Lane l loads U[r][16 bi +
-// l % 16] of row r = 4 s + l / 16 (128 contiguous bytes per 16 lanes).  The
-// partial tile has the layout of k_gram_mfma's; only its blocks bi < nbu,
-// bj < nbv are written, which hold every entry i < p, j < q.
-template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-k_gram_mfma_narrow(int64_t n, int64_t rows_per_wave, int nwaves, const T* __restrict__ U, int ldu, int p,
+// l % 16] of row r = 4 s + l / 16 (128 contiguous bytes per 16 lanes).
+// Bound by the latency of a wave's chain of loads, so a wave takes as few rows
+// as the launch allows (16: both loads of its two steps in flight at once) and
+// the workgroup's four waves add their tiles in LDS, which leaves one partial
+// tile per workgroup.  Loads are clamped and zeroed instead of branched around.
+// Gram of 16 to 48 columns, 642 rows: 13.2 -> 3.6 to
+// 6 us, 10,242 rows: 14.7 -> 4 to 7 (64 rows a wave, one partial tile a wave).
+// The partial tile has the layout of k_gram_mfma's; only its blocks bi < nbu,
+// bj < nbv are written, which hold every entry i < p, j < q.  One
+// instance per block count: with the counts as arguments the kernel had 9.5 kB
+// of code, and a cold fetch of it cost as much as the loads.
+constexpr int kNarrowBlocks = 9;
+template <int NBU, int NBV, typename T>
+__global__ void __launch_bounds__(256)
+k_gram_mfma_narrow(int64_t n, int64_t rows_per_wave, const T* __restrict__ U, int ldu, int p,
                    const T* __restrict__ V, int ldv, int q, double* __restrict__ part) {
     typedef typename Mf<T>::v4 v4;
-    const int lane = threadIdx.x & 63;
-    const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (w >= nwaves) return;  // whole wave exits together
+    __shared__ T sh[4][NBU * NBV * 256];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int il = lane & 15, kg = lane >> 4;
-    const int nbu = (p + 15) >> 4, nbv = (q + 15) >> 4;
-    const int64_t rb = (int64_t)w * rows_per_wave;
+    const int64_t rb = ((int64_t)blockIdx.x * 4 + wv) * rows_per_wave;
     const int64_t re = (rb + rows_per_wave < n) ? rb + rows_per_wave : n;
-    v4 acc[4][4];
+    v4 acc[NBU][NBV];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < NBU; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = zero4<T>();
-    auto load_rows = [&](int64_t r0, T (&a)[2][4], T (&b)[2][4]) {
+        for (int b = 0; b < NBV; ++b) acc[a][b] = zero4<T>();
+    auto load_rows = [&](int64_t r0, T (&a)[2][NBU], T (&b)[2][NBV]) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int64_t r = r0 + 4 * s + kg;
             const bool in = r < re;
+            const T* u = U + (in ? r : rb) * ldu;
+            const T* v = V + (in ? r : rb) * ldv;
+            // columns below 16 (NBU - 1) exist
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < NBU; ++c) {
                 const int cc = 16 * c + il;
-                a[s][c] = (c < nbu && in && cc < p) ? U[r * ldu + cc] : T(0);
-                b[s][c] = (c < nbv && in && cc < q) ? V[r * ldv + cc] : T(0);
+                const bool ok = c + 1 < NBU || cc < p;
+                const T x = u[ok ? cc : 0];
+                a[s][c] = in && ok ? x : T(0);
+            }
+#pragma unroll
+            for (int c = 0; c < NBV; ++c) {
+                const int cc = 16 * c + il;
+                const bool ok = c + 1 < NBV || cc < q;
+                const T x = v[ok ? cc : 0];
+                b[s][c] = in && ok ? x : T(0);
             }
         }
     };
-    T a[2][4], b[2][4];
-    if (rb < re) load_rows(rb, a, b);
-    for (int64_t r0 = rb; r0 < re; r0 += 8) {
-        T an[2][4], bn[2][4];
-        const bool more = r0 + 8 < re;
-        if (more) load_rows(r0 + 8, an, bn);
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-                for (int bj = 0; bj < 4; ++bj)
-                    if (bi < nbu && bj < nbv) acc[bi][bj] = Mf<T>::mma(a[s][bi], b[s][bj], acc[bi][bj]);
-        if (more) {
+    if (rb < re) {
+        T a[2][NBU], b[2][NBV];
+        load_rows(rb, a, b);
+        for (int64_t r0 = rb; r0 < re; r0 += 8) {
+            T an[2][NBU], bn[2][NBV];
+            load_rows(r0 + 8, an, bn);  // zeros past re
 #pragma unroll
             for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    a[s][c] = an[s][c];
-                    b[s][c] = bn[s][c];
-                }
+                for (int bi = 0; bi < NBU; ++bi)
+#pragma unroll
+                    for (int bj = 0; bj < NBV; ++bj) acc[bi][bj] = Mf<T>::mma(a[s][bi], b[s][bj], acc[bi][bj]);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int c = 0; c < NBU; ++c) a[s][c] = an[s][c];
+#pragma unroll
+                for (int c = 0; c < NBV; ++c) b[s][c] = bn[s][c];
+            }
         }
     }
-    double* dst = part + (int64_t)w * 4096;  // one tile
+    // register r of lane l of block (bi, bj) at sh[wave][(bi NBV + bj) 256 + 64 r + l]
 #pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
+    for (int bi = 0; bi < NBU; ++bi)
 #pragma unroll
-        for (int bj = 0; bj < 4; ++bj)
-            if (bi < nbu && bj < nbv) {
+        for (int bj = 0; bj < NBV; ++bj)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    dst[(16 * bi + Mf<T>::drow(kg, r)) * 64 + 16 * bj + il] = (double)acc[bi][bj][r];
-            }
+            for (int r = 0; r < 4; ++r) sh[wv][(bi * NBV + bj) * 256 + 64 * r + lane] = acc[bi][bj][r];
+    __syncthreads();
+    double* dst = part + (int64_t)blockIdx.x * 4096;  // one tile
+    // thread (r, l): wave wv writes register wv of every block
+    const int row = Mf<T>::drow(kg, wv);
+#pragma unroll
+    for (int e = 0; e < NBU * NBV; ++e) {
+        const int o = e * 256 + (int)threadIdx.x;
+        dst[(16 * (e / NBV) + row) * 64 + 16 * (e % NBV) + il] =
+            ((double)sh[0][o] + (double)sh[1][o]) + ((double)sh[2][o] + (double)sh[3][o]);
+    }
 }
 
 // C[i][j] = alpha * sum over waves (fixed order: 8 interleaved lane groups,
@@ -302,16 +326,18 @@ k_gram_mfma_reduce(int nwaves, int ntile, int p, int q, int tv, int sym, const d
 // GROUPED (q <= 256): a workgroup owns all column blocks of its rows, so the
 // rows of U are fetched from HBM once for all of them.  INPLACE (Y = U,
 // p = q <= 256, grouped): the workgroup writes only after every wave of it has
-// read its rows of U.  A wave's tile is 64 rows x 16 NB columns: NB = 4 for
-// large n; NB = 1 for small n, where 64-column tiles leave most of the GPU idle
-// and each wave's chain of dependent matrix-core steps is four times shorter
-// (U, small enough to stay in the caches, is then read once per 16 columns).
+// read its rows of U.  A wave's tile is 16 RB rows x 16 NB columns: 32 x 64, or
+// 16 x 16 where the larger tile leaves most of the GPU idle or pads q too far
+// (U, read once per 16 columns then, comes out of the caches).  Bound by the
+// latency of a step's loads at small n and by HBM at large; 64-row tiles had
+// half the waves to hide it behind and twice the code to fetch: 642 rows
+// 8 -> 4.5 us, 35,937 rows x 120 columns 33 -> 22, 131,072 rows 192 -> 64 89 -> 82.
 // nq counts the tile-wide column blocks.
 template <bool VEC, bool INPLACE, bool GROUPED, int NB, typename T>
-__global__ void __launch_bounds__(NB == 4 ? 256 : 512) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(NB == 4 ? 256 : 512) __attribute__((amdgpu_waves_per_eu(4)))
 k_gemm_mfma(int64_t n, int p, int q, const T* U, int ldu, const double* __restrict__ Cm, int ldc, T* Y, int ldy,
             double alpha, double beta, int upper, int nq) {
-    constexpr int TW = 16 * NB;
+    constexpr int RB = NB == 4 ? 2 : 1, TW = 16 * NB;
     typedef typename Mf<T>::v4 v4;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int il = lane & 15, kg = lane >> 4;
@@ -319,28 +345,30 @@ k_gemm_mfma(int64_t n, int p, int q, const T* U, int ldu, const double* __restri
     int n0;      // first column of this wave
     if (INPLACE || GROUPED) {
         const int rsub = (int)(blockDim.x >> 6) / nq;
-        rw = xcd_block() * 64 * rsub + (int64_t)(wv / nq) * 64;
+        rw = (xcd_block() * rsub + wv / nq) * (16 * RB);
         n0 = (wv % nq) * TW;
         if (!INPLACE && rw >= n) return;  // whole wave (no barrier follows)
     } else {
-        rw = xcd_block() * 256 + (int64_t)wv * 64;
+        rw = (xcd_block() * 4 + wv) * (16 * RB);
         n0 = blockIdx.y * TW;
         if (rw >= n) return;  // whole wave
     }
     const int kend = upper ? min(p, n0 + TW) : p;
-    v4 acc[4][NB];
+    v4 acc[RB][NB];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < RB; ++a)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = zero4<T>();
     // one K step's operands: 16 summed indices, this lane's 4 of them
-    auto load_step = [&](int k0, v4 (&a)[4], T (&b)[4][NB]) {
-        const int kc = k0 + 4 * kg;
+    auto load_a = [&](int k0, v4 (&a)[RB]) {
 #pragma unroll
-        for (int bi = 0; bi < 4; ++bi) {
+        for (int bi = 0; bi < RB; ++bi) {
             const int64_t r = rw + 16 * bi + il;
-            a[bi] = (r < n && k0 < kend) ? load4<VEC, T>(U + r * ldu, kc, kend) : zero4<T>();
+            a[bi] = (r < n && k0 < kend) ? load4<VEC, T>(U + r * ldu, k0 + 4 * kg, kend) : zero4<T>();
         }
+    };
+    auto load_b = [&](int k0, T (&b)[4][NB]) {
+        const int kc = k0 + 4 * kg;
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
@@ -349,11 +377,11 @@ k_gemm_mfma(int64_t n, int p, int q, const T* U, int ldu, const double* __restri
                 b[jj][bj] = (kc + jj < kend && col < q) ? (T)Cm[(int64_t)(kc + jj) * ldc + col] : T(0);
             }
     };
-    auto mma_step = [&](const v4 (&a)[4], const T (&b)[4][NB]) {
+    auto mma_step = [&](const v4 (&a)[RB], const T (&b)[4][NB]) {
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
+            for (int bi = 0; bi < RB; ++bi)
 #pragma unroll
                 for (int bj = 0; bj < NB; ++bj) acc[bi][bj] = Mf<T>::mma(a[bi][jj], b[jj][bj], acc[bi][bj]);
     };
@@ -361,14 +389,16 @@ k_gemm_mfma(int64_t n, int p, int q, const T* U, int ldu, const double* __restri
         // 16-column tiles serve small n, where a step's loads are not hidden
         // by other waves: the next step's operands are loaded before this
         // step's matrix-core products
-        v4 a[4], an[4];
+        v4 a[RB], an[RB];
         T b[4][NB], bn[4][NB];
-        load_step(0, a, b);
+        load_a(0, a);
+        load_b(0, b);
         for (int k0 = 0; k0 < kend; k0 += 16) {
-            load_step(k0 + 16, an, bn);  // zeros past kend
+            load_a(k0 + 16, an);  // zeros past kend
+            load_b(k0 + 16, bn);
             mma_step(a, b);
 #pragma unroll
-            for (int bi = 0; bi < 4; ++bi) a[bi] = an[bi];
+            for (int bi = 0; bi < RB; ++bi) a[bi] = an[bi];
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
@@ -376,9 +406,10 @@ k_gemm_mfma(int64_t n, int p, int q, const T* U, int ldu, const double* __restri
         }
     } else {
         for (int k0 = 0; k0 < kend; k0 += 16) {
-            v4 a[4];
+            v4 a[RB];
             T b[4][NB];
-            load_step(k0, a, b);
+            load_b(k0, b);
+            load_a(k0, a);
             mma_step(a, b);
         }
     }
@@ -387,7 +418,7 @@ k_gemm_mfma(int64_t n, int p, int q, const T* U, int ldu, const double* __restri
     // load cannot pass a store the compiler cannot prove distinct, so
     // interleaving them would cost one memory round trip per value)
 #pragma unroll
-    for (int bi = 0; bi < 4; ++bi) {
+    for (int bi = 0; bi < RB; ++bi) {
         T yv[4][NB];
         if (beta != 0.0) {
 #pragma unroll
@@ -429,32 +460,57 @@ bool vec_ok(const T* p, int ld) {
 namespace {
 
 // row split of a Gram: nw waves per output tile, rpw rows each (a multiple of
-// 16); part holds nw * ntile partial tiles of 64 x 64 doubles
+// 16; narrow blocks: nw workgroups of four such waves); part holds nw * ntile partial tiles of 64 x 64 doubles
 struct GramPlan {
     int tv = 0, ntile = 0;
     int64_t nw = 0, rpw = 0;
 };
 
-// about two waves per SIMD over all tiles, at least 64 rows per wave;
-// max_parts > 0 caps nw * ntile (the fixed scratch of lh_block_gram_noalloc)
+// one output tile of which at most 9 of the 16 matrix-core blocks are needed
+inline bool gram_narrow(int p, int q) {
+    return p <= 64 && q <= 64 && ((p + 15) / 16) * ((q + 15) / 16) <= kNarrowBlocks;
+}
+
+// f(nbu, nbv) with the block counts of a narrow Gram as compile-time constants
+template <int NU, typename F>
+void with_narrow_v(int nv, F&& f) {
+    std::integral_constant<int, NU> u;
+    switch (nv) {
+        case 1: f(u, std::integral_constant<int, 1>{}); break;
+        case 2: f(u, std::integral_constant<int, 2>{}); break;
+        case 3: if constexpr (NU * 3 <= kNarrowBlocks) f(u, std::integral_constant<int, 3>{}); break;
+        default: if constexpr (NU * 4 <= kNarrowBlocks) f(u, std::integral_constant<int, 4>{}); break;
+    }
+}
+template <typename F>
+void with_narrow(int nu, int nv, F&& f) {
+    switch (nu) {
+        case 1: with_narrow_v<1>(nv, f); break;
+        case 2: with_narrow_v<2>(nv, f); break;
+        case 3: with_narrow_v<3>(nv, f); break;
+        default: with_narrow_v<4>(nv, f); break;
+    }
+}
+
+// about two waves per SIMD over all tiles, at least 64 rows per wave (narrow
+// blocks: 16, and nw counts workgroups of four waves); max_parts > 0 caps
+// nw * ntile (the fixed scratch of lh_block_gram_noalloc)
 GramPlan gram_plan(const lh_ctx* ctx, int64_t n, int p, int q, bool sym, int64_t max_parts) {
     GramPlan g;
     const int tu = (p + 63) / 64;
     g.tv = (q + 63) / 64;
     g.ntile = sym ? tu * (tu + 1) / 2 : tu * g.tv;
-    const int64_t target = (int64_t)ctx->n_cu * 8;
+    const int waves = gram_narrow(p, q) ? 4 : 1;
+    const int64_t target = (int64_t)ctx->n_cu * 8 / waves;
     int64_t nw = std::max<int64_t>(1, target / g.ntile);
     nw = std::min<int64_t>(nw, (n + 63) / 64);
     if (max_parts > 0) nw = std::min<int64_t>(nw, std::max<int64_t>(1, max_parts / g.ntile));
-    int64_t rpw = (n + nw - 1) / nw;
+    int64_t rpw = (n + nw * waves - 1) / (nw * waves);
     rpw = ((rpw + 15) / 16) * 16;
     g.rpw = rpw;
-    g.nw = (n + rpw - 1) / rpw;  // <= the nw above
+    g.nw = (n + rpw * waves - 1) / (rpw * waves);  // <= the nw above
     return g;
 }
-
-// one output tile of which at most 9 of the 16 matrix-core blocks are needed
-inline bool gram_narrow(int p, int q) { return p <= 64 && q <= 64 && ((p + 15) / 16) * ((q + 15) / 16) <= 9; }
 
 template <typename T>
 void gram_launch(lh_ctx* ctx, const GramPlan& g, int64_t n, const T* U, int ldu, int p, const T* V, int ldv, int q,
@@ -462,7 +518,10 @@ void gram_launch(lh_ctx* ctx, const GramPlan& g, int64_t n, const T* U, int ldu,
     const bool vec = vec_ok(U, ldu) && vec_ok(V, ldv);
     dim3 grid((unsigned)((g.nw + 3) / 4), (unsigned)g.ntile);
     if (gram_narrow(p, q))
-        k_gram_mfma_narrow<T><<<grid, 256, 0, ctx->stream>>>(n, g.rpw, (int)g.nw, U, ldu, p, V, ldv, q, part);
+        with_narrow((p + 15) / 16, (q + 15) / 16, [&](auto nu, auto nv) {
+            k_gram_mfma_narrow<nu.value, nv.value, T>
+                <<<(unsigned)g.nw, 256, 0, ctx->stream>>>(n, g.rpw, U, ldu, p, V, ldv, q, part);
+        });
     else if (vec)
         k_gram_mfma<true, T><<<grid, 256, 0, ctx->stream>>>(n, g.rpw, (int)g.nw, U, ldu, p, V, ldv, q, g.tv,
                                                             sym ? 1 : 0, part);
@@ -486,64 +545,56 @@ void gram_mfma(lh_ctx* ctx, int64_t n, const T* U, int ldu, int p, const T* V, i
     gram_launch<T>(ctx, g, n, U, ldu, p, V, ldv, q, sym, ws.as<double>(), C, ldc, alpha);
 }
 
-// 16-column tiles when 64-column ones would give fewer than 512 waves
-inline bool gemm_narrow(int64_t n, int q) { return (n + 63) / 64 * ((q + 63) / 64) < 512; }
+// 16 x 16 tiles instead of 32 x 64 ones: while those are less than a wave or
+// two per SIMD, and at any n when 64-column padding wastes more than the larger
+// tile's reuse of U gains.  us at 64-column | 16-column tiles, FP64, p -> q
+// (in place: upper triangular): 10,242 rows 64 -> 128 14 | 13, 192 -> 64 27 | 20,
+// 48 -> 16 9.6 | 4.3; 29,160 rows 64 -> 128 22 | 29, 192 -> 64 34 | 39,
+// 128 in place 38 | 35; 131,072 rows 40 -> 80 51 | 54, 80 in place 76 | 64,
+// 120 -> 40 55 | 78, 48 -> 16 24 | 14, 32 in place 22 | 18.  Within a solve of
+// 35,937 rows, 40 -> 80 and 120 -> 40 together: 23.6 | 18.6.
+inline bool gemm_narrow(int64_t n, int q, bool inplace) {
+    const int q16 = (q + 15) / 16 * 16, q64 = (q + 63) / 64 * 64;
+    const int64_t waves = (n + 31) / 32 * (q64 / 64);
+    return waves < (inplace ? 2048 : 768) || q16 * (inplace ? 24 : 26) < q64 * 16 || (waves < 2400 && q16 * 20 < q64 * 16);
+}
+
+template <int NB, bool INPLACE, bool GROUPED, typename T>
+void gemm_launch(lh_ctx* ctx, int64_t n, int p, int q, const T* U, int ldu, const double* C, int ldc, T* Y, int ldy,
+                 double alpha, double beta, int up, int nq) {
+    constexpr int rows = NB == 4 ? 32 : 16;  // of a wave
+    dim3 grid;
+    int bs;
+    if (GROUPED) {
+        // nq column blocks x rsub row blocks per workgroup (at most 512 threads for NB = 1, 256 for NB = 4)
+        const int rsub = NB == 1 ? std::max(1, 8 / nq) : (nq == 1 ? 4 : (nq == 2 ? 2 : 1));
+        bs = 64 * nq * rsub;
+        grid = dim3(nblocks_xcd(n, rows * rsub));
+    } else {
+        bs = 256;
+        grid = dim3(nblocks_xcd(n, 4 * rows), (unsigned)nq);
+    }
+    if (vec_ok(U, ldu))
+        k_gemm_mfma<true, INPLACE, GROUPED, NB, T><<<grid, bs, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy, alpha,
+                                                                                beta, up, nq);
+    else
+        k_gemm_mfma<false, INPLACE, GROUPED, NB, T><<<grid, bs, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy,
+                                                                                 alpha, beta, up, nq);
+    LH_CHECK_LAUNCH();
+}
 
 template <typename T>
 void gemm_mfma(lh_ctx* ctx, int64_t n, int p, int q, const T* U, int ldu, const double* C, int ldc, T* Y, int ldy,
                double alpha, double beta, bool upper) {
     if (n == 0 || q == 0) return;
-    const bool vec = vec_ok(U, ldu);
     const int up = upper ? 1 : 0;
-    if (gemm_narrow(n, q)) {
-        const int nq = (q + 15) / 16;
-        if (nq > 1 && nq <= 8) {
-            // grouped: nq 16-column blocks x rsub row blocks of 64 per
-            // workgroup (at most 512 threads)
-            const int rsub = std::max(1, 8 / nq);
-            const int bs = 64 * nq * rsub;
-            const unsigned nb = nblocks_xcd(n, 64 * rsub);
-            if (vec)
-                k_gemm_mfma<true, false, true, 1, T><<<nb, bs, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy,
-                                                                                alpha, beta, up, nq);
-            else
-                k_gemm_mfma<false, false, true, 1, T><<<nb, bs, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy,
-                                                                                 alpha, beta, up, nq);
-        } else {
-            dim3 grid(nblocks_xcd(n, 256), (unsigned)nq);
-            if (vec)
-                k_gemm_mfma<true, false, false, 1, T><<<grid, 256, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy,
-                                                                                    alpha, beta, up, nq);
-            else
-                k_gemm_mfma<false, false, false, 1, T><<<grid, 256, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y,
-                                                                                     ldy, alpha, beta, up, nq);
-        }
-        LH_CHECK_LAUNCH();
-        return;
-    }
-    const int nq = (q + 63) / 64;
-    if (nq > 1 && nq <= 4) {
-        // grouped: nq column blocks x rsub row blocks of 64 per workgroup
-        const int rsub = nq == 2 ? 2 : 1;
-        const int bs = 64 * nq * rsub;
-        const unsigned nb = nblocks_xcd(n, 64 * rsub);
-        if (vec)
-            k_gemm_mfma<true, false, true, 4, T><<<nb, bs, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy, alpha,
-                                                                            beta, up, nq);
-        else
-            k_gemm_mfma<false, false, true, 4, T><<<nb, bs, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy, alpha,
-                                                                             beta, up, nq);
-        LH_CHECK_LAUNCH();
-        return;
-    }
-    dim3 grid(nblocks_xcd(n, 256), (unsigned)nq);
-    if (vec)
-        k_gemm_mfma<true, false, false, 4, T><<<grid, 256, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy, alpha,
-                                                                             beta, up, nq);
-    else
-        k_gemm_mfma<false, false, false, 4, T><<<grid, 256, 0, ctx->stream>>>(n, p, q, U, ldu, C, ldc, Y, ldy, alpha,
-                                                                              beta, up, nq);
-    LH_CHECK_LAUNCH();
+    const bool narrow = gemm_narrow(n, q, false);
+    const int nq = narrow ? (q + 15) / 16 : (q + 63) / 64;
+    const bool grouped = nq > 1 && nq <= (narrow ? 8 : 4);
+    if (narrow && grouped) gemm_launch<1, false, true, T>(ctx, n, p, q, U, ldu, C, ldc, Y, ldy, alpha, beta, up, nq);
+    else if (narrow) gemm_launch<1, false, false, T>(ctx, n, p, q, U, ldu, C, ldc, Y, ldy, alpha, beta, up, nq);
+    else if (grouped) gemm_launch<4, false, true, T>(ctx, n, p, q, U, ldu, C, ldc, Y, ldy, alpha, beta, up, nq);
+    else gemm_launch<4, false, false, T>(ctx, n, p, q, U, ldu, C, ldc, Y, ldy, alpha, beta, up, nq);
 }
 
 template <typename T>
@@ -551,35 +602,12 @@ void gemm_mfma_inplace(lh_ctx* ctx, int64_t n, int p, T* X, int ldx, const doubl
                        bool upper) {
     if (n == 0 || p == 0) return;
     if (p > 256) LH_THROW(LH_ERR_ARG, "in-place block update needs width <= 256, got %d", p);
-    const bool vec = vec_ok(X, ldx);
     const int up = upper ? 1 : 0;
-    if (p <= 128 && gemm_narrow(n, p)) {
-        // a workgroup covers all p columns of its rows: nq <= 8 waves of 16
-        // columns, rsub row blocks of 64 (at most 512 threads)
-        const int nq = (p + 15) / 16;
-        const int rsub = std::max(1, 8 / nq);
-        const int bs = 64 * nq * rsub;
-        const unsigned nb = nblocks_xcd(n, 64 * rsub);
-        if (vec)
-            k_gemm_mfma<true, true, true, 1, T><<<nb, bs, 0, ctx->stream>>>(n, p, p, X, ldx, C, ldc, X, ldx, alpha,
-                                                                           0.0, up, nq);
-        else
-            k_gemm_mfma<false, true, true, 1, T><<<nb, bs, 0, ctx->stream>>>(n, p, p, X, ldx, C, ldc, X, ldx, alpha,
-                                                                            0.0, up, nq);
-        LH_CHECK_LAUNCH();
-        return;
-    }
-    const int nq = (p + 63) / 64;
-    const int rsub = nq == 1 ? 4 : (nq == 2 ? 2 : 1);
-    const int bs = 64 * nq * rsub;
-    const unsigned nb = nblocks_xcd(n, 64 * rsub);
-    if (vec)
-        k_gemm_mfma<true, true, true, 4, T><<<nb, bs, 0, ctx->stream>>>(n, p, p, X, ldx, C, ldc, X, ldx, alpha, 0.0,
-                                                                        up, nq);
+    // a workgroup covers all p columns of its rows: at most 8 waves of 16, 4 of 64
+    if (p <= 128 && gemm_narrow(n, p, true))
+        gemm_launch<1, true, true, T>(ctx, n, p, p, X, ldx, C, ldc, X, ldx, alpha, 0.0, up, (p + 15) / 16);
     else
-        k_gemm_mfma<false, true, true, 4, T><<<nb, bs, 0, ctx->stream>>>(n, p, p, X, ldx, C, ldc, X, ldx, alpha, 0.0,
-                                                                         up, nq);
-    LH_CHECK_LAUNCH();
+        gemm_launch<4, true, true, T>(ctx, n, p, p, X, ldx, C, ldc, X, ldx, alpha, 0.0, up, (p + 63) / 64);
 }
 
 template void gram_mfma<double>(lh_ctx*, int64_t, const double*, int, int, const double*, int, int, double*, int,
