@@ -61,6 +61,25 @@ __host__ __device__ inline Cheb2 cheb2(double bmax) {
     return Cheb2{1.0 / th, rho1 * rho0, 2.0 * rho1 / de};
 }
 
+template <int V>
+struct IntC {
+    static constexpr int v = V;
+};
+// lanes for a row of the mean length: about four entries a lane
+int lanes_for(int64_t nnz, int64_t n) {
+    const int64_t avg = n > 0 ? nnz / n : 0;
+    return avg >= 40 ? 16 : avg >= 20 ? 8 : avg >= 8 ? 4 : 1;
+}
+template <typename F>
+void with_lanes(int g, F&& f) {
+    switch (g) {
+        case 1: f(IntC<1>{}); break;
+        case 4: f(IntC<4>{}); break;
+        case 8: f(IntC<8>{}); break;
+        default: f(IntC<16>{}); break;
+    }
+}
+
 __device__ __forceinline__ uint32_t mix32(uint32_t x) {
     x ^= x >> 16;
     x *= 0x7feb352du;
@@ -71,32 +90,49 @@ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
 }
 
 // ---- setup ------------------------------------------------------------------
+// The kernels over the rows of a level's matrix take G lanes a row (about the
+// row's entries): with a thread a row a wave's loads are scattered over 64 rows
+// and the longest row sets its time.  118k tet vertices (15 entries a row; 50 on
+// the next level): power step 26 -> 5.4 us, averaged over the levels, and the
+// spreading step 35 -> 4.4, which also stopped testing every entry's strength
+// again in each round.
+
 // dinv; bad[0] set when a row's diagonal is negative, missing or zero beside
 // non-zero entries; start vector of the power iteration (0 on zero rows)
-__global__ void k_amg_diag(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
-                           const double* __restrict__ kv, double* __restrict__ dinv, double* __restrict__ x,
-                           int* __restrict__ bad) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+template <int G>
+__global__ void __launch_bounds__(256)
+k_amg_diag(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl, const double* __restrict__ kv,
+           double* __restrict__ dinv, double* __restrict__ x, int* __restrict__ bad) {
+    const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
     if (i >= n) return;
     double d = 0.0, other = 0.0;
-    for (int32_t s = rp[i]; s < rp[i + 1]; ++s) {
+    for (int32_t s = rp[i] + (int32_t)(threadIdx.x % G); s < rp[i + 1]; s += G) {
         if (cl[s] == (int32_t)i) d = kv[s];
         else other = fmax(other, fabs(kv[s]));
     }
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) {
+        d += __shfl_xor(d, o, 64);  // zero in all lanes but one
+        other = fmax(other, __shfl_xor(other, o, 64));
+    }
+    if (threadIdx.x % G) return;
     if (!(d >= 0.0) || (d == 0.0 && other != 0.0)) bad[0] = 1;  // every writer stores the same value
     const bool pos = d > 0.0;
     dinv[i] = pos ? 1.0 / d : 0.0;
     x[i] = pos ? (double)(mix32((uint32_t)i * 2654435761u + 12345u) >> 8) * (1.0 / 8388608.0) - 1.0 : 0.0;
 }
-// y = D^-1 K x, one thread per row
-__global__ void k_amg_power(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
-                            const double* __restrict__ kv, const double* __restrict__ dinv,
-                            const double* __restrict__ x, double* __restrict__ y) {
-    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+// y = D^-1 K x
+template <int G>
+__global__ void __launch_bounds__(256)
+k_amg_power(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl, const double* __restrict__ kv,
+            const double* __restrict__ dinv, const double* __restrict__ x, double* __restrict__ y) {
+    const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
     if (i >= n) return;
     double a = 0.0;
-    for (int32_t s = rp[i]; s < rp[i + 1]; ++s) a += kv[s] * x[cl[s]];
-    y[i] = dinv[i] * a;
+    for (int32_t s = rp[i] + (int32_t)(threadIdx.x % G); s < rp[i + 1]; s += G) a += kv[s] * x[cl[s]];
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+    if (threadIdx.x % G == 0) y[i] = dinv[i] * a;
 }
 // block partials of x^T D x and x^T D y (y = D^-1 K x): 2 doubles a block
 __global__ void __launch_bounds__(256)
@@ -132,40 +168,60 @@ __global__ void k_mis_init(int64_t n, const double* __restrict__ dinv, unsigned 
                ? kUndecided | ((unsigned long long)(mix32((uint32_t)i + 0x9e3779b9u) >> 2) << 32) | (unsigned)i
                : kOut;
 }
-__device__ __forceinline__ bool strong(double k, double di, double dj, double th2) { return k * k * di * dj > th2; }
+// the strong neighbours of each row, k_ij^2 > theta^2 k_ii k_jj: the column, or
+// -1 for a weak entry
+template <int G>
+__global__ void __launch_bounds__(256)
+k_strong(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl, const double* __restrict__ kv,
+         const double* __restrict__ dinv, double th2, int32_t* __restrict__ sc) {
+    const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
+    if (i >= n) return;
+    const double di = dinv[i];
+    for (int32_t s = rp[i] + (int32_t)(threadIdx.x % G); s < rp[i + 1]; s += G) {
+        const int32_t j = cl[s];
+        sc[s] = kv[s] * kv[s] * di * dinv[j] > th2 ? j : -1;
+    }
+}
 
-// largest key among the row and its strong neighbours
+// largest key among the row and its strong neighbours, in every lane of the row
+template <int G>
 __device__ __forceinline__ unsigned long long mis_max(int64_t i, const int32_t* __restrict__ rp,
-                                                      const int32_t* __restrict__ cl, const double* __restrict__ kv,
-                                                      const double* __restrict__ dinv, double th2,
+                                                      const int32_t* __restrict__ sc,
                                                       const unsigned long long* __restrict__ t) {
     unsigned long long best = t[i];
-    const double di = dinv[i];
-    for (int32_t s = rp[i]; s < rp[i + 1]; ++s) {
-        const int32_t j = cl[s];
-        if (strong(kv[s], di, dinv[j], th2)) {
-            const unsigned long long q = t[j];
-            best = q > best ? q : best;
-        }
+    for (int32_t s = rp[i] + (int32_t)(threadIdx.x % G); s < rp[i + 1]; s += G) {
+        const int32_t j = sc[s];
+        const unsigned long long q = j >= 0 ? t[j] : 0ull;
+        best = q > best ? q : best;
+    }
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) {
+        const unsigned long long q = __shfl_xor(best, o, 64);
+        best = q > best ? q : best;
     }
     return best;
 }
-__global__ void k_mis_spread(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
-                             const double* __restrict__ kv, const double* __restrict__ dinv, double th2,
-                             const unsigned long long* __restrict__ t, unsigned long long* __restrict__ a) {
-    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = mis_max(i, rp, cl, kv, dinv, th2, t);
+template <int G>
+__global__ void __launch_bounds__(256)
+k_mis_spread(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ sc,
+             const unsigned long long* __restrict__ t, unsigned long long* __restrict__ a) {
+    const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
+    if (i >= n) return;
+    const unsigned long long best = mis_max<G>(i, rp, sc, t);
+    if (threadIdx.x % G == 0) a[i] = best;
 }
 // second spreading step and the decision: a row whose key is the largest
 // within distance 2 joins, one with a member within distance 2 leaves
-__global__ void k_mis_decide(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
-                             const double* __restrict__ kv, const double* __restrict__ dinv, double th2,
-                             const unsigned long long* __restrict__ a, unsigned long long* __restrict__ t) {
-    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+template <int G>
+__global__ void __launch_bounds__(256)
+k_mis_decide(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ sc,
+             const unsigned long long* __restrict__ a, unsigned long long* __restrict__ t) {
+    const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
     if (i >= n) return;
     const unsigned long long own = t[i];
-    if ((own >> 62) != 1) return;
-    const unsigned long long best = mis_max(i, rp, cl, kv, dinv, th2, a);
+    if ((own >> 62) != 1) return;  // all lanes of the row
+    const unsigned long long best = mis_max<G>(i, rp, sc, a);
+    if (threadIdx.x % G) return;
     if (best == own) t[i] = kIn | (own & ~(3ull << 62));
     else if ((best >> 62) == 2) t[i] = kOut;
 }
@@ -180,25 +236,36 @@ __global__ void k_agg_roots(int64_t n, const int32_t* __restrict__ flag, const i
 }
 // an unassigned row joins the aggregate of its strongest assigned neighbour
 // (the first of equals); in: the assignment before this pass
-__global__ void k_agg_join(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
-                           const double* __restrict__ kv, const double* __restrict__ dinv, double th2,
-                           const int32_t* __restrict__ in, int32_t* __restrict__ out) {
-    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
+template <int G>
+__global__ void __launch_bounds__(256)
+k_agg_join(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ sc, const double* __restrict__ kv,
+           const int32_t* __restrict__ in, int32_t* __restrict__ out) {
+    const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
     if (i >= n) return;
     int32_t g = in[i];
-    const double di = dinv[i];
-    if (g < 0 && di > 0.0) {
+    if (g < 0) {  // all lanes of the row
         double best = 0.0;
-        for (int32_t s = rp[i]; s < rp[i + 1]; ++s) {
-            const int32_t j = cl[s];
+        int32_t at = INT32_MAX;
+        for (int32_t s = rp[i] + (int32_t)(threadIdx.x % G); s < rp[i + 1]; s += G) {
+            const int32_t j = sc[s];
             const double w = fabs(kv[s]);
-            if (in[j] >= 0 && w > best && strong(w, di, dinv[j], th2)) {
+            if (j >= 0 && w > best && in[j] >= 0) {
                 best = w;
-                g = in[j];
+                at = s;
             }
         }
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) {
+            const double w = __shfl_xor(best, o, 64);
+            const int32_t q = __shfl_xor(at, o, 64);
+            if (w > best || (w == best && q < at)) {
+                best = w;
+                at = q;
+            }
+        }
+        if (at != INT32_MAX) g = in[sc[at]];
     }
-    out[i] = g;
+    if (threadIdx.x % G == 0) out[i] = g;
 }
 
 // P = (I - w D^-1 K) P_0 row by row: first the number of distinct aggregates
@@ -301,20 +368,42 @@ __global__ void k_scatter_cols(int64_t n, const int32_t* __restrict__ pp, const 
         tv[q] = pv[s];
     }
 }
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 // one wave per row: an entry's place is the number of smaller ones (a row's
-// entries are distinct)
+// entries are distinct), counted over the row's keys in LDS, four a read; a
+// row of more than 1,024 counts in memory.  118k
+// tet vertices: 109 -> 30 us a level (one key a read from memory before).
 __global__ void __launch_bounds__(256)
 k_sort_rows(int64_t nc, const int32_t* __restrict__ tp, const int32_t* __restrict__ ti, const double* __restrict__ vi,
             int32_t* __restrict__ to, double* __restrict__ vo) {
-    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= nc) return;
-    const int32_t a = tp[r], b = tp[r + 1];
-    for (int32_t e = a + (int32_t)(threadIdx.x & 63); e < b; e += 64) {
-        const int32_t key = ti[e];
+    constexpr int kKeys = 1024;
+    __shared__ __align__(16) int32_t s_keys[4][kKeys];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t r = (int64_t)blockIdx.x * 4 + wv;
+    if (r >= nc) return;  // no workgroup barrier follows
+    const int32_t a = tp[r], len = tp[r + 1] - a;
+    const bool in_lds = len <= kKeys;
+    int32_t* keys = s_keys[wv];
+    if (in_lds) {
+        for (int q = lane; q < (len + 3) / 4 * 4; q += 64) keys[q] = q < len ? ti[a + q] : INT32_MAX;
+        wave_fence();
+    }
+    for (int e = lane; e < len; e += 64) {
+        const int32_t key = ti[a + e];
         int32_t rank = 0;
-        for (int32_t q = a; q < b; ++q) rank += ti[q] < key;
+        if (in_lds) {
+            for (int q = 0; q < len; q += 4) {
+                const int4 k = *reinterpret_cast<const int4*>(keys + q);
+                rank += (k.x < key) + (k.y < key) + (k.z < key) + (k.w < key);
+            }
+        } else {
+            for (int q = 0; q < len; ++q) rank += ti[a + q] < key;
+        }
         to[a + rank] = key;
-        vo[a + rank] = vi[e];
+        vo[a + rank] = vi[a + e];
     }
 }
 
@@ -325,7 +414,10 @@ k_sort_rows(int64_t nc, const int32_t* __restrict__ tp, const int32_t* __restric
 // distinct columns, so a value's terms are summed in the order of X's
 // entries; an entry's place in the output row is the number of smaller
 // columns.  A row with more than 3/4 HS distinct columns sets over[0].
-// Bound by the latency of its dependent LDS steps (one per entry of X's row).
+// Bound by the latency of its dependent LDS steps (one per entry of X's row):
+// the rows of Y are on their way before their turn.  118k tet vertices, all six
+// products:
+// 1.40 -> 0.98 ms.
 template <int HS>
 __device__ __forceinline__ int hash_slot(volatile int32_t* keys, int32_t key) {
     int h = (int)(mix32((uint32_t)key) & (HS - 1));
@@ -340,10 +432,6 @@ __device__ __forceinline__ int hash_slot(volatile int32_t* keys, int32_t key) {
     }
     return -1;
 }
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 template <int HS, bool FILL>
 __global__ void __launch_bounds__(256)
@@ -354,7 +442,7 @@ k_spgemm(int64_t n, const int32_t* __restrict__ xp, const int32_t* __restrict__ 
     __shared__ int32_t s_keys[4][HS];
     __shared__ double s_vals[FILL ? 4 : 1][FILL ? HS : 1];
     __shared__ int32_t s_list[FILL ? 4 : 1][FILL ? HS : 1], s_slot[FILL ? 4 : 1][FILL ? HS : 1];
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + wv;
     if (row >= n) return;  // no workgroup barrier follows
     volatile int32_t* keys = s_keys[wv];
@@ -383,14 +471,51 @@ k_spgemm(int64_t n, const int32_t* __restrict__ xp, const int32_t* __restrict__ 
         if (lane == 0) count_or_cols[row] = cnt;
         return;
     }
-    for (int32_t e = a; e < b; ++e) {
-        const int32_t j = xc[e];
-        const double x = xv[e];
-        for (int32_t q = yp[j] + lane; q < yp[j + 1]; q += 64) {
-            const int h = hash_slot<HS>(keys, yc[q]);
-            if (h >= 0) vals[h] = vals[h] + x * yv[q];
+    // 64 entries of X's row and their rows' bounds side by side, then the rows of
+    // Y four at a time: the next four are loaded while these are added
+    for (int32_t e0 = a; e0 < b; e0 += 64) {
+        const bool in = e0 + lane < b;
+        const int32_t j = in ? xc[e0 + lane] : 0;
+        const double xl = in ? xv[e0 + lane] : 0.0;
+        const int32_t y0 = in ? yp[j] : 0, y1 = in ? yp[j + 1] : 0;
+        const int cnt = b - e0 < 64 ? b - e0 : 64;
+        int32_t c[4], cn[4];
+        double v[4], vn[4];
+        auto load4 = [&](int o0, int32_t (&cc)[4], double (&vv)[4]) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int o = o0 + u < 64 ? o0 + u : 63;
+                const int32_t q = __builtin_amdgcn_readlane(y0, o) + lane;
+                const bool ok = o0 + u < cnt && q < __builtin_amdgcn_readlane(y1, o);
+                cc[u] = ok ? yc[q] : -1;
+                vv[u] = ok ? yv[q] : 0.0;
+            }
+        };
+        load4(0, c, v);
+        for (int o0 = 0; o0 < cnt; o0 += 4) {
+            load4(o0 + 4, cn, vn);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int o = o0 + u < 64 ? o0 + u : 63;
+                const double x = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(xl), o),
+                                                  __builtin_amdgcn_readlane(__double2loint(xl), o));
+                if (c[u] >= 0) {
+                    const int h = hash_slot<HS>(keys, c[u]);
+                    if (h >= 0) vals[h] = vals[h] + x * v[u];
+                }
+                const int32_t r1 = o0 + u < cnt ? __builtin_amdgcn_readlane(y1, o) : 0;
+                for (int32_t q = __builtin_amdgcn_readlane(y0, o) + 64 + lane; q < r1; q += 64) {
+                    const int h = hash_slot<HS>(keys, yc[q]);
+                    if (h >= 0) vals[h] = vals[h] + x * yv[q];
+                }
+                wave_fence();
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                c[u] = cn[u];
+                v[u] = vn[u];
+            }
         }
-        wave_fence();
     }
     // the table's columns packed into a list, then ranked against it
     const int32_t base = cp[row], cnt = cp[row + 1] - base;
@@ -883,7 +1008,7 @@ double amg_condition(lh_ctx* ctx, int64_t n, const int32_t* rp, const int32_t* c
                      const double* dinv) {
     DevBuf x(n * 8), y(n * 8), part(2 * kRB * 8);
     k_fill_one<<<nblocks(n, 256), 256, 0, ctx->stream>>>(n, dinv, x.as<double>());
-    k_amg_power<<<nblocks_xcd(n, 256), 256, 0, ctx->stream>>>(n, rp, cl, kv, dinv, x.as<double>(), y.as<double>());
+    k_amg_power<8><<<nblocks_xcd(n * 8, 256), 256, 0, ctx->stream>>>(n, rp, cl, kv, dinv, x.as<double>(), y.as<double>());
     k_amg_rayleigh<<<kRB, 256, 0, ctx->stream>>>(n, dinv, x.as<double>(), y.as<double>(), part.as<double>());
     LH_CHECK_LAUNCH();
     double hp[2 * kRB], d = 0.0, k = 0.0;
@@ -915,7 +1040,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
     const int32_t *rp = rp0, *cl = cl0;
     const double* kv = kv0;
     DevBuf x(n0 * 8), y(n0 * 8), part(2 * kRB * 8), key(n0 * 8), key2(n0 * 8), agg(n0 * 4), agg2(n0 * 4),
-        cnt((n0 + 1) * 4), idx((n0 + 1) * 4);
+        cnt((n0 + 1) * 4), idx((n0 + 1) * 4), strong;
     double theta = kTheta;
     for (int l = 0; l < kMaxLevels; ++l) {
         levels.emplace_back();
@@ -933,7 +1058,9 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
             lv.ekv = ekv;
         }
         const unsigned nb = nblocks(n, 256), nbx = nblocks_xcd(n, 256);
-        k_amg_diag<<<nb, 256, 0, st>>>(n, rp, cl, kv, dinv, x.as<double>(), bad);
+        const int g = lanes_for(nnz, n);
+        const unsigned nbg = nblocks_xcd(n * g, 256);
+        with_lanes(g, [&](auto G) { k_amg_diag<G.v><<<nbg, 256, 0, st>>>(n, rp, cl, kv, dinv, x.as<double>(), bad); });
         LH_CHECK_LAUNCH();
         if (n <= kCoarsest) {
             // last level: its inverse
@@ -952,28 +1079,33 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         }
         double *xa = x.as<double>(), *ya = y.as<double>();
         for (int q = 0; q < kPowerSteps; ++q) {
-            k_amg_power<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, xa, ya);
+            with_lanes(g, [&](auto G) { k_amg_power<G.v><<<nbg, 256, 0, st>>>(n, rp, cl, kv, dinv, xa, ya); });
             if (q + 1 < kPowerSteps) std::swap(xa, ya);
         }
         k_amg_rayleigh<<<kRB, 256, 0, st>>>(n, dinv, xa, ya, part.as<double>());
         LH_CHECK_LAUNCH();
         // aggregates
+        strong.ensure((size_t)nnz * 4);
         const double th2 = theta * theta;
         theta *= 0.5;
         auto* ta = key.as<unsigned long long>();
         auto* tb = key2.as<unsigned long long>();
         k_mis_init<<<nb, 256, 0, st>>>(n, dinv, ta);
-        for (int r = 0; r < kMisRounds; ++r) {
-            k_mis_spread<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, th2, ta, tb);
-            k_mis_decide<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, th2, tb, ta);
-        }
+        int32_t* sc = strong.as<int32_t>();
+        with_lanes(g, [&](auto G) {
+            k_strong<G.v><<<nbg, 256, 0, st>>>(n, rp, cl, kv, dinv, th2, sc);
+            for (int r = 0; r < kMisRounds; ++r) {
+                k_mis_spread<G.v><<<nbg, 256, 0, st>>>(n, rp, sc, ta, tb);
+                k_mis_decide<G.v><<<nbg, 256, 0, st>>>(n, rp, sc, tb, ta);
+            }
+        });
         k_mis_flag<<<nb, 256, 0, st>>>(n, ta, cnt.as<int32_t>());
         LH_CHECK_LAUNCH();
         exclusive_scan_i32(ctx, cnt.as<int32_t>(), idx.as<int32_t>(), n);
         k_agg_roots<<<nb, 256, 0, st>>>(n, cnt.as<int32_t>(), idx.as<int32_t>(), agg.as<int32_t>());
         int32_t *ga = agg.as<int32_t>(), *gb = agg2.as<int32_t>();
         for (int r = 0; r < 3; ++r) {
-            k_agg_join<<<nbx, 256, 0, st>>>(n, rp, cl, kv, dinv, th2, ga, gb);
+            with_lanes(g, [&](auto G) { k_agg_join<G.v><<<nbg, 256, 0, st>>>(n, rp, sc, kv, ga, gb); });
             std::swap(ga, gb);
         }
         LH_CHECK_LAUNCH();
@@ -1161,25 +1293,6 @@ void Amg::prepare(int m_) {
 }
 
 namespace {
-
-template <int V>
-struct IntC {
-    static constexpr int v = V;
-};
-// lanes for a row of the mean length: about four entries a lane
-int lanes_for(int64_t nnz, int64_t n) {
-    const int64_t avg = n > 0 ? nnz / n : 0;
-    return avg >= 40 ? 16 : avg >= 20 ? 8 : avg >= 8 ? 4 : 1;
-}
-template <typename F>
-void with_lanes(int g, F&& f) {
-    switch (g) {
-        case 1: f(IntC<1>{}); break;
-        case 4: f(IntC<4>{}); break;
-        case 8: f(IntC<8>{}); break;
-        default: f(IntC<16>{}); break;
-    }
-}
 
 // lanes of four columns for a block row
 template <typename F>

@@ -125,6 +125,21 @@ def test_rows_with_many_entries():
     assert np.linalg.norm(b - a @ x) <= 1e-11 * np.linalg.norm(b)
 
 
+@pytest.mark.parametrize("spokes", [1000, 1024, 1025, 1500])  # entries of the longest row of P^T: about one a spoke
+def test_long_coarse_rows(spokes):
+    ctx = _lib.default_context()
+    n = 6001
+    i = np.arange(n - 1)
+    r, c = np.r_[i, np.full(spokes, n - 1)], np.r_[(i + 1) % (n - 1), np.arange(spokes)]
+    w = sparse.coo_matrix((np.r_[np.ones(n - 1), np.full(spokes, 0.01)], (r, c)), shape=(n, n)).tocsr()
+    w = w + w.T
+    a = sparse.csr_matrix(sparse.diags(np.asarray(w.sum(axis=1)).ravel() + 1e-4) - w)
+    b = np.random.default_rng(spokes).standard_normal(n)
+    x, st = _lib.pcg(ctx, _lib.DeviceCSR.from_scipy(ctx, a), None, 0.0, 1.0, b, rtol=1e-12)
+    assert st.fallback_used == 0 and st.iterations < 120
+    assert np.linalg.norm(b - a @ x) <= 1e-11 * np.linalg.norm(b)
+
+
 def _eig_problem(name):
     if name == "tail":  # 642 rows: every level in the one-launch tail
         return Solver(TriaMesh(*meshgen.perturbed_sphere(3, np.random.default_rng(1), axes=(1.3, 0.8, 1.0), sigma=0.02)))
