@@ -960,27 +960,37 @@ k_blk_restrict(int64_t n, int ld, const int32_t* __restrict__ mp, const int32_t*
         if (c0 < ld && part == 0) *reinterpret_cast<float4*>(out + row * ld + c0) = y;
     }
 }
-// b = W in FP32, columns m .. ld - 1 zero
+// b = the columns perm[0 .. m - 1] of W (all in order when perm is null) in
+// FP32, columns m .. ld - 1 zero
 template <typename WT>
-__global__ void k_blk_in(int64_t n, int m, int ld, const WT* __restrict__ W, int ldw, float* __restrict__ b) {
+__global__ void k_blk_in(int64_t n, int m, int ld, const WT* __restrict__ W, int ldw, const int32_t* __restrict__ perm,
+                         float* __restrict__ b) {
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= n * ld) return;
     const int64_t i = gid / ld;
     const int c = (int)(gid - i * ld);
-    b[gid] = c < m ? (float)W[i * ldw + c] : 0.f;
+    b[gid] = c < m ? (float)W[i * ldw + (perm ? perm[c] : c)] : 0.f;
 }
-// W = w1 x1 + w2 x2 (+ w3 x3)
+// the same columns of W = w1 x1 + w2 x2 (+ w3 x3); with perm, the total - m
+// other columns perm[m ..] times dinv (Jacobi)
 template <typename WT>
-__global__ void k_blk_out(int64_t n, int m, int ld, const float* __restrict__ x1, const float* __restrict__ x2,
-                          const float* __restrict__ x3, double w1, double w2, double w3, WT* __restrict__ W, int ldw) {
+__global__ void k_blk_out(int64_t n, int m, int total, int ld, const float* __restrict__ x1,
+                          const float* __restrict__ x2, const float* __restrict__ x3, double w1, double w2, double w3,
+                          const double* __restrict__ dinv, const int32_t* __restrict__ perm, WT* __restrict__ W,
+                          int ldw) {
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= n * m) return;
-    const int64_t i = gid / m;
-    const int c = (int)(gid - i * m);
+    if (gid >= n * total) return;
+    const int64_t i = gid / total;
+    const int c = (int)(gid - i * total);
+    WT* w = W + i * ldw + (perm ? perm[c] : c);
+    if (c >= m) {
+        *w = (WT)((double)*w * dinv[i]);
+        return;
+    }
     const int64_t o = i * ld + c;
     double v = w1 * (double)x1[o] + w2 * (double)x2[o];
     if (x3) v += w3 * (double)x3[o];
-    W[i * ldw + c] = (WT)v;
+    *w = (WT)v;
 }
 __global__ void k_narrow(int64_t cnt, const double* __restrict__ s, float* __restrict__ d) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1495,7 +1505,7 @@ void Amg::cycle_blocks(int l, int w, const float* b, float* x) {
 }
 
 template <typename WT>
-void Amg::apply_blocks(WT* W, int ldw, int cols) {
+void Amg::apply_blocks(WT* W, int ldw, int cols, int total, const int32_t* perm) {
     if (cols > m) LH_THROW(LH_ERR_ARG, "multigrid block width %d exceeds %d", cols, m);
     const int w = (cols + 3) / 4 * 4;
     const int64_t n = levels[0].n;
@@ -1503,24 +1513,26 @@ void Amg::apply_blocks(WT* W, int ldw, int cols) {
     const double th = 0.5 * (kBlkHi + lo), de = 0.5 * (kBlkHi - lo), sig = th / de;
     const double rho1 = 1.0 / sig, rho2 = 1.0 / (2.0 * sig - rho1), rho3 = 1.0 / (2.0 * sig - rho2);
     const double p2 = rho2 * rho1, q2 = 2.0 * rho2 / de, p3 = rho3 * rho2, q3 = 2.0 * rho3 / de;
-    k_blk_in<<<nblocks(n * w, 256), 256, 0, ctx->stream>>>(n, cols, w, W, ldw, bin);
+    k_blk_in<<<nblocks(n * w, 256), 256, 0, ctx->stream>>>(n, cols, w, W, ldw, perm, bin);
     LH_CHECK_LAUNCH();
     cycle_blocks(0, w, bin, bx1);
     blk_step<kBlkRes>(0, w, bin, bx1, fb[0], 0.f, 0.f, (float)(1.0 / th));
-    const unsigned nb = nblocks(n * cols, 256);
+    const unsigned nb = nblocks(n * total, 256);
+    const double* di = levels[0].d.dinv;
     if (cycles == 2) {
         cycle_blocks(0, w, fb[0], fx[0]);
-        k_blk_out<<<nb, 256, 0, ctx->stream>>>(n, cols, w, bx1, fx[0], nullptr, (1.0 + p2) / th, q2, 0.0, W, ldw);
+        k_blk_out<WT><<<nb, 256, 0, ctx->stream>>>(n, cols, total, w, bx1, fx[0], nullptr, (1.0 + p2) / th, q2, 0.0, di,
+                                                   perm, W, ldw);
     } else {
         cycle_blocks(0, w, fb[0], bx2);
         blk_step<kBlkMix>(0, w, fb[0], bx2, bin, (float)-p2, (float)(1.0 + p2), (float)q2);  // r_3 over b
         cycle_blocks(0, w, bin, fx[0]);
-        k_blk_out<<<nb, 256, 0, ctx->stream>>>(n, cols, w, bx1, bx2, fx[0], (1.0 + p2 + p3 * p2) / th,
-                                               (1.0 + p3) * q2, q3, W, ldw);
+        k_blk_out<WT><<<nb, 256, 0, ctx->stream>>>(n, cols, total, w, bx1, bx2, fx[0],
+                                                   (1.0 + p2 + p3 * p2) / th, (1.0 + p3) * q2, q3, di, perm, W, ldw);
     }
     LH_CHECK_LAUNCH();
 }
-template void Amg::apply_blocks<double>(double*, int, int);
-template void Amg::apply_blocks<float>(float*, int, int);
+template void Amg::apply_blocks<double>(double*, int, int, int, const int32_t*);
+template void Amg::apply_blocks<float>(float*, int, int, int, const int32_t*);
 
 }  // namespace lh

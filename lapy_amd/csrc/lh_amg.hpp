@@ -53,9 +53,11 @@ struct Amg {
     // the block cycle for at most m columns: FP32 copies and work blocks.
     // ell_w == 8: the columns of an ELL copy of the finest level's pattern
     void prepare_blocks(int m, int ell_w, const int32_t* ecl);
-    // W (n x cols, leading dimension ldw) <- p(M K) M W, in FP32
+    // columns perm[0 .. cols - 1] of W (leading dimension ldw; null: the first
+    // cols) <- p(M K) M times them, in FP32; columns perm[cols .. total - 1] <-
+    // D^-1 times them
     template <typename WT>  // double or float
-    void apply_blocks(WT* W, int ldw, int cols);
+    void apply_blocks(WT* W, int ldw, int cols, int total, const int32_t* perm);
 
     // products with the finest K in one application: four a cycle, one between two
     int block_products() const { return 5 * cycles - 1; }

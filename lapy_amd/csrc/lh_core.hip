@@ -81,6 +81,21 @@ void exclusive_scan_i32(lh_ctx* ctx, const int32_t* in, int32_t* out, int64_t n)
 // between device and pinned memory is one DMA (or kernel) on the stream,
 // where pageable memory takes the runtime's shared staging path, which
 // serialises the concurrent solver streams of the batched eigensolver.
+// up to kStageItems small device arrays into the pinned stage in one launch:
+// the copies of the iterations' scalars are pure launch cost, 4 to 5 us each as
+// separate blits
+constexpr int kStageItems = 4;
+constexpr size_t kStageBytes = 16 << 10;
+struct StageItems {
+    const uint32_t* src[kStageItems];
+    uint32_t words[kStageItems], at[kStageItems];
+};
+__global__ void __launch_bounds__(256) k_stage(StageItems q, uint32_t* __restrict__ stage) {
+#pragma unroll
+    for (int i = 0; i < kStageItems; ++i)
+        for (uint32_t w = threadIdx.x; w < q.words[i]; w += 256) stage[q.at[i] + w] = q.src[i][w];
+}
+
 void d2h_n(lh_ctx* ctx, const Xfer* x, int cnt) {
     size_t total = 0;
     for (int i = 0; i < cnt; ++i) total += (x[i].bytes + 63) & ~size_t(63);
@@ -92,7 +107,22 @@ void d2h_n(lh_ctx* ctx, const Xfer* x, int cnt) {
     }
     char* stage = static_cast<char*>(ctx->host_stage);
     size_t off = 0;
-    for (int i = 0; i < cnt; ++i) {
+    // whole words of several arrays, few enough for one workgroup
+    bool small = cnt > 1 && cnt <= kStageItems && total <= kStageBytes;
+    for (int i = 0; i < cnt && small; ++i)
+        small = x[i].bytes % 4 == 0 && (reinterpret_cast<uintptr_t>(x[i].dev) & 3) == 0;
+    if (small) {
+        StageItems q{};
+        for (int i = 0; i < cnt; ++i) {
+            q.src[i] = static_cast<const uint32_t*>(x[i].dev);
+            q.words[i] = (uint32_t)(x[i].bytes / 4);
+            q.at[i] = (uint32_t)(off / 4);
+            off += (x[i].bytes + 63) & ~size_t(63);
+        }
+        k_stage<<<1, 256, 0, ctx->stream>>>(q, reinterpret_cast<uint32_t*>(stage));
+        LH_CHECK_LAUNCH();
+    }
+    for (int i = 0; i < cnt && !small; ++i) {
         if (x[i].bytes) HIPX(hipMemcpyAsync(stage + off, x[i].dev, x[i].bytes, hipMemcpyDeviceToHost, ctx->stream));
         off += (x[i].bytes + 63) & ~size_t(63);
     }

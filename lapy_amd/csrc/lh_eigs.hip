@@ -394,16 +394,19 @@ struct Lobpcg {
                     std::memcpy(pin + (size_t)m * 8, perm.data(), (size_t)m * 4);
                     HIPX(hipMemcpyAsync(lockbuf.p, pin, (size_t)m * 12, hipMemcpyHostToDevice, ctx->stream));
                     T* W = Sp() + m;
-                    T* tmp = S2.as<T>() + m;  // S2 is free until the update below
-                    gather_cols<T>(ctx, n, m, W, ld, tmp, ld,
-                                   reinterpret_cast<const int32_t*>(lockbuf.as<char>() + (size_t)m * 8));
-                    copy_block<T, T>(ctx, n, m, tmp, ld, W, ld);
-                    if (amg_on) amg->apply_blocks<T>(W, ld, ma);
-                    else cheb->apply(W, ld, ma, lockbuf.as<double>());
-                    rowscale<T>(ctx, n, m - ma, W + ma, ld, dinv.as<double>());
+                    const int32_t* order = reinterpret_cast<const int32_t*>(lockbuf.as<char>() + (size_t)m * 8);
+                    if (amg_on) {  // takes and leaves the columns where they are
+                        amg->apply_blocks<T>(W, ld, ma, m, order);
+                    } else {
+                        T* tmp = S2.as<T>() + m;  // S2 is free until the update below
+                        gather_cols<T>(ctx, n, m, W, ld, tmp, ld, order);
+                        copy_block<T, T>(ctx, n, m, tmp, ld, W, ld);
+                        cheb->apply(W, ld, ma, lockbuf.as<double>());
+                        rowscale<T>(ctx, n, m - ma, W + ma, ld, dinv.as<double>());
+                    }
                     st.poly_columns += ma;
                 } else {
-                    if (amg_on) amg->apply_blocks<T>(Sp() + m, ld, m);
+                    if (amg_on) amg->apply_blocks<T>(Sp() + m, ld, m, m, nullptr);
                     else cheb->apply(Sp() + m, ld, m, cs1.as<double>());  // cs1: ||w_c||^2 from the test above
                     st.poly_columns += m;
                 }
