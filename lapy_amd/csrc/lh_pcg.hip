@@ -138,59 +138,46 @@ __device__ __forceinline__ double allsum_partials(const double* __restrict__ par
     return block_allsum(t, sh);
 }
 
-// two block sums with one pair of barriers (each formed as block_allsum forms
-// it); sh holds 2 * blockDim / 64 doubles
-__device__ __forceinline__ void block_allsum2(double a, double b, double* sh, double& ra, double& rb) {
+// N block sums with one pair of barriers (each formed as block_allsum forms
+// it), in every thread; sh holds N * blockDim / 64 doubles
+template <int N>
+__device__ __forceinline__ void block_allsum_n(double (&t)[N], double* sh) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        a += __shfl_down(a, o, 64);
-        b += __shfl_down(b, o, 64);
-    }
-    const int nw = (int)(blockDim.x >> 6);
-    __syncthreads();  // sh free (an earlier call's readers are done)
-    if ((threadIdx.x & 63) == 0) {
-        sh[threadIdx.x >> 6] = a;
-        sh[nw + (threadIdx.x >> 6)] = b;
-    }
-    __syncthreads();
-    double ta = 0.0, tb = 0.0;
-    for (int k = 0; k < nw; ++k) {
-        ta += sh[k];
-        tb += sh[nw + k];
-    }
-    ra = ta;
-    rb = tb;
-}
-
-// K such sums at once: every partial load is issued before the first
-// reduction waits, and one pair of barriers serves all K (each sum is formed
-// in the order allsum_partials uses, so the results are the same).  sh holds
-// K * blockDim / 64 doubles.
-template <int K>
-__device__ __forceinline__ void allsum_partials_k(const double* const (&part)[K], const int (&np)[K], int m, int c,
-                                                  double* sh, double (&out)[K]) {
-    double t[K];
+    for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
-    for (int q = 0; q < K; ++q) {
-        t[q] = 0.0;
-        for (int b = threadIdx.x; b < np[q]; b += blockDim.x) t[q] += part[q][(int64_t)b * m + c];
-    }
-#pragma unroll
-    for (int q = 0; q < K; ++q)
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) t[q] += __shfl_down(t[q], o, 64);
+        for (int q = 0; q < N; ++q) t[q] += __shfl_down(t[q], o, 64);
     const int nw = (int)(blockDim.x >> 6);
     __syncthreads();  // sh free (an earlier call's readers are done)
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
-        for (int q = 0; q < K; ++q) sh[q * nw + (threadIdx.x >> 6)] = t[q];
+        for (int q = 0; q < N; ++q) sh[q * nw + (threadIdx.x >> 6)] = t[q];
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < K; ++q) {
+    for (int q = 0; q < N; ++q) {
         double r = 0.0;
         for (int k = 0; k < nw; ++k) r += sh[q * nw + k];
-        out[q] = r;
+        t[q] = r;
     }
+}
+
+// K sums of partials of each of the columns c0 .. c0 + mc - 1 at once, out[K c + k]:
+// every partial load is issued before the first reduction waits, and one pair
+// of barriers serves all (each sum is formed in the order allsum_partials
+// uses, so the results do not depend on how many columns share the launch).
+// A pair of barriers a column cost 2.5 us a column at the head of each kernel.
+template <int K, int MC>
+__device__ __forceinline__ void allsum_partials_k(const double* const (&part)[K], const int (&np)[K], int m, int c0,
+                                                  int mc, double* sh, double (&out)[K * MC]) {
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+#pragma unroll
+        for (int c = 0; c < MC; ++c) out[K * c + q] = 0.0;
+        for (int b = threadIdx.x; b < np[q]; b += blockDim.x)
+#pragma unroll
+            for (int c = 0; c < MC; ++c)
+                if (c < mc) out[K * c + q] += part[q][(int64_t)b * m + c0 + c];
+    }
+    block_allsum_n<K * MC>(out, sh);
 }
 
 // CG state on the device (m columns).  Iteration k reads r_k.z_k and r_k.r_k
@@ -217,25 +204,23 @@ k_cg_dir(int64_t n, int m, int c0, int mc, int par, const int32_t* __restrict__ 
          const int32_t* __restrict__ cols, const double* __restrict__ kv, const double* __restrict__ Z,
          double* __restrict__ P, double* __restrict__ Q, const double* __restrict__ R, CgState s) {
     if (s.status[0]) return;  // converged: the enqueued iterations end here
-    __shared__ double sh[4 * kIBS / 64];
+    __shared__ double sh[3 * MC * kIBS / 64];
     constexpr int GPB = kIBS / LPR;
     const int lane = threadIdx.x % LPR, grp = threadIdx.x / LPR;
     const int64_t rpb = (n + gridDim.x - 1) / gridDim.x;
     const int64_t rb = xcd_block() * rpb, re = rb + rpb < n ? rb + rpb : n;
     double bet[MC], pq[MC], sr[MC];
+    {
+        const double* const pp[3] = {s.rz[par], s.rz[par ^ 1], s.rr[par]};
+        const int np[3] = {s.nb_rz, s.nb_rz, s.nb_upd};
+        double v[3 * MC];
+        allsum_partials_k<3, MC>(pp, np, m, c0, mc, sh, v);
+        // beta_k = rz_k / rz_{k-1}; 0 for a converged column (and at k = 0,
+        // where P and Q hold zeros anyway)
 #pragma unroll
-    for (int c = 0; c < MC; ++c) {
-        bet[c] = 0.0;
-        pq[c] = sr[c] = 0.0;
-        if (c < mc) {
-            // beta_k = rz_k / rz_{k-1}; 0 for a converged column (and at k = 0,
-            // where P and Q hold zeros anyway)
-            const double* const pp[3] = {s.rz[par], s.rz[par ^ 1], s.rr[par]};
-            const int np[3] = {s.nb_rz, s.nb_rz, s.nb_upd};
-            double v[3];
-            allsum_partials_k<3>(pp, np, m, c0 + c, sh, v);
-            const double rzk = v[0], rzo = v[1], rrk = v[2];
-            bet[c] = (rrk > s.tol2[c0 + c] && rzo != 0.0) ? rzk / rzo : 0.0;
+        for (int c = 0; c < MC; ++c) {
+            pq[c] = sr[c] = 0.0;
+            bet[c] = (c < mc && v[3 * c + 2] > s.tol2[c0 + c] && v[3 * c + 1] != 0.0) ? v[3 * c] / v[3 * c + 1] : 0.0;
         }
     }
     for (int64_t i = rb + grp; i < re; i += GPB) {
@@ -269,16 +254,21 @@ k_cg_dir(int64_t n, int m, int c0, int mc, int par, const int32_t* __restrict__ 
             }
         }
     }
+    constexpr int NS = SING ? 2 : 1;
+    double t[NS * MC];
 #pragma unroll
     for (int c = 0; c < MC; ++c) {
-        if (c >= mc) continue;
-        double bp, bs;
-        block_allsum2(pq[c], SING ? sr[c] : 0.0, sh, bp, bs);
-        if (threadIdx.x == 0) {
-            s.pq[(int64_t)blockIdx.x * m + c0 + c] = bp;
-            if (SING) s.sr[(int64_t)blockIdx.x * m + c0 + c] = bs;
-        }
+        t[NS * c] = pq[c];
+        if (SING) t[NS * c + NS - 1] = sr[c];
     }
+    block_allsum_n<NS * MC>(t, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int c = 0; c < MC; ++c) {
+            if (c >= mc) continue;
+            s.pq[(int64_t)blockIdx.x * m + c0 + c] = t[NS * c];
+            if (SING) s.sr[(int64_t)blockIdx.x * m + c0 + c] = t[NS * c + NS - 1];
+        }
 }
 
 // the same on the operator's ELL copy (W slots per row, padding slots point
@@ -286,30 +276,30 @@ k_cg_dir(int64_t n, int m, int c0, int mc, int par, const int32_t* __restrict__ 
 // and its slots loaded before the gathers, which then go out together;
 // 256-thread blocks, 8 waves per SIMD for W = 8.  A column's arithmetic (the
 // slots summed in order, the same blocks and partials) does not depend on how
-// many columns share the launch, so a block of right-hand sides gives what
-// one solve per column gives.
+// many columns share the launch.  MC columns exactly: tests of the column
+// count between the gathers had serialised them (10,242 rows x 3: 13.2 -> 10.0 us).
 constexpr int kEBS = 256;
 template <int W, int MC, bool SING>
 __global__ void __launch_bounds__(kEBS) __attribute__((amdgpu_waves_per_eu((W <= 8 && MC == 1) ? 8 : 4)))
-k_cg_dir_ell(int64_t n, int m, int c0, int mc, int par, const int32_t* __restrict__ ecols,
+k_cg_dir_ell(int64_t n, int m, int c0, int par, const int32_t* __restrict__ ecols,
              const double* __restrict__ ev, const double* __restrict__ Z, double* __restrict__ P,
              double* __restrict__ Q, const double* __restrict__ R, CgState s) {
     if (s.status[0]) return;
-    __shared__ double sh[4 * kEBS / 64];
+    __shared__ double sh[3 * MC * kEBS / 64];
     const int64_t rpb = (n + gridDim.x - 1) / gridDim.x;
     const int64_t rb = xcd_block() * rpb, re = rb + rpb < n ? rb + rpb : n;
     double bet[MC], pq[MC], sr[MC];
+    {
+        const double* const pp[3] = {s.rz[par], s.rz[par ^ 1], s.rr[par]};
+        const int np[3] = {s.nb_rz, s.nb_rz, s.nb_upd};
+        double v[3 * MC];
+        allsum_partials_k<3, MC>(pp, np, m, c0, MC, sh, v);
+        // beta_k = rz_k / rz_{k-1}; 0 for a converged column (and at k = 0,
+        // where P and Q hold zeros anyway)
 #pragma unroll
-    for (int c = 0; c < MC; ++c) {
-        bet[c] = 0.0;
-        pq[c] = sr[c] = 0.0;
-        if (c < mc) {
-            const double* const pp[3] = {s.rz[par], s.rz[par ^ 1], s.rr[par]};
-            const int np[3] = {s.nb_rz, s.nb_rz, s.nb_upd};
-            double v[3];
-            allsum_partials_k<3>(pp, np, m, c0 + c, sh, v);
-            const double rzk = v[0], rzo = v[1], rrk = v[2];
-            bet[c] = (rrk > s.tol2[c0 + c] && rzo != 0.0) ? rzk / rzo : 0.0;
+        for (int c = 0; c < MC; ++c) {
+            pq[c] = sr[c] = 0.0;
+            bet[c] = (v[3 * c + 2] > s.tol2[c0 + c] && v[3 * c + 1] != 0.0) ? v[3 * c] / v[3 * c + 1] : 0.0;
         }
     }
     for (int64_t i = rb + threadIdx.x; i < re; i += kEBS) {
@@ -317,16 +307,15 @@ k_cg_dir_ell(int64_t n, int m, int c0, int mc, int par, const int32_t* __restric
         double zo[MC], po[MC], qo[MC], ro[MC], acc[MC];
 #pragma unroll
         for (int c = 0; c < MC; ++c) {
-            zo[c] = po[c] = qo[c] = ro[c] = acc[c] = 0.0;
-            if (c < mc) {
-                zo[c] = Z[o + c];
-                po[c] = P[o + c];
-                qo[c] = Q[o + c];
-                if (SING) ro[c] = R[o + c];
-            }
+            acc[c] = 0.0;
+            zo[c] = Z[o + c];
+            po[c] = P[o + c];
+            qo[c] = Q[o + c];
+            ro[c] = SING ? R[o + c] : 0.0;
         }
-        // slots in groups of G (all W at once for one column), in order
-        constexpr int G = MC == 1 ? W : 8;
+        // slots in groups of G (all W at once for one column), in order: the
+        // gathers of a group go out before the first of them is used
+        constexpr int G = MC == 1 ? W : (MC <= 3 ? 8 : 4);
 #pragma unroll
         for (int k0 = 0; k0 < W; k0 += G) {
             int32_t col[G];
@@ -347,25 +336,18 @@ k_cg_dir_ell(int64_t n, int m, int c0, int mc, int par, const int32_t* __restric
                 val[2 * k] = v2.x;
                 val[2 * k + 1] = v2.y;
             }
-            if (MC == 1) {
-                double g[G];
+            double g[G][MC];
 #pragma unroll
-                for (int k = 0; k < G; ++k) g[k] = Z[(int64_t)col[k] * m + c0];
+            for (int k = 0; k < G; ++k)
 #pragma unroll
-                for (int k = 0; k < G; ++k) acc[0] += val[k] * g[k];
-            } else {
+                for (int c = 0; c < MC; ++c) g[k][c] = Z[(int64_t)col[k] * m + c0 + c];
 #pragma unroll
-                for (int k = 0; k < G; ++k) {
-                    const double* zr = Z + (int64_t)col[k] * m + c0;
+            for (int k = 0; k < G; ++k)
 #pragma unroll
-                    for (int c = 0; c < MC; ++c)
-                        if (c < mc) acc[c] += val[k] * zr[c];
-                }
-            }
+                for (int c = 0; c < MC; ++c) acc[c] += val[k] * g[k][c];
         }
 #pragma unroll
         for (int c = 0; c < MC; ++c) {
-            if (c >= mc) continue;
             const double pn = zo[c] + bet[c] * po[c];
             const double qn = acc[c] + bet[c] * qo[c];
             P[o + c] = pn;
@@ -374,27 +356,31 @@ k_cg_dir_ell(int64_t n, int m, int c0, int mc, int par, const int32_t* __restric
             if (SING) sr[c] += ro[c];
         }
     }
+    constexpr int NS = SING ? 2 : 1;
+    double t[NS * MC];
 #pragma unroll
     for (int c = 0; c < MC; ++c) {
-        if (c >= mc) continue;
-        double bp, bs;
-        block_allsum2(pq[c], SING ? sr[c] : 0.0, sh, bp, bs);
-        if (threadIdx.x == 0) {
-            s.pq[(int64_t)blockIdx.x * m + c0 + c] = bp;
-            if (SING) s.sr[(int64_t)blockIdx.x * m + c0 + c] = bs;
-        }
+        t[NS * c] = pq[c];
+        if (SING) t[NS * c + NS - 1] = sr[c];
     }
+    block_allsum_n<NS * MC>(t, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int c = 0; c < MC; ++c) {
+            s.pq[(int64_t)blockIdx.x * m + c0 + c] = t[NS * c];
+            if (SING) s.sr[(int64_t)blockIdx.x * m + c0 + c] = t[NS * c + NS - 1];
+        }
 }
 
 // ---- update: x += alpha p, r = r - mean - alpha q, (z = D^-1 r) -------------
 // alpha_k = rz_k / p.q for an active column (r_k.r_k > tol2), else 0
 template <int BS, int MC, bool SING, bool JAC>
 __global__ void __launch_bounds__(BS)
-k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict__ dinv, const double* __restrict__ P,
+k_cg_update(int64_t n, int m, int c0, int par, const double* __restrict__ dinv, const double* __restrict__ P,
             const double* __restrict__ Q, double* __restrict__ X, double* __restrict__ R, double* __restrict__ Z,
             CgState s, int last_chunk) {
     if (s.status[0]) return;
-    __shared__ double sh[4 * BS / 64];
+    __shared__ double sh[4 * MC * BS / 64];
     // contiguous rows per block, an even count; a thread takes two adjacent
     // rows per step (one 16-byte load per operand for one column)
     int64_t rpb = (n + gridDim.x - 1) / gridDim.x;
@@ -402,21 +388,30 @@ k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict_
     const int64_t rb = blockIdx.x * rpb, re = rb + rpb < n ? rb + rpb : n;
     double al[MC], mu[MC], rz[MC], rr[MC];
     int nact = 0;
+    {
+        constexpr int K = SING ? 4 : 3;
+        double v[K * MC];
+        if constexpr (SING) {
+            const double* const pp[K] = {s.rz[par], s.rr[par], s.pq, s.sr};
+            const int np[K] = {s.nb_rz, s.nb_upd, s.nb_dir, s.nb_dir};
+            allsum_partials_k<K, MC>(pp, np, m, c0, MC, sh, v);
+        } else {
+            const double* const pp[K] = {s.rz[par], s.rr[par], s.pq};
+            const int np[K] = {s.nb_rz, s.nb_upd, s.nb_dir};
+            allsum_partials_k<K, MC>(pp, np, m, c0, MC, sh, v);
+        }
 #pragma unroll
-    for (int c = 0; c < MC; ++c) {
-        al[c] = mu[c] = rz[c] = rr[c] = 0.0;
-        if (c < mc) {
-            const int cc = c0 + c;
-            const double* const pp[4] = {s.rz[par], s.rr[par], s.pq, s.sr};
-            const int np[4] = {s.nb_rz, s.nb_upd, s.nb_dir, SING ? s.nb_dir : 0};
-            double v[4];
-            allsum_partials_k<4>(pp, np, m, cc, sh, v);
-            const double rzk = v[0], rrk = v[1], pqk = v[2];
-            const bool act = rrk > s.tol2[cc];
-            nact += act ? 1 : 0;
-            al[c] = (act && pqk != 0.0) ? rzk / pqk : 0.0;
-            if (SING && act) mu[c] = v[3] / (double)n;
-            if (blockIdx.x == 0 && threadIdx.x == 0) s.rr_out[cc] = rrk;
+        for (int c = 0; c < MC; ++c) {
+            al[c] = mu[c] = rz[c] = rr[c] = 0.0;
+            {
+                const int cc = c0 + c;
+                const double rzk = v[K * c], rrk = v[K * c + 1], pqk = v[K * c + 2];
+                const bool act = rrk > s.tol2[cc];
+                nact += act ? 1 : 0;
+                al[c] = (act && pqk != 0.0) ? rzk / pqk : 0.0;
+                if (SING && act) mu[c] = v[K * c + K - 1] / (double)n;
+                if (blockIdx.x == 0 && threadIdx.x == 0) s.rr_out[cc] = rrk;
+            }
         }
     }
     for (int64_t i = rb + 2 * (int64_t)threadIdx.x; i < re; i += 2 * BS) {
@@ -446,13 +441,10 @@ k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict_
                 vd[h] = JAC ? dinv[row] : 0.0;
 #pragma unroll
                 for (int c = 0; c < MC; ++c) {
-                    vr[h][c] = vq[h][c] = vp[h][c] = vx[h][c] = 0.0;
-                    if (c < mc) {
-                        vr[h][c] = R[o + c];
-                        vq[h][c] = Q[o + c];
-                        vp[h][c] = P[o + c];
-                        vx[h][c] = X[o + c];
-                    }
+                    vr[h][c] = R[o + c];
+                    vq[h][c] = Q[o + c];
+                    vp[h][c] = P[o + c];
+                    vx[h][c] = X[o + c];
                 }
             }
         }
@@ -483,7 +475,6 @@ k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict_
                 const int64_t o = (i + h) * m + c0;
 #pragma unroll
                 for (int c = 0; c < MC; ++c) {
-                    if (c >= mc) continue;
                     R[o + c] = nr[h][c];
                     X[o + c] = nx[h][c];
                     if (JAC) Z[o + c] = nz[h][c];
@@ -491,16 +482,20 @@ k_cg_update(int64_t n, int m, int c0, int mc, int par, const double* __restrict_
             }
         }
     }
+    constexpr int NS = JAC ? 2 : 1;
+    double t[NS * MC];
 #pragma unroll
     for (int c = 0; c < MC; ++c) {
-        if (c >= mc) continue;
-        double b1, b2;
-        block_allsum2(rr[c], JAC ? rz[c] : 0.0, sh, b1, b2);
-        if (threadIdx.x == 0) {
-            s.rr[par ^ 1][(int64_t)blockIdx.x * m + c0 + c] = b1;
-            if (JAC) s.rz[par ^ 1][(int64_t)blockIdx.x * m + c0 + c] = b2;
-        }
+        t[NS * c] = rr[c];
+        if (JAC) t[NS * c + NS - 1] = rz[c];
     }
+    block_allsum_n<NS * MC>(t, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int c = 0; c < MC; ++c) {
+            s.rr[par ^ 1][(int64_t)blockIdx.x * m + c0 + c] = t[NS * c];
+            if (JAC) s.rz[par ^ 1][(int64_t)blockIdx.x * m + c0 + c] = t[NS * c + NS - 1];
+        }
     // status for the host (and the early exit of later launches): every block
     // reached the same decision from the same partials; block 0 records it.
     // The columns of this launch are all converged only if nact == 0; the
@@ -734,7 +729,7 @@ struct Launcher {
         if constexpr (MC <= 4) {
           if (ew) {
 #define LH_DIRE(W_, S) \
-    k_cg_dir_ell<W_, MC, S><<<nb_ell, kEBS, 0, ctx->stream>>>(n, m, c0, mc, par, ecols, ev, Z, P, Q, R, s)
+    k_cg_dir_ell<W_, MC, S><<<nb_ell, kEBS, 0, ctx->stream>>>(n, m, c0, par, ecols, ev, Z, P, Q, R, s)
             switch (ew) {
                 case 8: if (sing) LH_DIRE(8, true); else LH_DIRE(8, false); break;
                 case 16: if (sing) LH_DIRE(16, true); else LH_DIRE(16, false); break;
@@ -762,29 +757,33 @@ struct Launcher {
         for (int c0 = 0; c0 < m; c0 += w) {
             const int mc = std::min(w, m - c0);
             if (mc == 1) dir_mc<1>(c0, mc, par, sing, Z, P, Q, R, s);
-            else if (mc <= 4) dir_mc<4>(c0, mc, par, sing, Z, P, Q, R, s);
+            else if (mc == 2) dir_mc<2>(c0, mc, par, sing, Z, P, Q, R, s);
+            else if (mc == 3) dir_mc<3>(c0, mc, par, sing, Z, P, Q, R, s);
+            else if (mc == 4) dir_mc<4>(c0, mc, par, sing, Z, P, Q, R, s);
             else dir_mc<8>(c0, mc, par, sing, Z, P, Q, R, s);
         }
     }
     template <int MC>
-    void update_mc(int c0, int mc, int par, bool sing, bool jac, const double* dinv, const double* P,
+    void update_mc(int c0, int par, bool sing, bool jac, const double* dinv, const double* P,
                    const double* Q, double* X, double* R, double* Z, const CgState& s, int last) {
 #define LH_UPD(S, J)                                                                                              \
-    (small ? k_cg_update<kBS, MC, S, J><<<nb, kBS, 0, ctx->stream>>>(n, m, c0, mc, par, dinv, P, Q, X, R, Z, s, last) \
-           : k_cg_update<kIBS, MC, S, J><<<nb, kIBS, 0, ctx->stream>>>(n, m, c0, mc, par, dinv, P, Q, X, R, Z, s, last))
+    (small ? k_cg_update<kBS, MC, S, J><<<nb, kBS, 0, ctx->stream>>>(n, m, c0, par, dinv, P, Q, X, R, Z, s, last) \
+           : k_cg_update<kIBS, MC, S, J><<<nb, kIBS, 0, ctx->stream>>>(n, m, c0, par, dinv, P, Q, X, R, Z, s, last))
         if (sing) { if (jac) LH_UPD(true, true); else LH_UPD(true, false); }
         else { if (jac) LH_UPD(false, true); else LH_UPD(false, false); }
 #undef LH_UPD
         LH_CHECK_LAUNCH();
     }
-    // two columns per launch at most (two rows of four columns would spill)
+    // three columns per launch at most (two rows of four columns would spill)
     void update(int par, bool sing, bool jac, const double* dinv, const double* P, const double* Q, double* X,
                 double* R, double* Z, const CgState& s) {
-        for (int c0 = 0; c0 < m; c0 += 2) {
-            const int mc = std::min(2, m - c0);
-            const int last = c0 + 2 >= m;
-            if (mc == 1) update_mc<1>(c0, mc, par, sing, jac, dinv, P, Q, X, R, Z, s, last);
-            else update_mc<2>(c0, mc, par, sing, jac, dinv, P, Q, X, R, Z, s, last);
+        for (int c0 = 0; c0 < m;) {
+            const int mc = m - c0 == 4 ? 2 : std::min(3, m - c0);
+            const int last = c0 + mc >= m;
+            if (mc == 1) update_mc<1>(c0, par, sing, jac, dinv, P, Q, X, R, Z, s, last);
+            else if (mc == 2) update_mc<2>(c0, par, sing, jac, dinv, P, Q, X, R, Z, s, last);
+            else update_mc<3>(c0, par, sing, jac, dinv, P, Q, X, R, Z, s, last);
+            c0 += mc;
         }
     }
     // partials (nb per column) of r.z into part
