@@ -318,10 +318,10 @@ def run_workload(args, ctx, _lib, meshgen):
         k = 50
         gold = golden("batch_256_k50.json") if nb == 256 else None
         base = [_lib.DeviceMesh(ctx, v, t) for v, t in meshes]
-        # preconditioner: Chebyshev-Jacobi (default), plain Jacobi, or the
-        # learned network, trained first (untimed) on six other meshes of
+        # preconditioner: the default (multigrid cycles, the Chebyshev polynomial where they
+        # do not suit), plain Jacobi, or the learned network, trained first (untimed) on six other meshes of
         # the same family (levels 3 and 4, seeds outside the batch)
-        popts = {"cheb": {}, "jacobi": {"poly_degree": 1},
+        popts = {"default": {}, "cheb": {}, "jacobi": {"poly_degree": 1},
                  "learned": {"precond": _lib.LH_PRECOND_LEARNED},
                  "auto": {"precond": _lib.LH_PRECOND_AUTO}}[args.precond]
         net = None
@@ -416,7 +416,7 @@ def run_learned(args, ctx, _lib, meshgen, out):
     solver's own residuals of 512 seeded meshes of icosphere levels 4-7, then
     applied inside the batched LOBPCG (k = 50) and the heat PCG on 64
     held-out level-7 meshes (163,842 vertices each), against plain Jacobi
-    (the fallback and the plain form) and Chebyshev-Jacobi (the default).
+    (the fallback and the plain form) and the default (multigrid cycles).
     Every solve ends at the same FP64 residual test, so the eigenvalues of
     all forms agree; the line reports throughput, iterations and fallbacks of
     each form and the roofline of the network's layer kernel."""
@@ -460,7 +460,7 @@ def run_learned(args, ctx, _lib, meshgen, out):
     # first chunk only, to show how the network itself fares
     chunk = 16
     nall = len(mats)
-    forms = [("chebyshev_fp64", {}, nall), ("jacobi_fp64", {"poly_degree": 1}, nall),
+    forms = [("default_fp64", {}, nall), ("jacobi_fp64", {"poly_degree": 1}, nall),
              ("learned_fp64", {"precond": _lib.LH_PRECOND_LEARNED}, nall),
              ("learned_mixed", {"precond": _lib.LH_PRECOND_LEARNED, "precision": _lib.LH_PREC_MIXED}, nall),
              ("jacobi_mixed", {"poly_degree": 1, "precision": _lib.LH_PREC_MIXED}, nall),
@@ -497,7 +497,7 @@ def run_learned(args, ctx, _lib, meshgen, out):
         results[name] = {"meshes": cnt, "eigenpairs_per_s": round(k * cnt / dt, 3), "seconds": round(dt, 3),
                          "lobpcg_iterations_min_median_max": [int(min(its)), int(np.median(its)), int(max(its))],
                          "fallbacks_to_jacobi": fb, "not_converged": nconv,
-                         "eig_rel_diff_vs_chebyshev_fp64": err}
+                         "eig_rel_diff_vs_default_fp64": err}
     # heat PCG on each held-out mesh (lumped mass, t = avg edge length^2)
     heat = {"jacobi": [0, 0.0], "learned": [0, 0.0]}
     hfb = 0
@@ -572,8 +572,8 @@ def main():
     ap.add_argument("--batch-count", type=int, default=256, help="batch workload: number of meshes")
     ap.add_argument("--batch-workers", type=int, default=0,
                     help="batch workload: solver workers (0: autotuned on every eighth mesh)")
-    ap.add_argument("--precond", default="cheb", choices=["cheb", "jacobi", "learned", "auto"],
-                    help="batch workload: Chebyshev-Jacobi (default), plain Jacobi, the learned network, or auto "
+    ap.add_argument("--precond", default="default", choices=["default", "cheb", "jacobi", "learned", "auto"],
+                    help="batch workload: multigrid cycles (default; cheb: its earlier name), plain Jacobi, the learned network, or auto "
                          "(the network on the meshes where the polynomial would be plain Jacobi)")
     ap.add_argument("--kernels-only", action="store_true",
                     help="skip the eigensolves; only the roofline timings of the two measured kernels")
@@ -712,7 +712,22 @@ def main():
     m = base.clone()
     A, B = m.assemble(_lib.LH_TRIA, False, np.float64)
     nnz = A.nnz
-    # dominant kernel: one Chebyshev step of the preconditioner (FP32 arithmetic, block of m = 64 columns)
+    # dominant kernel: the FP64 matrix-core products of the tall-skinny blocks (a third of the device
+    # time); timed here in its most frequent form, the in-place Cholesky-QR update of [W P] (2 m columns
+    # of a basis of 3 m, upper triangular factor): every value read and written once
+    mb = args.block if args.block else 64
+    ld = 3 * mb
+    rng = np.random.default_rng(0)
+    _, us_g = _lib.block_gemm(ctx, None, 2 * mb, np.triu(rng.random((2 * mb, 2 * mb))), rng.random((nv, ld)),
+                              iters=20, upper=True, inplace=True)
+    gemm_bytes = 16 * nv * 2 * mb
+    ach_g = gemm_bytes / (us_g * 1e-6) / 1e9
+    roofline = {"bound": "hbm", "achieved": round(ach_g, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(ach_g / HBM_PEAK_GBS, 4), "traffic": None,
+                "kernel": f"k_gemm_mfma, in-place update of {2 * mb} FP64 columns",
+                "avg_us": round(us_g, 2), "algorithmic_bytes": int(gemm_bytes)}
+    # one Chebyshev step of the polynomial preconditioner (an explicit degree, or a matrix that multigrid
+    # does not suit; not in the default step): FP32 arithmetic, block of m = 64 columns
     mcols = args.block if args.block else 64
     half = storage == _lib.LH_STORE_F16 or (storage == _lib.LH_STORE_AUTO and mcols % 8 == 0)
     us_c = _lib.time_cheb_step(ctx, A, B, mcols, iters=50, reorder=True,
@@ -726,11 +741,11 @@ def main():
     kname = "k_cheb_step_e (ELL, FP16 storage)" if half else "k_cheb_step_v (FP32 storage)"
     # traffic: measured by rocprofv3 on exactly this configuration (L8, m = 64, FP16 storage)
     profiled = args.level == 8 and mcols == 64 and half
-    roofline = {"bound": "hbm", "achieved": round(ach_c, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(ach_c / HBM_PEAK_GBS, 4),
-                "traffic": profiled_traffic("cheb_step_e_l8_m64_traffic.txt") if profiled else None,
-                "kernel": f"{kname}, Chebyshev-Jacobi preconditioner step, m={mcols}",
-                "avg_us": round(us_c, 2), "algorithmic_bytes": int(cheb_bytes)}
+    roofline_cheb = {"bound": "hbm", "achieved": round(ach_c, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": round(ach_c / HBM_PEAK_GBS, 4),
+                     "traffic": profiled_traffic("cheb_step_e_l8_m64_traffic.txt") if profiled else None,
+                     "kernel": f"{kname}, Chebyshev-Jacobi preconditioner step, m={mcols}",
+                     "avg_us": round(us_c, 2), "algorithmic_bytes": int(cheb_bytes)}
     # the metric's second figure: numeric assembly
     # (rows in the pattern's locality order for meshes of >= 65,536 vertices, else in mesh order)
     us = m.time_assembly(_lib.LH_TRIA, False, A, B, iters=20)
@@ -770,9 +785,10 @@ def main():
                    "vertices": nv, "triangles": nf, "k": args.k, "precision": args.precision,
                    "lobpcg_iterations": st.iterations if st else None,
                    "lobpcg_iterations_fp32": st.iterations_fp32 if st else None,
-                   "chebyshev_block_columns": st.poly_columns if st else None, "eig_rel_err_vs_oracle": eig_err,
+                   "preconditioned_block_columns": st.poly_columns if st else None, "eig_rel_err_vs_oracle": eig_err,
                    "max_rel_resid": st.max_resid if st else None},
         "roofline": roofline,
+        "roofline_chebyshev": roofline_cheb,
         "roofline_assembly": roofline_asm,
         "cpu_baseline": cpu,
     }

@@ -587,7 +587,7 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
     const int auto_deg = std::min(128, (int)std::lround(std::sqrt((double)n) / 6.3));
     if (pc == LH_PRECOND_AUTO) {
         // the learned network where the automatic polynomial would be plain
-        // Jacobi (small meshes), Chebyshev-Jacobi elsewhere
+        // Jacobi (small meshes), the built-in preconditioner elsewhere
         const bool small = (opts && opts->poly_degree > 0) ? opts->poly_degree == 1 : auto_deg < 4;
         const bool fp64 = !opts || opts->precision == LH_PREC_FP64;  // auto picks the network for FP64 solves only
         pc = (ctx->mpnn && small && fp64) ? LH_PRECOND_LEARNED : LH_PRECOND_JACOBI;
