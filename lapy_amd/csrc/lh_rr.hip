@@ -582,8 +582,23 @@ k_rr_back(int N, int nev, double* __restrict__ work, unsigned long long* __restr
 // ---- 5. orthonormalisation in the small space and output --------------------
 typedef double d4_t __attribute__((ext_vector_type(4)));
 // rows of Z and E in LDS when the products run on the matrix cores: two
-// doubles longer than nev, against bank conflicts between rows
-__device__ __forceinline__ int pol_ld(int nev) { return nev >= 32 ? nev + 2 : nev; }
+// doubles longer than nev, against bank conflicts between rows, where that
+// fits (N = nev = 96 does not)
+__device__ __forceinline__ int pol_ld(int N, int nev) {
+    return nev >= 32 && (N + nev) * (nev + 2) <= PK ? nev + 2 : nev;
+}
+// 16 x 16 tiles of Z a wave updates: 60 at most wherever Z and E fit into LDS
+// (N = 192, nev = 65 .. 70 and N = 145 .. 147, nev = 81)
+constexpr int kPolTiles = 4;
+constexpr int pol_tiles_max() {
+    int most = 0;
+    for (int N = 1; N <= NMAX; ++N)
+        for (int nev = 1; nev <= N; ++nev)
+            if ((N + nev) * nev <= PK && (N + 15) / 16 * ((nev + 15) / 16) > most)
+                most = (N + 15) / 16 * ((nev + 15) / 16);
+    return most;
+}
+static_assert(pol_tiles_max() <= kPolTiles * (NB / 64), "a tile of Z without a wave");
 
 __global__ void __launch_bounds__(NB)
 k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, int* __restrict__ status,
@@ -593,8 +608,8 @@ k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, i
     stamp(prof, 5);
     RRWork W(work, N, nev);
     const int tid = threadIdx.x;
-    const int nz = N * nev, ld = pol_ld(nev);
-    if ((N + nev) * ld <= PK && ((N + 15) / 16) * ((nev + 15) / 16) <= 3 * (NB / 64)) {
+    const int nz = N * nev, ld = pol_ld(N, nev);
+    if ((N + nev) * ld <= PK) {
         double* E = Zs + N * ld;
         for (int idx = tid; idx < nz; idx += NB) Zs[(idx / nev) * ld + idx % nev] = W.Z[idx];
         __syncthreads();
@@ -646,11 +661,11 @@ k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, i
                 for (int w = 0; w < NB / 64; ++w) em = fmax(em, red[w]);
                 // Newton-Schulz needs ||E|| < 1; a basis that far off is left as it is
                 if (em >= 0.5 || (pass > 0 && em <= 1e-8)) break;
-                // Z <- Z - Z E / 2: up to three 16 x 16 tiles a wave, written
+                // Z <- Z - Z E / 2: up to kPolTiles 16 x 16 tiles a wave, written
                 // after a barrier once every tile has been read
-                d4_t acc[3];
+                d4_t acc[kPolTiles];
 #pragma unroll
-                for (int u = 0; u < 3; ++u) {
+                for (int u = 0; u < kPolTiles; ++u) {
                     acc[u] = (d4_t){0.0, 0.0, 0.0, 0.0};
                     const int t = wv + (NB / 64) * u;
                     if (t >= nupd) continue;
@@ -667,7 +682,7 @@ k_rr_polish(int N, int nev, double* __restrict__ work, double* __restrict__ C, i
                 }
                 __syncthreads();
 #pragma unroll
-                for (int u = 0; u < 3; ++u) {
+                for (int u = 0; u < kPolTiles; ++u) {
                     const int t = wv + (NB / 64) * u;
                     if (t >= nupd) continue;
                     const int col = 16 * (t % nt) + il;

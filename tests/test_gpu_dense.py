@@ -44,6 +44,21 @@ def test_random_spectrum(N, nev):
     check(sym_with_spectrum(lam, N), nev)
 
 
+# shapes whose vectors and Z^T Z fill the polish's LDS (nev = N, rows without
+# padding, more than three tiles a wave), and ordinary ones
+@pytest.mark.parametrize("N,nev", [(96, 96), (95, 95), (90, 90), (150, 75), (156, 73), (147, 81), (192, 70), (192, 65),
+                                   (192, 64), (129, 32), (60, 31)])
+def test_vectors_are_orthonormal_to_rounding(N, nev):
+    """The eigenvalues' gaps are 1e-6 of the norm and less, so inverse
+    iteration alone leaves 1e-11 to 1e-9.  The last polish step starts from
+    |Z^T Z - I| <= 1e-8 and squares it, which leaves the rounding of its
+    products and of the host's: N terms of 2^-53 each, twice that allowed."""
+    rng = np.random.default_rng(N + nev)
+    lam = np.sort(np.concatenate([[1e-12], rng.uniform(0.4, 60.0, N - 1 - N // 3), 10 ** rng.uniform(2, 5.7, N // 3)]))
+    _, Z = _lib.small_symeig(_lib.default_context(), sym_with_spectrum(lam, nev), nev)
+    assert np.abs(Z.T @ Z - np.eye(nev)).max() <= (N + 8) * 2.0**-52
+
+
 def test_clusters_and_multiplicities():
     lam = np.concatenate([[0.0, 1e-13], np.repeat([2.0, 6.0], 5), 6.0 + 1e-9 * np.arange(7),
                           np.linspace(7, 1e3, 192 - 19)])
