@@ -96,6 +96,11 @@ int  lh_ctx_create(int device, lh_ctx** out);
 void lh_ctx_destroy(lh_ctx* ctx);
 const char* lh_last_error(lh_ctx* ctx);
 int  lh_sync(lh_ctx* ctx);
+/* Iterations that the eigensolver (default 80; each phase of a mixed-precision
+ * solve counts its own) and the linear solver (200, looked at every fourth)
+ * keep their automatic multigrid cycle before they go on with the Chebyshev
+ * polynomial or Jacobi (stats.fallback_used = 1); 0: the default. */
+int  lh_ctx_set_cycle_limits(lh_ctx* ctx, int eig_iterations, int cg_iterations);
 /* Number of visible HIP devices (0 when no GPU is present). */
 int  lh_device_count(void);
 

@@ -131,6 +131,7 @@ SIGNATURES = {
     "lh_mpnn_get_params": (C.c_int, [_vp, _vp]),
     "lh_ctx_set_mpnn": (C.c_int, [_vp, _vp]),
     "lh_ctx_set_assembly_order": (C.c_int, [_vp, C.c_int]),
+    "lh_ctx_set_cycle_limits": (C.c_int, [_vp, C.c_int, C.c_int]),
     "lh_mpnn_apply": (C.c_int, [_vp, _vp, _vp, C.c_double, C.c_double, _vp, C.c_int, _vp]),
     "lh_mpnn_loss_grad": (C.c_int, [_vp, _vp, _vp, C.c_double, C.c_double, _vp, C.c_int, _dp, _vp]),
     "lh_mpnn_time_layer": (C.c_int, [_vp, _vp, _vp, C.c_double, C.c_double, C.c_int, C.c_int, C.c_int, _dp]),
@@ -249,6 +250,11 @@ class Context:
         """Row order of the triangle assembly (LH_ASM_ORDER_*); the values
         do not depend on it."""
         check(lib().lh_ctx_set_assembly_order(self.handle, int(order)), self, "lh_ctx_set_assembly_order")
+
+    def set_cycle_limits(self, eig: int = 0, cg: int = 0):
+        """Iterations the eigensolver and the linear solver keep their
+        multigrid cycle (lh_ctx_set_cycle_limits; 0: the default)."""
+        check(lib().lh_ctx_set_cycle_limits(self.handle, int(eig), int(cg)), self, "lh_ctx_set_cycle_limits")
 
 
 def content_hash(a):

@@ -47,7 +47,7 @@ double now_us() {
 // this many times the tolerance (they keep a plain Jacobi direction)
 constexpr double kPolyLockFactor = 1.0;
 // iterations with the multigrid cycle before the polynomial takes over (13 to
-// 25 are usual)
+// 25 are usual) where the context sets no other limit
 constexpr int kAmgMaxIters = 80;
 
 // T: the block type.  double for the FP64 solve; float for the first phase
@@ -79,11 +79,13 @@ struct Lobpcg {
     LearnedPrecond learned;
     ChebPrecond own_cheb;
     ChebPrecond* cheb = &own_cheb;  // a second phase shares the first one's
-    bool cheb_ready = false;
+    bool cheb_ready = false;  // set up (by this phase or the one before)
     bool use_amg = false;  // the multigrid cycle; the polynomial (or Jacobi) where it finds no hierarchy
     Amg own_amg;
     Amg* amg = &own_amg;   // a second phase shares the first one's
     bool amg_ready = false;
+    bool amg_on = false;   // in use: false from the iteration on that drops it
+    int amg_max_iters = kAmgMaxIters;
     DevBuf kshift;         // K = A - sigma B, what the cycle is built from
     // locality reordering (solver-internal)
     std::shared_ptr<Reorder> ro;      // the pattern's (kept with it)
@@ -267,9 +269,11 @@ struct Lobpcg {
         HIPX(hipMemsetAsync(S.p, 0, n * ld * sizeof(T), ctx->stream));
         jacobi_diag(ctx, A, B, -sigma, 1.0, dinv.as<double>());
         auto set_polynomial = [&]() {
-            if (poly_degree > 1 && !cheb_ready) cheb->setup(ctx, A, B, sigma, poly_degree, poly_ratio, n, m, poly_half);
+            if (poly_degree <= 1 || cheb_ready) return;
+            cheb->setup(ctx, A, B, sigma, poly_degree, poly_ratio, n, m, poly_half);
+            cheb_ready = true;
         };
-        bool amg_on = use_amg;
+        amg_on = use_amg;
         if (amg_on && !amg_ready) {
             form_shifted(ctx, A, B, -sigma, 1.0, kshift);
             amg_on = amg->setup(ctx, n, A->nnz(), A->pat->rowptr.as<int32_t>(), A->pat->cols.as<int32_t>(),
@@ -362,7 +366,7 @@ struct Lobpcg {
                 if (it >= kMinFp32Iters && gm_hist[it] > 0.55 * gm_hist[it - 1]) break;
             }
             // an operator that the cycle does not suit
-            if (amg_on && it >= kAmgMaxIters) {
+            if (amg_on && it >= amg_max_iters) {
                 amg_on = false;
                 st.fallback_used = 1;
                 set_polynomial();
@@ -599,6 +603,7 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
     const bool jac = pc == LH_PRECOND_JACOBI;
     int deg = opts ? opts->poly_degree : 0;
     L.use_amg = jac && deg <= 0;
+    if (ctx->eig_cycle_limit > 0) L.amg_max_iters = ctx->eig_cycle_limit;
     if (!jac) deg = 1;
     if (deg <= 0) deg = auto_deg < 4 ? 1 : auto_deg;
     deg = std::max(1, std::min(deg, 1024));
@@ -642,6 +647,7 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
         L1.poly_ratio = L.poly_ratio;
         L1.poly_half = L.poly_half;
         L1.use_amg = L.use_amg;
+        L1.amg_max_iters = L.amg_max_iters;
         L1.phase_one = true;
         L1.run(nullptr, nullptr);
         DevBuf X0((size_t)n * m * 8);
@@ -650,14 +656,15 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
         L.B = L1.B;
         L.ext_ro = L1.reordered ? L1.ro.get() : nullptr;
         L.cheb = L1.cheb;
-        L.cheb_ready = L.poly_degree > 1;
+        L.cheb_ready = L1.cheb_ready;
         L.amg = L1.amg;
         L.amg_ready = L1.amg_ready;
-        L.use_amg = L1.amg_ready;
+        L.use_amg = L1.amg_on;  // not a cycle that the first phase has dropped
         L.x0 = X0.as<double>();
         L.x0_ld = m;
         L.max_iter = std::max(1, L.max_iter - L1.st.iterations);
         L.run(e->evals.data(), &e->evecs);
+        L.st.fallback_used |= L1.st.fallback_used;
         L.st.iterations += L1.st.iterations;
         L.st.iterations_fp32 = L1.st.iterations;
         L.st.spmm_calls += L1.st.spmm_calls;
@@ -720,6 +727,7 @@ void solve_batch(lh_ctx* ctx, int nmesh, lh_csr* const* A, lh_csr* const* B, con
     for (int w = 0; w < nw; ++w) {
         lh_ctx* wc = ctx->workers[w];
         wc->mpnn = ctx->mpnn;  // the learned preconditioner's weights are shared read-only
+        wc->eig_cycle_limit = ctx->eig_cycle_limit;
         if (wc->arena_mem.bytes < abytes) {
             wc->arena_mem.alloc(abytes);
             wc->arena.base = wc->arena_mem.as<char>();
@@ -919,6 +927,13 @@ int lh_tune_set(lh_ctx* ctx, const lh_tune_entry* e) {
 int lh_ctx_get_workers(lh_ctx* ctx, int* workers) {
     if (!ctx || !workers) return LH_ERR_ARG;
     *workers = ctx->tuned_workers;
+    return LH_OK;
+}
+
+int lh_ctx_set_cycle_limits(lh_ctx* ctx, int eig_iterations, int cg_iterations) {
+    if (!ctx || eig_iterations < 0 || cg_iterations < 0) return LH_ERR_ARG;
+    ctx->eig_cycle_limit = eig_iterations;
+    ctx->cg_cycle_limit = cg_iterations;
     return LH_OK;
 }
 

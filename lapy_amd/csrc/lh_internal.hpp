@@ -156,6 +156,7 @@ struct lh_ctx {
     size_t host_stage_bytes = 0;
     void* blas = nullptr;  // rocBLAS handle of the wide Rayleigh-Ritz solver, made on first use
     int asm_order = 0;     // LH_ASM_ORDER_*: row order of the triangle assembly
+    int eig_cycle_limit = 0, cg_cycle_limit = 0;  // lh_ctx_set_cycle_limits (0: the solvers' own)
     std::shared_ptr<TuneTable> tune = std::make_shared<TuneTable>();
 };
 

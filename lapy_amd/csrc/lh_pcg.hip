@@ -68,7 +68,7 @@ constexpr int kBS = 256;    // threads per block of the set-up kernels
 constexpr int kIBS = 1024;  // threads per block of the iteration kernels
 constexpr int kMC = 8;      // right-hand sides per launch (wider blocks: several launches)
 constexpr double kAmgMinIters = 350.0;  // expected Jacobi-CG iterations from which the multigrid cycle takes over
-constexpr int kAmgMaxIters = 200;       // iterations with the cycle before Jacobi takes over again
+constexpr int kAmgMaxIters = 200;       // iterations with the cycle before Jacobi takes over again (no context limit)
 
 // K = beta * A + alpha * B on A's pattern
 template <typename VT>
@@ -1062,6 +1062,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     // condition estimate 2 tr(D) / 1^T K 1 with one
     Amg amg;
     bool amg_on = false;
+    const int amg_max_iters = ctx->cg_cycle_limit > 0 ? ctx->cg_cycle_limit : kAmgMaxIters;
     if (precond == LH_PRECOND_JACOBI && pdeg_opt == 0) {
         const double dn = (double)n;
         double expect = (double)nnz > 10.0 * dn ? 14.4 * std::cbrt(dn) : 5.4 * std::sqrt(dn);
@@ -1214,7 +1215,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
             }
         }
         // an operator that the cycle does not suit: on with Jacobi (CG restarted)
-        if (amg_on && !done && enq >= kAmgMaxIters) {
+        if (amg_on && !done && enq >= amg_max_iters) {
             amg_on = false;
             s.rz[0] = rz_plain[0];
             s.rz[1] = rz_plain[1];

@@ -175,6 +175,35 @@ def test_eigenpairs_with_the_block_cycle(name, k, block):
     assert np.all(np.abs(lam - lo) <= 1e-10 * lo[-1])
 
 
+@pytest.fixture
+def cycle_limits():
+    ctx = _lib.default_context()
+    yield ctx.set_cycle_limits
+    ctx.set_cycle_limits()
+
+
+# limit 3: the FP32 phase drops the cycle and the FP64 one starts without it;
+# 11: the FP64 phase drops it; tol 1e-15, which nothing reaches: the default
+# limit of 80 iterations, results of the last one
+@pytest.mark.parametrize("limit,tol,max_iter", [(3, 0.0, 0), (11, 1e-13, 200), (0, 1e-15, 110)])
+@pytest.mark.parametrize("name", ["tail", "cap"])  # 642 rows: degree 4; 4,403: 11
+def test_mixed_solves_past_the_cycles_limit(name, limit, tol, max_iter, cycle_limits):
+    fem = _eig_problem(name)
+    a, b = fem.device_matrices()
+    lam, _ = fem.eigs(k=12)
+    cycle_limits(eig=limit)
+    mixed, x, st = _lib.eigs(_lib.default_context(), a, b, 12, -0.01, precision=_lib.LH_PREC_MIXED, tol=tol,
+                             max_iter=max_iter, allow_noconv=True)
+    fp64 = st.iterations - st.iterations_fp32
+    print(name, "FP32 iterations", st.iterations_fp32, "FP64", fp64, "residual", st.max_resid)
+    assert st.fallback_used == 1
+    assert st.iterations_fp32 > limit if limit == 3 else fp64 > (limit or 80) >= st.iterations_fp32
+    assert np.all(np.abs(mixed - lam) <= 1e-10 * lam[-1])
+    bx = fem.mass @ x
+    res = np.linalg.norm(fem.stiffness @ x - bx * mixed, axis=0) / np.linalg.norm(bx, axis=0)
+    assert np.all(res <= 1e-8 * np.maximum(np.abs(mixed), 1e-2 * mixed[-1]))
+
+
 def test_eigenpairs_the_same_with_and_without_the_cycle():
     """The mixed-precision solve shares one hierarchy between its phases; an
     explicit degree keeps the polynomial."""
