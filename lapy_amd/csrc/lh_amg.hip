@@ -24,10 +24,17 @@
 // sizes are nothing but launch latency), and the last level (at most 128
 // rows) multiplies with its inverse.
 //
-// The coarsest matrix of a pure Neumann operator is singular (constants):
-// its unit diagonal is raised by 1e-9, which leaves the other components
-// unchanged to that accuracy and bounds the constant one, which the
-// right-hand sides of such systems do not have.
+// The coarsest matrix of a pure Neumann operator is singular (constants), and
+// that of A - sigma B nearly so where sigma is small against the eigenvalues
+// (a mesh in small units): its unit diagonal is raised by 1e-9 in FP64, which
+// leaves the other components unchanged to that accuracy and bounds the
+// constant one, which the right-hand sides of such systems have only to
+// rounding.  The eigensolver's blocks are raised by 1e-5 (the other components'
+// eigenvalues are (pi / 128)^2 / 2 = 3e-4 and more, a chain's; about 0.04 on a
+// sphere): its first residuals hold the constant components in full, and
+// columns that are the same to 1e-6 after the cycle fail in the Cholesky-QR,
+// whose pivots are squares (with 1e-6 at radius 1e-8, with 1e-9 at 0.01).  The
+// inverse and its sums stay in FP64 there too.
 #include "lh_amg.hpp"
 
 #include <cmath>
@@ -715,7 +722,7 @@ template <typename T>
 struct TailDesc {
     int count;  // levels, the last one with the inverse
     TailLevel<T> lv[kMaxLevels];
-    const T* ginv;
+    const double* ginv;
 };
 constexpr int kTailThreads = 1024;
 
@@ -738,7 +745,7 @@ k_amg_tail(int ld, const TailDesc<T>* __restrict__ desc, const T* __restrict__ b
            const int* __restrict__ status) {
     if (status && status[0]) return;
     __shared__ T sb[kTailSum], sx[kTailSum], sy[kTailSum];
-    __shared__ T red[kTailThreads];
+    __shared__ double red[kTailThreads];
     const int tid = threadIdx.x, col = blockIdx.x;
     const int count = desc->count;
     {
@@ -769,16 +776,16 @@ k_amg_tail(int ld, const TailDesc<T>* __restrict__ desc, const T* __restrict__ b
         const TailLevel<T>& lv = desc->lv[count - 1];
         const int n = lv.n;  // <= 128
         const int i = tid & 127, part = tid >> 7;
-        T a = T(0);
+        double a = 0.0;
         if (i < n)
-            for (int k = part; k < n; k += kTailThreads / 128) a += desc->ginv[k * n + i] * sb[lv.off + k];
+            for (int k = part; k < n; k += kTailThreads / 128) a += desc->ginv[k * n + i] * (double)sb[lv.off + k];
         red[tid] = a;
         __syncthreads();
         if (tid < n) {
-            T t = T(0);
+            double t = 0.0;
 #pragma unroll
             for (int p = 0; p < kTailThreads / 128; ++p) t += red[tid + 128 * p];
-            sx[lv.off + tid] = t;
+            sx[lv.off + tid] = (T)t;
         }
         __syncthreads();
     }
@@ -1037,7 +1044,7 @@ X* Amg::own(size_t count) {
 }
 
 bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const int32_t* cl0, const double* kv0,
-                int ell_w, const int32_t* ecl, const double* ekv) {
+                int ell_w, const int32_t* ecl, const double* ekv, double coarse_shift) {
     ctx = c;
     levels.clear();
     keep.clear();
@@ -1078,7 +1085,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
             ginv.alloc((size_t)n * n * 8);
             k_amg_dense<<<(unsigned)n, 128, 0, st>>>((int)n, rp, cl, kv, g.as<double>());
             LH_CHECK_LAUNCH();
-            cholinv(ctx, (int)n, g.as<double>(), t.as<double>(), 1e-9, stt.as<int>());
+            cholinv(ctx, (int)n, g.as<double>(), t.as<double>(), coarse_shift, stt.as<int>());
             k_amg_inverse<<<(unsigned)n, 128, 0, st>>>((int)n, t.as<double>(), ginv.as<double>());
             LH_CHECK_LAUNCH();
             int hs = 0, hb[2] = {0, 0};
@@ -1249,11 +1256,11 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
 }
 
 template <typename T>
-void Amg::describe_tail(const T* inverse) {
+void Amg::describe_tail() {
     const int last = (int)levels.size() - 1;
     TailDesc<T> d{};
     d.count = last - tail + 1;
-    d.ginv = inverse;
+    d.ginv = ginv.as<double>();
     int off = 0;
     for (int l = tail; l <= last; ++l) {
         const AmgLevel& lv = levels[l];
@@ -1283,7 +1290,7 @@ void Amg::describe_tail(const T* inverse) {
 
 void Amg::prepare(int m_) {
     m = m_;
-    describe_tail<double>(ginv.as<double>());
+    describe_tail<double>();
     size_t total = 0;
     for (int l = 0; l <= tail; ++l) total += 4 * (size_t)levels[l].n * m;
     work.alloc(total * 8);
@@ -1433,7 +1440,7 @@ void Amg::prepare_blocks(int m_, int ell_w, const int32_t* ecl) {
         l0.ecl = ecl;
         l0.ekv32 = e;
     }
-    describe_tail<float>(narrow(ginv.as<double>(), levels[last].n * levels[last].n));
+    describe_tail<float>();
     cycles = l0.n >= kManyRows ? 3 : 2;
     size_t total = cycles * (size_t)l0.n * ld;
     for (int l = 0; l <= tail; ++l) total += (l == 0 || l < tail ? 4 : 2) * (size_t)levels[l].n * ld;

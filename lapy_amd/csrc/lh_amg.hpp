@@ -40,8 +40,11 @@ struct Amg {
     // ekv) for the products of the finest level.  Returns false (nothing to
     // free) when no useful hierarchy exists: a negative diagonal, coarsening
     // that stalls, or a coarsest matrix that does not factorise.
+    // coarse_shift: what raises the unit diagonal of the equilibrated
+    // coarsest matrix, kShiftF64 or kShiftBlocks.
     bool setup(lh_ctx* ctx, int64_t n, int64_t nnz, const int32_t* rp, const int32_t* cl, const double* kv, int ell_w,
-               const int32_t* ecl, const double* ekv);
+               const int32_t* ecl, const double* ekv, double coarse_shift);
+    static constexpr double kShiftF64 = 1e-9, kShiftBlocks = 1e-5;
     // work blocks for m columns in double precision
     void prepare(int m);
     // Z <- M R, row-major n x m; a set status[0] makes every launch return at
@@ -77,7 +80,7 @@ struct Amg {
     int cycles = 2;            // combined in one application
     float *bin = nullptr, *bx1 = nullptr, *bx2 = nullptr;
     std::vector<float*> fb, fx, fy, fr;
-    template <typename T> void describe_tail(const T* inverse);
+    template <typename T> void describe_tail();
     template <int MODE> void blk_step(int l, int w, const float* b, const float* x, float* out, float w0, float w1, float g);
     void cycle_blocks(int l, int w, const float* b, float* x);
     template <typename X> X* own(size_t count);

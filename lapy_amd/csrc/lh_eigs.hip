@@ -277,7 +277,7 @@ struct Lobpcg {
         if (amg_on && !amg_ready) {
             form_shifted(ctx, A, B, -sigma, 1.0, kshift);
             amg_on = amg->setup(ctx, n, A->nnz(), A->pat->rowptr.as<int32_t>(), A->pat->cols.as<int32_t>(),
-                                kshift.as<double>(), 0, nullptr, nullptr);
+                                kshift.as<double>(), 0, nullptr, nullptr, Amg::kShiftBlocks);
             if (amg_on) amg->prepare_blocks(m, ell.W, ell.cols.as<int32_t>());
             amg_ready = amg_on;
         }

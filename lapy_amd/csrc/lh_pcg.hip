@@ -1072,7 +1072,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
             expect = std::min(expect, 0.5 * std::sqrt(kappa) * std::log(2.0 / rtol));
         }
         if (expect > kAmgMinIters) {
-            amg_on = amg.setup(ctx, n, nnz, L.rp, L.cl, L.kv, L.ew, L.ecols, L.ev);
+            amg_on = amg.setup(ctx, n, nnz, L.rp, L.cl, L.kv, L.ew, L.ecols, L.ev, Amg::kShiftF64);
             if (amg_on) amg.prepare(m);
         }
     }

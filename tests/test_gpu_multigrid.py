@@ -175,6 +175,30 @@ def test_eigenpairs_with_the_block_cycle(name, k, block):
     assert np.all(np.abs(lam - lo) <= 1e-10 * lo[-1])
 
 
+def _two_spheres():
+    v, t = meshgen.perturbed_sphere(4, np.random.default_rng(2), axes=(1.3, 0.8, 1.0), sigma=0.02)
+    return np.r_[v, v + 3.0], np.r_[t, t + len(v)]  # a constant of its own on each part
+
+
+@pytest.mark.parametrize("unit,sigma", [(1e-2, -0.01), (1e-3, -0.01), (1e-4, -0.01), (1.0, 0.0), (1.0, -1e-12)])
+@pytest.mark.parametrize("name", ["sphere", "two spheres"])
+def test_eigenpairs_in_small_units(name, unit, sigma):
+    """The shift sigma far below the spectrum, so that A - sigma B is singular
+    to rounding: eigenvalues and iterations are those of the same mesh in
+    ordinary units."""
+    v, t = meshgen.perturbed_sphere(5, np.random.default_rng(2), axes=(1.3, 0.8, 1.0), sigma=0.02) \
+        if name == "sphere" else _two_spheres()
+    fem = Solver(TriaMesh(v, t))
+    lam, _ = fem.eigs(k=10)
+    its = fem.last_stats.iterations
+    fem = Solver(TriaMesh(v * unit, t))
+    small, _ = fem.eigs(k=10, sigma=sigma)
+    st = fem.last_stats
+    print(name, unit, sigma, "iterations", its, st.iterations)
+    assert st.fallback_used == 0 and st.iterations <= its + 3
+    assert np.all(np.abs(small * unit**2 - lam) <= 1e-10 * lam[-1])
+
+
 @pytest.fixture
 def cycle_limits():
     ctx = _lib.default_context()
