@@ -435,6 +435,11 @@ int lh_small_symeig(lh_ctx* ctx, int N, int nev, const double* H, double* evals,
  * numerically positive definite (a pivot <= 1e-12 relative to its unit
  * diagonal). */
 int lh_small_cholinv(lh_ctx* ctx, int m, const double* G, double shift, double* T, double* min_pivot);
+/* One multigrid cycle of the linear solves on its own (no counterpart in the
+ * reference; exposed for its tests): Z = M R for the FP64 matrix A and host
+ * R, Z (n x nc row-major), the hierarchy set up in the call.  LH_ERR_NUMERIC
+ * where A has no hierarchy (the solves use Jacobi or the polynomial then). */
+int lh_cycle_apply(lh_ctx* ctx, lh_csr* A, const double* R, int nc, double* Z);
 
 #ifdef __cplusplus
 }

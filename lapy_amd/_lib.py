@@ -113,6 +113,7 @@ SIGNATURES = {
     "lh_time_spmm": (C.c_int, [_vp, _vp, _vp, C.c_int, C.c_int, C.c_int, _dp]),
     "lh_small_symeig": (C.c_int, [_vp, C.c_int, C.c_int, _vp, _vp, _vp, _vp]),
     "lh_small_cholinv": (C.c_int, [_vp, C.c_int, _vp, C.c_double, _vp, _dp]),
+    "lh_cycle_apply": (C.c_int, [_vp, _vp, _vp, C.c_int, _vp]),
     "lh_time_cheb_step": (C.c_int, [_vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, _dp]),
     "lh_eigs_batched": (C.c_int, [_vp, C.c_int, _vp, _vp, _vp, C.c_double, _vp, C.c_int, _vp, _vp, _vp]),
     "lh_eigs_autotune": (C.c_int, [_vp, C.c_int, _vp, _vp, _vp, C.c_double, _vp, _vp, _vp]),
@@ -724,6 +725,15 @@ def small_cholinv(ctx: Context, G, shift: float = 0.0):
     check(lib().lh_small_cholinv(ctx.handle, m, _ptr(G), float(shift), _ptr(T), C.byref(mp)), ctx,
           "lh_small_cholinv")
     return T, mp.value
+
+
+def cycle_apply(ctx: Context, A: DeviceCSR, R):
+    """One multigrid cycle of the linear solves for A applied to the columns
+    of R (lh_cycle_apply)."""
+    R = np.ascontiguousarray(np.asarray(R, dtype=np.float64).reshape(A.n, -1))
+    Z = np.empty_like(R)
+    check(lib().lh_cycle_apply(ctx.handle, A.handle, _ptr(R), R.shape[1], _ptr(Z)), ctx, "lh_cycle_apply")
+    return Z
 
 
 def curvature(ctx: Context, dm: "DeviceMesh", smoothit: int):

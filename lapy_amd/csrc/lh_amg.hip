@@ -3,7 +3,9 @@
 // mass + t stiffness).
 //
 // Setup (once per solve, all on the device, deterministic), level by level:
-//  * lambda_max of D^-1 K from ten power steps;
+//  * lambda_max of D^-1 K from ten power steps, bmax = 1.1 times it and 2 at
+//    most, and D raised in the rows whose Gershgorin sum exceeds 1.16 bmax, so
+//    that no eigenvalue does;
 //  * aggregates around the roots of a maximal independent set of distance 2
 //    in the graph of strong connections (k_ij^2 > theta^2 k_ii k_jj), found
 //    with hashed keys in a fixed number of rounds; the roots are numbered in
@@ -17,8 +19,15 @@
 //    depend on scheduling).
 //
 // Cycle: V(1,1) with the Chebyshev polynomial of degree 2 on [bmax / 6, bmax]
-// as the smoother before and after, hence a symmetric positive definite
-// preconditioner, as conjugate gradients need.  A level is six launches; all
+// as the smoother before and after.  Its error polynomial is at most 1 in
+// magnitude on [0, 7/6 bmax], which holds the spectrum, hence a symmetric
+// positive definite preconditioner, as conjugate gradients need.  (Power steps
+// alone miss the mode of one bad element among good ones: a vertex of an
+// icosphere of 40,962 moved to 0.08 of its height has lambda_max 2.01, the
+// steps find 1.50, and the cycle was indefinite.  Raising D where the
+// row asks for it leaves the other rows' smoothing as it is, and takes bad
+// elements' modes out of bmax: CG on 4,913 tet vertices jittered by a quarter
+// of the spacing took 35 iterations with bmax 4.1, 28 now.)  A level is six launches; all
 // levels of at most kTailRows rows run in one workgroup per column with
 // their vectors in LDS (one launch instead of six a level, which at these
 // sizes are nothing but launch latency), and the last level (at most 128
@@ -53,6 +62,8 @@ constexpr int kTailNnz = 24576;      // and its entries: one CU reads them from 
 constexpr int kTailSum = 2560;       // rows of all of them together at most
 constexpr int kLongRow = 20;         // mean row length from which a wave forms a row of P
 constexpr double kSmoothRatio = 6.0; // the smoother's interval is [bmax / ratio, bmax]
+constexpr double kSmoothTop = 2.0;   // bmax at most (good elements: 1.5 to 1.9 on the finest level, 1.3 to 1.5 below)
+constexpr double kGuard = 1.16;      // rows' Gershgorin sums are held to this many bmax (7/6: the smoother's limit)
 
 static_assert(kCoarsest <= kCholMax, "the coarsest level is factorised by cholinv");
 
@@ -104,29 +115,36 @@ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
 // spreading step 35 -> 4.4, which also stopped testing every entry's strength
 // again in each round.
 
-// dinv; bad[0] set when a row's diagonal is negative, missing or zero beside
+// dinv and the row sums of |D^-1 K|; bad[0] set when a row's diagonal is negative, missing or zero beside
 // non-zero entries; start vector of the power iteration (0 on zero rows)
 template <int G>
 __global__ void __launch_bounds__(256)
 k_amg_diag(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl, const double* __restrict__ kv,
-           double* __restrict__ dinv, double* __restrict__ x, int* __restrict__ bad) {
+           double* __restrict__ dinv, double* __restrict__ gersh, double* __restrict__ x, int* __restrict__ bad) {
     const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
     if (i >= n) return;
-    double d = 0.0, other = 0.0;
+    double d = 0.0, other = 0.0;  // other: sum of the magnitudes beside the diagonal
     for (int32_t s = rp[i] + (int32_t)(threadIdx.x % G); s < rp[i + 1]; s += G) {
         if (cl[s] == (int32_t)i) d = kv[s];
-        else other = fmax(other, fabs(kv[s]));
+        else other += fabs(kv[s]);
     }
 #pragma unroll
     for (int o = G / 2; o > 0; o >>= 1) {
         d += __shfl_xor(d, o, 64);  // zero in all lanes but one
-        other = fmax(other, __shfl_xor(other, o, 64));
+        other += __shfl_xor(other, o, 64);
     }
     if (threadIdx.x % G) return;
     if (!(d >= 0.0) || (d == 0.0 && other != 0.0)) bad[0] = 1;  // every writer stores the same value
     const bool pos = d > 0.0;
     dinv[i] = pos ? 1.0 / d : 0.0;
+    gersh[i] = pos ? 1.0 + other / d : 0.0;
     x[i] = pos ? (double)(mix32((uint32_t)i * 2654435761u + 12345u) >> 8) * (1.0 / 8388608.0) - 1.0 : 0.0;
+}
+// D raised where the row's sum exceeds the limit: by Gershgorin's theorem no
+// eigenvalue of the new D^-1 K does
+__global__ void k_amg_guard(int64_t n, const double* __restrict__ gersh, double limit, double* __restrict__ dinv) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && gersh[i] > limit) dinv[i] *= limit / gersh[i];
 }
 // y = D^-1 K x
 template <int G>
@@ -1056,7 +1074,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
     int64_t n = n0, nnz = nnz0;
     const int32_t *rp = rp0, *cl = cl0;
     const double* kv = kv0;
-    DevBuf x(n0 * 8), y(n0 * 8), part(2 * kRB * 8), key(n0 * 8), key2(n0 * 8), agg(n0 * 4), agg2(n0 * 4),
+    DevBuf x(n0 * 8), y(n0 * 8), part(2 * kRB * 8), gersh(n0 * 8), key(n0 * 8), key2(n0 * 8), agg(n0 * 4), agg2(n0 * 4),
         cnt((n0 + 1) * 4), idx((n0 + 1) * 4), strong;
     double theta = kTheta;
     for (int l = 0; l < kMaxLevels; ++l) {
@@ -1077,7 +1095,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         const unsigned nb = nblocks(n, 256), nbx = nblocks_xcd(n, 256);
         const int g = lanes_for(nnz, n);
         const unsigned nbg = nblocks_xcd(n * g, 256);
-        with_lanes(g, [&](auto G) { k_amg_diag<G.v><<<nbg, 256, 0, st>>>(n, rp, cl, kv, dinv, x.as<double>(), bad); });
+        with_lanes(g, [&](auto G) { k_amg_diag<G.v><<<nbg, 256, 0, st>>>(n, rp, cl, kv, dinv, gersh.as<double>(), x.as<double>(), bad); });
         LH_CHECK_LAUNCH();
         if (n <= kCoarsest) {
             // last level: its inverse
@@ -1142,7 +1160,9 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         const int64_t nc = nc32;
         // a stalled coarsening, a bad diagonal or a meaningless estimate: no hierarchy
         if (hb[0] || hb[1] || nc < 1 || nc > n * 7 / 10 || !(lmax > 0.0) || !std::isfinite(lmax)) return false;
-        lv.bmax = 1.1 * lmax;
+        lv.bmax = std::min(1.1 * lmax, kSmoothTop);
+        k_amg_guard<<<nb, 256, 0, st>>>(n, gersh.as<double>(), kGuard * lv.bmax, dinv);
+        LH_CHECK_LAUNCH();
         const double w = 4.0 / (3.0 * lv.bmax);
         // P
         int32_t* pp = own<int32_t>(n + 1);
@@ -1543,3 +1563,21 @@ template void Amg::apply_blocks<double>(double*, int, int, int, const int32_t*);
 template void Amg::apply_blocks<float>(float*, int, int, int, const int32_t*);
 
 }  // namespace lh
+
+extern "C" int lh_cycle_apply(lh_ctx* ctx, lh_csr* A, const double* R, int nc, double* Z) {
+    if (!ctx || !A || !R || !Z || nc < 1 || A->dtype != LH_F64) return LH_ERR_ARG;
+    LH_API_BEGIN(ctx)
+    HIPX(hipSetDevice(ctx->device));
+    const int64_t n = A->n();
+    lh::Amg amg;
+    if (!amg.setup(ctx, n, A->nnz(), A->pat->rowptr.as<int32_t>(), A->pat->cols.as<int32_t>(), A->vals.as<double>(), 0,
+                   nullptr, nullptr, lh::Amg::kShiftF64))
+        LH_THROW(LH_ERR_NUMERIC, "lh_cycle_apply: no multigrid hierarchy for this matrix");
+    amg.prepare(nc);
+    const size_t bytes = (size_t)n * nc * 8;
+    DevBuf r(bytes), z(bytes);
+    lh::h2d(ctx, r.p, R, bytes);
+    amg.apply(r.as<double>(), z.as<double>(), nullptr, nullptr);
+    lh::d2h(ctx, Z, z.p, bytes);
+    LH_API_END(ctx)
+}

@@ -175,6 +175,67 @@ def test_eigenpairs_with_the_block_cycle(name, k, block):
     assert np.all(np.abs(lam - lo) <= 1e-10 * lo[-1])
 
 
+def _bad_element(name):
+    """A regular mesh with one bad element: the vertex moved."""
+    if name == "sliver":  # to 0.08 of its height over an edge
+        v, t = meshgen.icosphere(6)
+        tri = t[(t == 20000).any(axis=1)][0]
+        mid = v[tri[tri != 20000]].mean(axis=0)
+        v[20000] = mid + 0.08 * (v[20000] - mid)
+        return Solver(TriaMesh(v, t))
+    v, t = meshgen.tet_cube(24)
+    v[25**3 // 2] += 0.48 / 24 * np.array([1.0, -1.0, 0.0])  # almost into a face
+    return Solver(TetMesh(v, t))
+
+
+@pytest.mark.parametrize("name", ["sliver", "flat tet"])
+def test_cycle_is_positive_definite_on_bad_elements(name):
+    """On the top eigenvector x of D^-1 K, which one element's mode is here,
+    the smoother's error polynomial is largest.  0 < x K M K x <= x K x says
+    that M is positive and does not overshoot there; 1e-8 allows for the
+    rounding of x."""
+    from scipy.sparse.linalg import eigsh
+
+    fem = _bad_element(name)
+    k = sparse.csr_matrix(fem.stiffness)
+    k = k + sparse.diags(1e-6 * k.diagonal())  # regular
+    s = sparse.diags(1.0 / np.sqrt(k.diagonal()))
+    lam, x = eigsh(s @ k @ s, k=1, which="LA", tol=1e-6)
+    kx = k @ (s @ x)
+    ctx = _lib.default_context()
+    z = _lib.cycle_apply(ctx, _lib.DeviceCSR.from_scipy(ctx, k), kx)
+    part = float(kx[:, 0] @ z[:, 0]) / float((s @ x)[:, 0] @ kx[:, 0])
+    print(name, "top eigenvalue", lam[0], "x K M K x / x K x", part)
+    assert 0.0 < part <= 1.0 + 1e-8
+
+
+@pytest.mark.parametrize("name", ["tail", "rough surface", "rough tets", "flat tets"])
+def test_cycle_spectrum(name):
+    """M symmetric and M K's eigenvalues in (0, 1], from the whole matrices:
+    as far as rounding goes, which the condition number (1e7 at most) raises
+    to about 1e-9."""
+    from scipy.linalg import cholesky, eigvalsh
+
+    if name == "tail":
+        fem = _eig_problem("tail")
+    elif name == "rough surface":
+        fem = Solver(TriaMesh(*meshgen.perturbed_sphere(4, np.random.default_rng(5), sigma=0.06)))
+    elif name == "rough tets":
+        fem = Solver(TetMesh(*meshgen.tet_cube(12, jitter=0.2)))
+    else:
+        fem = Solver(TetMesh(*meshgen.tet_cube(11, jitter=0.28)))
+    k = sparse.csr_matrix(fem.stiffness)
+    k = k + sparse.diags(1e-5 * k.diagonal())
+    n = k.shape[0]
+    ctx = _lib.default_context()
+    m = _lib.cycle_apply(ctx, _lib.DeviceCSR.from_scipy(ctx, k), np.eye(n))
+    assert np.abs(m - m.T).max() <= 1e-9 * np.abs(m).max()
+    c = cholesky(k.toarray(), lower=True)
+    w = eigvalsh(c.T @ (0.5 * (m + m.T)) @ c)
+    print(name, n, "M K in", w[0], w[-1])
+    assert w[0] > 0.02 and w[-1] <= 1.0 + 1e-8
+
+
 def _two_spheres():
     v, t = meshgen.perturbed_sphere(4, np.random.default_rng(2), axes=(1.3, 0.8, 1.0), sigma=0.02)
     return np.r_[v, v + 3.0], np.r_[t, t + len(v)]  # a constant of its own on each part
