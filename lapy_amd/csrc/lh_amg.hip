@@ -1160,6 +1160,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         const int64_t nc = nc32;
         // a stalled coarsening, a bad diagonal or a meaningless estimate: no hierarchy
         if (hb[0] || hb[1] || nc < 1 || nc > n * 7 / 10 || !(lmax > 0.0) || !std::isfinite(lmax)) return false;
+        if (l == 0) rough = lmax;
         lv.bmax = std::min(1.1 * lmax, kSmoothTop);
         k_amg_guard<<<nb, 256, 0, st>>>(n, gersh.as<double>(), kGuard * lv.bmax, dinv);
         LH_CHECK_LAUNCH();
@@ -1428,8 +1429,15 @@ void Amg::apply(const double* R, double* Z, double* part, const int* status) { c
 // with the inverse, 21 with two).  Three from kManyRows rows on, where an
 // iteration's other work is ten times a cycle's; two below, where a cycle is
 // launch latency and costs a seventh of an iteration.
+// Three too where the estimate of lambda_max(D^-1 K) is above kRough (surfaces
+// reach 2.3 with noise of two edge lengths, tets jittered by 0.18 of the spacing
+// 2.1, by 0.2, which makes flat ones, 2.8 to 3.8): the cycle leaves a few of the
+// flat elements' modes (eigenvalues 0.03), so 35,937 vertices jittered by 0.25 took
+// 41 iterations and 24 ms (10 pairs), by 0.28 33 and 37 (30 pairs) with two, 31
+// and 22, 22 and 29 with three; by 0.2, 20 and 12.5 against 18 and 13.3.
 constexpr double kBlkHi = 1.02, kBlkLo2 = 0.35, kBlkLo3 = 0.2;
 constexpr int64_t kManyRows = 65536;
+constexpr double kRough = 2.5;
 
 void Amg::prepare_blocks(int m_, int ell_w, const int32_t* ecl) {
     m = m_;
@@ -1461,7 +1469,7 @@ void Amg::prepare_blocks(int m_, int ell_w, const int32_t* ecl) {
         l0.ekv32 = e;
     }
     describe_tail<float>();
-    cycles = l0.n >= kManyRows ? 3 : 2;
+    cycles = l0.n >= kManyRows || rough > kRough ? 3 : 2;
     size_t total = cycles * (size_t)l0.n * ld;
     for (int l = 0; l <= tail; ++l) total += (l == 0 || l < tail ? 4 : 2) * (size_t)levels[l].n * ld;
     work.alloc(total * 4);

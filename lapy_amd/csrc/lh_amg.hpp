@@ -76,6 +76,7 @@ struct Amg {
     DevBuf work;
     DevBuf tail_desc;          // the tail's levels, for its kernel
     std::vector<double*> wb, wx, wy, wr;  // per level: right-hand side, iterate, second iterate, residual
+    double rough = 0.0;        // the finest level's estimate of lambda_max(D^-1 K)
     int ld = 0;                // block cycle: columns rounded up to 4
     int cycles = 2;            // combined in one application
     float *bin = nullptr, *bx1 = nullptr, *bx2 = nullptr;

@@ -260,6 +260,22 @@ def test_eigenpairs_in_small_units(name, unit, sigma):
     assert np.all(np.abs(small * unit**2 - lam) <= 1e-10 * lam[-1])
 
 
+@pytest.mark.parametrize("jitter", [0.2, 0.25, 0.28])  # of the spacing: elements from bad to almost flat
+def test_eigenpairs_on_flat_tets(jitter):
+    """The block cycle that rough elements get: about the iterations that the
+    Chebyshev polynomial takes (21 to 27), held to the solver's own bar."""
+    fem = Solver(TetMesh(*meshgen.tet_cube(25, jitter=jitter)))
+    lam, x = fem.eigs(k=10)
+    st = fem.last_stats
+    poly, _ = fem.eigs(k=10, poly_degree=21)
+    print(jitter, "iterations", st.iterations, "polynomial", fem.last_stats.iterations)
+    assert st.fallback_used == 0 and st.iterations <= 27
+    bx = fem.mass @ x
+    res = np.linalg.norm(fem.stiffness @ x - bx * lam, axis=0) / np.linalg.norm(bx, axis=0)
+    assert np.all(res <= 1e-8 * np.maximum(np.abs(lam), 1e-2 * lam[-1]))
+    assert np.all(np.abs(poly - lam) <= 1e-10 * lam[-1])
+
+
 @pytest.fixture
 def cycle_limits():
     ctx = _lib.default_context()
