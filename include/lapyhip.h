@@ -224,10 +224,10 @@ typedef struct lh_eig_opts {
                               polynomial in D^-1 (A - sigma B) applied on top
                               of Jacobi; 1: plain Jacobi; 0: automatic: two or
                               three smoothed-aggregation multigrid cycles, and
-                              where those find no hierarchy, or have not
-                              converged after 80 iterations (fallback_used =
-                              1), the polynomial of degree ~sqrt(n)/6.3, at
-                              most 128                                       */
+                              where those find no hierarchy, have not
+                              converged after 80 iterations or leave a rank
+                              deficient block (fallback_used = 1), the
+                              polynomial of degree ~sqrt(n)/6.3, at most 128 */
     double  poly_ratio;    /* Chebyshev interval [lmax/ratio, lmax]
                               (0: automatic, 2 * degree^2)                   */
     int32_t poly_storage;  /* LH_STORE_* for the Chebyshev work blocks        */

@@ -282,6 +282,12 @@ struct Lobpcg {
             amg_ready = amg_on;
         }
         if (!amg_on) set_polynomial();
+        auto drop_cycle = [&](int at) {
+            amg_on = false;
+            st.fallback_used = 1;
+            set_polynomial();
+            if (verbose) fprintf(stderr, "[lobpcg] it %d: multigrid -> polynomial\n", at);
+        };
         bool learned_on = false;
         if (precond == LH_PRECOND_LEARNED) {
             learned.setup(ctx, ctx->mpnn, A, B, -sigma, 1.0);  // K = A - sigma B
@@ -366,12 +372,7 @@ struct Lobpcg {
                 if (it >= kMinFp32Iters && gm_hist[it] > 0.55 * gm_hist[it - 1]) break;
             }
             // an operator that the cycle does not suit
-            if (amg_on && it >= amg_max_iters) {
-                amg_on = false;
-                st.fallback_used = 1;
-                set_polynomial();
-                if (verbose) fprintf(stderr, "[lobpcg] it %d: multigrid -> polynomial\n", it);
-            }
+            if (amg_on && it >= amg_max_iters) drop_cycle(it);
             // precondition W
             if (learned_on) {
                 learned.apply(Sp() + m, ld, m);
@@ -424,15 +425,19 @@ struct Lobpcg {
             project_out(0, m, m, nb);
             // joint Cholesky-QR of [W P]; P is dropped if [W P] is numerically rank deficient
             spmm_B(Sp() + m, MSp() + m, nb);
-            if (!cholqr(m, nb, true)) {
-                if (nb == 2 * m) {
-                    st.restarts++;
-                    nb = m;
-                    if (!cholqr(m, nb, true))
-                        LH_THROW(LH_ERR_NUMERIC, "Cholesky-QR of the residual block failed at iteration %d", it);
-                } else {
-                    LH_THROW(LH_ERR_NUMERIC, "Cholesky-QR of the residual block failed at iteration %d", it);
-                }
+            bool full_rank = cholqr(m, nb, true);
+            if (!full_rank && nb == 2 * m) {
+                st.restarts++;
+                nb = m;
+                full_rank = cholqr(m, nb, true);
+            }
+            if (!full_rank) {
+                if (!amg_on) LH_THROW(LH_ERR_NUMERIC, "Cholesky-QR of the residual block failed at iteration %d", it);
+                // the cycle's W is rank deficient or not finite: X and its
+                // products stand, the next iteration forms W again without it
+                drop_cycle(it);
+                have_p = false;
+                continue;
             }
             const int N = m + nb;
             {

@@ -260,6 +260,21 @@ def test_eigenpairs_in_small_units(name, unit, sigma):
     assert np.all(np.abs(small * unit**2 - lam) <= 1e-10 * lam[-1])
 
 
+def test_cycle_that_overflows_gives_way():
+    """A and B near the largest FP32 number: the finest level fits, the coarse
+    matrices of a volume, whose entries grow with the spacing, do not.  The
+    solve goes on without the cycle (block of 18: FP32 work blocks; FP16 ones
+    underflow here, as they did before there was a cycle)."""
+    fem = Solver(TetMesh(*meshgen.tet_cube(17, jitter=0.1)), lump=True)
+    lam, _ = fem.eigs(k=10)
+    scale = 2.0**127 / np.abs(fem.stiffness).max()
+    fem.stiffness, fem.mass = fem.stiffness * scale, fem.mass * scale
+    big, x = fem.eigs(k=10, block=18)
+    print("iterations", fem.last_stats.iterations)
+    assert fem.last_stats.fallback_used == 1
+    assert np.all(np.abs(big - lam) <= 1e-10 * lam[-1])
+
+
 @pytest.mark.parametrize("jitter", [0.2, 0.25, 0.28])  # of the spacing: elements from bad to almost flat
 def test_eigenpairs_on_flat_tets(jitter):
     """The block cycle that rough elements get: about the iterations that the
