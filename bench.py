@@ -319,9 +319,9 @@ def run_workload(args, ctx, _lib, meshgen):
         gold = golden("batch_256_k50.json") if nb == 256 else None
         base = [_lib.DeviceMesh(ctx, v, t) for v, t in meshes]
         # preconditioner: the default (multigrid cycles, the Chebyshev polynomial where they
-        # do not suit), plain Jacobi, or the learned network, trained first (untimed) on six other meshes of
+        # do not suit), the polynomial (asked for by its storage), plain Jacobi, or the learned network, trained first (untimed) on six other meshes of
         # the same family (levels 3 and 4, seeds outside the batch)
-        popts = {"default": {}, "cheb": {}, "jacobi": {"poly_degree": 1},
+        popts = {"default": {}, "cheb": {"poly_storage": _lib.LH_STORE_F16}, "jacobi": {"poly_degree": 1},
                  "learned": {"precond": _lib.LH_PRECOND_LEARNED},
                  "auto": {"precond": _lib.LH_PRECOND_AUTO}}[args.precond]
         net = None
@@ -573,7 +573,7 @@ def main():
     ap.add_argument("--batch-workers", type=int, default=0,
                     help="batch workload: solver workers (0: autotuned on every eighth mesh)")
     ap.add_argument("--precond", default="default", choices=["default", "cheb", "jacobi", "learned", "auto"],
-                    help="batch workload: multigrid cycles (default; cheb: its earlier name), plain Jacobi, the learned network, or auto "
+                    help="batch workload: multigrid cycles (default), the Chebyshev polynomial of automatic degree (cheb), plain Jacobi, the learned network, or auto "
                          "(the network on the meshes where the polynomial would be plain Jacobi)")
     ap.add_argument("--kernels-only", action="store_true",
                     help="skip the eigensolves; only the roofline timings of the two measured kernels")

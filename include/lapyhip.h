@@ -227,7 +227,9 @@ typedef struct lh_eig_opts {
                               where those find no hierarchy, have not
                               converged after 80 iterations or leave a rank
                               deficient block (fallback_used = 1), the
-                              polynomial of degree ~sqrt(n)/6.3, at most 128 */
+                              polynomial of degree ~sqrt(n)/6.3, at most 128;
+                              that polynomial from the start where poly_ratio
+                              or poly_storage is given                       */
     double  poly_ratio;    /* Chebyshev interval [lmax/ratio, lmax]
                               (0: automatic, 2 * degree^2)                   */
     int32_t poly_storage;  /* LH_STORE_* for the Chebyshev work blocks        */

@@ -607,7 +607,9 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
     L.no_fallback = opts && opts->no_fallback;
     const bool jac = pc == LH_PRECOND_JACOBI;
     int deg = opts ? opts->poly_degree : 0;
-    L.use_amg = jac && deg <= 0;
+    // an interval or a storage for the polynomial asks for the polynomial
+    const bool shaped = opts && (opts->poly_ratio > 1.0 || opts->poly_storage != LH_STORE_AUTO);
+    L.use_amg = jac && deg <= 0 && !shaped;
     if (ctx->eig_cycle_limit > 0) L.amg_max_iters = ctx->eig_cycle_limit;
     if (!jac) deg = 1;
     if (deg <= 0) deg = auto_deg < 4 ? 1 : auto_deg;

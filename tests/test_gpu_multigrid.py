@@ -260,6 +260,19 @@ def test_eigenpairs_in_small_units(name, unit, sigma):
     assert np.all(np.abs(small * unit**2 - lam) <= 1e-10 * lam[-1])
 
 
+@pytest.mark.parametrize("shape", [{"poly_ratio": 50.0}, {"poly_storage": _lib.LH_STORE_F32},
+                                   {"poly_storage": _lib.LH_STORE_F16}])
+def test_shaped_polynomial_runs(shape):
+    """An interval or storage for the automatic polynomial is an explicit choice
+    of it: bit for bit the solve with its degree spelled out."""
+    ctx = _lib.default_context()
+    a, b = Solver(TriaMesh(*meshgen.perturbed_sphere(5, np.random.default_rng(2), sigma=0.02))).device_matrices()
+    lam, x, st = _lib.eigs(ctx, a, b, 10, -0.01, **shape)
+    lam16, x16, st16 = _lib.eigs(ctx, a, b, 10, -0.01, poly_degree=16, **shape)  # round(sqrt(10,242) / 6.3)
+    assert (st.iterations, st.spmm_calls, st.fallback_used) == (st16.iterations, st16.spmm_calls, 0)
+    assert np.array_equal(lam, lam16) and np.array_equal(x, x16)
+
+
 def test_cycle_that_overflows_gives_way():
     """A and B near the largest FP32 number: the finest level fits, the coarse
     matrices of a volume, whose entries grow with the spacing, do not.  The
