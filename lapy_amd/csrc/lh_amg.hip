@@ -60,7 +60,8 @@ constexpr int kCoarsest = 128;       // rows of the inverted level at most (kCho
 constexpr int kTailRows = 2048;      // rows of a one-workgroup level at most
 constexpr int kTailNnz = 24576;      // and its entries: one CU reads them from L2 for every product
 constexpr int kTailSum = 2560;       // rows of all of them together at most
-constexpr int kLongRow = 20;         // mean row length from which a wave forms a row of P
+constexpr int kLongRow = 20;         // mean row length from which a wave forms a row of P,
+constexpr int kLongestRow = 128;     // and the longest from which it does whatever the mean
 constexpr double kSmoothRatio = 6.0; // the smoother's interval is [bmax / ratio, bmax]
 constexpr double kSmoothTop = 2.0;   // bmax at most (good elements: 1.5 to 1.9 on the finest level, 1.3 to 1.5 below)
 constexpr double kGuard = 1.16;      // rows' Gershgorin sums are held to this many bmax (7/6: the smoother's limit)
@@ -116,11 +117,13 @@ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
 // again in each round.
 
 // dinv and the row sums of |D^-1 K|; bad[0] set when a row's diagonal is negative, missing or zero beside
-// non-zero entries; start vector of the power iteration (0 on zero rows)
+// non-zero entries; start vector of the power iteration (0 on zero rows);
+// longest: raised to the length of the rows above kLongestRow, if any
 template <int G>
 __global__ void __launch_bounds__(256)
 k_amg_diag(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl, const double* __restrict__ kv,
-           double* __restrict__ dinv, double* __restrict__ gersh, double* __restrict__ x, int* __restrict__ bad) {
+           double* __restrict__ dinv, double* __restrict__ gersh, double* __restrict__ x, int* __restrict__ bad,
+           int* __restrict__ longest) {
     const int64_t i = (xcd_block() * 256 + threadIdx.x) / G;
     if (i >= n) return;
     double d = 0.0, other = 0.0;  // other: sum of the magnitudes beside the diagonal
@@ -136,6 +139,7 @@ k_amg_diag(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict_
     if (threadIdx.x % G) return;
     if (!(d >= 0.0) || (d == 0.0 && other != 0.0)) bad[0] = 1;  // every writer stores the same value
     const bool pos = d > 0.0;
+    if (rp[i + 1] - rp[i] > kLongestRow) atomicMax(longest, rp[i + 1] - rp[i]);
     dinv[i] = pos ? 1.0 / d : 0.0;
     gersh[i] = pos ? 1.0 + other / d : 0.0;
     x[i] = pos ? (double)(mix32((uint32_t)i * 2654435761u + 12345u) >> 8) * (1.0 / 8388608.0) - 1.0 : 0.0;
@@ -296,7 +300,9 @@ k_agg_join(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict_
 // P = (I - w D^-1 K) P_0 row by row: first the number of distinct aggregates
 // among a row's columns, then the entries in the order of first appearance.
 // One thread per row for short rows; for long ones (below) the quadratic
-// search is spread over a wave.
+// search is spread over a wave, also where a single row is long: the pole of a
+// sphere of meridians has an entry and a third of an aggregate for each, and
+// at 1,000 of them one thread's search took about 100 ms, twice.
 template <bool FILL>
 __global__ void k_prolongator(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ cl,
                               const double* __restrict__ kv, const double* __restrict__ dinv, double w,
@@ -480,11 +486,11 @@ k_spgemm(int64_t n, const int32_t* __restrict__ xp, const int32_t* __restrict__ 
     const int32_t a = xp[row], b = xp[row + 1];
     if (!FILL) {
         int mine = 0;
-        // lanes over X's entries; more than HS distinct columns: hash_slot gives up
-        for (int32_t e = a + lane; e < b; e += 64) {
+        // lanes over X's entries; more than HS distinct columns: hash_slot gives
+        // up after a search of the whole table, and the lane with it
+        for (int32_t e = a + lane; e < b && !mine; e += 64) {
             const int32_t j = xc[e];
-            for (int32_t q = yp[j]; q < yp[j + 1]; ++q)
-                if (hash_slot<HS>(keys, yc[q]) < 0) mine = 1;
+            for (int32_t q = yp[j]; q < yp[j + 1] && !mine; ++q) mine = hash_slot<HS>(keys, yc[q]) < 0;
         }
         wave_fence();
         int cnt = 0;
@@ -1067,7 +1073,8 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
     levels.clear();
     keep.clear();
     hipStream_t st = ctx->stream;
-    DevBuf flags(64);         // [0] bad diagonal, [1] hash table too small
+    DevBuf flags(64);         // [0] bad diagonal, [1] hash table too small, [2 + level] longest row
+    static_assert((2 + kMaxLevels) * 4 <= 64, "flags");
     memset_d(ctx, flags.p, 0, 64);
     int* bad = flags.as<int>();
     int* over = bad + 1;
@@ -1095,7 +1102,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         const unsigned nb = nblocks(n, 256), nbx = nblocks_xcd(n, 256);
         const int g = lanes_for(nnz, n);
         const unsigned nbg = nblocks_xcd(n * g, 256);
-        with_lanes(g, [&](auto G) { k_amg_diag<G.v><<<nbg, 256, 0, st>>>(n, rp, cl, kv, dinv, gersh.as<double>(), x.as<double>(), bad); });
+        with_lanes(g, [&](auto G) { k_amg_diag<G.v><<<nbg, 256, 0, st>>>(n, rp, cl, kv, dinv, gersh.as<double>(), x.as<double>(), bad, bad + 2 + l); });
         LH_CHECK_LAUNCH();
         if (n <= kCoarsest) {
             // last level: its inverse
@@ -1146,9 +1153,9 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         LH_CHECK_LAUNCH();
         double hp[2 * kRB];
         int32_t nc32 = 0;
-        int hb[2] = {0, 0};
+        int hb[2 + kMaxLevels] = {};
         {
-            const Xfer q[3] = {{hp, part.p, sizeof(hp)}, {&nc32, idx.as<int32_t>() + n, 4}, {hb, flags.p, 8}};
+            const Xfer q[3] = {{hp, part.p, sizeof(hp)}, {&nc32, idx.as<int32_t>() + n, 4}, {hb, flags.p, sizeof(hb)}};
             d2h_n(ctx, q, 3);
         }
         double xdx = 0.0, xkx = 0.0;
@@ -1167,7 +1174,7 @@ bool Amg::setup(lh_ctx* c, int64_t n0, int64_t nnz0, const int32_t* rp0, const i
         const double w = 4.0 / (3.0 * lv.bmax);
         // P
         int32_t* pp = own<int32_t>(n + 1);
-        const bool long_rows = nnz > kLongRow * n;
+        const bool long_rows = nnz > kLongRow * n || hb[2 + l] > 0;
         if (long_rows)
             k_prolongator_wave<false><<<nblocks(n, 4), 256, 0, st>>>(n, rp, cl, kv, dinv, w, ga, nullptr,
                                                                      cnt.as<int32_t>(), nullptr);
