@@ -13,6 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("level,keep,k", [
+    (2, 1.0, 7),     # 162 rows: the dense solver's own columns
+    (2, 0.93, 40),   # an odd number of them, past one tile of columns
     (3, 1.0, 31),    # 642 rows: the caller's order, below one tile of columns
     (3, 0.61, 33),   # an odd number of rows, one column into the second tile
     (5, 0.413, 32),  # above 4,096 rows: the locality order undone

@@ -100,28 +100,36 @@ def test_systems_left_to_jacobi():
     weak = sparse.diags([-1e-3 * np.ones(n - 1), np.ones(n), -1e-3 * np.ones(n - 1)], [-1, 0, 1], format="csr")
     b = rng.standard_normal(n)
     for m in (-lap, sparse.csr_matrix(sparse.diags(rng.uniform(1, 2, n))), weak):
-        x, _ = _lib.pcg(ctx, _lib.DeviceCSR.from_scipy(ctx, m), None, 0.0, 1.0, b, rtol=1e-12)
+        a = _lib.DeviceCSR.from_scipy(ctx, m)
+        x, st = _lib.pcg(ctx, a, None, 0.0, 1.0, b, rtol=1e-12)
         assert np.linalg.norm(b - m @ x) <= 1e-11 * np.linalg.norm(b)
+        xj, st_j = _lib.pcg(ctx, a, None, 0.0, 1.0, b, rtol=1e-12, poly_degree=1)
+        assert (st.iterations, st.fallback_used) == (st_j.iterations, 0) and np.array_equal(x, xj)
 
 
 def test_rows_with_many_entries():
-    """A graph Laplacian with rows of 3 to ~60 entries, not from a mesh: CSR
-    products, long rows in every setup kernel, hash tables of both sizes."""
+    """A graph Laplacian with rows of 3 to ~300 entries, not from a mesh: CSR
+    products, long rows in every setup kernel, hash tables of both sizes (a hub
+    couples most of the ~700 aggregates, weakly)."""
     ctx = _lib.default_context()
     n = 5003
     rng = np.random.default_rng(6)
-    i = np.repeat(np.arange(n), 14)
-    j = (i + np.rint(rng.normal(0, 60, len(i))).astype(int)) % n
-    hub = rng.choice(n, 40, replace=False)
-    i = np.concatenate([i, np.repeat(hub, 30)])
-    j = np.concatenate([j, rng.integers(0, n, 40 * 30)])
+    i = np.repeat(np.arange(n), 3)
+    j = (i + np.rint(rng.normal(0, 3, len(i))).astype(int)) % n
+    hub = rng.choice(n, 8, replace=False)
+    i = np.concatenate([i, np.repeat(hub, 300)])
+    j = np.concatenate([j, rng.integers(0, n, 8 * 300)])
+    wt = np.where(np.arange(len(i)) < 3 * n, rng.uniform(0.5, 1.5, len(i)), 0.01)
     keep = i != j
-    w = sparse.coo_matrix((rng.uniform(0.5, 1.5, keep.sum()), (i[keep], j[keep])), shape=(n, n)).tocsr()
+    w = sparse.coo_matrix((wt[keep], (i[keep], j[keep])), shape=(n, n)).tocsr()
     w = w + w.T
     a = sparse.csr_matrix(sparse.diags(np.asarray(w.sum(axis=1)).ravel() + 1e-3) - w)
     b = rng.standard_normal(n)
-    x, st = _lib.pcg(ctx, _lib.DeviceCSR.from_scipy(ctx, a), None, 0.0, 1.0, b, rtol=1e-12)
-    print("iterations", st.iterations, "longest row", np.diff(a.indptr).max())
+    d = _lib.DeviceCSR.from_scipy(ctx, a)
+    x, st = _lib.pcg(ctx, d, None, 0.0, 1.0, b, rtol=1e-12)
+    _, st_j = _lib.pcg(ctx, d, None, 0.0, 1.0, b, rtol=1e-12, poly_degree=1)
+    print("iterations", st.iterations, "jacobi", st_j.iterations, "longest row", np.diff(a.indptr).max())
+    assert st.fallback_used == 0 and 4 * st.iterations < st_j.iterations  # the cycle ran
     assert np.linalg.norm(b - a @ x) <= 1e-11 * np.linalg.norm(b)
 
 
@@ -332,6 +340,43 @@ def test_cycle_that_overflows_gives_way():
     print("iterations", fem.last_stats.iterations)
     assert fem.last_stats.fallback_used == 1
     assert np.all(np.abs(big - lam) <= 1e-10 * lam[-1])
+
+
+# partials of r.z from the cycle (up to four columns) and from a launch of
+# their own: both go back to Jacobi's after the limit
+@pytest.mark.parametrize("m", [1, 3, 4, 6])
+@pytest.mark.parametrize("singular", [False, True])
+def test_linear_solves_past_the_cycles_limit(m, singular, cycle_limits):
+    ctx = _lib.default_context()
+    _, fem, _ = next(_systems())
+    a = sparse.csr_matrix(fem.stiffness)
+    n = a.shape[0]
+    rng = np.random.default_rng(m)
+    dmask = np.zeros(n, np.uint8)
+    if not singular:
+        dmask[rng.choice(n, 20, replace=False)] = 1
+    free = np.flatnonzero(dmask == 0)
+    b = rng.standard_normal((n, m))
+    if singular:
+        b -= b.mean(axis=0)
+    dm = None if singular else dmask
+    _, full = _lib.pcg(ctx, fem.device_matrices()[0], None, 0.0, 1.0, b, dmask=dm, rtol=1e-12)
+    cycle_limits(cg=8)
+    x, st = _lib.pcg(ctx, fem.device_matrices()[0], None, 0.0, 1.0, b, dmask=dm, rtol=1e-12)
+    print("columns", m, "iterations", full.iterations, "with the limit", st.iterations)
+    assert full.fallback_used == 0 and st.fallback_used == 1 and st.iterations > 100
+    for c in range(m):
+        assert np.linalg.norm(b[free, c] - a[free][:, free] @ x[free, c]) <= 1e-11 * np.linalg.norm(b[free, c])
+
+
+@pytest.mark.parametrize("limit", [1, 5])
+def test_eigensolve_past_the_cycles_limit(limit, cycle_limits):
+    fem = _eig_problem("cap")
+    lam, _ = fem.eigs(k=12)
+    cycle_limits(eig=limit)
+    late, _ = fem.eigs(k=12)
+    assert fem.last_stats.fallback_used == 1 and fem.last_stats.iterations > limit
+    assert np.all(np.abs(late - lam) <= 1e-10 * lam[-1])
 
 
 @pytest.mark.parametrize("jitter", [0.2, 0.25, 0.28])  # of the spacing: elements from bad to almost flat
