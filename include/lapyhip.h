@@ -96,6 +96,11 @@ int  lh_ctx_create(int device, lh_ctx** out);
 void lh_ctx_destroy(lh_ctx* ctx);
 const char* lh_last_error(lh_ctx* ctx);
 int  lh_sync(lh_ctx* ctx);
+/* A context keeps the work memory of lh_eigs and lh_pcg between calls (at most
+ * 1 GiB), and that of lh_eigs_batched's workers (as large as the largest
+ * problem needed).  lh_ctx_trim gives all of it back; an allocation on the
+ * context that would fail without the former gives that back by itself. */
+int  lh_ctx_trim(lh_ctx* ctx);
 /* Iterations that the eigensolver (default 80; each phase of a mixed-precision
  * solve counts its own) and the linear solver (200, looked at every fourth)
  * keep their automatic multigrid cycle before they go on with the Chebyshev

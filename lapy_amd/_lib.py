@@ -89,6 +89,7 @@ SIGNATURES = {
     "lh_ctx_destroy": (None, [_vp]),
     "lh_last_error": (C.c_char_p, [_vp]),
     "lh_sync": (C.c_int, [_vp]),
+    "lh_ctx_trim": (C.c_int, [_vp]),
     "lh_content_hash": (C.c_int, [_vp, C.c_uint64, C.POINTER(C.c_uint64)]),
     "lh_mesh_create": (C.c_int, [_vp, _vp, C.c_int, _i64, _vp, _i64, C.c_int, C.POINTER(_vp)]),
     "lh_mesh_create_device": (C.c_int, [_vp, _vp, C.c_int, _i64, _vp, _i64, C.c_int, C.POINTER(_vp)]),
@@ -217,6 +218,10 @@ class Context:
                 self.handle = None
         except Exception:
             pass
+
+    def trim(self):
+        """Give back the device memory kept between calls (lh_ctx_trim)."""
+        check(lib().lh_ctx_trim(self.handle), self, "lh_ctx_trim")
 
     def sync(self):
         check(lib().lh_sync(self.handle), self, "lh_sync")

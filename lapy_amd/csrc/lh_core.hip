@@ -226,6 +226,28 @@ void refresh_dense_diag(lh_ctx* ctx, lh_csr* a) {
 using namespace lh;
 
 thread_local Arena* lh_thread_arena = nullptr;
+thread_local lh_ctx* lh_api_ctx = nullptr;
+
+static bool release_arena(lh_ctx* c) {
+    if (!c || c->arena_busy || !c->arena_mem.p) return false;
+    c->arena = Arena{};
+    c->arena_mem.release();  // waits for the device
+    return true;
+}
+bool lh_release_idle_arena() { return release_arena(lh_api_ctx); }
+
+extern "C" int lh_ctx_trim(lh_ctx* ctx) {
+    if (!ctx) return LH_ERR_ARG;
+    LH_API_BEGIN(ctx)
+    HIPX(hipSetDevice(ctx->device));
+    HIPX(hipStreamSynchronize(ctx->stream));
+    release_arena(ctx);
+    for (lh_ctx* w : ctx->workers) {
+        HIPX(hipStreamSynchronize(w->stream));
+        release_arena(w);
+    }
+    LH_API_END(ctx)
+}
 
 extern "C" {
 

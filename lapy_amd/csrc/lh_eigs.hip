@@ -558,8 +558,9 @@ int block_width(int k, const lh_eig_opts* opts) {
 // one generalized eigenproblem on ctx's stream; throws lh_error on bad
 // arguments or failures, returns the result with code LH_OK or
 // LH_ERR_NOCONV (results of the last iteration)
+// lean: without the multigrid hierarchy (and, where the caller made none, an arena)
 lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const lh_eig_opts* opts, lh_stats& st,
-                  int& code) {
+                  int& code, bool lean) {
     const int64_t n = A->n();
     if (B->n() != n) LH_THROW(LH_ERR_ARG, "A and B differ in size (%lld vs %lld)", (long long)n, (long long)B->n());
     if (k <= 0 || k >= n) LH_THROW(LH_ERR_ARG, "k must satisfy 0 < k < n (k=%d, n=%lld)", k, (long long)n);
@@ -609,7 +610,7 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
     int deg = opts ? opts->poly_degree : 0;
     // an interval or a storage for the polynomial asks for the polynomial
     const bool shaped = opts && (opts->poly_ratio > 1.0 || opts->poly_storage != LH_STORE_AUTO);
-    L.use_amg = jac && deg <= 0 && !shaped;
+    L.use_amg = jac && deg <= 0 && !shaped && !lean;
     if (ctx->eig_cycle_limit > 0) L.amg_max_iters = ctx->eig_cycle_limit;
     if (!jac) deg = 1;
     if (deg <= 0) deg = auto_deg < 4 ? 1 : auto_deg;
@@ -757,7 +758,16 @@ void solve_batch(lh_ctx* ctx, int nmesh, lh_csr* const* A, lh_csr* const* B, con
             int code = LH_OK;
             lh_eig* e = nullptr;
             try {
-                e = eigs_impl(wc, A[i], B[i], k[i], sigma, opts, sti, code);
+                try {
+                    e = eigs_impl(wc, A[i], B[i], k[i], sigma, opts, sti, code, false);
+                } catch (const lh_error& ex) {
+                    if (ex.code != LH_ERR_OOM) throw;
+                    (void)hipGetLastError();
+                    (void)hipStreamSynchronize(wc->stream);
+                    wc->arena.top = mark;  // every buffer of the attempt is released
+                    sti = lh_stats{};
+                    e = eigs_impl(wc, A[i], B[i], k[i], sigma, opts, sti, code, true);
+                }
                 if (e) e->ctx = ctx;
             } catch (const lh_error& ex) {
                 code = ex.code;
@@ -798,8 +808,18 @@ int lh_eigs(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const lh_eig
     HIPX(hipSetDevice(ctx->device));
     lh_stats st{};
     int code = LH_OK;
-    CallArena arena(ctx, arena_bytes(A->n(), block_width(k, opts)));
-    *out = eigs_impl(ctx, A, B, k, sigma, opts, st, code);
+    try {
+        CallArena arena(ctx, arena_bytes(A->n(), block_width(k, opts)));
+        *out = eigs_impl(ctx, A, B, k, sigma, opts, st, code, false);
+    } catch (const lh_error& e) {
+        if (e.code != LH_ERR_OOM) throw;
+    }
+    if (!*out) {  // again with what the polynomial needs
+        (void)hipGetLastError();
+        lh_release_idle_arena();
+        st = lh_stats{};
+        *out = eigs_impl(ctx, A, B, k, sigma, opts, st, code, true);
+    }
     if (stats) *stats = st;
     if (code == LH_ERR_NOCONV) {
         ctx->last_error = "LOBPCG did not converge within max_iter";

@@ -58,6 +58,9 @@ struct Arena {
     }
 };
 extern thread_local Arena* lh_thread_arena;
+// gives back the memory that the context of this thread's entry point keeps
+// between calls, unless the call itself is using it; false: nothing to give
+bool lh_release_idle_arena();
 
 struct DevBuf {
     void* p = nullptr;
@@ -94,7 +97,12 @@ struct DevBuf {
             }
         }
         hipError_t e = hipMalloc(&p, n);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();  // or the next launch check would report it
+            if (lh_release_idle_arena()) e = hipMalloc(&p, n);
+        }
         if (e != hipSuccess) {
+            (void)hipGetLastError();
             p = nullptr;
             LH_THROW(LH_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", n, hipGetErrorString(e));
         }
@@ -147,6 +155,7 @@ struct lh_ctx {
     std::vector<lh_ctx*> workers;
     DevBuf arena_mem;
     Arena arena;
+    bool arena_busy = false;  // a CallArena is on it
     int tuned_workers = 0;  // 0: not tuned
     lh_mpnn* mpnn = nullptr;  // network used by LH_PRECOND_LEARNED (not owned)
     void* host_small = nullptr;   // pinned host memory (hipHostMalloc): the PCG's status polling, the
@@ -161,8 +170,10 @@ struct lh_ctx {
 };
 
 // A solve's temporaries from its context's own arena (bounded by kMost, kept
-// until the context ends): without it a small solve spends as long in
-// hipMalloc and hipFree as on the device.  Does nothing where the thread has
+// until the context ends, lh_ctx_trim or an allocation of the context that
+// would fail without it): without it a small solve spends as long in
+// hipMalloc and hipFree as on the device (a pair of them takes 0.3 ms from 200 MiB
+// up, of a solve of 4 to 10).  Does nothing where the thread has
 // an arena already (the batched solver's workers).  What does not fit comes
 // from hipMalloc as before.  One call at a time uses a context and its stream,
 // so the memory is reused in stream order.
@@ -170,14 +181,13 @@ struct CallArena {
     static constexpr size_t kLeast = size_t(64) << 20, kMost = size_t(1) << 30;
     lh_ctx* ctx = nullptr;
     CallArena(lh_ctx* c, size_t want) {
-        if (lh_thread_arena) return;
+        if (!c || lh_thread_arena) return;
         want = want < kLeast ? kLeast : want > kMost ? kMost : want;
         if (c->arena_mem.bytes < want) {
             c->arena.base = nullptr;
             try {
                 c->arena_mem.alloc(want);
             } catch (const lh_error&) {  // no room: plain allocations, which may still fit
-                (void)hipGetLastError();
                 return;
             }
         }
@@ -186,11 +196,13 @@ struct CallArena {
         c->arena.top = 0;
         lh_thread_arena = &c->arena;
         ctx = c;
+        ctx->arena_busy = true;
     }
     ~CallArena() {
         if (!ctx) return;
         lh_thread_arena = nullptr;
         ctx->arena.top = 0;
+        ctx->arena_busy = false;
     }
     CallArena(const CallArena&) = delete;
     CallArena& operator=(const CallArena&) = delete;
@@ -409,7 +421,17 @@ inline int vec_lanes(int ncol, int vec) {
 }  // namespace lh
 
 // C-ABI guard
-#define LH_API_BEGIN(ctx) try {
+// the context whose entry point this thread is in
+extern thread_local lh_ctx* lh_api_ctx;
+struct ApiCall {
+    lh_ctx* saved;
+    explicit ApiCall(lh_ctx* c) : saved(lh_api_ctx) { lh_api_ctx = c; }
+    ~ApiCall() { lh_api_ctx = saved; }
+    ApiCall(const ApiCall&) = delete;
+    ApiCall& operator=(const ApiCall&) = delete;
+};
+
+#define LH_API_BEGIN(ctx) try { ApiCall lh_api_call_(ctx);
 #define LH_API_END(ctx)                                                       \
     }                                                                         \
     catch (const lh_error& e) {                                               \

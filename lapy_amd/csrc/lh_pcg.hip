@@ -873,13 +873,11 @@ struct Launcher {
 
 }  // namespace
 
-extern "C" {
+namespace {
 
-int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const double* b, int nrhs,
-           const uint8_t* dmask, double* x, const lh_pcg_opts* opts, lh_stats* stats) {
-    if (!ctx || !A || !b || !x || nrhs <= 0) return LH_ERR_ARG;
-    LH_API_BEGIN(ctx)
-    HIPX(hipSetDevice(ctx->device));
+// lean: without the call arena and the multigrid hierarchy
+int pcg_solve(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const double* b, int nrhs,
+              const uint8_t* dmask, double* x, const lh_pcg_opts* opts, lh_stats* stats, bool lean) {
     const double t0 = now_us();
     const int64_t n = A->n(), nnz = A->nnz();
     if (B && B->n() != n) LH_THROW(LH_ERR_ARG, "A and B differ in size");
@@ -891,7 +889,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     const int precond = opts ? opts->precond : LH_PRECOND_JACOBI;
     if (precond != LH_PRECOND_JACOBI && precond != LH_PRECOND_LEARNED && precond != LH_PRECOND_NONE)
         LH_THROW(LH_ERR_ARG, "preconditioner %d unknown", precond);
-    // Chebyshev-Jacobi degree (Jacobi only): 0 or 1 plain Jacobi
+    // Chebyshev-Jacobi degree (Jacobi only): 1 plain Jacobi, 0 the automatic choice
     const int pdeg_opt = opts ? opts->poly_degree : 0;
     if (pdeg_opt < 0 || pdeg_opt > 256) LH_THROW(LH_ERR_ARG, "poly_degree must be in [0, 256], got %d", pdeg_opt);
     if (precond == LH_PRECOND_LEARNED && !ctx->mpnn)
@@ -900,7 +898,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     lh_stats st{};
     // values, reordered and ELL copies, the multigrid hierarchy (~100 bytes an
     // entry) and the block vectors
-    CallArena arena(ctx, (size_t)nnz * 100 + (size_t)n * 8 * (20 + 14 * (size_t)m));
+    CallArena arena(lean ? nullptr : ctx, (size_t)nnz * 100 + (size_t)n * 8 * (20 + 14 * (size_t)m));
     // operator values on A's pattern
     DevBuf kv(nnz * 8), missing(8);
     memset_d(ctx, missing.p, 0, 4);
@@ -1063,7 +1061,7 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
     Amg amg;
     bool amg_on = false;
     const int amg_max_iters = ctx->cg_cycle_limit > 0 ? ctx->cg_cycle_limit : kAmgMaxIters;
-    if (precond == LH_PRECOND_JACOBI && pdeg_opt == 0) {
+    if (precond == LH_PRECOND_JACOBI && pdeg_opt == 0 && !lean) {
         const double dn = (double)n;
         double expect = (double)nnz > 10.0 * dn ? 14.4 * std::cbrt(dn) : 5.4 * std::sqrt(dn);
         expect *= std::log(2.0 / rtol) / std::log(2e12);
@@ -1253,7 +1251,24 @@ int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const d
         ctx->last_error = "PCG did not converge within max_iter";
         return LH_ERR_NOCONV;
     }
-    LH_API_END(ctx)
+    return LH_OK;
 }
 
-}  // extern "C"
+}  // namespace
+
+extern "C" int lh_pcg(lh_ctx* ctx, lh_csr* A, lh_csr* B, double alpha, double beta, const double* b, int nrhs,
+                      const uint8_t* dmask, double* x, const lh_pcg_opts* opts, lh_stats* stats) {
+    if (!ctx || !A || !b || !x || nrhs <= 0) return LH_ERR_ARG;
+    LH_API_BEGIN(ctx)
+    HIPX(hipSetDevice(ctx->device));
+    try {
+        return pcg_solve(ctx, A, B, alpha, beta, b, nrhs, dmask, x, opts, stats, false);
+    } catch (const lh_error& e) {
+        if (e.code != LH_ERR_OOM) throw;
+    }
+    // x holds its start until a solve ends: again with what Jacobi needs
+    (void)hipGetLastError();
+    lh_release_idle_arena();
+    return pcg_solve(ctx, A, B, alpha, beta, b, nrhs, dmask, x, opts, stats, true);
+    LH_API_END(ctx)
+}
