@@ -99,6 +99,7 @@ void with_lanes(int g, F&& f) {
     }
 }
 
+// C. Wellons' "lowbias32" (hash prospector, 2018), a 32-bit integer mixer
 __device__ __forceinline__ uint32_t mix32(uint32_t x) {
     x ^= x >> 16;
     x *= 0x7feb352du;
@@ -1435,7 +1436,10 @@ void Amg::apply(const double* R, double* Z, double* part, const int* status) { c
 // and 24; on a surface with noise of two edge lengths 15 with three cycles, 14
 // with the inverse, 21 with two).  Three from kManyRows rows on, where an
 // iteration's other work is ten times a cycle's; two below, where a cycle is
-// launch latency and costs a seventh of an iteration.
+// launch latency and costs a seventh of an iteration.  Whole solves of caps of an
+// ellipsoid with two | three cycles, ms, 10 pairs and 50: 52,418 rows 8.7 | 9.6, 31.9 | 33.5;
+// 104,853 11.5 | 11.9, 50.2 | 54.0; 163,842 17.2 | 17.7, 77.5 | 75.7; 655,362,
+// 50 pairs, 28 | 22 iterations.
 // Three too where the estimate of lambda_max(D^-1 K) is above kRough (surfaces
 // reach 2.3 with noise of two edge lengths, tets jittered by 0.18 of the spacing
 // 2.1, by 0.2, which makes flat ones, 2.8 to 3.8): the cycle leaves a few of the
@@ -1443,7 +1447,7 @@ void Amg::apply(const double* R, double* Z, double* part, const int* status) { c
 // 41 iterations and 24 ms (10 pairs), by 0.28 33 and 37 (30 pairs) with two, 31
 // and 22, 22 and 29 with three; by 0.2, 20 and 12.5 against 18 and 13.3.
 constexpr double kBlkHi = 1.02, kBlkLo2 = 0.35, kBlkLo3 = 0.2;
-constexpr int64_t kManyRows = 65536;
+constexpr int64_t kManyRows = 131072;
 constexpr double kRough = 2.5;
 
 void Amg::prepare_blocks(int m_, int ell_w, const int32_t* ecl) {

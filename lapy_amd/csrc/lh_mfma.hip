@@ -19,7 +19,8 @@
 // Narrow blocks (at most 9 useful blocks of 16 x 16) use a variant whose
 // blocks hold contiguous columns, so the blocks beyond p or q are skipped.
 //
-// Update: a wave owns 64 rows x 64 columns of Y (64 x 16 for small n); per
+// Update: a wave owns 32 rows x 64 columns of Y (16 x 16 for small n and for
+// widths that 64 columns would pad too far, gemm_narrow); per
 // group of 16 columns of U (the summed index) each lane loads 4 consecutive
 // values of its row (one 32-byte load), which serve as the A operand of 4
 // successive MFMAs, and the matching 4 rows of C (L2-resident) as B.
@@ -551,12 +552,16 @@ void gram_mfma(lh_ctx* ctx, int64_t n, const T* U, int ldu, int p, const T* V, i
 // (in place: upper triangular): 10,242 rows 64 -> 128 14 | 13, 192 -> 64 27 | 20,
 // 48 -> 16 9.6 | 4.3; 29,160 rows 64 -> 128 22 | 29, 192 -> 64 34 | 39,
 // 128 in place 38 | 35; 131,072 rows 40 -> 80 51 | 54, 80 in place 76 | 64,
-// 120 -> 40 55 | 78, 48 -> 16 24 | 14, 32 in place 22 | 18.  Within a solve of
-// 35,937 rows, 40 -> 80 and 120 -> 40 together: 23.6 | 18.6.
+// 120 -> 40 55 | 78, 48 -> 16 24 | 14, 32 in place 22 | 18.  Moderate padding
+// (q = 33 .. 48, 65 .. 96) pays below 1,600 waves of the larger tile: 120 -> 40 at 24,577,
+// 35,937, 45,000, 60,000 and 90,000 rows (769 to 2,813 waves) 23 | 21, 32 | 27, 33 | 31,
+// 33 | 40, 43 | 56; 96 -> 96 at 18,000, 24,577 and 30,000 rows (1,126 to 1,876) 25 | 21,
+// 27 | 28, 28 | 32.  In place to 2,400: 48 at 60,000, 66,000 and 76,000 rows (1,875 to
+// 2,375) 18 | 17, 21 | 18, 23 | 20.
 inline bool gemm_narrow(int64_t n, int q, bool inplace) {
     const int q16 = (q + 15) / 16 * 16, q64 = (q + 63) / 64 * 64;
     const int64_t waves = (n + 31) / 32 * (q64 / 64);
-    return waves < (inplace ? 2048 : 768) || q16 * (inplace ? 24 : 26) < q64 * 16 || (waves < 2400 && q16 * 20 < q64 * 16);
+    return waves < (inplace ? 2048 : 768) || q16 * (inplace ? 24 : 26) < q64 * 16 || (waves < (inplace ? 2400 : 1600) && q16 * 20 < q64 * 16);
 }
 
 template <int NB, bool INPLACE, bool GROUPED, typename T>
