@@ -11,7 +11,7 @@
 //    with hashed keys in a fixed number of rounds; the roots are numbered in
 //    row order, so the coarse rows keep the fine rows' locality;
 //  * P = (I - w D^-1 K) P_0, P_0 the aggregates' indicator, w = 4 / (3
-//    lambda_max): the smoothing that makes the interpolated coarse functions
+//    bmax): the smoothing that makes the interpolated coarse functions
 //    continuous, without which the cycle's quality decays with every level;
 //  * K_c = P^T (K P): two sparse products, one wave per output row, the
 //    row's entries gathered in a hash table in LDS whose values are summed

@@ -10,7 +10,7 @@ namespace lh {
 template <typename T>
 struct AmgOps {
     const T* kv = nullptr;    // K (the level's CSR slots; level 0 with an ELL copy: its slots)
-    const T* dinv = nullptr;  // 1 / diag K (0 on a zero row)
+    const T* dinv = nullptr;  // 1 / diag K, smaller in the guarded rows (0 on a zero row)
     const T* pv = nullptr;    // P
     const T* rv = nullptr;    // P^T
 };
@@ -23,7 +23,7 @@ struct AmgLevel {
     const int32_t* ecl = nullptr;
     const double* ekv = nullptr;
     const float* ekv32 = nullptr;
-    double bmax = 2.0;  // upper end of the smoother's interval (estimate of lambda_max(D^-1 K))
+    double bmax = 2.0;  // upper end of the smoother's interval
     // transfer to the next level (absent on the last one)
     int64_t nc = 0, pnnz = 0;
     const int32_t *pp = nullptr, *pc = nullptr;  // P (n x nc), CSR

@@ -586,7 +586,9 @@ lh_eig* eigs_impl(lh_ctx* ctx, lh_csr* A, lh_csr* B, int k, double sigma, const 
     // 21 -> 13, 8.4 -> 5.4 ms; 10,242, 10 pairs 27 -> 15, 13.7 -> 8.7; 29,000,
     // 50 pairs 20 -> 19, 42.9 -> 41.0; 655,362, 50 pairs 25 -> 22, 402 -> 242
     // (the polynomial's 128 products an iteration against 14 with FP32
-    // blocks).  Otherwise: Jacobi, accelerated by a Chebyshev polynomial on
+    // blocks); 386 to 485 vertices, 10 pairs, 48 to 57 -> 11 to 13, 18 to 21 -> 3.2 to
+    // 4.0 ms against plain Jacobi, which is FP64 where the cycle's blocks are FP32: the
+    // residuals that set the accuracy are FP64 with either.  Otherwise: Jacobi, accelerated by a Chebyshev polynomial on
     // [lmax / (2 d^2), lmax] whose degree d grows with sqrt(n) (the condition
     // number of a mesh Laplacian grows like n^(2/dim)) until the iteration
     // count stops falling (128 at 655k vertices: beyond it the block's own

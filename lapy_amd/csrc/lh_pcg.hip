@@ -20,10 +20,10 @@
 //
 // Large ill-conditioned systems are preconditioned by a multigrid cycle
 // (lh_amg.hip), the others by Jacobi.  Against Jacobi-CG, a whole call: a
-// singular Poisson solve on a closed surface of 163,842 vertices 2,496 -> 32
-// iterations (46 -> 7 ms on the device), a Dirichlet one of 40,962 1,168 -> 24
-// (17.4 -> 4.0 ms), three columns of mass + stiffness at 10,242 715 -> 28 (28 ->
-// 5 ms), and the solutions' error against 64-bit references is 2 to 10 times
+// singular Poisson solve on a closed surface of 163,842 vertices 2,496 -> 26 to 32
+// iterations (46 -> 6.3 ms), a Dirichlet one of 40,962 1,168 -> 20 to 24
+// (17.4 -> 3.7 ms), three columns of mass + stiffness at 10,242 715 -> 22 to 28 (28 ->
+// 3 to 5 ms), and the solutions' error against 64-bit references is 2 to 10 times
 // smaller, since the residual left over lies in the high frequencies.  Below
 // ~350 Jacobi iterations the hierarchy's setup (1.5 ms at 40,962 rows, bound
 // by the latency of ~400 small launches) costs more than it saves.
