@@ -158,6 +158,34 @@ struct Lobpcg {
         return true;
     }
 
+    // the same for a block whose Gram matrix is not positive definite to
+    // rounding though its columns differ: a first factorisation with the unit
+    // diagonal raised by more than the Gram's rounding, which shortens the
+    // condition number by the shift's root, then the ordinary one (shifted
+    // Cholesky QR; Fukaya, Kannan, Nakatsukasa, Yamamoto, Yanagisawa 2020).
+    // The cycles' first W needs it, above all in FP32: the near-null
+    // components (a constant on each part of a mesh) are 1e4 to 1e5 times the
+    // others until X holds them.
+    bool cholqr_shifted(int off, int c) {
+        constexpr double kShift = sizeof(T) == 8 ? 1e-10 : 1e-5;
+        if (c > kCholMax) {
+            const int c1 = (c + 1) / 2, c2 = c - c1;
+            if (!cholqr_shifted(off, c1)) return false;
+            project_out(off, c1, off + c1, c2);
+            project_out(off, c1, off + c1, c2);
+            return cholqr_shifted(off + c1, c2);
+        }
+        T* X = Sp() + off;
+        T* MX = MSp() + off;
+        spmm_B(X, MX, c);
+        gram<T>(ctx, n, X, ld, c, MX, ld, c, Gs.as<double>(), c, wsg, 1.0, true);
+        cholinv(ctx, c, Gs.as<double>(), Ts.as<double>(), kShift, status.as<int>());
+        if (read_status()) return false;  // a zero or not finite column
+        gemm_mfma_inplace(ctx, n, c, X, ld, Ts.as<double>(), c, 1.0, true);
+        spmm_B(X, MX, c);
+        return cholqr(off, c, true);
+    }
+
     // Y -= X C with C = (B X)^T Y  (X block at xoff, Y block at yoff, widths cx, cy)
     void project_out(int xoff, int cx, int yoff, int cy) {
         gram<T>(ctx, n, MSp() + xoff, ld, cx, Sp() + yoff, ld, cy, Cm.as<double>(), cy, wsg);
@@ -431,6 +459,7 @@ struct Lobpcg {
                 nb = m;
                 full_rank = cholqr(m, nb, true);
             }
+            if (!full_rank && amg_on) full_rank = cholqr_shifted(m, m);
             if (!full_rank) {
                 if (!amg_on) LH_THROW(LH_ERR_NUMERIC, "Cholesky-QR of the residual block failed at iteration %d", it);
                 // the cycle's W is rank deficient or not finite: X and its

@@ -194,15 +194,17 @@ def test_rejected_hierarchy_costs_little():
     assert st.iterations > 200 and best[0] < 1.5 * best[1]
 
 
-def _eig_problem(name):
+def _eig_problem(name, unit=1.0):
     if name == "tail":  # 642 rows: every level in the one-launch tail
-        return Solver(TriaMesh(*meshgen.perturbed_sphere(3, np.random.default_rng(1), axes=(1.3, 0.8, 1.0), sigma=0.02)))
-    if name == "one level":  # 2,562 rows: the finest level launched, lumped mass
-        return Solver(TriaMesh(*meshgen.perturbed_sphere(4, np.random.default_rng(2), axes=(1.3, 0.8, 1.0), sigma=0.05)),
-                      lump=True)
-    if name == "cap":  # odd rows, the locality order, 8 slots a row
-        return Solver(TriaMesh(*_cap(5, 0.43)))
-    return Solver(TetMesh(*meshgen.tet_cube(17, jitter=0.15)))  # 5,832 rows of ~15 entries
+        v, t = meshgen.perturbed_sphere(3, np.random.default_rng(1), axes=(1.3, 0.8, 1.0), sigma=0.02)
+    elif name == "one level":  # 2,562 rows: the finest level launched, lumped mass
+        v, t = meshgen.perturbed_sphere(4, np.random.default_rng(2), axes=(1.3, 0.8, 1.0), sigma=0.05)
+    elif name == "cap":  # odd rows, the locality order, 8 slots a row
+        v, t = _cap(5, 0.43)
+    else:
+        v, t = meshgen.tet_cube(17, jitter=0.15)  # 5,832 rows of ~15 entries
+        return Solver(TetMesh(unit * v, t))
+    return Solver(TriaMesh(unit * v, t), lump=name == "one level")
 
 
 @pytest.mark.parametrize("name,k,block", [("tail", 5, 0), ("tail", 10, 13), ("one level", 9, 18), ("one level", 33, 0),
@@ -288,6 +290,23 @@ def test_cycle_spectrum(name):
     w = eigvalsh(c.T @ (0.5 * (m + m.T)) @ c)
     print(name, n, "M K in", w[0], w[-1])
     assert w[0] > 0.02 and w[-1] <= 1.0 + 1e-8
+
+
+@pytest.mark.parametrize("unit", [1.0, 1e-2, 1e-3])
+@pytest.mark.parametrize("name,k", [("tets", 20), ("tets", 77), ("cap", 50), ("tail", 10)])
+def test_mixed_precision_keeps_the_cycle(name, k, unit):
+    """FP32 blocks whose first preconditioned columns are the same to 1e-4 or
+    less (near-null components): orthonormalised in two steps instead of
+    refused, so that the solve takes the FP64 one's iterations, a few more for
+    the hand-over."""
+    fem = _eig_problem(name, unit)
+    lam, _ = fem.eigs(k=k)
+    its = fem.last_stats.iterations
+    mixed, _ = fem.eigs(k=k, precision="mixed")
+    st = fem.last_stats
+    print(name, k, unit, "iterations", its, "mixed", st.iterations)
+    assert st.fallback_used == 0 and st.iterations <= its + 8
+    assert np.all(np.abs(mixed - lam) <= 1e-10 * lam[-1])
 
 
 def _two_spheres():
