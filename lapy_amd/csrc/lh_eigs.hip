@@ -123,6 +123,10 @@ struct Lobpcg {
         return s;
     }
 
+    // smallest pivot that the factorisations since the last reset met first;
+    // normalising a direction of pivot p raises its rounding to u / sqrt(p)
+    double min_pivot = 1.0;
+
     // X block (cols [off, off+c)) <- X T with T^T (X^T B X) T = I; B X must be
     // current on entry.  A second pass follows when the first one met a small
     // pivot (Cholesky-QR2).  Returns false when the block is numerically rank
@@ -149,6 +153,7 @@ struct Lobpcg {
             double stv[2];
             d2h(ctx, stv, status.p, sizeof(stv));
             if (reinterpret_cast<int*>(stv)[0]) return false;
+            min_pivot = std::min(min_pivot, stv[1]);
             gemm_mfma_inplace(ctx, n, c, X, ld, Ts.as<double>(), c, 1.0, true);  // T is upper triangular
             if (stv[1] > 1e-2) break;
             gemm_mfma_inplace(ctx, n, c, MX, ld, Ts.as<double>(), c, 1.0, true);
@@ -183,6 +188,7 @@ struct Lobpcg {
         if (read_status()) return false;  // a zero or not finite column
         gemm_mfma_inplace(ctx, n, c, X, ld, Ts.as<double>(), c, 1.0, true);
         spmm_B(X, MX, c);
+        min_pivot = 0.0;
         return cholqr(off, c, true);
     }
 
@@ -328,7 +334,12 @@ struct Lobpcg {
         if (x0) copy_block<T, T>(ctx, n, m, x0, x0_ld, Sp(), ld);
         else randn<T>(ctx, n, m, Sp(), ld, seed);
         spmm_B(Sp(), MSp(), m);
-        if (!cholqr(0, m, true)) LH_THROW(LH_ERR_NUMERIC, "start block is rank deficient");
+        if (!cholqr(0, m, true)) {
+            if (!x0) LH_THROW(LH_ERR_NUMERIC, "start block is rank deficient");
+            randn<T>(ctx, n, m, Sp(), ld, seed);  // the first phase's is of no use
+            spmm_B(Sp(), MSp(), m);
+            if (!cholqr(0, m, true)) LH_THROW(LH_ERR_NUMERIC, "start block is rank deficient");
+        }
         if (!rayleigh_ritz(m)) LH_THROW(LH_ERR_NUMERIC, "initial Rayleigh-Ritz failed");
         gemm_mfma_inplace<T>(ctx, n, m, Sp(), ld, Cm.as<double>(), m, 1.0, false);
         spmm_AB(Sp(), ASp(), MSp(), m);
@@ -453,6 +464,7 @@ struct Lobpcg {
             project_out(0, m, m, nb);
             // joint Cholesky-QR of [W P]; P is dropped if [W P] is numerically rank deficient
             spmm_B(Sp() + m, MSp() + m, nb);
+            min_pivot = 1.0;
             bool full_rank = cholqr(m, nb, true);
             if (!full_rank && nb == 2 * m) {
                 st.restarts++;
@@ -460,6 +472,14 @@ struct Lobpcg {
                 full_rank = cholqr(m, nb, true);
             }
             if (!full_rank && amg_on) full_rank = cholqr_shifted(m, m);
+            // short directions have brought their rounding along, parts of X
+            // with it: out of the trial basis, whose Rayleigh-Ritz takes it for
+            // orthonormal (u / sqrt(p) above 1e-4 in FP32, 1e-10 in FP64)
+            if (full_rank && min_pivot < (sizeof(T) == 8 ? 1e-12 : 1e-6)) {
+                project_out(0, m, m, nb);
+                spmm_B(Sp() + m, MSp() + m, nb);
+                full_rank = cholqr(m, nb, true);
+            }
             if (!full_rank) {
                 if (!amg_on) LH_THROW(LH_ERR_NUMERIC, "Cholesky-QR of the residual block failed at iteration %d", it);
                 // the cycle's W is rank deficient or not finite: X and its

@@ -309,6 +309,21 @@ def test_mixed_precision_keeps_the_cycle(name, k, unit):
     assert np.all(np.abs(mixed - lam) <= 1e-10 * lam[-1])
 
 
+@pytest.mark.parametrize("cells,seed,unit", [(10, 2, 1e-2), (11, 3, 1e-2), (11, 3, 1e-3)])
+def test_mixed_precision_basis_stays_orthonormal(cells, seed, unit):
+    """Short directions of the first blocks, made long, carry parts of X: with
+    those left in, the FP32 phase ended in a block that the FP64 phase refused."""
+    v, t = meshgen.tet_cube(cells, jitter=0.2, seed=seed)
+    fem = Solver(TetMesh(unit * v, t))
+    lam, _ = fem.eigs(k=50)
+    its = fem.last_stats.iterations
+    mixed, _ = fem.eigs(k=50, precision="mixed")
+    st = fem.last_stats
+    print(cells, seed, unit, "iterations", its, "mixed", st.iterations, "FP32", st.iterations_fp32)
+    assert st.fallback_used == 0 and st.iterations <= its + 8
+    assert np.all(np.abs(mixed - lam) <= 1e-10 * lam[-1])
+
+
 def _two_spheres():
     v, t = meshgen.perturbed_sphere(4, np.random.default_rng(2), axes=(1.3, 0.8, 1.0), sigma=0.02)
     return np.r_[v, v + 3.0], np.r_[t, t + len(v)]  # a constant of its own on each part
