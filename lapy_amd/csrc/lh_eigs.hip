@@ -14,7 +14,8 @@
 //                    sigma*B (lh_amg.hip), nearly K^-1; or D^-1 and a
 //                    Chebyshev polynomial in D^-1 K, D = diag(K) (lh_poly.hip)
 //   W <- W - X (BX)^T W (twice),  Cholesky-QR in the B inner product
-//   P <- P - X (BX)^T P - W (BW)^T P,  Cholesky-QR (dropped on breakdown)
+//   P <- P - X (BX)^T P - W (BW)^T P,  Cholesky-QR (dropped on breakdown;
+//                    a W that breaks down: the shifted factorisation first)
 //   Rayleigh-Ritz on span(S) with the one-workgroup FP64 solver (lh_rr.hip)
 //   X <- S C,  P <- S[:, m:] C[m:]
 //
