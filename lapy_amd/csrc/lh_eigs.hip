@@ -466,12 +466,14 @@ struct Lobpcg {
             // joint Cholesky-QR of [W P]; P is dropped if [W P] is numerically rank deficient
             spmm_B(Sp() + m, MSp() + m, nb);
             min_pivot = 1.0;
-            bool full_rank = cholqr(m, nb, true);
-            if (!full_rank && nb == 2 * m) {
+            auto orthonormalise = [&]() {
+                if (cholqr(m, nb, true)) return true;
+                if (nb == m) return false;
                 st.restarts++;
                 nb = m;
-                full_rank = cholqr(m, nb, true);
-            }
+                return cholqr(m, nb, true);
+            };
+            bool full_rank = orthonormalise();
             if (!full_rank && amg_on) full_rank = cholqr_shifted(m, m);
             // short directions have brought their rounding along, parts of X
             // with it: out of the trial basis, whose Rayleigh-Ritz takes it for
@@ -479,7 +481,7 @@ struct Lobpcg {
             if (full_rank && min_pivot < (sizeof(T) == 8 ? 1e-12 : 1e-6)) {
                 project_out(0, m, m, nb);
                 spmm_B(Sp() + m, MSp() + m, nb);
-                full_rank = cholqr(m, nb, true);
+                full_rank = orthonormalise();
             }
             if (!full_rank) {
                 if (!amg_on) LH_THROW(LH_ERR_NUMERIC, "Cholesky-QR of the residual block failed at iteration %d", it);
